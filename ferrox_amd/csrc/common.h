@@ -273,6 +273,36 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
     return v;
 }
 
+// ---- the order in which float32 products add an output's terms ------------------
+// K is cut into F32_PARTS parts whose sums are added in their order.  Inside a part 16 k at a time: instruction u = 0..3 of
+// v_mfma_f32_16x16x4_f32 takes k = 4 g + u for g = 0..3, in that order, each product added with one rounding.
+#define F32_PARTS 8
+__host__ __device__ __forceinline__ int f32_part_length(int K) { return ((K + F32_PARTS - 1) / F32_PARTS + 31) / 32 * 32; }
+// the sum over k of x(k) * w(k) in that order, for kernels whose few rows must have the bits of the tiled product
+template <typename X, typename W>
+__device__ __forceinline__ float f32_ordered_dot(int K, X&& x, W&& w) {
+    const int part = f32_part_length(K);
+    float total = 0.f;
+    for (int k0 = 0; k0 < K; k0 += part) {
+        const int end = k0 + part < K ? k0 + part : K;
+        float acc = 0.f;
+        int c = k0;
+        for (; c + 16 <= end; c += 16) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) acc = fmaf(w(c + 4 * g + u), x(c + 4 * g + u), acc);
+        }
+        if (c < end) {
+            for (int u = 0; u < 4; ++u)
+                for (int g = 0; g < 4; ++g)
+                    if (c + 4 * g + u < end) acc = fmaf(w(c + 4 * g + u), x(c + 4 * g + u), acc);
+        }
+        total += acc;
+    }
+    return total;
+}
+
 static inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
 // Compute units of the current device, asked for once per device.  Dispatch decisions that weigh a launch's

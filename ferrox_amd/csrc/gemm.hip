@@ -3,11 +3,11 @@
 // for plain and for expert-grouped rows.
 //
 //  * bfloat16: MFMA 16x16x32 tiles, float32 accumulators.
-//  * float32 : FMA in float32 only (no reduced-precision matrix mode).
+//  * float32 : MFMA 16x16x4 in float32 (no reduced-precision matrix mode).
 //
-// In both, one output element is accumulated over k in ascending order with a
-// single accumulator, whatever the tile shape and whatever else is in the batch,
-// so a row's result does not depend on how many rows are computed with it.
+// In both, one output element's products are added in an order that the sizes of the
+// weights fix, whatever the tile shape and whatever else is in the batch, so a float32
+// row's result does not depend on how many rows are computed with it.
 //
 // Grouped mode: rows are sorted by expert; expert e owns rows
 // [expert_offsets[e], expert_offsets[e+1]) and the weights at W + e * w_stride.
@@ -72,6 +72,7 @@ struct GemmArgs {
     long ld_gate;            //   (m % gate_div) * N + n
     int gate_div;
     int vec_ok;  // 16-byte loads are legal for A and W
+    int c_vec;   // float32: so are 16-byte loads and stores of C
     int n_col_tiles, n_row_tiles;  // tiled kernels: the grid they decode block ids with
 };
 
@@ -1174,94 +1175,301 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
 }
 
 // ===========================================================================
-// float32 with FMA
+// float32 on MFMA
 // ===========================================================================
-#define FK 16
-// 64 x 64 outputs per block, 256 threads, 4 x 4 per thread.
+// v_mfma_f32_16x16x4_f32 multiplies and adds in float32 (twice the rate of v_fma_f32, whose packed form is not used here).
+// Both kernels below add an output's products in the same order, so a row's bits do not depend on which of them
+// computes it: K is cut into F32_PARTS parts; inside a part 16 k at a time, four instructions of 4 k each, instruction u
+// taking k = 4 g + u for g = 0..3 (the order is stated in common.h; a lane of group g holds four consecutive k in one 16-byte register group); the parts'
+// sums are added in their order.  The weights are the instruction's first operand, so that a lane ends with four
+// consecutive columns of one row.
+
+// four k steps of one tile: w and x hold k = 4 g .. 4 g + 3 of the lane's weight row and activation row
+template <int MT, int NT>
+__device__ __forceinline__ void f32_multiply(f32x4_t (&acc)[MT][NT], const f32x4_t (&w)[NT], const f32x4_t (&x)[MT]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][u], x[i][u], acc[i][j], 0, 0, 0);
+}
+// k .. k + 3 of a row; guarded: zeros from K on (VEC: the row is 16-byte aligned and K a multiple of 4).  Inside the loops
+// the loads are unconditional (a step past the end reads the last one again): behind a branch the compiler waits for them
+// on the spot, and the loop has no load in flight (tiles of 64 x 64 against 2,048 k: 84 -> 47 us).
+template <bool VEC>
+__device__ __forceinline__ f32x4_t f32_fetch(const float* p) {
+    if (VEC) return *(const f32x4_t*)p;
+    return (f32x4_t){p[0], p[1], p[2], p[3]};
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4_t f32_fetch_guarded(const float* row, int k, int K) {
+    f32x4_t v = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        if (k < K) v = *(const f32x4_t*)(row + k);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (k + r < K) v[r] = row[k + r];
+    }
+    return v;
+}
+// columns n .. n + 3 of logical row ml on their way out
 template <bool DUAL, int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs g) {
-    __shared__ float As[FK][64 + 4];
-    __shared__ float Bs[DUAL ? 2 : 1][FK][64 + 4];
-    int r0, r_end, expert;
-    locate_rows<64>(g, blockIdx.y, r0, r_end, expert);
-    if (r0 < 0) return;
-    const int n0 = blockIdx.x * 64;
-    const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-    const float* Abase = (const float*)g.A;
-    const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
-
-    // loader: element idx = tid + i*256 of a 64 x 16 tile, k fastest
-    const float* a_src[4];
-    const float* b_src[4];
+__device__ __forceinline__ void f32_store4(const GemmArgs& g, int ml, int n, f32x4_t v, f32x4_t v2) {
+    if (n >= g.N) return;
+    const int m = g.c_rows ? g.c_rows[ml] : ml;
+    float* out = (float*)g.C + (size_t)m * g.ldc + n;
+    const int cnt = g.N - n < 4 ? g.N - n : 4;
+    f32x4_t y;
+    if constexpr (DUAL) {
+        const float ps = FX_PRE_SCALE(g, ml);
+        with_activation(g.act, [&](auto ac) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (tid + i * 256) >> 4;
-        a_src[i] = nullptr;
-        b_src[i] = nullptr;
-        if (r0 + row < r_end) {
-            const int m = r0 + row;
-            a_src[i] = Abase + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda;
+            for (int r = 0; r < 4; ++r) y[r] = gated_c<decltype(ac)::value>(v[r] * ps, v2[r] * ps, g.act_limit, g.act_alpha);
+        });
+    } else {
+        if (g.bias) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += load_as_float(g.bias, g.bias_dtype, n + r < g.N ? n + r : g.N - 1);
         }
-        if (n0 + row < g.N) b_src[i] = Wbase + (size_t)(n0 + row) * g.K;
-    }
-    const int kk = tid & 15;
-
-    float acc[4][4] = {}, acc2[4][4] = {};
-    for (int k0 = 0; k0 < g.K; k0 += FK) {
-        __syncthreads();
+        if constexpr (EPI == EPI_RESID) {
+            const float rs = g.row_scale ? g.row_scale[ml] : 1.0f;
+            if (g.row_scale) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = (tid + i * 256) >> 4;
-            const bool kin = k0 + kk < g.K;
-            As[kk][row] = (a_src[i] && kin) ? a_src[i][k0 + kk] : 0.f;
-            Bs[0][kk][row] = (b_src[i] && kin) ? b_src[i][k0 + kk] : 0.f;
-            if (DUAL) Bs[DUAL ? 1 : 0][kk][row] = (b_src[i] && kin) ? b_src[i][g.up_offset + k0 + kk] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < FK; ++k) {
-            float a[4], b[4], b2[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[0][k][tx * 4 + j];
-            if (DUAL) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b2[j] = Bs[DUAL ? 1 : 0][k][tx * 4 + j];
+                for (int r = 0; r < 4; ++r) v[r] *= rs;
             }
+            if (g.c_vec && cnt == 4) {
+                const f32x4_t old = *(const f32x4_t*)out;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-                    if (DUAL) acc2[i][j] = fmaf(a[i], b2[j], acc2[i][j]);
-                }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int ml = r0 + ty * 4 + i;
-        if (ml >= r_end) continue;
-        const int m = g.c_rows ? g.c_rows[ml] : ml;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= g.N) continue;
-            float v = acc[i][j];
-            float* out = (float*)g.C + (size_t)m * g.ldc + n;
-            if (DUAL) {
-                const float ps = FX_PRE_SCALE(g, ml);
-                with_activation(g.act, [&](auto ac) { *out = gated_c<decltype(ac)::value>(v * ps, acc2[i][j] * ps, g.act_limit, g.act_alpha); });
+                for (int r = 0; r < 4; ++r) y[r] = old[r] + v[r];
             } else {
-                if (g.bias) v += load_as_float(g.bias, g.bias_dtype, n);
-                if (EPI == EPI_RESID) {
-                    if (g.row_scale) v *= g.row_scale[ml];
-                    *out += v;
-                } else {
-                    *out = stored_f(g, v, gate_of(g, m, n));      // (the host sets store_act for stored products only)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y[r] = r < cnt ? out[r] + v[r] : 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y[r] = r < cnt ? stored_f(g, v[r], gate_of(g, m, n + r)) : 0.f;   // (the host sets store_act for stored products only)
+        }
+    }
+    if (g.c_vec && cnt == 4) *(f32x4_t*)out = y;
+    else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r < cnt) out[r] = y[r];
+    }
+}
+
+// Many rows: TM x TN outputs a block (DUAL: TN / 2 columns of both matrices, their blocks of 16 in turn), four waves of
+// TM/2 x TN/2, operands 32 k at a time through LDS in two stages, 16-byte pieces swizzled by the row, the loads two steps
+// ahead.  Bound by the matrix units and the waits between barriers: 1,500 x 6,144 x 2,048 in 327 us, 115 of the 157
+// TFLOP/s of the instruction (the FMA kernel before it: 700 x 6,144 x 2,048 in 379 us, this one 186).
+template <int TM, int TN, bool DUAL, int EPI, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(GemmArgs g) {
+    constexpr int MT = TM / 32, NT = TN / 32;
+    static_assert(!DUAL || NT % 2 == 0, "a wave holds both matrices' blocks of its columns");
+    __shared__ f32x4_t As[2][TM][8];
+    __shared__ f32x4_t Bs[2][TN][8];
+    int r0, r_end, expert;
+    locate_rows<TM>(g, blockIdx.y, r0, r_end, expert);
+    if (r0 < 0) return;
+    const int n0 = blockIdx.x * (DUAL ? TN / 2 : TN);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
+    const int wm = wave & 1, wn = wave >> 1;
+    const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
+    // (a row or column past the end reads the last one; what comes of it is not stored)
+    const int piece = tid & 7;
+    const float* a_src[MT];
+    const float* b_src[NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        int m = r0 + (tid >> 3) + 32 * i;
+        m = m < r_end ? m : r_end - 1;
+        a_src[i] = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int r = (tid >> 3) + 32 * j;
+        int n = DUAL ? n0 + (r >> 5) * 16 + (r & 15) : n0 + r;
+        n = n < g.N ? n : g.N - 1;
+        b_src[j] = Wbase + (size_t)n * g.K + (DUAL && (r & 16) ? g.up_offset : 0);
+    }
+    f32x4_t ra[2][MT], rb[2][NT];
+    const int n_full = g.K / 32;
+    auto fetch = [&](int set, int step) {
+        const int k = (step < n_full ? step : n_full - 1) * 32 + piece * 4;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) ra[set][i] = f32_fetch<VEC>(a_src[i] + k);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) rb[set][j] = f32_fetch<VEC>(b_src[j] + k);
+    };
+    auto keep = [&](int set) {
+        const int row = tid >> 3, at = piece ^ (row & 7);      // (32 rows on: the same swizzle)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) As[set][row + 32 * i][at] = ra[set][i];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) Bs[set][row + 32 * j][at] = rb[set][j];
+    };
+    f32x4_t acc[MT][NT], total[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = total[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int part = f32_part_length(g.K);
+    int next_end = part;
+    auto multiply = [&](int buf, int k0) {
+        if (k0 == next_end) {
+            next_end += part;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    total[i][j] += acc[i][j];
+                    acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
                 }
+        }
+        f32x4_t w[2][NT], x[2][MT];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int at = (s * 4 + gq) ^ (li & 7);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) w[s][j] = Bs[buf][(wn * NT + j) * 16 + li][at];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) x[s][i] = As[buf][(wm * MT + i) * 16 + li][at];
+        }
+        f32_multiply(acc, w[0], x[0]);
+        f32_multiply(acc, w[1], x[1]);
+    };
+    if (n_full > 0) {
+        fetch(0, 0);
+        fetch(1, 1);
+        keep(0);
+        int step = 0;
+        for (; step + 1 < n_full; step += 2) {
+            lds_barrier();
+            fetch(0, step + 2);
+            multiply(0, step * 32);
+            keep(1);
+            lds_barrier();
+            fetch(1, step + 3);
+            multiply(1, step * 32 + 32);
+            keep(0);
+        }
+        if (step < n_full) {
+            lds_barrier();
+            multiply(0, step * 32);
+        }
+    }
+    if (n_full * 32 < g.K) {           // the last, partial step
+        const int k = n_full * 32 + piece * 4;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) ra[0][i] = f32_fetch_guarded<VEC>(a_src[i], k, g.K);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) rb[0][j] = f32_fetch_guarded<VEC>(b_src[j], k, g.K);
+        lds_barrier();
+        keep(0);
+        lds_barrier();
+        multiply(0, n_full * 32);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int ml = r0 + (wm * MT + i) * 16 + li;
+        if (ml >= r_end) continue;
+#pragma unroll
+        for (int j = 0; j < NT; j += DUAL ? 2 : 1) {
+            const int t = wn * NT + j;
+            const int n = n0 + (DUAL ? t >> 1 : t) * 16 + 4 * gq;
+            f32_store4<DUAL, EPI>(g, ml, n, total[i][j] + acc[i][j], DUAL ? total[i][j + (DUAL ? 1 : 0)] + acc[i][j + (DUAL ? 1 : 0)] : acc[i][j]);
+        }
+    }
+}
+
+// Few rows: the weights go from memory straight into operands, every wave a part of K, 16 * MT rows and NW sets of 16
+// weight rows a block (DUAL: the sets alternate between the two matrices); 64 k a step, the next step's loads issued
+// before this step's products; the parts' sums meet in LDS.  Bound by the stream of the weights: 4 rows against 6,144 x
+// 2,048 17 us (3 TB/s, launch included; the FMA kernel's tile of 64 rows took 253).
+template <int MT, int NW, bool DUAL, int EPI, bool VEC>
+__global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
+    static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
+    __shared__ f32x4_t red[F32_PARTS][MT * NW][64];
+    int r0, r_end, expert;
+    locate_rows<16 * MT>(g, blockIdx.y, r0, r_end, expert);
+    if (r0 < 0) return;
+    const int n0 = blockIdx.x * (DUAL ? 8 * NW : 16 * NW);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
+    const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
+    const float* x_src[MT];
+    const float* w_src[NW];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        int m = r0 + i * 16 + li;
+        m = m < r_end ? m : r_end - 1;
+        x_src[i] = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda;
+    }
+#pragma unroll
+    for (int a = 0; a < NW; ++a) {
+        int n = n0 + (DUAL ? a >> 1 : a) * 16 + li;
+        n = n < g.N ? n : g.N - 1;
+        w_src[a] = Wbase + (size_t)n * g.K + (DUAL && (a & 1) ? g.up_offset : 0);
+    }
+    const int part = f32_part_length(g.K);
+    const int k_first = wave * part, k_end = k_first + part < g.K ? k_first + part : g.K;
+    constexpr int STEP = MT > 1 ? 2 : 4;       // groups of 16 k that are on their way together
+    f32x4_t w[2][STEP][NW], x[2][STEP][MT];
+    const int k_full = k_first + (k_end - k_first) / 16 * 16;
+    auto fetch = [&](int b, int k0) {
+#pragma unroll
+        for (int c = 0; c < STEP; ++c) {
+            const int kc = k0 + c * 16, k = (kc < k_full ? kc : k_full - 16) + gq * 4;
+#pragma unroll
+            for (int a = 0; a < NW; ++a) w[b][c][a] = f32_fetch<VEC>(w_src[a] + k);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) x[b][c][i] = f32_fetch<VEC>(x_src[i] + k);
+        }
+    };
+    f32x4_t acc[MT][NW];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int a = 0; a < NW; ++a) acc[i][a] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    if (k_first < k_full) {
+        fetch(0, k_first);
+        for (int k0 = k_first; k0 < k_full; k0 += 2 * STEP * 16) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const int kb = k0 + b * STEP * 16;
+                fetch(b ^ 1, kb + STEP * 16);
+#pragma unroll
+                for (int c = 0; c < STEP; ++c)
+                    if (kb + c * 16 < k_full) f32_multiply(acc, w[b][c], x[b][c]);
             }
         }
+    }
+    if (k_first < k_end && k_full < k_end) {       // the last, partial group of K
+#pragma unroll
+        for (int a = 0; a < NW; ++a) w[0][0][a] = f32_fetch_guarded<VEC>(w_src[a], k_full + gq * 4, k_end);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) x[0][0][i] = f32_fetch_guarded<VEC>(x_src[i], k_full + gq * 4, k_end);
+        f32_multiply(acc, w[0][0], x[0][0]);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int a = 0; a < NW; ++a) red[wave][i * NW + a][lane] = acc[i][a];
+    __syncthreads();
+    constexpr int PER = DUAL ? 2 : 1;
+    for (int t = wave; t < MT * NW / PER; t += F32_PARTS) {
+        const int i = t * PER / NW, a = t * PER % NW;
+        f32x4_t v = red[0][i * NW + a][lane], v2 = v;
+#pragma unroll
+        for (int p = 1; p < F32_PARTS; ++p) v += red[p][i * NW + a][lane];
+        if (DUAL) {
+            v2 = red[0][i * NW + a + PER - 1][lane];
+#pragma unroll
+            for (int p = 1; p < F32_PARTS; ++p) v2 += red[p][i * NW + a + PER - 1][lane];
+        }
+        const int ml = r0 + i * 16 + li;
+        if (ml < r_end) f32_store4<DUAL, EPI>(g, ml, n0 + (DUAL ? a >> 1 : a) * 16 + 4 * gq, v, v2);
     }
 }
 
@@ -1297,6 +1505,7 @@ static int g_tile64_rows = 20; // "tile64_rows": experts with up to this many ro
 static int g_no_wide = 0;      // "wide": 0 sends many-row products to the register-staged tiled kernel, 1 (default) by the sizes,
 static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to the product for few rows whatever the weight rows (0: by the sizes)
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
+static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
 static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
@@ -1309,8 +1518,9 @@ FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "wide")) { g_no_wide = !value; g_wide_force = value > 1 ? value : 0; return 0; }
     if (!strcmp(key, "wide_grouped")) { g_wide_grouped = value > 1 ? value : 0; return 0; }
     if (!strcmp(key, "stream_w")) { g_stream_w = value; return 0; }
+    if (!strcmp(key, "f32_tile")) { g_f32_tile = value; return 0; }
     if (!strcmp(key, "plain_rows")) { g_plain_rows = value; return 0; }
-    FX_REQUIRE(false, "gemm: no debug switch '%s' (skinny_sets, skinny_row_tiles, skinny_waves, few_rows, head_rows, tile64_rows, wide, wide_grouped, stream_w, plain_rows)", key);
+    FX_REQUIRE(false, "gemm: no debug switch '%s' (skinny_sets, skinny_row_tiles, skinny_waves, few_rows, head_rows, tile64_rows, wide, wide_grouped, stream_w, plain_rows, f32_tile)", key);
     return 1;
 }
 
@@ -1338,6 +1548,15 @@ static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
         }
     }
     launch_wide_as<TMB, TN, NS, NSA, false>(g, epi, grid, s);
+}
+
+template <bool DUAL, int EPI, bool VEC>
+static void launch_f32(const GemmArgs& g, int tile, int mt, int nw, dim3 grid, hipStream_t s) {
+    if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
+    else if (tile == 32) gemm_f32_tiled_kernel<32, DUAL ? 64 : 32, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
+    else if (mt == 2) gemm_f32_skinny_kernel<2, 2, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
+    else if (nw == 2 || DUAL) gemm_f32_skinny_kernel<1, 2, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
+    else gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
 }
 
 template <int MT, int WAVES, int NW>
@@ -1494,15 +1713,41 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     hipStream_t s = (hipStream_t)stream;
     const int nonempty = expert_offsets ? (E < M ? E : M) : 0;
     if (dtype == FX_F32) {
-        g.vec_ok = 0;
-        const int m_tiles = M / 64 + (expert_offsets ? nonempty : (M % 64 != 0));
-        dim3 grid(ceil_div(N, 64), m_tiles);
+        g.vec_ok = K % 4 == 0 && lda % 4 == 0 && w_stride % 4 == 0 && up_offset % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) % 16 == 0);
+        g.c_vec = ldc % 4 == 0 && ((uintptr_t)C % 16) == 0;
+        const bool dual = epi == EPI_GATED;
+        const long group = expert_offsets ? (M + E - 1) / E : M, cus = fx_compute_units();
+        auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
+        // Up to 32 plain rows: the kernel for few rows (2,048 x 2,048 weights, 4 rows: 10 us against 30 with tiles of 32 and 45
+        // of 64; 32 rows: 22, 30 and 47), but where the weight rows are so many that tiles of 32 fill the GPU many times
+        // (the head's 151,936: 260 against 272 us at 4 rows, 240 the other way at one).  Tiles of 64 once they are two and
+        // a half a CU (6,144 weight rows: 512 rows 121 against 139 us, 256 rows 76 against 71; 2,048 weight rows: 1,500
+        // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: tiles of 32 up to 36 rows an expert (60 experts'
+        // gate/up product of 2,048: 4.3 rows 263 us against 277 for few rows and 428 with tiles of 64; 34 rows 396 and
+        // 437; 47 rows 496 and 424).
+        int tile = 0, mt = 1, nw = 2;
+        if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
+        else if (expert_offsets) tile = group <= 36 ? 32 : 64;
+        else {
+            const bool many_columns = ceil_div(N, 32) >= 8 * cus && M > 2;
+            if (M > 32 || many_columns) tile = M > 32 && 2 * (long)ceil_div(N, 64) * ceil_div(M, 64) >= 5 * cus ? 64 : 32;
+        }
+        if (!tile) {
+            mt = group <= 16 ? 1 : 2;
+            if (mt == 1 && !dual && (long)ceil_div(N, 32) * row_tiles(16) < cus) nw = 1;
+        }
+        const int tm = tile ? tile : 16 * mt, tn = tile ? (tile == 32 && dual ? 64 : tile) : 16 * nw;
+        dim3 grid(ceil_div(N, dual ? tn / 2 : tn), row_tiles(tm));
+#define FX_F32(DUAL_, EPI_)                                                            \
+    if (g.vec_ok) launch_f32<DUAL_, EPI_, true>(g, tile, mt, nw, grid, s);             \
+    else launch_f32<DUAL_, EPI_, false>(g, tile, mt, nw, grid, s)
         switch (epi) {
             case EPI_STORE:
-            case EPI_STORE_F32: gemm_f32_kernel<false, EPI_STORE_F32><<<grid, 256, 0, s>>>(g); break;
-            case EPI_RESID: gemm_f32_kernel<false, EPI_RESID><<<grid, 256, 0, s>>>(g); break;
-            default: gemm_f32_kernel<true, EPI_GATED><<<grid, 256, 0, s>>>(g); break;
+            case EPI_STORE_F32: FX_F32(false, EPI_STORE_F32); break;
+            case EPI_RESID: FX_F32(false, EPI_RESID); break;
+            default: FX_F32(true, EPI_GATED); break;
         }
+#undef FX_F32
         FX_CHECK_LAUNCH("gemm_f32");
         return 0;
     }

@@ -198,8 +198,8 @@ FX_API int fx_delta_prepare(void* stream, const float* q, long ldq, const float*
 }
 
 // ---------------------------------------------------------------------------
-// Two small float32 products of few rows in one launch: out_i[t, n] = sum_k x_i[t, k] * wt_i[k, n], i = 0, 1, k
-// ascending in one accumulator (the sums of the float32 product kernel, so a row gets the same bits from either).
+// Two small float32 products of few rows in one launch: out_i[t, n] = sum_k x_i[t, k] * wt_i[k, n], i = 0, 1,
+// added in the order of the tiled float32 product (so a row gets the same bits from either).
 // These are the second halves of the delta rule's two low-rank projections (decay and output gate): K is the
 // inner size (tens to a few hundred), the weights are kept transposed [K, N] so that neighbouring lanes read
 // neighbouring columns, and a decode step's few rows make them two launches' worth of waiting otherwise.
@@ -222,10 +222,7 @@ __global__ __launch_bounds__(256) void small_rows_pair_kernel(const float* __res
     for (int k = threadIdx.x; k < K; k += 256) xs[k] = x[(size_t)t * ldx + k];
     __syncthreads();
     if (n >= N) return;
-    float acc = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < K; ++k) acc = fmaf(xs[k], wt[(size_t)k * N + n], acc);
-    out[(size_t)t * ldo + n] = acc;
+    out[(size_t)t * ldo + n] = f32_ordered_dot(K, [&](int k) { return xs[k]; }, [&](int k) { return wt[(size_t)k * N + n]; });
 }
 
 FX_API int fx_small_rows_pair(void* stream, const float* x0, long ldx0, const float* wt0, float* out0, long ldo0, int K0, int N0,
@@ -243,7 +240,7 @@ FX_API int fx_small_rows_pair(void* stream, const float* x0, long ldx0, const fl
 
 // ---------------------------------------------------------------------------
 // A block-diagonal float32 product of few rows in one launch: the K-wide part j of row t, times the transposed matrix
-// wt[j] [K, N] of that part, out[t, j, n] = sum_k x[t, j K + k] * wt[j, k, n], k ascending in one accumulator.  These
+// wt[j] [K, N] of that part, out[t, j, n] = sum_k x[t, j K + k] * wt[j, k, n], added in the order of the tiled float32 product.  These
 // are the gates of a recurrent unit whose channels are cut into parts with a square matrix each; a decode step's few
 // rows would wait in a tiled product's launch for nothing.  Grid: (ceil(N / 256), rows, parts).
 // ---------------------------------------------------------------------------
@@ -255,10 +252,7 @@ __global__ __launch_bounds__(256) void small_rows_parts_kernel(const float* __re
     __syncthreads();
     if (n >= N) return;
     const float* w = wt + (size_t)j * K * N;
-    float acc = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < K; ++k) acc = fmaf(xs[k], w[(size_t)k * N + n], acc);
-    out[((size_t)t * parts + j) * N + n] = acc;
+    out[((size_t)t * parts + j) * N + n] = f32_ordered_dot(K, [&](int k) { return xs[k]; }, [&](int k) { return w[(size_t)k * N + n]; });
 }
 
 FX_API int fx_small_rows_parts(void* stream, const float* x, long ldx, const float* wt, float* out, int K, int N, int parts, int T) {

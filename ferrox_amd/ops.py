@@ -1283,7 +1283,7 @@ def gated_head_norm(o, gate, weight, eps: float, n_heads: int, v_dim: int, out_d
 def small_rows_parts(x, wt):
     """A block-diagonal float32 product of few rows, one launch: x float32 rows [T, parts * K] (any row stride), wt
     contiguous float32 [parts, K, N] (every part's matrix transposed); returns contiguous [T, parts, N] with
-    out[t, j] = x[t, j K:(j + 1) K] @ wt[j], the sums over k ascending in one accumulator, as `gemm` does in float32."""
+    out[t, j] = x[t, j K:(j + 1) K] @ wt[j], the sums over k in the order in which `gemm` adds them in float32."""
     T = x.shape[0]
     if wt.dtype != torch.float32 or wt.dim() != 3 or not wt.is_contiguous() or wt.shape[1] > SMALL_ROWS_MAX_K:
         raise KernelError(f"small_rows_parts: transposed weights {tuple(wt.shape)} ({wt.dtype})")
@@ -1459,8 +1459,8 @@ SMALL_ROWS_MAX_K = 512
 
 def small_rows_pair(x0, wt0, x1, wt1):
     """(x0 @ wt0, x1 @ wt1) in float32 for few rows, one launch: x_i float32 rows [T, K_i] (any row stride),
-    wt_i contiguous float32 [K_i, N_i] (the weights transposed).  The sums run over k ascending in one accumulator,
-    as `gemm` does in float32."""
+    wt_i contiguous float32 [K_i, N_i] (the weights transposed).  The sums run over k in the order
+    in which `gemm` adds them in float32."""
     T = x0.shape[0]
     for x, wt in ((x0, wt0), (x1, wt1)):
         _f32_rows(x, "small_rows_pair: x", wt.shape[0])

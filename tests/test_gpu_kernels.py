@@ -46,6 +46,54 @@ def test_gemm_plain_and_epilogues(dtype, M, N, K):
     close(h, h0.double() + ref * scale.double()[:, None], dtype, "residual")
 
 
+@pytest.mark.parametrize("N,K", [(16, 16), (61, 37), (100, 70), (130, 96), (96, 2052), (2048, 264)])
+def test_float32_products_have_the_same_bits_in_every_kernel(N, K):
+    """The kernel for few rows and the tiles of 32 and 64 rows, at their edges (rows, columns, the last step of K, operands
+    that are not 16-byte aligned): each close to float64, and the same bits row for row however many rows there are."""
+    from ferrox_amd import debug, ops
+    M = 130
+    a, w, bias = rnd(M, K), rnd(N, K, seed=1), rnd(N, seed=2)
+    w2, scale = rnd(2 * N, K, seed=3, scale=0.3), rnd(M, seed=4)
+    ref, ref2 = a.double() @ w.double().T, a.double() @ w2.double().T
+    whole = ops.gemm(a, w, bias=bias)
+    close(whole, ref + bias.double(), torch.float32, "stored")
+    gated = ops.gemm(a, w2, epilogue=ops.EPI_GATED)
+    close(gated, plain.silu(ref2[:, :N]) * ref2[:, N:], torch.float32, "silu(gate)*up")
+    h0 = rnd(M, N, seed=5)
+    for tile in (1, 32, 64, 0):
+        with debug.kernel_switch("gemm", "f32_tile", tile):
+            for rows in (1, 16, 17, 32, 33, 64, 65, M):
+                assert torch.equal(ops.gemm(a[:rows], w, bias=bias), whole[:rows]), (tile, rows)
+                assert torch.equal(ops.gemm(a[:rows], w2, epilogue=ops.EPI_GATED), gated[:rows]), (tile, rows)
+            h = h0.clone()
+            ops.gemm(a, w, epilogue=ops.EPI_RESID, out=h, row_scale=scale)
+            close(h, h0.double() + ref * scale.double()[:, None], torch.float32, "residual")
+    # rows that begin at an odd multiple of four bytes
+    wide = rnd(M, K + 3, seed=6)
+    wide[:, 1:K + 1] = a
+    assert torch.equal(ops.gemm(wide[:, 1:K + 1], w, bias=bias), whole)
+
+
+@pytest.mark.parametrize("T,E,k,I,H", [(1, 5, 2, 20, 36), (3, 60, 4, 96, 128), (90, 7, 3, 33, 50), (700, 4, 2, 64, 96)])
+def test_float32_grouped_products_have_the_same_bits_in_every_kernel(T, E, k, I, H):
+    from ferrox_amd import debug, ops
+    x, w = rnd(T, H), rnd(E, 2 * I, H, seed=1, scale=0.3)
+    g = torch.Generator().manual_seed(7)
+    ids = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(torch.int32).to(DEV)
+    offsets, sorted_token, sorted_pair, inv = ops.moe_align(ids, E)
+    got = {}
+    for tile in (0, 1, 32, 64):
+        with debug.kernel_switch("gemm", "f32_tile", tile):
+            got[tile] = ops.gemm(x, w, epilogue=ops.EPI_GATED, a_rows=sorted_token, expert_offsets=offsets, n_rows=T * k)
+        assert torch.equal(got[tile], got[0]), tile
+    xs, off = x.double()[sorted_token.long()], offsets.cpu().tolist()
+    for e in range(E):
+        r = slice(off[e], off[e + 1])
+        if r.start == r.stop:
+            continue
+        close(got[0][r], plain.silu(xs[r] @ w[e, :I].double().T) * (xs[r] @ w[e, I:].double().T), torch.float32, f"expert {e}")
+
+
 @pytest.mark.parametrize("T,H,N,k,S", [(1, 2048, 6144, 4, 4), (8, 2048, 6144, 4, 4), (16, 264, 100, 3, 0), (5, 520, 72, 1, 2)])
 def test_combine_that_leaves_the_scale_to_the_product(T, H, N, k, S):
     """combine -> rows times the norm's weight and sums of squares -> product that scales its rows,

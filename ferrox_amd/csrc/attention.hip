@@ -802,6 +802,237 @@ struct WaveAttn {
     }
 };
 
+// ---------------------------------------------------------------------------
+// float32 on MFMA (head sizes that are multiples of 4 up to 256, pages of a multiple of 4 keys): one wave owns 16 rows
+// that share a kv head, 16 consecutive queries of a head (prefill) or the query heads of a kv group at one token
+// (decode).  v_mfma_f32_16x16x4_f32 multiplies and adds in float32.  S^T = K Q^T with keys as the first operand leaves
+// lane (row = lane % 16, g = lane / 16) the scores of keys 16 kb + 4 g + r of its own row, and the same registers are the
+// second operand of O^T += V^T P^T, whose first operand is four consecutive keys of a transposed value row: keys and
+// values go from memory straight into operands, no LDS and no barrier.  A unit (16 keys x up to 128 numbers, or 32 value
+// rows x 64 keys) is on its way while the one before it is multiplied; page ids are asked for a tile ahead.
+// (A lane per key that reads its row number by number, as the kernels for any shape do, took 514 us a layer for 700
+// tokens of 16 heads and 124 us for four single queries at 1,030 keys; these take 111 and 30 us.  What bounds them now is
+// one wave's chain: 512 products of 32 cycles a tile of 64 keys x 128 numbers, 7 us, and few waves a SIMD to hide its waits.)
+// ---------------------------------------------------------------------------
+template <int HDM>
+struct F32Attention {
+    static constexpr int NC = HDM / 16;                         // groups of 16 numbers in a row
+    static constexpr int UC = NC < 8 ? NC : 8, NU = NC / UC;    // a unit's groups, units of a key block
+    f32x4_t q[NC];     // the row's query, scaled: numbers 16 c + 4 g + u
+    f32x4_t o[NC];     // the row's outputs 16 c + 4 g + u
+    float m, l;
+
+    // `query`: the row's query or null (a row that does not exist)
+    __device__ __forceinline__ void begin(const AttnArgs& a, const float* query, int g) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            o[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int d = 16 * c + 4 * g + u;
+                q[c][u] = (query && d < a.hd) ? query[d] * a.scale : 0.f;
+            }
+        }
+        m = NEG_INF;
+        l = 0.f;
+    }
+    __device__ __forceinline__ static int next_tile(const KeySpan& span, int kt0) {
+        return (kt0 >= span.keep && kt0 + 64 <= span.begin) ? span.begin & ~63 : kt0;
+    }
+    // Tiles of 64 keys from `first` (a multiple of 64) to the span's end.  The row stands at `pos`, head `h`, and sees keys
+    // from `lo` on (and the kept first ones).
+    __device__ __forceinline__ void walk(const AttnArgs& a, const int* bt, int kvh, const KeySpan& span, int first, int pos, int lo, int h) {
+        const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+        const bool shaped = shapes_scores(a);
+        const float slope = a.slopes ? a.slopes[h] : 0.f;
+        // (a key outside the span may have lost its page: its lane reads a key of the span instead, and its score is masked)
+        const int safe = span.begin < span.end ? span.end - 1 : min(span.keep, span.end) - 1;
+        const float* kp[4];       // the tile's key rows of this lane, from number 4 g on
+        const float* vp[4];       // row li of the values, at keys 16 c + 4 g
+        int kpage[4], kslot[4], vpage[4], vslot[4];
+        auto ask_pages = [&](int kt0) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                int t = kt0 + 16 * c + li, blk;
+                t = span.has(t) ? t : safe;
+                page_slot(a, t, blk, kslot[c]);
+                kpage[c] = bt[blk];
+                t = kt0 + 16 * c + 4 * g;
+                // (four keys of one page: the page is there if any of them is in the span)
+                t = span.touches(t, 4) ? t : (safe & ~3);
+                page_slot(a, t, blk, vslot[c]);
+                vpage[c] = bt[blk];
+            }
+        };
+        auto point_keys = [&]() {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                kp[c] = (const float*)a.k_pages + (((size_t)kpage[c] * a.nkv + kvh) * a.bs + kslot[c]) * a.hd + min(4 * g, a.hd - 4);
+        };
+        auto point_values = [&]() {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                vp[c] = (const float*)a.v_pages + (((size_t)vpage[c] * a.nkv + kvh) * a.vd + min(li, a.vd - 1)) * a.bs + vslot[c];
+        };
+        f32x4_t kb[2][UC];
+        auto fetch_keys = [&](int set, int unit) {       // unit: key block, then the part of its numbers
+            const int c0 = unit % NU * UC;
+            const int at = min(4 * g, a.hd - 4);
+#pragma unroll
+            for (int i = 0; i < UC; ++i) kb[set][i] = *(const f32x4_t*)(kp[unit / NU] + (min(16 * (c0 + i) + 4 * g, a.hd - 4) - at));
+        };
+        f32x4_t vb[2][8];
+        auto fetch_values = [&](int set, int pair) {     // value rows 32 pair .. 32 pair + 31
+            const int v0 = min(li, a.vd - 1);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) vb[set][4 * i + c] = *(const f32x4_t*)(vp[c] + (size_t)(min(32 * pair + 16 * i + li, a.vd - 1) - v0) * a.bs);
+        };
+        int kt0 = next_tile(span, first);
+        if (kt0 >= span.end) return;
+        ask_pages(kt0);
+        point_keys();
+        point_values();
+        fetch_keys(0, 0);
+        while (true) {
+            const int after = next_tile(span, kt0 + 64);
+            const bool more = after < span.end;
+            ask_pages(more ? after : kt0);
+            f32x4_t s[4];
+#pragma unroll
+            for (int unit = 0; unit < 4 * NU; ++unit) {
+                if (unit + 1 < 4 * NU) fetch_keys((unit + 1) & 1, unit + 1);
+                else fetch_values(0, 0);
+                // (two chains of sums: an instruction that waits for the one before it takes longer than its turn)
+                f32x4_t part[2] = {(f32x4_t){0.f, 0.f, 0.f, 0.f}, (f32x4_t){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int i = 0; i < UC; ++i)
+                        part[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[unit & 1][i][u], q[unit % NU * UC + i][u], part[i & 1], 0, 0, 0);
+                s[unit / NU] = unit % NU == 0 ? part[0] + part[1] : s[unit / NU] + (part[0] + part[1]);
+            }
+            float top = NEG_INF;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = kt0 + 16 * c + 4 * g + r;
+                    const bool sees = t <= pos && span.has(t) && (t >= lo || t < a.keep_first);
+                    float v = s[c][r];
+                    if (shaped) v = shaped_score(a, h, slope, v, pos - t);
+                    s[c][r] = sees ? v : NEG_INF;
+                    top = fmaxf(top, s[c][r]);
+                }
+            const float m_new = fmaxf(m, quad_max(top));
+            const float al = m_new == NEG_INF ? 1.f : expf(m - m_new);
+            float sum = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    s[c][r] = s[c][r] == NEG_INF ? 0.f : expf(s[c][r] - m_new);
+                    sum += s[c][r];
+                }
+            l = l * al + quad_sum(sum);
+            m = m_new;
+            const bool whole = span.holds_tile(kt0);
+#pragma unroll
+            for (int pair = 0; pair < (NC + 1) / 2; ++pair) {
+                if (pair + 1 < (NC + 1) / 2) fetch_values((pair + 1) & 1, pair + 1);
+                f32x4_t (&v)[8] = vb[pair & 1];
+                if (!whole) {          // memory of keys outside the span may hold anything
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (!span.has(kt0 + 16 * c + 4 * g + r)) v[c][r] = v[4 + c][r] = 0.f;
+                }
+                o[2 * pair] *= al;
+                o[2 * pair + 1] *= al;
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        o[2 * pair] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c][r], s[c][r], o[2 * pair], 0, 0, 0);
+                        o[2 * pair + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[4 + c][r], s[c][r], o[2 * pair + 1], 0, 0, 0);
+                    }
+                if (pair == 0) {
+                    // (the next tile's first keys: their pages were asked for a tile ago)
+                    point_keys();
+                    fetch_keys(0, 0);
+                }
+            }
+            if (!more) return;
+            point_values();
+            kt0 = after;
+        }
+    }
+};
+
+// prefill: block = (item of up to 64 queries, head), a wave per 16 queries
+template <int HDM>
+__global__ __launch_bounds__(256) void attn_f32_block_kernel(AttnArgs a) {
+    const int item = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int kvh = h / (a.nh / a.nkv);
+    const int tok0 = a.item_tok[item] + 16 * wave, n = min(16, a.item_n[item] - 16 * wave);
+    if (n <= 0) return;
+    const int* bt = a.block_table + (size_t)a.item_seq[item] * a.max_blocks;
+    const int tok = tok0 + min(li, n - 1);
+    const int pos = a.positions[tok], pmin = a.positions[tok0], pmax = a.positions[tok0 + n - 1];
+    const KeySpan span = {first_visible(a, pmin), pmax + 1, a.keep_first};
+    F32Attention<HDM> w;
+    w.begin(a, li < n ? (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd : nullptr, g);
+    w.walk(a, bt, kvh, span, 0, pos, first_visible(a, pos), h);
+    if (li >= n) return;
+    const float fin = finish_row<false>(a, h, w.m, w.l);
+#pragma unroll
+    for (int c = 0; c < HDM / 16; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int d = 16 * c + 4 * g + r;
+            if (d >= a.vd) continue;
+            float v = w.o[c][r] * fin;
+            if (a.turns) v = turned_back(a, tok, d, v, w.o[c][r ^ 1] * fin);
+            store_out<float>(a, tok, h, d, v);
+        }
+}
+// decode: block = one wave = (item, kv head x block of 16 of its query heads, chunk of keys); results merge as those of
+// attn_decode_kernel do
+template <int HDM>
+__global__ __launch_bounds__(64) void attn_f32_decode_kernel(AttnArgs a) {
+    const int item = blockIdx.x, split = blockIdx.z, lane = threadIdx.x, li = lane & 15, g = lane >> 4;
+    const int group = a.nh / a.nkv, group_blocks = (group + 15) / 16;
+    const int kvh = blockIdx.y / group_blocks, row = blockIdx.y % group_blocks * 16 + li;
+    const bool there = row < group;
+    const int h = kvh * group + min(row, group - 1);
+    const int tok = a.item_tok[item];
+    const int* bt = a.block_table + (size_t)a.item_seq[item] * a.max_blocks;
+    const int p = a.positions[tok], s0 = split * a.chunk, lo = first_visible(a, p);
+    const KeySpan span = {max(lo, s0), min(p + 1, s0 + a.chunk), a.keep_first};
+    F32Attention<HDM> w;
+    w.begin(a, nullptr, g);
+    if (s0 < span.end && (span.begin < span.end || s0 < span.keep)) {
+        w.begin(a, there ? (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd : nullptr, g);
+        w.walk(a, bt, kvh, span, s0, p, lo, h);
+    }
+    if (!there) return;
+    const size_t at = ((size_t)item * a.nh + h) * a.splits + split;
+    if (g == 0) {
+        a.part_ml[2 * at] = w.m;
+        a.part_ml[2 * at + 1] = w.l;
+    }
+    if (w.m == NEG_INF) return;
+#pragma unroll
+    for (int c = 0; c < HDM / 16; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int d = 16 * c + 4 * g + r;
+            if (d < a.vd) a.part_o[at * a.vd + d] = w.o[c][r];
+        }
+}
+
 // prefill: item = up to 16 consecutive queries of one sequence; block = one wave = (item, head)
 template <int HD, int SHAPE>
 __global__ __launch_bounds__(64) void attn_mfma_tile_kernel(AttnArgs a) {
@@ -1489,6 +1720,11 @@ static int check_common(const char* who, int dtype, int nh, int nkv, int hd, int
     return 0;
 }
 
+// float32 heads that the matrix-unit kernels take: keys and values in 16-byte pieces, a head's numbers in registers
+static bool f32_mfma_ok(int hd, int vd, int bs, const void* k_pages, const void* v_pages) {
+    return hd % 4 == 0 && bs % 4 == 0 && hd <= HD_MAX && vd <= HD_MAX && (((uintptr_t)k_pages | (uintptr_t)v_pages) % 16) == 0;
+}
+
 // Items of up to 128 queries are for bfloat16 with head_dim 64 or 128 and pages of a multiple of 64 keys.
 static bool wide_items_ok(int dtype, int hd, int bs) {
     return dtype == FX_BF16 && bs % 64 == 0 && (hd == 64 || hd == 128) && g_direct == 2;
@@ -1533,7 +1769,12 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
     // group and two blocks to a CU are as fast or faster)
     const bool two_groups = g_groups ? g_groups == 2 : (long)n_items * nh <= fx_compute_units();
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
-    if (dtype == FX_F32 && beyond)
+    if (dtype == FX_F32 && f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
+        const dim3 grid_items(n_items, nh);
+        if (hd <= 64 && vd <= 64) attn_f32_block_kernel<64><<<grid_items, 256, 0, s>>>(a);
+        else if (hd <= 128 && vd <= 128) attn_f32_block_kernel<128><<<grid_items, 256, 0, s>>>(a);
+        else attn_f32_block_kernel<256><<<grid_items, 256, 0, s>>>(a);
+    } else if (dtype == FX_F32 && beyond)
         attn_tile_kernel<float, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
     else if (dtype == FX_F32)
         attn_tile_kernel<float><<<grid, 64, 0, s>>>(a);
@@ -1590,7 +1831,12 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
     hipStream_t s = (hipStream_t)stream;
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
     if (dtype == FX_F32) {
-        if (beyond) attn_decode_kernel<float, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
+        if (f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
+            const dim3 gridf(n_items, nkv * ((nh / nkv + 15) / 16), splits);
+            if (hd <= 64 && vd <= 64) attn_f32_decode_kernel<64><<<gridf, 64, 0, s>>>(a);
+            else if (hd <= 128 && vd <= 128) attn_f32_decode_kernel<128><<<gridf, 64, 0, s>>>(a);
+            else attn_f32_decode_kernel<256><<<gridf, 64, 0, s>>>(a);
+        } else if (beyond) attn_decode_kernel<float, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
         else attn_decode_kernel<float><<<grid, 64, 0, s>>>(a);
         attn_decode_merge_kernel<float><<<grid2, 128, splits * sizeof(float), s>>>(a);
     } else if (beyond) {

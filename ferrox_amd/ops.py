@@ -968,7 +968,7 @@ def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq,
                      gate=None, softcap: float = 0.0, slopes=None, gate_per_head: bool = False, turns=None,
                      distance_bias=None) -> None:
     """Single queries.  The keys go to ceil(max_kv_len / chunk) blocks whose results are merged in ascending
-    order.  float32 cuts them at multiples of `chunk`, 256 by default (so that a result does not depend on the
+    order.  float32 cuts them at multiples of `chunk`, 128 by default (so that a result does not depend on the
     batch); bfloat16, whose blocks of up to eight waves share a chunk, cuts every sequence's own range of keys (from
     its window's first key to its position) into that many equal chunks of whole tiles of 64, `chunk` by default as
     `decode_attention_chunk` picks it.  `waves`: waves per block, 0 for the launch's own choice."""
@@ -978,7 +978,7 @@ def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq,
     _check_attention_extras(out, n_heads, 1 if gate_per_head else v_dim, window, keep_first, sinks, gate, softcap, slopes, distance_bias)
     _check_turns(turns, q.shape[0], v_dim, "attention")
     if chunk is None:
-        chunk = 256
+        chunk = 128 if q.dtype == torch.float32 else 256
         if q.dtype == torch.bfloat16:
             chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device))
     splits = max(1, -(-max_kv_len // chunk))

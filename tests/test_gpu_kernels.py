@@ -690,6 +690,62 @@ def test_attention_kernels(dtype, nh, nkv, hd, bs, window):
         close(out2[last], ref[last], dtype, f"decode attention chunk {chunk}")
 
 
+@pytest.mark.parametrize("nh,nkv,hd,vd", [(2, 1, 4, 4), (34, 2, 20, 36), (4, 2, 64, 64), (3, 3, 68, 48), (16, 4, 128, 128),
+                                          (2, 2, 132, 96), (2, 1, 192, 256)])
+@pytest.mark.parametrize("form", ["plain", "window", "window_keep", "chunk", "shaped", "gated", "turned"])
+def test_float32_attention_on_the_matrix_units_against_the_kernels_for_any_shape(nh, nkv, hd, vd, form):
+    """The same sequences in pages of 8 keys (the matrix-unit kernels) and of 7 (the kernels for any shape): every form of
+    mask and score, group sizes on both sides of 16, edge tiles beside slots that hold NaN.  Both sum float32 products in
+    orders of their own: they differ by roundings of sums of up to a few hundred terms."""
+    from ferrox_amd import ops
+    lens = [1, 70, 197]
+    T = sum(lens)
+    q, k, v = rnd(T, nh * hd), rnd(T, nkv, hd, seed=1), rnd(T, nkv, vd, seed=2)
+    starts = [0, 1, 71, 268]
+    pos = torch.cat([torch.arange(n) for n in lens]).to(torch.int32).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    kw = dict(v_dim=vd)
+    window = 0
+    if form.startswith("window"):
+        window = 50
+        kw.update(keep_first=20 if form == "window_keep" else 0, sinks=rnd(nh, seed=3))
+    elif form == "chunk":
+        kw.update(mask_chunk=48)
+    elif form == "shaped":
+        kw.update(softcap=3.0, slopes=torch.rand(nh, device=DEV) * 0.2, distance_bias=ops.distance_bias_rows(rnd(nh, 30, seed=4)))
+    elif form == "gated":
+        kw.update(gate=rnd(T, nh * vd, seed=5))
+    elif form == "turned":
+        angle = torch.rand(T, vd // 2, device=DEV) * 6.0
+        kw.update(turns=torch.stack([angle.cos(), angle.sin()], -1).contiguous())
+    got = {}
+    for bs in (8, 7):
+        blocks = [-(-n // bs) for n in lens]
+        table = torch.zeros(3, max(blocks), dtype=torch.int32)
+        kp = torch.full((sum(blocks), nkv, bs, hd), float("nan"), device=DEV)
+        vp = torch.full((sum(blocks), nkv, vd, bs), float("nan"), device=DEV)
+        page = 0
+        for s, n in enumerate(lens):
+            for b in range(blocks[s]):
+                table[s, b] = page
+                rows = slice(starts[s] + b * bs, min(starts[s] + (b + 1) * bs, starts[s + 1]))
+                kp[page, :, :rows.stop - rows.start] = k[rows].transpose(0, 1)
+                vp[page, :, :, :rows.stop - rows.start] = v[rows].permute(1, 2, 0)
+                page += 1
+        items = [(s, starts[s] + o, min(64, n - o)) for s, n in enumerate(lens) for o in range(0, n, 64)]
+        out, single = torch.zeros(T, nh * vd, device=DEV), torch.zeros(T, nh * vd, device=DEV)
+        args = (nh, nkv, hd, bs, window, 0.7 * hd ** -0.5)
+        ops.attention_tiles(q, out, kp, vp, table.to(DEV), pos, *(i32(list(x)) for x in zip(*items)), *args, **kw)
+        last = [x - 1 for x in starts[1:]] + [starts[2] + 100]
+        ops.attention_decode(q, single, kp, vp, table.to(DEV), pos, i32([0, 1, 2, 2]), i32(last), *args, max_kv_len=max(lens), **kw)
+        got[bs] = out, single[last]
+        # (rounding errors of a decode row: another order than the tiles', the same numbers)
+        assert torch.allclose(single[last], out[last], rtol=2e-5, atol=2e-5)
+    assert torch.isfinite(got[8][0]).all()
+    for a, b in zip(got[8], got[7]):
+        assert torch.allclose(a, b, rtol=2e-5, atol=2e-5), float((a - b).abs().max())
+
+
 @pytest.mark.parametrize("hd,bs,window", [(64, 16, 0), (64, 64, 0), (128, 64, 40000), (32, 16, 9000)])
 def test_attention_over_more_pages_than_a_block_copies(hd, bs, window):
     """A sequence of more than 1024 pages (the kernels copy that many page ids into LDS and read the rest of

@@ -27,14 +27,7 @@ from .. import debug, ops
 from .base import MIXERS, Mixer, ParamSpec
 from .latent import head_groups
 from .linear import Linear, matmul, same_dtype
-from .recurrent import sequence_starts
-
-
-def longest_portion(ctx) -> int:
-    """The most tokens that one sequence brings to this step (1 in a recorded step)."""
-    if ctx.recorded:
-        return 1
-    return max((ctx.q_starts[s + 1] - ctx.q_starts[s] for s in range(ctx.n_seqs)), default=0)
+from .recurrent import longest_portion, sequence_starts
 
 
 def _add_out(o_proj, y, ctx, residual, out_scale, fresh=False):

@@ -38,6 +38,13 @@ def sequence_starts(ctx) -> torch.Tensor:
                     .to(ctx.device, non_blocking=True))
 
 
+def longest_portion(ctx) -> int:
+    """The most tokens that one sequence brings to this step (1 in a recorded step)."""
+    if ctx.recorded:
+        return 1
+    return max((ctx.q_starts[s + 1] - ctx.q_starts[s] for s in range(ctx.n_seqs)), default=0)
+
+
 @MIXERS.register("channel_delta")
 class ChannelDelta(Mixer):
     kernel_libraries = ("elementwise", "gemm", "recurrent")
@@ -131,7 +138,8 @@ class ChannelDelta(Mixer):
 class HeadDelta(ChannelDelta):
     """The gated delta rule with one decay per head (W_a: [heads, hidden], dt_bias: [heads]) and an output gate
     silu(W_g h) of full rank (W_g: [heads * v_dim, hidden]).  State, convolution, unit vectors, step sizes and the
-    recurrence are `channel_delta`'s, through the same kernels: the decay of a head is handed to all its key channels."""
+    recurrence are `channel_delta`'s.  Short portions go through its kernels too (the decay of a head is handed to all its key channels),
+    long ones by chunks of 64 tokens."""
     TENSORS = {"q": "q", "k": "k", "v": "v", "q_conv": "q.conv", "k_conv": "k.conv", "v_conv": "v.conv", "beta": "b",
                "A_log": "A_log", "dt_bias": "dt_bias", "decay": "a", "gate": "g", "norm": "norm", "o": "o"}
 
@@ -176,11 +184,17 @@ class HeadDelta(ChannelDelta):
         debug.region("delta conv")
         conv = ops.short_conv(proj[:, :C], self.taps, cache.state["conv"], ctx.token_seq, starts, ctx.slot_ids, ctx.n_seqs)
         debug.region("delta gates")
+        longest = longest_portion(ctx)
+        chunks = ops.can_head_delta_chunks(longest, D, V)
         qn, kn, decay, beta, kq = ops.delta_prepare(conv[:, :QK], conv[:, QK:2 * QK], proj[:, o1:o2], proj[:, C:o1], self.A_log,
-                                                    self.dt_bias, H, G, D, per_head=True)
+                                                    self.dt_bias, H, G, D, per_head=True, compact=chunks)
         debug.region("delta rule")
-        o = ops.channel_delta(qn, kn, decay, beta, kq, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
-                              H, G, D, V)
+        if chunks:
+            o = ops.head_delta_chunks(qn, kn, decay, beta, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
+                                      longest, H, G, D, V)
+        else:
+            o = ops.channel_delta(qn, kn, decay, beta, kq, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
+                                  H, G, D, V)
         debug.region("delta out")
         y = ops.gated_head_norm(o, proj[:, o2:o2 + self.v_width], self.norm_w, self.norm_eps, H, V, ctx.act_dtype,
                                 gate_activation=self.gate_activation)

@@ -272,6 +272,37 @@ def main_requests():
     return {f"r{n}": u.random_tokens(u.CFG_MAIN["vocab"], n, 40 + n) for n in LENGTHS}
 
 
+@pytest.mark.parametrize("H,G,D,V,lens", [(2, 1, 64, 16, [1]), (4, 2, 64, 48, [63, 64, 65, 1]), (2, 2, 128, 32, [128, 3, 200]),
+                                          (9, 3, 128, 16, [257])])
+def test_delta_rule_by_chunks_against_the_recurrence(H, G, D, V, lens):
+    """Portions around whole chunks of 64 tokens, from and into slots in another order, a token that forgets everything,
+    heads that do not divide among eight: outputs and states of the token-by-token kernel up to the roundings of sums of at
+    most 64 + 128 terms, and in two portions what one gives."""
+    from ferrox_amd import ops
+    T, n = sum(lens), len(lens)
+    gen = torch.Generator().manual_seed(T)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda()
+    unit = lambda x: torch.nn.functional.normalize(x, dim=-1)
+    qn, kn = unit(rand(T, G, D)).reshape(T, -1) * D ** -0.5, unit(rand(T, G, D)).reshape(T, -1).contiguous()
+    qn = qn.contiguous()
+    decay, beta, v = torch.exp(-0.3 * torch.rand(T, H, generator=gen)).cuda(), torch.sigmoid(rand(T, H)), rand(T, H * V + 3)[:, :H * V]
+    decay[T // 2] = 0.0
+    kq = (qn.view(T, G, D) * kn.view(T, G, D)).sum(-1).contiguous()
+    slots = torch.arange(n, dtype=torch.int32).flip(0).contiguous().cuda()
+    starts = lambda ls: torch.tensor([0] + torch.tensor(ls).cumsum(0).tolist(), dtype=torch.int32).cuda()
+    first = rand(n, H, V, D)
+    wide = decay[:, :, None].expand(T, H, D).reshape(T, H * D).contiguous()
+    s1, s2, s3 = first.clone(), first.clone(), first.clone()
+    want = ops.channel_delta(qn, kn, wide, beta, kq, v, s1, starts(lens), slots, n, H, G, D, V)
+    got = ops.head_delta_chunks(qn, kn, decay, beta, v, s2, starts(lens), slots, n, max(lens), H, G, D, V)
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5) and torch.allclose(s2, s1, rtol=1e-5, atol=1e-5)
+    if n == 1 and T > 100:
+        cut = lambda x, a, b: x[a:b].contiguous()
+        parts = [ops.head_delta_chunks(cut(qn, a, b), cut(kn, a, b), cut(decay, a, b), cut(beta, a, b), v[a:b], s3, starts([b - a]),
+                                       slots, 1, b - a, H, G, D, V) for a, b in ((0, 100), (100, T))]
+        assert torch.allclose(torch.cat(parts), want, rtol=1e-5, atol=1e-5) and torch.allclose(s3, s1, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_whole_prompts_and_decoding(tmp_path_factory, dtype):
     weights, model = model_for(tmp_path_factory, "main", u.CFG_MAIN, 3, dtype)

@@ -1471,8 +1471,13 @@ typedef __attribute__((address_space(3))) void* fx_lds_ptr;
 // ones, group 1 the odd ones), each with stages, running maxima, sums and outputs of its own; group 1 hands its
 // results over through LDS at the end and group 0 merges them.  An item's chain of tiles is then half as long,
 // which is what bounds a prompt portion of few items over many keys.
+// HD = 256 (a latent that all heads read): the stages take 128 KB, one block of eight waves on a CU, and value heads may be
+// narrower than key heads (vd a multiple of 16).  The same bits as items of 64 queries whose four waves stage through
+// registers, which took 135 us for 1,337 tokens of 16 heads, 256 + 192 numbers; this takes 72.  Every wave reads the whole
+// tile out of LDS, 8 x 56 KB a tile, which is what bounds it.
 template <int HD, int NS, int W, int G, int SHAPE>
-__global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(AttnArgs a) {      // two blocks on a CU, or one of two groups
+__global__ __launch_bounds__(W * G * 64, HD > 128 ? 2 : W / 2) void attn_mfma_direct_kernel(AttnArgs a) {      // two blocks on a CU, or one of two groups
+    const int vd = HD > 128 ? a.vd : HD;
     static_assert(G == 1 || (G == 2 && NS == 2), "one group, or two with two stages each");
     constexpr int KS = HD / 32, CB = HD / 16;
     constexpr int NCH = HD / 8;                 // 16-byte chunks of a key row
@@ -1546,7 +1551,7 @@ __global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(Att
         const int j = wave + W * i;                          // wave-load j of HD / 8
         const int row = KROWS * j + lane / NCH;              // LDS key row 16 kb + 4 a + b
         const int key = 16 * ((row >> 2) & 3) + 4 * (row >> 4) + (row & 3);
-        k_src[i] = key * HD + (((lane % NCH) ^ (NCH == 16 ? (row & 15) : ((row >> 1) & 7))) * 8);
+        k_src[i] = key * HD + (((lane % NCH) ^ (NCH >= 16 ? (row & 15) : ((row >> 1) & 7))) * 8);
         const int d = 8 * j + (lane >> 3);                   // value row
         v_src[i] = d * bs + (((lane & 7) ^ ((d >> 1) & 7)) * 8);
     }
@@ -1555,19 +1560,20 @@ __global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(Att
         page_slot(a, kt0, blk, slot);
         const size_t page = (size_t)__builtin_amdgcn_readfirstlane(pl.page(blk));
         const bf16* kbase = (const bf16*)a.k_pages + ((page * a.nkv + kvh) * bs + slot) * HD;
-        const bf16* vbase = (const bf16*)a.v_pages + (page * a.nkv + kvh) * HD * bs + slot;
+        const bf16* vbase = (const bf16*)a.v_pages + (page * a.nkv + kvh) * vd * bs + slot;
         bf16* st = tiles + (grp * NS + stage) * TILE;
 #pragma unroll
         for (int i = 0; i < NLOAD; ++i)
             __builtin_amdgcn_global_load_lds((fx_global_ptr)(kbase + k_src[i]), (fx_lds_ptr)(st + (wave + W * i) * 512), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < NLOAD; ++i)
-            __builtin_amdgcn_global_load_lds((fx_global_ptr)(vbase + v_src[i]),
+            if (HD <= 128 || 8 * (wave + W * i) < vd)          // (value rows that exist)
+                __builtin_amdgcn_global_load_lds((fx_global_ptr)(vbase + v_src[i]),
                                              (fx_lds_ptr)(st + 64 * HD + (wave + W * i) * 512), 16, 0, 0);
     };
     // operands: key row 16 kb + li, chunk 4 u + g; value row 16 cb + li, chunks 2 g and 2 g + 1
     const int k_at = li * HD, v_at = 64 * HD + li * 64;
-    const int ksw = NCH == 16 ? li : (li >> 1) & 7, vsw = (li >> 1) & 7;
+    const int ksw = NCH >= 16 ? li : (li >> 1) & 7, vsw = (li >> 1) & 7;
 
     // Every wave of the block goes through the same barriers: the loop runs over rounds of G tiles, of which group
     // grp takes tile grp (a round's last tiles may not exist: that group then only keeps step).
@@ -1592,7 +1598,7 @@ __global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(Att
             any_edge = any_edge || (round + q < walk.n && !span.holds_tile(walk.start(round + q)));
         if (any_edge) {
             if (kt0 < kv_end && !span.holds_tile(kt0)) {
-                for (int idx = tid; idx < HD * 64; idx += W * 64) {
+                for (int idx = tid; idx < vd * 64; idx += W * 64) {
                     const int d = idx >> 6, key = idx & 63;
                     if (!span.has(kt0 + key))
                         st[64 * HD + d * 64 + (((key >> 3) ^ ((d >> 1) & 7)) * 8) + (key & 7)].bits = 0;
@@ -1629,8 +1635,9 @@ __global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(Att
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
             const bf16* vr = st + v_at + cb * 16 * 64;
-            o[cb] = pv_step(o[cb], rescale, al, p_lo, p_hi, *(const uint4*)(vr + (((2 * g) ^ vsw) * 8)),
-                            *(const uint4*)(vr + (((2 * g + 1) ^ vsw) * 8)));
+            if (HD <= 128 || 16 * cb < vd)
+                o[cb] = pv_step(o[cb], rescale, al, p_lo, p_hi, *(const uint4*)(vr + (((2 * g) ^ vsw) * 8)),
+                                *(const uint4*)(vr + (((2 * g + 1) ^ vsw) * 8)));
         }
     }
     if constexpr (G == 2) {
@@ -1670,7 +1677,8 @@ __global__ __launch_bounds__(W * G * 64, W / 2) void attn_mfma_direct_kernel(Att
             for (int cb = 0; cb < CB; ++cb) y[cb] = o[cb][r] * fr;
             turn_back_row(a, tok0 + row, li, y);
 #pragma unroll
-            for (int cb = 0; cb < CB; ++cb) store_out<bf16>(a, tok0 + row, h, 16 * cb + li, y[cb]);
+            for (int cb = 0; cb < CB; ++cb)
+                if (HD <= 128 || 16 * cb < vd) store_out<bf16>(a, tok0 + row, h, 16 * cb + li, y[cb]);
         }
     }
 }
@@ -1725,9 +1733,9 @@ static bool f32_mfma_ok(int hd, int vd, int bs, const void* k_pages, const void*
     return hd % 4 == 0 && bs % 4 == 0 && hd <= HD_MAX && vd <= HD_MAX && (((uintptr_t)k_pages | (uintptr_t)v_pages) % 16) == 0;
 }
 
-// Items of up to 128 queries are for bfloat16 with head_dim 64 or 128 and pages of a multiple of 64 keys.
+// Items of up to 128 queries are for bfloat16 with head_dim 64, 128 or 256 and pages of a multiple of 64 keys.
 static bool wide_items_ok(int dtype, int hd, int bs) {
-    return dtype == FX_BF16 && bs % 64 == 0 && (hd == 64 || hd == 128) && g_direct == 2;
+    return dtype == FX_BF16 && bs % 64 == 0 && (hd == 64 || hd == 128 || hd == 256) && g_direct == 2;
 }
 FX_API int fx_attn_tile_queries(int dtype, int hd, int bs) { return wide_items_ok(dtype, hd, bs) ? 128 : 64; }
 
@@ -1745,7 +1753,7 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
     FX_REQUIRE(!turns || vd % 2 == 0, "attn_tiles: outputs that are turned back come in pairs, a value head has %d", vd);
     FX_REQUIRE(softcap >= 0.f && softcap < INFINITY, "attn_tiles: a cap of %g on the scores", (double)softcap);
     if (check_common("attn_tiles", dtype, nh, nkv, hd, bs, window, scale, vd, mask_chunk, keep_first)) return 1;
-    FX_REQUIRE(tile_q == 64 || (tile_q == 128 && wide_items_ok(dtype, hd, bs) && mfma_ok(dtype, hd, bs, q, ldq, k_pages, v_pages, vd)),
+    FX_REQUIRE(tile_q == 64 || (tile_q == 128 && (vd == hd || hd == 256) && wide_items_ok(dtype, hd, bs) && mfma_ok(dtype, hd, bs, q, ldq, k_pages, v_pages, vd)),
                "attn_tiles: items of %d queries (64, or 128 where fx_attn_tile_queries says so)", tile_q);
     FX_REQUIRE(tile_q == 64 || !bias || bias_n + 2 * BIAS_PAD <= BIAS_LDS_MAX, "attn_tiles: items of %d queries with biases for %d distances", tile_q, bias_n);
     if (n_items <= 0) return 0;
@@ -1783,7 +1791,8 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
     else if (mfma_ok(dtype, hd, bs, q, ldq, k_pages, v_pages, vd) && shm <= BIAS_LDS_MAX * sizeof(float)) by_shape(a, [&](auto shape) {
         constexpr int SH = decltype(shape)::value;
         // the widest heads: tiles of 64 keys (34 KB) and their values (36 KB) staged in LDS for the block's 64 queries
-        if (hd > 128) attn_mfma_block_kernel<256, SH><<<grid_blocks, 256, shm, s>>>(a);
+        if (hd > 128 && tile_q == 128) attn_mfma_direct_kernel<256, 2, 8, 1, SH><<<grid_blocks, 512, shm, s>>>(a);
+        else if (hd > 128) attn_mfma_block_kernel<256, SH><<<grid_blocks, 256, shm, s>>>(a);
         else if (vd != hd && hd <= 64) attn_mfma_tile_kernel<64, SH><<<grid, 64, 0, s>>>(a);
         else if (vd != hd) attn_mfma_tile_kernel<128, SH><<<grid, 64, 0, s>>>(a);
         else if (tile_q == 128 && hd == 128 && two_groups) attn_mfma_direct_kernel<128, 2, 8, 2, SH><<<grid_blocks, 1024, shm, s>>>(a);

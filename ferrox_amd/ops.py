@@ -855,9 +855,11 @@ def compute_units(device) -> int:
     return _compute_units[key]
 
 
-def attention_tile_queries(dtype, head_dim: int, block_size: int) -> int:
+def attention_tile_queries(dtype, head_dim: int, block_size: int, v_dim: int | None = None) -> int:
     """The most consecutive queries of a sequence that one item of attention_tiles may cover at these sizes: 64,
-    or 128 where the kernel has a block of eight waves for them."""
+    or 128 where the kernel has a block of eight waves for them (value heads of another size only beside key heads of 256)."""
+    if v_dim is not None and v_dim != head_dim and not (head_dim == 256 and v_dim < 256 and v_dim % 16 == 0):
+        return 64
     f, _ = _fn("attention", "fx_attn_tile_queries")
     return int(f(dtype_code(dtype), int(head_dim), int(block_size)))
 

@@ -272,6 +272,47 @@ def main_requests():
     return {f"r{n}": u.random_tokens(u.CFG_MAIN["vocab"], n, 40 + n) for n in LENGTHS}
 
 
+@pytest.mark.parametrize("nh,nkv,vd,bs,window,keep", [(16, 1, 192, 64, 0, 0), (2, 1, 256, 64, 0, 0), (3, 3, 16, 128, 90, 0),
+                                                      (4, 2, 208, 64, 100, 70)])
+def test_latents_of_256_numbers_in_items_of_128_queries(nh, nkv, vd, bs, window, keep):
+    """Items of 128 queries (tiles straight into LDS) give the bits of items of 64 (tiles through registers) where key heads
+    hold 256 numbers: ragged items, windows and kept keys inside tiles, value heads of other sizes, slots that hold NaN."""
+    from ferrox_amd import ops
+    lens, hd = [1, 127, 130, 300], 256
+    T, starts = sum(lens), [0, 1, 128, 258]
+    gen = torch.Generator().manual_seed(vd)
+    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda().to(torch.bfloat16)
+    blocks = [-(-n // bs) for n in lens]
+    table = torch.zeros(len(lens), max(blocks), dtype=torch.int32)
+    kp = torch.full((sum(blocks), nkv, bs, hd), float("nan"), dtype=torch.bfloat16, device="cuda")
+    vp = torch.full((sum(blocks), nkv, vd, bs), float("nan"), dtype=torch.bfloat16, device="cuda")
+    page = sum(blocks)
+    for s, n in enumerate(lens):
+        for b in range(blocks[s]):
+            page -= 1
+            table[s, b] = page
+            rows = min(bs, n - b * bs)
+            kp[page, :, :rows], vp[page, :, :, :rows] = rand(nkv, rows, hd), rand(nkv, vd, rows)
+    q = rand(T, nh * hd)
+    pos = torch.cat([torch.arange(n) for n in lens]).to(torch.int32).cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    assert ops.attention_tile_queries(torch.bfloat16, hd, bs, v_dim=vd) == 128
+    assert ops.attention_tile_queries(torch.bfloat16, hd, bs, v_dim=vd - 8) == ops.attention_tile_queries(torch.bfloat16, 128, bs, v_dim=64) == 64
+    with pytest.raises(ops.KernelError):       # narrower key heads with values of another size take items of 64
+        ops.attention_tiles(torch.zeros(4, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros(4, 64, dtype=torch.bfloat16, device="cuda"),
+                            torch.zeros(1, 1, 64, 128, dtype=torch.bfloat16, device="cuda"), torch.zeros(1, 1, 64, 64, dtype=torch.bfloat16, device="cuda"),
+                            torch.zeros(1, 1, dtype=torch.int32, device="cuda"), torch.arange(4, dtype=torch.int32, device="cuda"),
+                            *(torch.tensor([x], dtype=torch.int32, device="cuda") for x in (0, 0, 4)), 1, 1, 128, 64, 0, 0.1, tile_q=128, v_dim=64)
+    got = []
+    for tq in (64, 128):
+        items = [(s, starts[s] + o, min(tq, n - o)) for s, n in enumerate(lens) for o in range(0, n, tq)]
+        out = torch.zeros(T, nh * vd, dtype=torch.bfloat16, device="cuda")
+        ops.attention_tiles(q, out, kp, vp, table.cuda(), pos, *(i32(list(x)) for x in zip(*items)), nh, nkv, hd, bs, window,
+                            hd ** -0.5, tile_q=tq, v_dim=vd, keep_first=keep, sinks=torch.randn(nh, generator=gen).cuda() * 0)
+        got.append(out)
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("H,G,D,V,lens", [(2, 1, 64, 16, [1]), (4, 2, 64, 48, [63, 64, 65, 1]), (2, 2, 128, 32, [128, 3, 200]),
                                           (9, 3, 128, 16, [257])])
 def test_delta_rule_by_chunks_against_the_recurrence(H, G, D, V, lens):

@@ -14,6 +14,7 @@
 // Dual mode: two weight matrices (gate, up) are multiplied at once and the
 // epilogue stores silu(gate) * up  (ferrox-moe/src/lib.rs:655-658).
 #include "common.h"
+#include <climits>
 #include <type_traits>
 #include <utility>
 
@@ -1507,7 +1508,7 @@ static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
 static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
-static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows) picks that tile of the LDS-tiled kernel
+static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128) or 8128 (128 x 128 in two stages) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "skinny_sets")) { g_skinny_nw = value; return 0; }
     if (!strcmp(key, "skinny_row_tiles")) { g_skinny_mt = value; return 0; }
@@ -1769,17 +1770,21 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     // holds an expert's share, streams the weights at the same speed whatever the rows (400 us at 5.9 TB/s); decode
     // steps of 48 and 64 sequences 10.3 -> 10.0 and 12.0 -> 11.4 ms, of 17 to 64 of the larger model's sizes 8-24 %
     // less; with three rows an expert the product for few rows is still 1-2 % ahead of the tiles of 64 rows.
-    // 65 to 256 plain rows against so few weight rows that the tiled kernel, whose smallest tiles are 128 x 128, would
-    // run on 32 CUs or fewer (the attention's output product): its chain of K steps takes 20-25 us whatever the rows,
-    // the product for few rows, 32 or 64 rows a block, streams the weights through every CU (2,048 x 2,048 weights:
-    // 11 us up to 128 rows and 18 us up to 256 against 20-24 us; 3,584 x 3,584: 26-30 us up to 128 rows against 31-39;
-    // with 48 tiles, the q/k/v product, the tiled kernel is ahead)
-    const bool few_tiles = !expert_offsets && !pair_ids && M > 64 && M <= 256 && (long)ceil_div(N, 128) * ceil_div(M, 128) <= 32 && !g_wide_force;
-    // More rows against very few weight rows (a low-rank projection, a router): tiles of 128 rows leave most CUs idle
+    // 65 to 128 plain rows against few weight rows (the attention's output product): the product for few rows, 32 or 64 rows
+    // a block, still streams the weights faster than tiles of 64 x 64 (2,048 x 2,048 weights 12 against 13 us, 2,048 x 5,632
+    // 25 against 28-30; 3,584 x 3,584 the other way, 31 against 20)
+    // (where the tiled kernel is the register-staged one, K no multiple of 64: up to 256 rows and 32 tiles of 128 x 128)
+    const bool few_tiles = !expert_offsets && !pair_ids && M > 64 && !g_wide_force &&
+                           (wide_ok ? M <= 128 && ceil_div(N, 128) <= 16 : M <= 256 && (long)ceil_div(N, 128) * ceil_div(M, 128) <= 32);
+    // More rows against very few weight rows (a low-rank projection, a router): tiles leave most CUs idle
     // through the whole chain of K steps, the product for few rows covers them (2,048 rows of K = 2,048 against 64 weight
-    // rows: 9 against 24 us, against 256: 18 against 25 us; against 512 it falls behind)
-    const bool narrow = !expert_offsets && !pair_ids && M > 256 && (long)M * N <= 524288 && !g_wide_force;
-    const long plain_limit = g_plain_rows > 0 ? g_plain_rows : (few_tiles ? 256 : (narrow ? M : 64));
+    // rows: 9 against 13 us; 512 rows against 512 11.3 against 12.5, 768 rows 18.8 against 12.7)
+    const bool narrow = !expert_offsets && !pair_ids && M > (wide_ok ? 128 : 256) && (long)M * N <= (wide_ok ? 262144 : 524288) && !g_wide_force;
+    // 33 to 64 plain rows of a wide gate/up product: the product for few rows fetches every row's operands in every block,
+    // tiles of 64 rows bring them to LDS once (gate/up of 11,264 x 2,048, 64 rows 27.5 -> 19 us, of 40,960 x 3,584 125 -> 70).
+    // (Stored products of so many rows keep the bits of the one that rotates in its epilogue.)
+    const bool tiles_of_64 = epi == EPI_GATED && !expert_offsets && !pair_ids && wide_ok && M > 32 && M <= 64 && 2 * N >= 8192;
+    const long plain_limit = g_plain_rows > 0 ? g_plain_rows : (few_tiles || narrow ? M : (tiles_of_64 ? 32 : 64));
     // Groups with little weight of their own (a head's up-projection of a latent): the product for few rows up to 16 rows a
     // group, tiles of 128 x 128 beyond (tiles 256 columns wide would be half empty).  16 heads of 128 x 192: 8 rows a head
     // 5.0 against 6.9 us, 2,048 rows a head 12.6 against 21.0 us.
@@ -1859,7 +1864,20 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three, the same bits: decode
         // at 64 sequences 11.2 -> 11.0 ms, a 192-token step 6.8 -> 6.4 ms; from 25 rows on average on, steps of 384
         // tokens, more and more experts need a second tile and it falls behind)
-        if (!force && small_groups)
+        // Plain rows whose tiles of 128 x 128 are fewer than the CUs: a block's chain of K steps takes the same 23-25 us (2,048
+        // k) whatever the rows, so smaller tiles on more CUs: 64 x 64 while they are one a CU (2,048 x 2,048 weights, 512 rows
+        // 23 -> 13 us; 5,632 k 55 -> 29; 6,144 weight rows, 128 rows 25 -> 14), then 64 x 128 (6,144 weight rows, 256 rows 25 ->
+        // 19; 2,048 x 5,632, 1,024 rows 56 -> 41).  Beyond that the larger tiles are ahead until 128 x 128 in two stages, two
+        // blocks to a CU, fill one round of them: 6,144 weight rows, 768 rows 40 -> 34 us; 4,608 x 3,584, 1,337 rows 61 -> 55;
+        // gate/up of 11,264, 384 rows 41 -> 35, 1,337 rows (two rounds, 95 % full) 94 -> 80.  The same bits in every tile.
+        const bool plain = !expert_offsets && !force;
+        const long t64 = dual ? LONG_MAX : (long)ceil_div(N, 64) * ceil_div(M, 64), t64w = tiles(64, 128), t128 = tiles(128, 128);
+        const bool small_square = plain && t64 <= cus, small_wide = plain && !small_square && t64w <= cus;
+        const bool two_a_cu = plain && ((t128 > cus && t128 <= 2 * cus) || (t128 > 3.72 * cus && t128 <= 4 * cus));
+        if (force == 464 ? !dual : small_square) launch_wide<4, 64, 4>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);
+        else if (force == 4128 || small_wide) launch_wide<4, 128, 3>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);
+        else if (force == 8128 || two_a_cu) launch_wide<8, 128, 2>(g, epi, M / 128 + (expert_offsets ? nonempty : (M % 128 != 0)), s);
+        else if (!force && small_groups)
             launch_wide<8, 128, 4>(g, epi, M / 128 + nonempty, s);
         else if (force == 4 || (!force && expert_offsets && per_group <= g_tile64_rows))
             launch_wide<4, 256, 4, 2>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);

@@ -146,7 +146,8 @@ def test_combine_of_many_rows_equals_that_of_few(T, H, k, S, sorted_rows):
     close(h_all, want, torch.float32, "combined rows")
 
 
-@pytest.mark.parametrize("tile", [256, 192, 128, 64, 12, 4])      # 12, 4: tiles of 192 and of 64 rows x 256 weight rows
+# 12, 4: tiles of 192 and of 64 rows x 256 weight rows; 464, 4128: 64 x 64 and 64 x 128; 8128: 128 x 128 in two stages
+@pytest.mark.parametrize("tile", [256, 192, 128, 64, 12, 4, 464, 4128, 8128])
 @pytest.mark.parametrize("M,N,K", [(300, 400, 192), (513, 200, 64), (70, 520, 448)])
 def test_gemm_every_wide_tile(tile, M, N, K):
     """The many-row kernel picks its tile by the sizes; here each tile shape is made to run the same products."""
@@ -164,6 +165,24 @@ def test_gemm_every_wide_tile(tile, M, N, K):
     close(got, ref + bias.double(), dtype, "store+bias")
     close(h, h0.double() + ref, dtype, "residual")
     close(act, plain.silu(a.double() @ w2[:N].double().T) * (a.double() @ w2[N:].double().T), dtype, "silu(gate)*up")
+
+
+@pytest.mark.parametrize("M,N", [(33, 4096), (64, 8200), (129, 64), (257, 1000), (513, 2048), (700, 3000)])
+def test_plain_products_have_the_same_bits_in_every_tile(M, N):
+    """The tile that the sizes choose (64 x 64 to 256 x 256, edges inside tiles) against one that is forced: every tile adds an
+    element's products in ascending order."""
+    from ferrox_amd import debug, ops
+    K, dtype = 192, torch.bfloat16
+    a, w, bias = rnd(M, K, dtype=dtype), rnd(N, K, dtype=dtype, seed=1), rnd(N, dtype=dtype, seed=2)
+    chosen = ops.gemm(a, w, bias=bias)
+    close(chosen, a.double() @ w.double().T + bias.double(), dtype, "chosen tile")
+    with debug.kernel_switch("gemm", "plain_rows", 32):      # (no product for few rows beyond 32 rows)
+        gated = ops.gemm(a, w[:N // 2 * 2], epilogue=ops.EPI_GATED)
+        chosen = ops.gemm(a, w, bias=bias)
+        for tile in (464, 4128, 8128, 64, 256):
+            with debug.kernel_switch("gemm", "wide", tile):
+                assert torch.equal(ops.gemm(a, w, bias=bias), chosen), tile
+                assert torch.equal(ops.gemm(a, w[:N // 2 * 2], epilogue=ops.EPI_GATED), gated), tile
 
 
 @pytest.mark.parametrize("tile", [12, 256, 4])

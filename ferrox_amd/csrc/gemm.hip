@@ -1800,16 +1800,13 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // rows the four row tiles a block stay ahead, 17.3 against 20.1 us)
         const bool spread_rows = mt == 4 && !expert_offsets && !norm_w && epi == EPI_RESID && ceil_div(N, 16) * (long)ceil_div(M, 64) < 192;
         if (spread_rows) mt = 1;
-        // 33 and more plain rows against so few weight rows that blocks of several row tiles are a fraction of the CUs (a
-        // router of 61 rows as the rows, the step's tokens as the weights): a block per row tile, or per two, while the blocks
-        // stay about one a CU (2,048 k: 512 tokens 12.1 -> below 8.7 us, 2,048 tokens 12.7 -> 9.2; 3,584 k, 65 rows, 512 tokens
-        // 13.0 -> 9.7; at 4,096 tokens the larger blocks are ahead, 13.2 against 14.6-17.8)
-        int fewest = 0;
-        if (!expert_offsets && !pair_ids && !norm_w && (epi == EPI_STORE || epi == EPI_STORE_F32) && M > 32 && M <= 128) {
-            for (int t = 1; t < mt && !fewest; t *= 2)
-                if (4L * ceil_div(N, 16) * ceil_div(M, 16 * t) <= 5L * fx_compute_units()) fewest = t;
-            if (fewest) mt = fewest;
-        }
+        // 33 to 128 plain rows against so few weight rows that blocks of several row tiles are a fraction of the CUs (a
+        // router of 61 rows as the rows, the step's tokens as the weights): a block per row tile while they stay about one a CU
+        // (2,048 k, 512 tokens 16.8 -> 10.4 us in a step; 3,584 k, 65 rows, 512 tokens 13.0 -> 9.7).  Two row tiles a block for 2,048
+        // tokens took 10.6 instead of 14.9 us, but the step, whose routing runs beside the shared expert, 0.5 % longer.
+        const bool row_tile_blocks = !expert_offsets && !pair_ids && !norm_w && (epi == EPI_STORE || epi == EPI_STORE_F32) && M > 32 &&
+                                     M <= 128 && mt > 1 && 4L * ceil_div(N, 16) * ceil_div(M, 16) <= 5L * fx_compute_units();
+        if (row_tile_blocks) mt = 1;
         if (g_skinny_mt && !pair_ids) mt = g_skinny_mt;
         const int m_tiles = pair_ids ? (M < E ? M : E) + M / 16 + n_always
                                      : M / (16 * mt) + (expert_offsets ? nonempty : (M % (16 * mt) != 0));
@@ -1819,7 +1816,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         int nw = (dual || (long)ceil_div(N, 32) * m_tiles >= 160) ? 2 : 1;
         if (!dual && (norm_w || (M <= 2 && (long)ceil_div(N, 16) * m_tiles >= 4096))) nw = 1;
         if (spread_rows) nw = 2;
-        if (fewest) nw = 1;
+        if (row_tile_blocks) nw = 1;
         if ((g_skinny_nw == 1 && !dual) || (g_skinny_nw == 2 && !norm_w)) nw = g_skinny_nw;
         // Waves per block: four, a part of K each, for unsorted pairs too.  (Those ran with one wave that went
         // through all four parts, or two, while a wave found its tile with a loop over the experts and each such

@@ -139,7 +139,7 @@ FX_API int fx_short_conv(void* stream, const void* x, int x_dtype, long ldx, voi
 //   qn = q / sqrt(sum(q^2) + 1e-6) * D^-1/2,  kn = k / sqrt(sum(k^2) + 1e-6)        per q/k head
 //   decay[h, i] = exp(-exp(A_log[h]) * softplus(a[h, i] + dt_bias[h, i]))             per head and key channel
 //                 (per_head: a and dt_bias hold one number a head, a[h] and dt_bias[h], and all D channels of a
-//                 head receive the same decay; per_head 2: the decays are [T, H] too)
+//                 head receive the same decay)
 //   beta[h] = sigmoid(b[h])
 //   kq[g] = kn[g] . qn[g]                                                             per q/k head (the recurrence needs it per token)
 // Blocks (token, part): part p makes 256 of the token's decays and, a wave each, heads 4p .. 4p+3 of q and k (a
@@ -174,12 +174,11 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const float* __restr
         dot = wave_sum(dot);
         if (lane == 0) kq[(size_t)t * G + g] = dot;
     }
-    const int copies = per_head == 2 ? 1 : D;
-    for (int idx = part * 256 + threadIdx.x; idx < H * copies; idx += 256 * gridDim.y) {
-        const int h = idx / copies, src = per_head ? h : idx;
+    for (int idx = part * 256 + threadIdx.x; idx < H * D; idx += 256 * gridDim.y) {
+        const int h = idx / D, src = per_head ? h : idx;
         const float rate = expf(load_as_float(A_log, w_dtype, h));
         const float step = softplus_f(a[(size_t)t * lda + src] + load_as_float(dt_bias, w_dtype, src));
-        decay[(size_t)t * H * copies + idx] = expf(-rate * step);
+        decay[(size_t)t * H * D + idx] = expf(-rate * step);
     }
     if (part == 0)
         for (int h = threadIdx.x; h < H; h += 256) beta[(size_t)t * H + h] = 1.0f / (1.0f + expf(-b[(size_t)t * ldb + h]));
@@ -191,7 +190,7 @@ FX_API int fx_delta_prepare(void* stream, const float* q, long ldq, const float*
     FX_REQUIRE(T >= 0 && H > 0 && G > 0 && D > 0 && H % G == 0, "delta_prepare: bad sizes T=%d H=%d G=%d D=%d", T, H, G, D);
     FX_REQUIRE(w_dtype == FX_F32 || w_dtype == FX_BF16, "delta_prepare: unknown dtype %d", w_dtype);
     if (T == 0) return 0;
-    const int parts = (int)fminl(1024, fmaxl((H * (long)(per_head == 2 ? 1 : D) + 255) / 256, (G + 3) / 4));
+    const int parts = (int)fminl(1024, fmaxl((H * (long)D + 255) / 256, (G + 3) / 4));
     delta_prepare_kernel<<<dim3(T, parts), 256, 0, (hipStream_t)stream>>>(q, ldq, k, ldk, a, lda, b, ldb, A_log, dt_bias, w_dtype, qn, kn,
                                                              decay, beta, kq, H, G, D, per_head);
     FX_CHECK_LAUNCH("delta_prepare");
@@ -454,310 +453,6 @@ FX_API int fx_channel_delta(void* stream, const float* qn, const float* kn, cons
     else FX_DELTA(8, 32, 8);
 #undef FX_DELTA
     FX_CHECK_LAUNCH("channel_delta");
-    return 0;
-}
-
-// ---------------------------------------------------------------------------
-// The delta rule with one decay per head over a long portion, 64 tokens at a time on the float32 matrix instructions
-// (the recurrence above is a chain of a quarter of a microsecond a token whatever the GPU has to spare).  Inside a chunk,
-// with c_t the product of the decays up to token t, M[t][s] = decay_{s+1} .. decay_t, and S the state in front of it:
-//     u_t = beta_t (v_t - c_t S^T k_t - sum_{s < t} M[t][s] (k_t . k_s) u_s)
-//     o_t = c_t S^T q_t + sum_{s <= t} M[t][s] (q_t . k_s) u_s
-//     S' = c_last S + sum_s M[last][s] k_s u_s^T
-// so with A[t][s] = beta_t M[t][s] (k_t . k_s), s < t:  (I + A) U = beta V - (beta c K) S.  The first kernel, a block per
-// (chunk, head), solves (I + A) X = [beta c K | beta V] by forward substitution, a column per thread, and leaves
-// W = X's first part, U0 = its second (transposed), P[t][s] = M[t][s] (q_t . k_s) and the transpose of M[last][s] k_s; the
-// second, a block per (head, 16 columns of the state), walks over the chunks: U = U0 - W S, O = c (Q S) + P U,
-// S = c_last S + (..)^T U, four waves of 16 tokens each, operands from memory two chunks ahead, the state in registers.
-// Products of decays are made by multiplying (no logarithms): a decay of zero is as good as another.
-// Everything is float32: against 64 bits the state is off by 9e-8 and the outputs by 1.4e-7 (norms; 1e-7 and 1.2e-7 token by token).
-// 1,337 tokens of 16 heads of 128 x 128: 54 + 83 us against 355 (4,096 tokens: 343 against 1,090).  The second kernel is bound by its
-// 112 products of 32 cycles a chunk and wave and by the 112 KB a block reads for them, the first by a thread's 2,016 dependent steps.
-// ---------------------------------------------------------------------------
-#define DELTA_CHUNK 64
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-
-// what the first kernel leaves per (chunk, head)
-struct DeltaChunks {
-    float* w;        // [64][D]
-    float* kt;       // [D][64]
-    float* p;        // [64][64]
-    float* u0;       // [V][64]
-    float* c;        // [64]
-    __host__ __device__ static size_t floats(int D, int V) { return (size_t)DELTA_CHUNK * (2 * D + DELTA_CHUNK + V + 1); }
-    __device__ DeltaChunks(float* work, size_t at, int D, int V) {
-        w = work + at * floats(D, V);
-        kt = w + DELTA_CHUNK * D;
-        p = kt + DELTA_CHUNK * D;
-        u0 = p + DELTA_CHUNK * DELTA_CHUNK;
-        c = u0 + DELTA_CHUNK * V;
-    }
-};
-// where the chunks of sequence s, which begins at token t0, begin: a sequence of n tokens has no more than
-// (t0 + n) / 64 - t0 / 64 + 1 of them
-__device__ __forceinline__ int first_chunk(int t0, int s) { return t0 / DELTA_CHUNK + s; }
-
-template <int D>
-__global__ __launch_bounds__(256) void head_delta_chunk_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
-                                                               const float* __restrict__ decay, const float* __restrict__ beta,
-                                                               const float* __restrict__ v, long ldv, const int* __restrict__ seq_starts,
-                                                               int H, int G, int V, float* __restrict__ work) {
-    constexpr int C = DELTA_CHUNK, NC = D / 16;
-    __shared__ float M[C][C + 1];
-    __shared__ __attribute__((aligned(16))) float A[C][C];
-    __shared__ __attribute__((aligned(16))) float gs[C], bs[C], cs[C];
-    const int h = blockIdx.y, s = blockIdx.z, g0 = h / (H / G), tid = threadIdx.x;
-    const int t0 = seq_starts[s] + blockIdx.x * C, n = min(C, seq_starts[s + 1] - t0);
-    if (n <= 0) return;
-    const DeltaChunks to(work, (size_t)(first_chunk(seq_starts[s], s) + blockIdx.x) * H + h, D, V);
-    if (tid < C) {
-        gs[tid] = tid < n ? decay[(size_t)(t0 + tid) * H + h] : 1.f;
-        bs[tid] = tid < n ? beta[(size_t)(t0 + tid) * H + h] : 0.f;
-    }
-    __syncthreads();
-    const int lane = tid & 63, wave = tid >> 6, li = lane & 15, g = lane >> 4;
-    if (tid < C) {
-        // (products of up to 64 factors: in 64 bits, rounded once)
-        float gv[C];
-#pragma unroll
-        for (int i = 0; i < C; i += 4) *(f32x4_t*)(gv + i) = *(const f32x4_t*)(gs + i);
-        double r = 1.0;
-#pragma unroll
-        for (int i = C - 1; i >= 0; --i) {
-            M[tid][i] = (float)r;                   // (entries above the diagonal: 1, never used)
-            r *= i <= tid ? (double)gv[i] : 1.0;
-        }
-        cs[tid] = (float)r;
-        to.c[tid] = (float)r;
-    }
-    __syncthreads();
-    {
-        // rows 16 wave .. + 15 of K K^T and Q K^T (rows past the end read the last token; nothing of them is kept)
-        const size_t mine = ((size_t)(t0 + min(16 * wave + li, n - 1)) * G + g0) * D + 4 * g;
-        f32x4_t kr[NC], qr[NC];
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            kr[i] = *(const f32x4_t*)(kn + mine + 16 * i);
-            qr[i] = *(const f32x4_t*)(qn + mine + 16 * i);
-        }
-        f32x4_t b[4][NC];
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            const float* col = kn + ((size_t)(t0 + min(16 * ct + li, n - 1)) * G + g0) * D + 4 * g;
-#pragma unroll
-            for (int i = 0; i < NC; ++i) b[ct][i] = *(const f32x4_t*)(col + 16 * i);
-        }
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) {
-            const f32x4_t zero = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-            f32x4_t kks[4] = {zero, zero, zero, zero}, qks[4] = {zero, zero, zero, zero};
-            if (ct <= wave) {
-#pragma unroll
-                for (int i = 0; i < NC; ++i)
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        kks[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[i][u], b[ct][i][u], kks[u], 0, 0, 0);
-                        qks[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(qr[i][u], b[ct][i][u], qks[u], 0, 0, 0);
-                    }
-            }
-            const f32x4_t kk = (kks[0] + kks[1]) + (kks[2] + kks[3]), qk = (qks[0] + qks[1]) + (qks[2] + qks[3]);
-            const int c = 16 * ct + li;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * wave + 4 * g + r;
-                const bool in = t < n && c <= t;
-                const float m = in ? M[t][c] : 0.f;
-                A[t][c] = in && c < t ? bs[t] * (m * kk[r]) : 0.f;
-                to.p[(size_t)t * C + c] = in ? m * qk[r] : 0.f;
-            }
-        }
-    }
-    __syncthreads();
-    for (int j = tid; j < D + V; j += 256) {
-        const bool key = j < D;
-        float x[C];
-        // (a running pointer that stops at the last token: 64 addresses worked out ahead do not fit the scalar registers)
-        const float* src = key ? kn + ((size_t)t0 * G + g0) * D + j : v + (size_t)t0 * ldv + (size_t)h * V + (j - D);
-        const size_t stride = key ? (size_t)G * D : (size_t)ldv;
-#pragma unroll
-        for (int t = 0; t < C; ++t) {
-            x[t] = *src;
-            src += t + 1 < n ? stride : 0;
-        }
-        if (key) {
-#pragma unroll
-            for (int t = 0; t < C; t += 4) {
-                f32x4_t y;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) y[r] = t + r < n ? M[C - 1][t + r] * x[t + r] : 0.f;
-                *(f32x4_t*)(to.kt + (size_t)j * C + t) = y;
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < C; ++t) x[t] = t < n ? x[t] * (key ? bs[t] * cs[t] : bs[t]) : 0.f;
-#pragma unroll
-        for (int t = 1; t < C; ++t) {
-            float part[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int i = 0; i < t; i += 4) {
-                const f32x4_t a = *(const f32x4_t*)&A[t][i];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (i + r < t) part[r] = fmaf(a[r], x[i + r], part[r]);
-            }
-            x[t] -= (part[0] + part[1]) + (part[2] + part[3]);
-        }
-        if (key) {
-#pragma unroll
-            for (int t = 0; t < C; ++t) to.w[(size_t)t * D + j] = x[t];
-        } else {
-#pragma unroll
-            for (int t = 0; t < C; t += 4) *(f32x4_t*)(to.u0 + (size_t)(j - D) * C + t) = (f32x4_t){x[t], x[t + 1], x[t + 2], x[t + 3]};
-        }
-    }
-}
-
-// one chunk's operands of a lane
-template <int D>
-struct DeltaOperands {
-    f32x4_t w[D / 16], q[D / 16], p[4], kt[D / 64][4], u0;
-    float c, c_last;
-};
-
-template <int D>
-__global__ __launch_bounds__(256) void head_delta_scan_kernel(const float* __restrict__ qn, float* __restrict__ out, long ldo,
-                                                              float* __restrict__ state, const int* __restrict__ seq_starts,
-                                                              const int* __restrict__ slots, int H, int G, int V, float* __restrict__ work) {
-    constexpr int C = DELTA_CHUNK, NC = D / 16, JJ = D / 64;
-    __shared__ __attribute__((aligned(16))) float St[2][16][D + 4];      // the state's columns, transposed
-    __shared__ f32x4_t U[4][64];
-    // blocks go to the eight XCDs in turn: the column blocks of a head, which read the same operands, on one of them
-    const int nvb = V / 16, id = blockIdx.x, along = id / 8;
-    const int h = id % 8 + along / nvb * 8, vb = along % nvb, s = blockIdx.y;
-    if (h >= H) return;
-    const int g0 = h / (H / G), t0 = seq_starts[s], n_all = seq_starts[s + 1] - t0;
-    if (n_all <= 0) return;
-    const int n_chunks = (n_all + C - 1) / C, base = first_chunk(t0, s);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, g = lane >> 4;
-    const int col = 16 * vb + li;
-    auto load = [&](DeltaOperands<D>& o, int chunk) {
-        chunk = min(chunk, n_chunks - 1);
-        const DeltaChunks from(work, (size_t)(base + chunk) * H + h, D, V);
-        const int t = min(chunk * C + 16 * wave + li, n_all - 1);
-        const float* qrow = qn + ((size_t)(t0 + t) * G + g0) * D + 4 * g;
-        const float* wrow = from.w + (size_t)(16 * wave + li) * D + 4 * g;
-#pragma unroll
-        for (int i = 0; i < NC; ++i) o.w[i] = *(const f32x4_t*)(wrow + 16 * i);
-#pragma unroll
-        for (int i = 0; i < NC; ++i) o.q[i] = *(const f32x4_t*)(qrow + 16 * i);
-        o.u0 = *(const f32x4_t*)(from.u0 + (size_t)col * C + 16 * wave + 4 * g);
-        o.c = from.c[16 * wave + li];
-        o.c_last = from.c[C - 1];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o.p[i] = *(const f32x4_t*)(from.p + (size_t)(16 * wave + li) * C + 16 * i + 4 * g);
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) o.kt[jj][i] = *(const f32x4_t*)(from.kt + (size_t)(16 * (wave * JJ + jj) + li) * C + 16 * i + 4 * g);
-    };
-    float* S_g = state + (((size_t)slots[s] * H + h) * V + col) * D + 4 * g;
-    f32x4_t S[JJ];
-#pragma unroll
-    for (int jj = 0; jj < JJ; ++jj) {
-        S[jj] = *(const f32x4_t*)(S_g + 16 * (wave * JJ + jj));
-        *(f32x4_t*)&St[0][li][16 * (wave * JJ + jj) + 4 * g] = S[jj];
-    }
-    auto step = [&](const DeltaOperands<D>& o, int chunk) {
-        const int buf = chunk & 1;
-        // (four chains of sums each: the shorter a chain, the less it rounds)
-        const f32x4_t zero = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-        f32x4_t ws[4] = {zero, zero, zero, zero}, qs[4] = {zero, zero, zero, zero};
-        f32x4_t b[NC];
-#pragma unroll
-        for (int i = 0; i < NC; ++i) b[i] = *(const f32x4_t*)&St[buf][li][16 * i + 4 * g];
-#pragma unroll
-        for (int i = 0; i < NC; ++i)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                ws[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[i][u], b[i][u], ws[u], 0, 0, 0);
-                qs[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[i][u], o.q[i][u], qs[u], 0, 0, 0);
-            }
-        // the loads of the chunk after next, which stand in front of this step, go out between its products: a burst of them
-        // keeps the wave from issuing anything for half a microsecond
-        __builtin_amdgcn_sched_group_barrier(0x100, NC, 0);                            // reads of LDS
-#pragma unroll
-        for (int i = 0; i < 2 * NC + 4 * JJ + 7; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, D == 128 ? 2 : 1, 0);      // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                     // a load from memory
-        }
-        U[wave][lane] = o.u0 - ((ws[0] + ws[1]) + (ws[2] + ws[3]));
-        // (outputs transposed: a lane holds four neighbouring columns of token 16 wave + li, one store a chunk.  With the tokens
-        // along a lane's registers the four stores took as long as all the rest, 100 against 50 us for 21 chunks)
-        const f32x4_t y0 = o.c * ((qs[0] + qs[1]) + (qs[2] + qs[3]));
-        f32x4_t ys[4] = {zero, zero, zero, zero}, ks[JJ][2];
-        lds_barrier();
-        f32x4_t u4[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) u4[i] = U[i][lane];
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj) ks[jj][0] = ks[jj][1] = zero;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-#pragma unroll
-                for (int jj = 0; jj < JJ; ++jj) ks[jj][u & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[jj][i][u], u4[i][u], ks[jj][u & 1], 0, 0, 0);
-                ys[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(u4[i][u], o.p[i][u], ys[u], 0, 0, 0);      // (zeros above the diagonal)
-            }
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj) S[jj] = S[jj] * o.c_last + (ks[jj][0] + ks[jj][1]);
-        const f32x4_t y = y0 + ((ys[0] + ys[1]) + (ys[2] + ys[3]));
-#pragma unroll
-        for (int jj = 0; jj < JJ; ++jj) *(f32x4_t*)&St[buf ^ 1][li][16 * (wave * JJ + jj) + 4 * g] = S[jj];
-        const int t = chunk * C + 16 * wave + li;
-        if (t < n_all) *(f32x4_t*)(out + (size_t)(t0 + t) * ldo + (size_t)h * V + 16 * vb + 4 * g) = y;
-        lds_barrier();
-    };
-    // (operands two chunks ahead: a chunk's work is shorter than a trip to memory)
-    DeltaOperands<D> a, b, c;
-    load(a, 0);
-    load(b, 1);
-    lds_barrier();
-    int chunk = 0;
-    for (; chunk + 2 < n_chunks; chunk += 3) {
-        load(c, chunk + 2);
-        step(a, chunk);
-        load(a, chunk + 3);
-        step(b, chunk + 1);
-        load(b, chunk + 4);
-        step(c, chunk + 2);
-    }
-    if (chunk < n_chunks) step(a, chunk);
-    if (chunk + 1 < n_chunks) step(b, chunk + 1);
-#pragma unroll
-    for (int jj = 0; jj < JJ; ++jj) *(f32x4_t*)(S_g + 16 * (wave * JJ + jj)) = S[jj];
-}
-
-// decay, beta: [T, H].  `longest`: the most tokens any sequence brings.  work: (T / 64 + n_seqs) H 64 (2 D + V + 65) floats.
-FX_API int fx_head_delta_chunks(void* stream, const float* qn, const float* kn, const float* decay, const float* beta,
-                                const float* v, long ldv, float* out, long ldo, float* state, const int* seq_starts,
-                                const int* slots, int n_seqs, int longest, int H, int G, int D, int V, float* work) {
-    FX_REQUIRE(n_seqs >= 0 && H > 0 && G > 0 && H % G == 0, "head_delta: bad sizes sequences=%d H=%d G=%d", n_seqs, H, G);
-    FX_REQUIRE((D == 64 || D == 128) && V >= 16 && V % 16 == 0, "head_delta: key size %d (64 or 128) and value size %d (a multiple of 16)", D, V);
-    FX_REQUIRE(ldv >= (long)H * V && ldo >= (long)H * V, "head_delta: rows of %ld and %ld hold fewer than %d values", ldv, ldo, H * V);
-    FX_REQUIRE(n_seqs <= 65535 && H <= 65535 && longest >= 0, "head_delta: %d sequences of %d heads are more than a launch takes", n_seqs, H);
-    FX_REQUIRE(((((uintptr_t)state | (uintptr_t)qn | (uintptr_t)kn | (uintptr_t)work | (uintptr_t)out) % 16) == 0) && ldo % 4 == 0, "head_delta: operands not aligned to 16 bytes");
-    if (n_seqs == 0 || longest == 0) return 0;
-    hipStream_t s = (hipStream_t)stream;
-    const dim3 grid_a(ceil_div(longest, DELTA_CHUNK), H, n_seqs), grid_b(8 * ceil_div(H, 8) * (V / 16), n_seqs);
-    if (D == 128) {
-        head_delta_chunk_kernel<128><<<grid_a, 256, 0, s>>>(qn, kn, decay, beta, v, ldv, seq_starts, H, G, V, work);
-        head_delta_scan_kernel<128><<<grid_b, 256, 0, s>>>(qn, out, ldo, state, seq_starts, slots, H, G, V, work);
-    } else {
-        head_delta_chunk_kernel<64><<<grid_a, 256, 0, s>>>(qn, kn, decay, beta, v, ldv, seq_starts, H, G, V, work);
-        head_delta_scan_kernel<64><<<grid_b, 256, 0, s>>>(qn, out, ldo, state, seq_starts, slots, H, G, V, work);
-    }
-    FX_CHECK_LAUNCH("head_delta");
     return 0;
 }
 

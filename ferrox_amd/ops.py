@@ -114,8 +114,6 @@ _sigs = {
                                         c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int],
     ("recurrent", "fx_small_rows_pair"): [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_long, c_int, c_int,
                                           c_void_p, c_long, c_void_p, c_void_p, c_long, c_int, c_int, c_int],
-    ("recurrent", "fx_head_delta_chunks"): [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long,
-                                            c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
     ("recurrent", "fx_small_rows_parts"): [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int],
     ("recurrent", "fx_gated_head_norm"): [c_void_p, c_int, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_int, c_void_p,
                                           c_long, c_int, c_int, c_int, c_float, c_int, c_void_p, c_void_p],
@@ -1211,12 +1209,11 @@ def short_conv(x, taps, state, token_seq, seq_starts, slot_ids, n_seqs: int, act
     return y
 
 
-def delta_prepare(q, k, a, b, A_log, dt_bias, n_heads: int, n_kv_heads: int, key_dim: int, per_head: bool = False,
-                  compact: bool = False):
+def delta_prepare(q, k, a, b, A_log, dt_bias, n_heads: int, n_kv_heads: int, key_dim: int, per_head: bool = False):
     """From convolved q, k [T, G*D], the decay's projection a [T, H*D] and the step size's b [T, H] (float32 rows):
     (q / |q| / sqrt(D), k / |k|, exp(-exp(A_log[h]) softplus(a + dt_bias)), sigmoid(b), the normed k . q per q/k head
     [T, G]), all float32 contiguous.  `per_head`: a is [T, H] and dt_bias [H], one decay per head, which all D
-    channels of the head receive (the decays returned are [T, H*D] either way, or [T, H] if `compact`)."""
+    channels of the head receive (the decays returned are [T, H*D] either way)."""
     T = q.shape[0]
     H, G, D = int(n_heads), int(n_kv_heads), int(key_dim)
     Dd = 1 if per_head else D
@@ -1228,14 +1225,12 @@ def delta_prepare(q, k, a, b, A_log, dt_bias, n_heads: int, n_kv_heads: int, key
     dev = q.device
     qn = torch.empty((T, G * D), dtype=torch.float32, device=dev)
     kn = torch.empty((T, G * D), dtype=torch.float32, device=dev)
-    if compact and not per_head:
-        raise KernelError("delta_prepare: compact decays are those of one decay per head")
-    decay = torch.empty((T, H if compact else H * D), dtype=torch.float32, device=dev)
+    decay = torch.empty((T, H * D), dtype=torch.float32, device=dev)
     beta = torch.empty((T, H), dtype=torch.float32, device=dev)
     kq = torch.empty((T, G), dtype=torch.float32, device=dev)
     _call("recurrent", "fx_delta_prepare", _stream(), _p(q), q.stride(0), _p(k), k.stride(0), _p(a), a.stride(0), _p(b),
           b.stride(0), _p(A_log), _p(dt_bias), dtype_code(A_log.dtype), _p(qn), _p(kn), _p(decay), _p(beta), _p(kq), T, H, G, D,
-          2 if compact else (1 if per_head else 0))
+          1 if per_head else 0)
     return qn, kn, decay, beta, kq
 
 
@@ -1257,38 +1252,6 @@ def channel_delta(qn, kn, decay, beta, kq, v, state, seq_starts, slot_ids, n_seq
     out = torch.empty((T, H * V), dtype=torch.float32, device=qn.device)
     _call("recurrent", "fx_channel_delta", _stream(), _p(qn), _p(kn), _p(decay), _p(beta), _p(kq), _p(v), v.stride(0), _p(out),
           out.stride(0), _p(state), _p(_i32(seq_starts, "seq_starts")), _p(_i32(slot_ids, "slot_ids")), int(n_seqs), H, G, D, V)
-    return out
-
-
-HEAD_DELTA_CHUNKS_FROM = 128     # tokens of the longest portion from which the delta rule with one decay per head goes by chunks
-
-
-def can_head_delta_chunks(longest: int, key_dim: int, v_dim: int) -> bool:
-    """Whether `head_delta_chunks` is the way for a step of so many tokens: portions that are long enough (16 heads of
-    128 x 128, the recurrence against the chunks: 64 tokens 21 and 36 us, 128 38 and 39, 256 74 and 50, 4,096 1,090 and 343) of
-    heads that it takes."""
-    return longest >= HEAD_DELTA_CHUNKS_FROM and key_dim in (64, 128) and v_dim % 16 == 0
-
-
-def head_delta_chunks(qn, kn, decay, beta, v, state, seq_starts, slot_ids, n_seqs: int, longest: int, n_heads: int,
-                      n_kv_heads: int, key_dim: int, v_dim: int) -> torch.Tensor:
-    """The gated delta rule with one decay per head (`decay` [T, H]), 64 tokens at a time; else as `channel_delta`.
-    `longest`: the most tokens any sequence brings."""
-    T = qn.shape[0]
-    H, G, D, V = int(n_heads), int(n_kv_heads), int(key_dim), int(v_dim)
-    for t, cols, what in ((qn, G * D, "q"), (kn, G * D, "k"), (decay, H, "decay"), (beta, H, "beta")):
-        if t.dtype != torch.float32 or not t.is_contiguous() or tuple(t.shape) != (T, cols):
-            raise KernelError(f"head_delta_chunks: {what} must be contiguous float32 [{T}, {cols}]")
-    _f32_rows(v, "head_delta_chunks: v", H * V)
-    if v.shape[0] != T or state.dtype != torch.float32 or not state.is_contiguous() or tuple(state.shape[1:]) != (H, V, D):
-        raise KernelError(f"head_delta_chunks: v {tuple(v.shape)} / state {tuple(state.shape)} for [slots, {H}, {V}, {D}]")
-    if seq_starts.numel() < n_seqs + 1 or slot_ids.numel() < n_seqs or not 0 <= longest <= T:
-        raise KernelError("head_delta_chunks: the step's index tensors are shorter than its sequences, or a portion longer than the step")
-    out = torch.empty((T, H * V), dtype=torch.float32, device=qn.device)
-    work = torch.empty(((T // 64 + int(n_seqs)) * H, 64 * (2 * D + V + 65)), dtype=torch.float32, device=qn.device)
-    _call("recurrent", "fx_head_delta_chunks", _stream(), _p(qn), _p(kn), _p(decay), _p(beta), _p(v), v.stride(0), _p(out),
-          out.stride(0), _p(state), _p(_i32(seq_starts, "seq_starts")), _p(_i32(slot_ids, "slot_ids")), int(n_seqs), int(longest),
-          H, G, D, V, _p(work))
     return out
 
 

@@ -138,8 +138,7 @@ class ChannelDelta(Mixer):
 class HeadDelta(ChannelDelta):
     """The gated delta rule with one decay per head (W_a: [heads, hidden], dt_bias: [heads]) and an output gate
     silu(W_g h) of full rank (W_g: [heads * v_dim, hidden]).  State, convolution, unit vectors, step sizes and the
-    recurrence are `channel_delta`'s.  Short portions go through its kernels too (the decay of a head is handed to all its key channels),
-    long ones by chunks of 64 tokens."""
+    recurrence are `channel_delta`'s, through the same kernels: the decay of a head is handed to all its key channels."""
     TENSORS = {"q": "q", "k": "k", "v": "v", "q_conv": "q.conv", "k_conv": "k.conv", "v_conv": "v.conv", "beta": "b",
                "A_log": "A_log", "dt_bias": "dt_bias", "decay": "a", "gate": "g", "norm": "norm", "o": "o"}
 
@@ -184,17 +183,11 @@ class HeadDelta(ChannelDelta):
         debug.region("delta conv")
         conv = ops.short_conv(proj[:, :C], self.taps, cache.state["conv"], ctx.token_seq, starts, ctx.slot_ids, ctx.n_seqs)
         debug.region("delta gates")
-        longest = longest_portion(ctx)
-        chunks = ops.can_head_delta_chunks(longest, D, V)
         qn, kn, decay, beta, kq = ops.delta_prepare(conv[:, :QK], conv[:, QK:2 * QK], proj[:, o1:o2], proj[:, C:o1], self.A_log,
-                                                    self.dt_bias, H, G, D, per_head=True, compact=chunks)
+                                                    self.dt_bias, H, G, D, per_head=True)
         debug.region("delta rule")
-        if chunks:
-            o = ops.head_delta_chunks(qn, kn, decay, beta, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
-                                      longest, H, G, D, V)
-        else:
-            o = ops.channel_delta(qn, kn, decay, beta, kq, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
-                                  H, G, D, V)
+        o = ops.channel_delta(qn, kn, decay, beta, kq, conv[:, 2 * QK:], cache.state["S"], starts, ctx.slot_ids, ctx.n_seqs,
+                              H, G, D, V)
         debug.region("delta out")
         y = ops.gated_head_norm(o, proj[:, o2:o2 + self.v_width], self.norm_w, self.norm_eps, H, V, ctx.act_dtype,
                                 gate_activation=self.gate_activation)

@@ -313,35 +313,20 @@ def test_latents_of_256_numbers_in_items_of_128_queries(nh, nkv, vd, bs, window,
     assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
 
 
-@pytest.mark.parametrize("H,G,D,V,lens", [(2, 1, 64, 16, [1]), (4, 2, 64, 48, [63, 64, 65, 1]), (2, 2, 128, 32, [128, 3, 200]),
-                                          (9, 3, 128, 16, [257])])
-def test_delta_rule_by_chunks_against_the_recurrence(H, G, D, V, lens):
-    """Portions around whole chunks of 64 tokens, from and into slots in another order, a token that forgets everything,
-    heads that do not divide among eight: outputs and states of the token-by-token kernel up to the roundings of sums of at
-    most 64 + 128 terms, and in two portions what one gives."""
-    from ferrox_amd import ops
-    T, n = sum(lens), len(lens)
-    gen = torch.Generator().manual_seed(T)
-    rand = lambda *shape: torch.randn(*shape, generator=gen).cuda()
-    unit = lambda x: torch.nn.functional.normalize(x, dim=-1)
-    qn, kn = unit(rand(T, G, D)).reshape(T, -1) * D ** -0.5, unit(rand(T, G, D)).reshape(T, -1).contiguous()
-    qn = qn.contiguous()
-    decay, beta, v = torch.exp(-0.3 * torch.rand(T, H, generator=gen)).cuda(), torch.sigmoid(rand(T, H)), rand(T, H * V + 3)[:, :H * V]
-    decay[T // 2] = 0.0
-    kq = (qn.view(T, G, D) * kn.view(T, G, D)).sum(-1).contiguous()
-    slots = torch.arange(n, dtype=torch.int32).flip(0).contiguous().cuda()
-    starts = lambda ls: torch.tensor([0] + torch.tensor(ls).cumsum(0).tolist(), dtype=torch.int32).cuda()
-    first = rand(n, H, V, D)
-    wide = decay[:, :, None].expand(T, H, D).reshape(T, H * D).contiguous()
-    s1, s2, s3 = first.clone(), first.clone(), first.clone()
-    want = ops.channel_delta(qn, kn, wide, beta, kq, v, s1, starts(lens), slots, n, H, G, D, V)
-    got = ops.head_delta_chunks(qn, kn, decay, beta, v, s2, starts(lens), slots, n, max(lens), H, G, D, V)
-    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5) and torch.allclose(s2, s1, rtol=1e-5, atol=1e-5)
-    if n == 1 and T > 100:
-        cut = lambda x, a, b: x[a:b].contiguous()
-        parts = [ops.head_delta_chunks(cut(qn, a, b), cut(kn, a, b), cut(decay, a, b), cut(beta, a, b), v[a:b], s3, starts([b - a]),
-                                       slots, 1, b - a, H, G, D, V) for a, b in ((0, 100), (100, T))]
-        assert torch.allclose(torch.cat(parts), want, rtol=1e-5, atol=1e-5) and torch.allclose(s3, s1, rtol=1e-5, atol=1e-5)
+def test_a_delta_rule_does_not_depend_on_neighbours_or_cuts(tmp_path_factory):
+    """float32: a request that decodes has the same bits alone and beside a portion of 300 tokens, and the portion the
+    same bits whole and in two, at head sizes of the named shape: the recurrence knows nothing of a step's other
+    sequences.  Kept states included (the tokens after the mixed step read them)."""
+    cfg = u.config([u.parallel_layer(heads=2, kv_heads=1, dim=16, window=0, r_heads=2, r_kv_heads=1, r_dim=64, r_vdim=32, conv=4, mlp=u.dense(32))])
+    _, model = model_for(tmp_path_factory, "neighbours", cfg, 31, "float32")
+    reqs = {"d": u.random_tokens(cfg["vocab"], 9, 1), "p": u.random_tokens(cfg["vocab"], 300, 2)}
+    before, after = [[("d", 6)]], [[("d", 1)]] * 2
+    run = lambda sched: u.run_schedule(runner_of(model), reqs, sched)[0]
+    alone = run(before + [[("d", 1)]] + after + [[("p", 300)]])
+    beside = run(before + [[("d", 1), ("p", 300)]] + after)
+    cut = run(before + [[("d", 1), ("p", 100)], [("p", 200)]] + after)
+    for r in reqs:
+        assert torch.equal(beside[r], alone[r]) and torch.equal(cut[r], alone[r]), r
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

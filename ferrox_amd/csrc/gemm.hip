@@ -1776,10 +1776,14 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     // (where the tiled kernel is the register-staged one, K no multiple of 64: up to 256 rows and 32 tiles of 128 x 128)
     const bool few_tiles = !expert_offsets && !pair_ids && M > 64 && !g_wide_force &&
                            (wide_ok ? M <= 128 && ceil_div(N, 128) <= 16 : M <= 256 && (long)ceil_div(N, 128) * ceil_div(M, 128) <= 32);
-    // More rows against very few weight rows (a low-rank projection, a router): tiles leave most CUs idle
-    // through the whole chain of K steps, the product for few rows covers them (2,048 rows of K = 2,048 against 64 weight
-    // rows: 9 against 13 us; 512 rows against 512 11.3 against 12.5, 768 rows 18.8 against 12.7)
-    const bool narrow = !expert_offsets && !pair_ids && M > (wide_ok ? 128 : 256) && (long)M * N <= (wide_ok ? 262144 : 524288) && !g_wide_force;
+    // More rows against very few weight rows (a low-rank projection): tiles leave most CUs idle through the whole chain of K
+    // steps, the product for few rows covers them while its blocks are one round of the CUs (K = 2,048: 1,024 rows against
+    // 256 weight rows 11.2 against 12.4 us, 512 against 512 the same, 1,337 against 256 18.5 against 12.5, 768 against 512 18.7 against
+    // 12.5; K = 3,584: 2,048 rows against 128 weight rows 16.9 against 18.1, 1,337 against 256 29.2 against 18.2).
+    // A router's logits (float32, up to 128 outputs) stay with it up to twice as many outputs, 4,096 tokens and 65 rows of 3,584 k
+    // 33 against 18.6 us beside the shared expert: which experts a token takes must not move with the tiles.
+    const bool router = epi == EPI_STORE_F32 && N <= 128;
+    const bool narrow = !expert_offsets && !pair_ids && M > (wide_ok ? 128 : 256) && (long)M * N <= (wide_ok && !router ? 262144 : 524288) && !g_wide_force;
     // 33 to 64 plain rows of a wide gate/up product: the product for few rows fetches every row's operands in every block,
     // tiles of 64 rows bring them to LDS once (gate/up of 11,264 x 2,048, 64 rows 27.5 -> 19 us, of 40,960 x 3,584 125 -> 70).
     // (Stored products of so many rows keep the bits of the one that rotates in its epilogue.)

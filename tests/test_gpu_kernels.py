@@ -185,6 +185,17 @@ def test_plain_products_have_the_same_bits_in_every_tile(M, N):
                 assert torch.equal(ops.gemm(a, w[:N // 2 * 2], epilogue=ops.EPI_GATED), gated), tile
 
 
+@pytest.mark.parametrize("T,E", [(2048, 65), (4096, 65), (4096, 128), (8065, 65)])
+def test_a_routers_logits_keep_their_order_of_sums(T, E):
+    """Up to 524,288 logits come from the product for few rows, whose bits decide between experts that stand close."""
+    from ferrox_amd import debug, ops
+    a, w = rnd(T, 1024, dtype=torch.bfloat16), rnd(E, 1024, dtype=torch.bfloat16, seed=1)
+    got = ops.gemm(a, w, epilogue=ops.EPI_STORE_F32)
+    with debug.kernel_switch("gemm", "plain_rows", T):
+        assert torch.equal(got, ops.gemm(a, w, epilogue=ops.EPI_STORE_F32))
+    close(got, a.double() @ w.double().T, torch.bfloat16, "logits")
+
+
 @pytest.mark.parametrize("tile", [12, 256, 4])
 def test_grouped_gemm_tiles_agree(tile):
     """An expert's rows in tiles of 192 (weights three steps deep), of 256 and of 64 (weights four steps deep) give

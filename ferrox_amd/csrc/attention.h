@@ -6,7 +6,8 @@ extern "C" {
 #endif
 
 // Queries in blocks: item i covers item_n[i] <= tile_q consecutive tokens of one sequence.  tile_q is 64, or 128
-// where fx_attn_tile_queries says so (bfloat16, head_dim 64 or 128, pages of a multiple of 64 keys).
+// where fx_attn_tile_queries says so (bfloat16, head_dim 64, 128 or 256, pages of a multiple of 64 keys; value heads of
+// another size only beside key heads of 256).
 int fx_attn_tile_queries(int dtype, int hd, int bs);
 int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void* out, long ldo, const void* k_pages,
                   const void* v_pages, const int* block_table, int max_blocks, const int* positions, const int* item_seq,

@@ -382,8 +382,11 @@ class PagedAttention(Mixer):
         tiles; so: items of 64 while they number no more than the CUs; else items of 128 if those do (a 2,048-token
         portion deep in a prompt: 603 against 784 us at 16 heads); else items of 128 if they still number about
         one evenly loaded block per CU (blocks of a portion that starts a prompt differ in work up to the portion's
-        length in keys and count by their mean share of the longest; +8-26 % from 448 such blocks on); else 64."""
-        if ctx.recorded or self.v_dim != self.head_dim or \
+        length in keys and count by their mean share of the longest; +8-26 % from 448 such blocks on); else 64.
+        Measured with heads of 64 and 128.  Heads of 256 take items of 64: their block of 128 queries is alone on its CU
+        and has no second group of waves, so none of the above holds for it (latents, one key head for all, have a
+        rule of their own)."""
+        if ctx.recorded or self.v_dim != self.head_dim or self.head_dim > 128 or \
                 (self.distance_bias is not None and self.distance_bias.shape[1] > ops.BIAS_ROW_MAX):
             # (the kernels for unequal head sizes, and for rows of biases that LDS does not hold, take items of 64)
             return 64

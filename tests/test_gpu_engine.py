@@ -606,6 +606,17 @@ def test_how_many_queries_an_item_of_a_prompt_portion_takes(model_folders):
     assert ask([(4096, 0)], bs=16) == 64
 
 
+@pytest.mark.parametrize("hd,want", [(64, 128), (128, 128), (256, 64)])
+def test_ordinary_heads_of_256_take_items_of_64_queries(hd, want):
+    """The rule is for heads whose items of 128 were measured against items of 64."""
+    from types import SimpleNamespace as NS
+    from ferrox_amd.parts.attention import PagedAttention
+    from ferrox_amd.parts.base import PartSpec
+    att = PagedAttention(256, 16, 1, hd, False, PartSpec("none", {}))
+    ctx = NS(recorded=False, n_seqs=1, q_starts=[0, 2048], kv_lens=[4096], device=torch.device("cuda:0"))
+    assert att.tile_queries(ctx, torch.bfloat16, 64) == want
+
+
 def test_recorded_decode_steps_equal_launched_ones(model_folders):
     """bfloat16 decode steps replayed from a HIP graph, several times with other work between the
     replays, against the same steps launched kernel by kernel (the bound on the sequence length

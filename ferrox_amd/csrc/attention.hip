@@ -415,9 +415,11 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(AttnArgs a) {
 // Merges the chunks' partial results in ascending order.  One block per (token, head): first
 // the weights exp(m_s - m) / sum of all chunks (kept in LDS), then every thread sums its head
 // dimensions over the chunks with several loads in flight.
+#define MERGE_KEPT 8192        // weights that LDS holds
+#define MERGE_MOST 16384       // chunks that are merged: two million keys by 128
 template <typename T>
 __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
-    extern __shared__ float wsm[];   // splits weights
+    extern __shared__ float wsm[];   // the weights of up to MERGE_KEPT chunks
     __shared__ float red[2];
     const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const int tok = a.item_tok[item];
@@ -436,13 +438,20 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
     if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
     m = fmaxf(red[0], red[1]);
-    for (int s = tid; s < S; s += 128) {
+    // (chunks beyond those that LDS holds: their weights are worked out where they are used, the same numbers)
+    auto weight_of = [&](int s) {
         const float ms = pml[2 * s];
-        wsm[s] = (ms == NEG_INF) ? 0.f : expf(ms - m);
-    }
+        return (ms == NEG_INF) ? 0.f : expf(ms - m);
+    };
+    const int kept = min(S, MERGE_KEPT);
+    for (int s = tid; s < kept; s += 128) wsm[s] = weight_of(s);
     __syncthreads();
     float l = 0.f;
-    for (int s = 0; s < S; ++s) l += wsm[s] * ((wsm[s] > 0.f) ? pml[2 * s + 1] : 0.f);   // ascending, the same in every thread
+    for (int s = 0; s < kept; ++s) l += wsm[s] * ((wsm[s] > 0.f) ? pml[2 * s + 1] : 0.f);   // ascending, the same in every thread
+    for (int s = kept; s < S; ++s) {
+        const float w = weight_of(s);
+        l += w * ((w > 0.f) ? pml[2 * s + 1] : 0.f);
+    }
     const float fin = finish_row<false>(a, h, m, l);
     for (int d = tid; d < hd; d += 128) {
         float acc = 0.f;
@@ -456,10 +465,14 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
             s0 = min(S, EARLY);
         }
 #pragma unroll 8
-        for (int s = s0; s < S; ++s) {
+        for (int s = s0; s < kept; ++s) {
             const float w = wsm[s];
             const float v = (w > 0.f) ? po[(size_t)s * hd + d] : 0.f;   // an empty chunk wrote nothing
             acc = fmaf(w, v, acc);
+        }
+        for (int s = kept; s < S; ++s) {
+            const float w = weight_of(s);
+            acc = fmaf(w, (w > 0.f) ? po[(size_t)s * hd + d] : 0.f, acc);
         }
         store_lane<T>(a, tok, h, d, acc * fin);
     }
@@ -1838,6 +1851,7 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
     a.part_o = part_o; a.part_ml = part_ml; a.splits = splits; a.chunk = chunk;
     dim3 grid(n_items, nh, splits), grid2(n_items, nh);
     hipStream_t s = (hipStream_t)stream;
+    const size_t merge_lds = (splits < MERGE_KEPT ? splits : MERGE_KEPT) * sizeof(float);
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
     if (dtype == FX_F32) {
         if (f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
@@ -1847,10 +1861,10 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
             else attn_f32_decode_kernel<256><<<gridf, 64, 0, s>>>(a);
         } else if (beyond) attn_decode_kernel<float, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
         else attn_decode_kernel<float><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<float><<<grid2, 128, splits * sizeof(float), s>>>(a);
+        attn_decode_merge_kernel<float><<<grid2, 128, merge_lds, s>>>(a);
     } else if (beyond) {
         attn_decode_kernel<bf16, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<bf16><<<grid2, 128, splits * sizeof(float), s>>>(a);
+        attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
     } else if (mfma_ok(dtype, hd, bs, q, ldq, k_pages, v_pages, vd)) {
         const int group = nh / nkv;
         dim3 gridm(nkv * ((group + 15) / 16), n_items, splits);
@@ -1880,10 +1894,10 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
             else if (hd <= 128) attn_mfma_decode_block_kernel<128, 512, SH><<<gridm, nw * 64, shm, s>>>(a);
             else attn_mfma_decode_block_kernel<256, 256, SH><<<gridm, nw * 64, shm, s>>>(a);
         });
-        if (splits > 1) attn_decode_merge_kernel<bf16><<<grid2, 128, splits * sizeof(float), s>>>(a);
+        if (splits > 1) attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
     } else {
         attn_decode_kernel<bf16><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<bf16><<<grid2, 128, splits * sizeof(float), s>>>(a);
+        attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
     }
     FX_CHECK_LAUNCH("attn_decode");
     return 0;
@@ -1892,7 +1906,7 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
 static int attn_decode_check(int dtype, int nh, int nkv, int hd, int bs, int window, float scale, int splits, int chunk) {
     if (check_common("attn_decode", dtype, nh, nkv, hd, bs, window, scale)) return 1;
     FX_REQUIRE(splits > 0 && chunk > 0 && chunk % 64 == 0, "attn_decode: chunk %d must be a positive multiple of 64", chunk);
-    FX_REQUIRE(splits <= 8192, "attn_decode: %d chunks are more than the merge kernel takes (8192)", splits);
+    FX_REQUIRE(splits <= MERGE_MOST, "attn_decode: %d chunks are more than the merge kernel takes (%d)", splits, MERGE_MOST);
     return 0;
 }
 

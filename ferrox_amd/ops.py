@@ -980,8 +980,7 @@ def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq,
     _check_attention_extras(out, n_heads, 1 if gate_per_head else v_dim, window, keep_first, sinks, gate, softcap, slopes, distance_bias)
     _check_turns(turns, q.shape[0], v_dim, "attention")
     if chunk is None:
-        # (longer than the merge's 8,192 chunks of 128 reach: 256)
-        chunk = 128 if q.dtype == torch.float32 and max_kv_len <= 128 * 8192 else 256
+        chunk = 128 if q.dtype == torch.float32 else 256
         if q.dtype == torch.bfloat16:
             chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device))
     splits = max(1, -(-max_kv_len // chunk))

@@ -776,6 +776,30 @@ def test_float32_attention_on_the_matrix_units_against_the_kernels_for_any_shape
         assert torch.allclose(a, b, rtol=2e-5, atol=2e-5), float((a - b).abs().max())
 
 
+@pytest.mark.parametrize("bs", [8, 7])
+@pytest.mark.parametrize("longest", [128 * 8192, 128 * 8192 + 1, 128 * 16384])
+def test_float32_single_queries_beside_a_very_long_sequence(bs, longest):
+    """The chunks of a float32 sequence, hence its bits, do not depend on the longest sequence that a launch is told of: up to
+    the most chunks that are merged, of which LDS holds the weights of 8,192.  (bs 8: the matrix units; 7: any shape)"""
+    from ferrox_amd import ops
+    nh, hd, n = 2, 16, 700
+    q, k, v = rnd(1, nh * hd), rnd(n, 1, hd, seed=1), rnd(n, 1, hd, seed=2)
+    blocks = -(-n // bs)
+    kp, vp = torch.zeros(blocks, 1, bs, hd, device=DEV), torch.zeros(blocks, 1, hd, bs, device=DEV)
+    for t in range(blocks):
+        rows = slice(t * bs, min((t + 1) * bs, n))
+        kp[t, 0, :rows.stop - rows.start], vp[t, 0, :, :rows.stop - rows.start] = k[rows, 0], v[rows, 0].T
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table, out = i32([list(range(blocks))]), []
+    for bound in (n, longest):
+        y = torch.zeros(1, nh * hd, device=DEV)
+        ops.attention_decode(q, y, kp, vp, table, i32([n - 1]), i32([0]), i32([0]), nh, 1, hd, bs, 0, hd ** -0.5, max_kv_len=bound)
+        out.append(y)
+    assert torch.equal(out[0], out[1])
+    with pytest.raises(ops.KernelError):
+        ops.attention_decode(q, y, kp, vp, table, i32([n - 1]), i32([0]), i32([0]), nh, 1, hd, bs, 0, hd ** -0.5, max_kv_len=128 * 16384 + 1)
+
+
 @pytest.mark.parametrize("hd,bs,window", [(64, 16, 0), (64, 64, 0), (128, 64, 40000), (32, 16, 9000)])
 def test_attention_over_more_pages_than_a_block_copies(hd, bs, window):
     """A sequence of more than 1024 pages (the kernels copy that many page ids into LDS and read the rest of

@@ -12,6 +12,7 @@ the step, by whoever schedules it.
 from __future__ import annotations
 
 import gc
+import sys
 
 from dataclasses import dataclass, field
 
@@ -38,10 +39,14 @@ class DecodeGraph:
     int32 device buffer at a fixed address that is refreshed before each replay; everything a
     kernel launch depends on beside that (number of sequences, width of the block tables, the
     bound on the sequence lengths that sets the number of attention splits) is fixed per graph.
+
+    It does not hold its runner: a runner that is dropped lets go of its recorded steps there and then, not whenever
+    the cycle collector finds them.  Whoever drops a recorded step, it waits for the device before its memory goes: steps
+    are launched ahead of their results.
     """
 
     def __init__(self, runner, n_seqs: int, kv_bound: int):
-        self.runner, self.n, self.kv_bound = runner, n_seqs, kv_bound
+        self.n, self.kv_bound = n_seqs, kv_bound
         mgr = runner.manager
         self.max_blocks = max(1, mgr.blocks_for(kv_bound))
         self.keys = list(mgr.groups)
@@ -58,33 +63,39 @@ class DecodeGraph:
         self.logits = None
         self.trace_calls = None        # where an active routing trace's copies went while this step was recorded
 
-    def _context(self) -> StepContext:
+    def __del__(self):
+        graph = getattr(self, "graph", None)
+        if graph is not None and not sys.is_finalizing():
+            torch.cuda.synchronize(self.meta.device)
+            graph.reset()
+
+    def _context(self, runner) -> StepContext:
         n, mb, m = self.n, self.max_blocks, self.meta
         tables, o = {}, 5 * n
         for key in self.keys:
             tables[key] = m[o:o + n * mb].view(n, mb)
             o += n * mb
-        ctx = StepContext(n_tokens=n, n_seqs=n, act_dtype=self.runner.act_dtype, device=self.runner.device,
+        ctx = StepContext(n_tokens=n, n_seqs=n, act_dtype=runner.act_dtype, device=runner.device,
                           token_ids=m[0:n], positions=m[n:2 * n], token_seq=m[2 * n:3 * n],
                           q_starts=list(range(n + 1)), kv_lens=[self.kv_bound] * n, slot_ids=m[3 * n:4 * n],
-                          slots=None, block_tables=tables, block_size=self.runner.block_size,
+                          slots=None, block_tables=tables, block_size=runner.block_size,
                           logit_rows=m[4 * n:5 * n], recorded=True, kv_bound=self.kv_bound)
         return ctx
 
-    def run(self, entries, feed=None) -> torch.Tensor:
+    def run(self, runner, entries, feed=None) -> torch.Tensor:
         """The logits of the entries' tokens (one each).  Fewer entries than the step was recorded for are
-        filled up with stand-in rows, which write to a page and a slot that no request owns.  `feed` as in
-        `ModelRunner.step`."""
+        filled up with stand-in rows, which write to a page and a slot that no request owns.  `runner`: the one it was
+        made for.  `feed` as in `ModelRunner.step`."""
         self.copied.synchronize()                  # the last upload has left the staging buffer
         for e in entries:
             if e.want[0] != 0:
                 raise ValueError(f"request {e.req!r}: wanted place {e.want[0]} is outside its one token")
-        storage = self.runner.storage
-        self.runner.manager.pack_decode([e.req for e in entries], [e.tokens[0] for e in entries], self.runner.vocab_size,
-                                        self._host_ptr, self._host_words, self.max_blocks, pad_to=self.n,
-                                        pad_pages=storage.pad_pages, pad_slot=storage.pad_slot)
-        if self.runner.before_launch is not None:
-            self.runner.before_launch()
+        storage = runner.storage
+        runner.manager.pack_decode([e.req for e in entries], [e.tokens[0] for e in entries], runner.vocab_size,
+                                   self._host_ptr, self._host_words, self.max_blocks, pad_to=self.n,
+                                   pad_pages=storage.pad_pages, pad_slot=storage.pad_slot)
+        if runner.before_launch is not None:
+            runner.before_launch()
         words = self._host_words
         if feed:
             ids, pairs = feed
@@ -96,12 +107,12 @@ class DecodeGraph:
         else:
             self.meta[:words].copy_(self.host[:words], non_blocking=True)
         self.copied.record()
-        model, caches = self.runner.model, self.runner.storage.caches
+        model, caches = runner.model, runner.storage.caches
         if self.graph is None:
             # This step runs eagerly (which also loads the kernels), then the same launches are recorded for the
             # steps to come.  Recording executes nothing, and the recorded step is not replayed now: a mixer that
             # carries state from token to token must see every token once.
-            first = model.forward(self._context(), caches)
+            first = model.forward(self._context(runner), caches)
             torch.cuda.synchronize()
             graph = torch.cuda.CUDAGraph()
             # no garbage collection while the stream is recording: a tensor of an earlier step that is freed
@@ -113,13 +124,13 @@ class DecodeGraph:
             # (capture_begin / capture_end on a stream of its own rather than `with torch.cuda.graph(...)`: that
             # context manager also gives the allocator's cached memory back to the driver first, which with tens of
             # GB in the cache costs a recording several hundred milliseconds)
-            main, side = torch.cuda.current_stream(), self.runner.capture_stream
+            main, side = torch.cuda.current_stream(), runner.capture_stream
             side.wait_stream(main)
             try:
                 with torch.cuda.stream(side):
                     graph.capture_begin()
                     try:
-                        self.logits = model.forward(self._context(), caches)
+                        self.logits = model.forward(self._context(runner), caches)
                     finally:
                         graph.capture_end()
             finally:
@@ -221,13 +232,11 @@ class ModelRunner:
                 self._graphs[key] = self._graphs.pop(key)          # kept in the order of last use
             else:
                 if len(self._graphs) >= 32:
-                    # the step that goes is the one unused for longest; the device may still be running it (steps
-                    # are launched ahead of their results), and its memory goes with it
-                    torch.cuda.current_stream(self.device).synchronize()
+                    # the step that goes is the one unused for longest
                     self._graphs.pop(next(iter(self._graphs)))
                 self._graphs[key] = DecodeGraph(self, n_rec, bound)
             try:
-                logits = self._graphs[key].run(entries, feed)
+                logits = self._graphs[key].run(self, entries, feed)
             except RuntimeError as err:
                 # recording is an optimisation of how kernels are launched, not another code path:
                 # if the runtime refuses it, the same kernels are launched one by one from here on

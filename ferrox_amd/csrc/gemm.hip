@@ -1657,6 +1657,18 @@ FX_API int fx_qkv_rope(void* stream, const void* A, long lda, const void* W, lon
     return 0;
 }
 
+// ---- decisions by sizes that are plain arithmetic (the compute units are an argument: they can be asked for without a GPU) ----
+// 33 to 128 plain rows against so few weight rows that blocks of several row tiles are a fraction of the CUs (a router of 61
+// rows as the rows, the step's tokens as the weights): whether a block takes one row tile and one set of weight rows.  Up to 64 rows,
+// where the other way is four row tiles a block, while such blocks are at most one and a quarter a CU (2,048 k, 61 rows: 1,024
+// weight rows 7.4 against 12.3 us, 1,280 10.2 against 12.2); beyond, where it is two, at most one a CU (96 rows: 640 weight rows 7.2 against
+// 8.6 us, 768 10.4 against 8.8; 4,096 k 10.9 against 14.1 and 17.6 against 14.4).  (2,048 tokens with two row tiles a block instead of four
+// took 10.6 instead of 14.9 us, but the step, whose routing runs beside the shared expert, 0.5 % longer.)
+FX_API int fx_gemm_row_tile_blocks(int M, int N, int cus) {
+    const long blocks = (long)ceil_div(N, 16) * ceil_div(M, 16);
+    return M > 32 && M <= 128 && (M <= 64 ? 4 * blocks <= 5L * cus : blocks <= cus);
+}
+
 // dtype: type of A and W.  C is: T for EPI_STORE and EPI_GATED, float32 otherwise.
 // rows_hint: in grouped mode, the expected number of rows per expert (chooses the tile).
 FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, const void* W, long w_stride,
@@ -1804,12 +1816,8 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // rows the four row tiles a block stay ahead, 17.3 against 20.1 us)
         const bool spread_rows = mt == 4 && !expert_offsets && !norm_w && epi == EPI_RESID && ceil_div(N, 16) * (long)ceil_div(M, 64) < 192;
         if (spread_rows) mt = 1;
-        // 33 to 128 plain rows against so few weight rows that blocks of several row tiles are a fraction of the CUs (a
-        // router of 61 rows as the rows, the step's tokens as the weights): a block per row tile while they stay about one a CU
-        // (2,048 k, 512 tokens 16.8 -> 10.4 us in a step; 3,584 k, 65 rows, 512 tokens 13.0 -> 9.7).  Two row tiles a block for 2,048
-        // tokens took 10.6 instead of 14.9 us, but the step, whose routing runs beside the shared expert, 0.5 % longer.
-        const bool row_tile_blocks = !expert_offsets && !pair_ids && !norm_w && (epi == EPI_STORE || epi == EPI_STORE_F32) && M > 32 &&
-                                     M <= 128 && mt > 1 && 4L * ceil_div(N, 16) * ceil_div(M, 16) <= 5L * fx_compute_units();
+        const bool row_tile_blocks = !expert_offsets && !pair_ids && !norm_w && (epi == EPI_STORE || epi == EPI_STORE_F32) && mt > 1 &&
+                                     fx_gemm_row_tile_blocks(M, N, fx_compute_units());
         if (row_tile_blocks) mt = 1;
         if (g_skinny_mt && !pair_ids) mt = g_skinny_mt;
         const int m_tiles = pair_ids ? (M < E ? M : E) + M / 16 + n_always

@@ -31,6 +31,16 @@ def test_decode_attention_chunks_fill_the_gpu_and_avoid_partial_rounds():
     assert splits(8, 16, 16, 2560, cus=128) == 1 and splits(12, 16, 16, 2560, cus=128) == 8
 
 
+def test_a_block_per_row_tile_while_such_blocks_are_one_a_cu():
+    """The product of 33 to 128 plain rows: beyond 64 rows a second round of blocks is behind two row tiles a block."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, n, cus=256: bool(load_library("gemm").fx_gemm_row_tile_blocks(m, n, cus))
+    assert not rule(32, 64) and rule(33, 64) and rule(128, 64) and not rule(129, 64)
+    assert rule(61, 1280) and not rule(61, 1296) and rule(40, 1696)
+    assert rule(96, 672) and not rule(96, 688) and not rule(96, 768) and rule(128, 512) and not rule(128, 528)
+    assert rule(128, 1024, cus=512) and not rule(128, 512, cus=128)
+
+
 def test_the_chunk_rule_leaves_the_callers_arguments_alone():
     """The rule counts waves per block; it once did so in a variable named like the `waves` argument of
     `attention_decode`, which then reached the launch instead of the caller's value."""

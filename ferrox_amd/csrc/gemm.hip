@@ -14,7 +14,6 @@
 // Dual mode: two weight matrices (gate, up) are multiplied at once and the
 // epilogue stores silu(gate) * up  (ferrox-moe/src/lib.rs:655-658).
 #include "common.h"
-#include <climits>
 #include <type_traits>
 #include <utility>
 
@@ -1669,6 +1668,62 @@ FX_API int fx_gemm_row_tile_blocks(int M, int N, int cus) {
     return M > 32 && M <= 128 && (M <= 64 ? 4 * blocks <= 5L * cus : blocks <= cus);
 }
 
+// The tile of the LDS-tiled kernel for plain rows, as the debug switch "wide" names them; all give the same bits.  `dual`: N
+// columns of two matrices.
+FX_API int fx_gemm_plain_tile(int M, int N, int K, int dual, int cus) {
+    auto tiles = [&](int tm, int tn) { return (long)ceil_div(N, dual ? tn / 2 : tn) * ceil_div(M, tm); };
+    // Fewer tiles of 128 x 128 than CUs: a block's chain of K steps takes the same 23-25 us (2,048 k) whatever the rows, so
+    // smaller tiles on more CUs: 64 x 64 while they are one a CU (2,048 x 2,048 weights, 512 rows 23 -> 13 us; 5,632 k 55 -> 29;
+    // 6,144 weight rows, 128 rows 25 -> 14), then 64 x 128 (6,144 weight rows, 256 rows 25 -> 19; 2,048 x 5,632, 1,024 rows 56 -> 41).
+    if (!dual && tiles(64, 64) <= cus) return 464;
+    if (tiles(64, 128) <= cus) return 4128;
+    // One round of 128 x 128 in two stages, two blocks to a CU, whether half or all of it is there (2,048 k: 6,144 weight rows, 768 to
+    // 1,280 rows 43 -> 34-36 us, gate/up of 11,264, 384 and 640 rows 40 -> 35 and 48 -> 38, 2,048 weight rows, 2,432 and 4,096 rows 49
+    // -> 38 and 49 -> 42; 8,192 k: 3-24 % less).  But beyond 14,336 rows (of at most 512 weight rows then) of long K the
+    // tiles of 256 x 128 read the rows fewer times (16,384 rows: 4,096 k 79 against 86 us, 5,632 k 104 against 117; 3,584 k 67 and 66).
+    const long t128 = tiles(128, 128);
+    if (t128 > cus && t128 <= 2L * cus && (M <= 14336 || K < 4096)) return 8128;
+    // More: the widest tile that still gives the CUs (one block each) an even share of the work; a tile's score is the share of
+    // its rounds that is there, of its rows that exist, and what it reaches when full.  Tiles of 192 x 256 where they divide the work more
+    // evenly (2,048 rows against 11,264 weight rows: 484 tiles for two rounds of the 256 CUs instead of 352 tiles of 256 x 256).
+    auto score = [&](int tm, int tn, double quality) {
+        const long t = tiles(tm, tn);
+        const double rows = (double)M / (double)((long)ceil_div(M, tm) * tm);
+        return quality * rows * (double)t / (double)((t + cus - 1) / cus * cus);
+    };
+    const double s256 = score(256, 256, 1.0), s192 = dual ? 0.0 : score(256, 192, 0.92), s128 = score(256, 128, 0.85),
+                 s64 = score(128, 128, 0.7), s12 = score(192, 256, 0.92);
+    if (s12 > s256 && s12 > s192 && s12 > s128 && s12 > s64) return 12;
+    if (s192 > s256 && s192 >= s128 && s192 >= s64) return 192;
+    if (s256 >= s128 && s256 >= s64) return 256;
+    if (s128 >= s64) return 128;
+    // Where that is 128 x 128, several rounds of it run two blocks to a CU in two stages as well (6,144 weight rows, 2,688 rows
+    // 88 -> 71 us; gate/up of 11,264, 1,337 rows 91 -> 79).  (Not ahead of the other tiles in general: four rounds' worth of tiles of 128 x 128,
+    // 2,048 rows' gate/up of 8,192 73 against 67 us, 3,456 rows against 4,608 weight rows of 3,584 k 111 against 101.)
+    return t128 > cus ? 8128 : 64;
+}
+// The same for rows sorted by expert.
+static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, int cus) {
+    // an expert's share of up to 20 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
+    // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three, the same bits: decode
+    // at 64 sequences 11.2 -> 11.0 ms, a 192-token step 6.8 -> 6.4 ms; from 25 rows on average on, steps of 384
+    // tokens, more and more experts need a second tile and it falls behind)
+    if (per_group <= g_tile64_rows) return 4;
+    // a share of up to 192 rows: the product streams the weights once and multiplies little, so it
+    // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows
+    // (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of
+    // 256 do, 273 rows an expert as 2 x 192 instead of 2 x 256: the down product of a 4,096-token step 173
+    // against 190 us)
+    const long pad192 = ceil_div(per_group, 192) * 192L, pad256 = ceil_div(per_group, 256) * 256L;
+    if (per_group <= 176 || pad192 < pad256) return 12;
+    auto score = [&](int tm, int tn, double quality) {
+        const long t = (long)ceil_div(N, dual ? tn / 2 : tn) * (M / tm + nonempty);
+        return quality * (double)t / (double)((t + cus - 1) / cus * cus);
+    };
+    const double s256 = score(256, 256, 1.0), s128 = score(256, 128, 0.85), s64 = score(128, 128, 0.7);
+    return s256 >= s128 && s256 >= s64 ? 256 : (s128 >= s64 ? 128 : 64);
+}
+
 // dtype: type of A and W.  C is: T for EPI_STORE and EPI_GATED, float32 otherwise.
 // rows_hint: in grouped mode, the expected number of rows per expert (chooses the tile).
 FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, const void* W, long w_stride,
@@ -1847,70 +1902,26 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         const int m_tiles = M / 64 + (expert_offsets ? nonempty : (M % 64 != 0));
         launch_bf16<64, 64, 32, 32>(g, epi, m_tiles, s);
     } else if (g.vec_ok && K % 64 == 0 && !g_no_wide) {
-        // the widest tile that still gives the CUs (one block each) an even share of the work
         const bool dual = epi == EPI_GATED;
-        const long cus = fx_compute_units();
-        const int force = expert_offsets && g_wide_grouped ? g_wide_grouped : g_wide_force;
         // weights that are read about once (an expert's rows fit one row tile on average; plain rows: one row tile)
         // are loaded with the non-temporal hint
         g.stream_w = g_stream_w >= 0 ? g_stream_w : (expert_offsets ? per_group <= 128 : M <= 128);
-        auto tiles = [&](int tm, int tn) {
-            return (long)ceil_div(N, dual ? tn / 2 : tn) * (M / tm + (expert_offsets ? nonempty : (M % tm != 0)));
-        };
-        auto score = [&](int tm, int tn, double quality) {
-            const long t = tiles(tm, tn);
-            // plain rows: the share of a tile's rows that exist (an expert's missing row blocks are skipped)
-            const double rows = expert_offsets ? 1.0 : (double)M / (double)((long)ceil_div(M, tm) * tm);
-            return quality * rows * (double)t / (double)(ceil_div(t, cus) * cus);
-        };
-        double s256 = score(256, 256, 1.0), s192 = dual || expert_offsets ? 0.0 : score(256, 192, 0.92), s128 = score(256, 128, 0.85),
-               s64 = score(128, 128, 0.7);
-        if (force) {
-            s256 = force == 256; s192 = force == 192 && !dual; s128 = force == 128; s64 = 0.5 * (force == 64);
+        int tile = expert_offsets && g_wide_grouped ? g_wide_grouped : g_wide_force;
+        if (dual && (tile == 464 || tile == 192)) tile = 256;       // (no such tiles of two matrices)
+        if (!tile && !expert_offsets) tile = fx_gemm_plain_tile(M, N, K, dual, fx_compute_units());
+        else if (!tile) tile = small_groups ? 64 : grouped_tile(per_group, M, N, nonempty, dual, fx_compute_units());
+        auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
+        switch (tile) {
+            case 464: launch_wide<4, 64, 4>(g, epi, row_tiles(64), s); break;
+            case 4128: launch_wide<4, 128, 3>(g, epi, row_tiles(64), s); break;
+            case 8128: launch_wide<8, 128, 2>(g, epi, row_tiles(128), s); break;
+            case 4: launch_wide<4, 256, 4, 2>(g, epi, row_tiles(64), s); break;
+            case 12: launch_wide<12, 256, 3, 2>(g, epi, row_tiles(192), s); break;
+            case 192: launch_wide<16, 192, 2>(g, epi, row_tiles(256), s); break;
+            case 128: launch_wide<16, 128, 3>(g, epi, row_tiles(256), s); break;
+            case 64: launch_wide<8, 128, 4>(g, epi, row_tiles(128), s); break;
+            default: launch_wide<16, 256, 2>(g, epi, row_tiles(256), s); break;
         }
-        // an expert's share of up to 192 rows: the product streams the weights once and multiplies little, so it
-        // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows
-        // plain rows: tiles of 192 x 256 where they divide the work more evenly (2,048 rows against 11,264 weight
-        // rows: 484 tiles for two rounds of the 256 CUs instead of 352 tiles of 256 x 256)
-        const double s12 = expert_offsets ? 0.0 : score(192, 256, 0.92);
-        // (an expert's share beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of
-        // 256 do, 273 rows an expert as 2 x 192 instead of 2 x 256: the down product of a 4,096-token step 173
-        // against 190 us)
-        const long pad192 = ceil_div(per_group, 192) * 192L, pad256 = ceil_div(per_group, 256) * 256L;
-        const bool few_rows = force ? force == 12
-                                           : (expert_offsets ? (per_group <= 176 || pad192 < pad256)
-                                                             : (s12 > s256 && s12 > s192 && s12 > s128 && s12 > s64));
-        // an expert's share of up to 20 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
-        // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three, the same bits: decode
-        // at 64 sequences 11.2 -> 11.0 ms, a 192-token step 6.8 -> 6.4 ms; from 25 rows on average on, steps of 384
-        // tokens, more and more experts need a second tile and it falls behind)
-        // Plain rows whose tiles of 128 x 128 are fewer than the CUs: a block's chain of K steps takes the same 23-25 us (2,048
-        // k) whatever the rows, so smaller tiles on more CUs: 64 x 64 while they are one a CU (2,048 x 2,048 weights, 512 rows
-        // 23 -> 13 us; 5,632 k 55 -> 29; 6,144 weight rows, 128 rows 25 -> 14), then 64 x 128 (6,144 weight rows, 256 rows 25 ->
-        // 19; 2,048 x 5,632, 1,024 rows 56 -> 41).  Beyond that the larger tiles are ahead until 128 x 128 in two stages, two
-        // blocks to a CU, fill one round of them: 6,144 weight rows, 768 rows 40 -> 34 us; 4,608 x 3,584, 1,337 rows 61 -> 55;
-        // gate/up of 11,264, 384 rows 41 -> 35, 1,337 rows (two rounds, 95 % full) 94 -> 80.  The same bits in every tile.
-        const bool plain = !expert_offsets && !force;
-        const long t64 = dual ? LONG_MAX : (long)ceil_div(N, 64) * ceil_div(M, 64), t64w = tiles(64, 128), t128 = tiles(128, 128);
-        const bool small_square = plain && t64 <= cus, small_wide = plain && !small_square && t64w <= cus;
-        const bool two_a_cu = plain && ((t128 > cus && t128 <= 2 * cus) || (t128 > 3.72 * cus && t128 <= 4 * cus));
-        if (force == 464 ? !dual : small_square) launch_wide<4, 64, 4>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);
-        else if (force == 4128 || small_wide) launch_wide<4, 128, 3>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);
-        else if (force == 8128 || two_a_cu) launch_wide<8, 128, 2>(g, epi, M / 128 + (expert_offsets ? nonempty : (M % 128 != 0)), s);
-        else if (!force && small_groups)
-            launch_wide<8, 128, 4>(g, epi, M / 128 + nonempty, s);
-        else if (force == 4 || (!force && expert_offsets && per_group <= g_tile64_rows))
-            launch_wide<4, 256, 4, 2>(g, epi, M / 64 + (expert_offsets ? nonempty : (M % 64 != 0)), s);
-        else if (few_rows)
-            launch_wide<12, 256, 3, 2>(g, epi, M / 192 + (expert_offsets ? nonempty : (M % 192 != 0)), s);
-        else if (s192 > s256 && s192 >= s128 && s192 >= s64)
-            launch_wide<16, 192, 2>(g, epi, M / 256 + (expert_offsets ? nonempty : (M % 256 != 0)), s);
-        else if (s256 >= s128 && s256 >= s64)
-            launch_wide<16, 256, 2>(g, epi, M / 256 + (expert_offsets ? nonempty : (M % 256 != 0)), s);
-        else if (s128 >= s64)
-            launch_wide<16, 128, 3>(g, epi, M / 256 + (expert_offsets ? nonempty : (M % 256 != 0)), s);
-        else
-            launch_wide<8, 128, 4>(g, epi, M / 128 + (expert_offsets ? nonempty : (M % 128 != 0)), s);
     } else {
         const int m_tiles = M / 128 + (expert_offsets ? nonempty : (M % 128 != 0));
         const bool dual = epi == EPI_GATED;

@@ -41,6 +41,23 @@ def test_a_block_per_row_tile_while_such_blocks_are_one_a_cu():
     assert rule(128, 1024, cus=512) and not rule(128, 512, cus=128)
 
 
+def test_tiles_of_plain_products():
+    """One round of 128 x 128 tiles in two stages goes two to a CU; more rounds go to the tiles that share the work most
+    evenly, and to two stages only in place of 128 x 128 in four."""
+    from ferrox_amd.csrc.build import load_library
+    tile = lambda m, n, k=2048, dual=0, cus=256: load_library("gemm").fx_gemm_plain_tile(m, n, k, dual, cus)
+    assert tile(512, 2048) == 464 and tile(513, 2048) == 4128 and tile(1024, 2048) == 4128
+    assert tile(512, 2048, dual=1) == 4128                               # no 64 x 64 of two matrices
+    assert tile(768, 6144) == tile(1280, 6144) == tile(2432, 2048) == tile(4096, 2048) == 8128
+    assert tile(16384, 512) == tile(14336, 512, 8192) == 8128 and tile(16384, 512, 4096) == 128
+    # four rounds' worth of 128 x 128, nearly full
+    assert tile(2560, 6144) == tile(7680, 2048) == tile(8192, 2048) == 256
+    assert tile(3456, 4608, 3584) == tile(4480, 3584, 3584) == tile(2048, 4096, dual=1) == 256
+    assert tile(2688, 6144) == tile(1337, 5632, dual=1) == 8128
+    assert tile(2048, 5632, dual=1) == 12 and tile(4096, 6144) == 192
+    assert tile(4096, 2048, cus=128) == tile(8192, 2048)
+
+
 def test_the_chunk_rule_leaves_the_callers_arguments_alone():
     """The rule counts waves per block; it once did so in a variable named like the `waves` argument of
     `attention_decode`, which then reached the launch instead of the caller's value."""

@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void small_rows_pair_kernel(const float* __res
     for (int k = threadIdx.x; k < K; k += 256) xs[k] = x[(size_t)t * ldx + k];
     __syncthreads();
     if (n >= N) return;
-    out[(size_t)t * ldo + n] = f32_ordered_dot(K, [&](int k) { return xs[k]; }, [&](int k) { return wt[(size_t)k * N + n]; });
+    out[(size_t)t * ldo + n] = f32_ordered_dot(K, xs, wt + n, N);
 }
 
 FX_API int fx_small_rows_pair(void* stream, const float* x0, long ldx0, const float* wt0, float* out0, long ldo0, int K0, int N0,
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void small_rows_parts_kernel(const float* __re
     __syncthreads();
     if (n >= N) return;
     const float* w = wt + (size_t)j * K * N;
-    out[((size_t)t * parts + j) * N + n] = f32_ordered_dot(K, [&](int k) { return xs[k]; }, [&](int k) { return w[(size_t)k * N + n]; });
+    out[((size_t)t * parts + j) * N + n] = f32_ordered_dot(K, xs, w + n, N);
 }
 
 FX_API int fx_small_rows_parts(void* stream, const float* x, long ldx, const float* wt, float* out, int K, int N, int parts, int T) {

@@ -776,6 +776,31 @@ def test_float32_attention_on_the_matrix_units_against_the_kernels_for_any_shape
         assert torch.allclose(a, b, rtol=2e-5, atol=2e-5), float((a - b).abs().max())
 
 
+@pytest.mark.parametrize("hd", [20, 64, 80, 132])
+def test_a_float32_key_at_minus_infinity_is_not_attended_to(hd):
+    """A key whose last four numbers (the ones that stand in for numbers that a narrow head does not have) are minus infinity scores
+    minus infinity with positive queries: weight 0 beside finite scores, as in the kernels for any shape (pages of 7 keys)."""
+    from ferrox_amd import ops
+    nh, n, at = 2, 150, 40
+    q, k, v = rnd(n, nh * hd).abs() + 0.1, rnd(n, 1, hd, seed=1), rnd(n, 1, hd, seed=2)
+    k[at, 0, hd - 4:] = -float("inf")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    pos, got = torch.arange(n, dtype=torch.int32, device=DEV), {}
+    for bs in (8, 7):
+        blocks = -(-n // bs)
+        kp, vp = torch.zeros(blocks, 1, bs, hd, device=DEV), torch.zeros(blocks, 1, hd, bs, device=DEV)
+        for t in range(blocks):
+            rows = slice(t * bs, min((t + 1) * bs, n))
+            kp[t, 0, :rows.stop - rows.start], vp[t, 0, :, :rows.stop - rows.start] = k[rows, 0], v[rows, 0].T
+        table, args = i32([list(range(blocks))]), (nh, 1, hd, bs, 0, hd ** -0.5)
+        out, single = torch.zeros(n, nh * hd, device=DEV), torch.zeros(n, nh * hd, device=DEV)
+        ops.attention_tiles(q, out, kp, vp, table, pos, i32([0, 0, 0]), i32([0, 64, 128]), i32([64, 64, 22]), *args)
+        ops.attention_decode(q, single, kp, vp, table, pos, i32([0]), i32([n - 1]), *args, max_kv_len=n)
+        got[bs] = out, single[n - 1]
+    for a, b in zip(got[8], got[7]):
+        assert torch.isfinite(a).all() and torch.allclose(a, b, rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("bs", [8, 7])
 @pytest.mark.parametrize("longest", [128 * 8192, 128 * 8192 + 1, 128 * 16384])
 def test_float32_single_queries_beside_a_very_long_sequence(bs, longest):

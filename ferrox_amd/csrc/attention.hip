@@ -917,6 +917,11 @@ struct F32Attention {
             for (int unit = 0; unit < 4 * NU; ++unit) {
                 if (unit + 1 < 4 * NU) fetch_keys((unit + 1) & 1, unit + 1);
                 else fetch_values(0, 0);
+                if (a.hd < HDM) {      // numbers that the head does not have: zeros, for 0 (the query's) times infinity is none
+#pragma unroll
+                    for (int i = 0; i < UC; ++i)
+                        if (16 * (unit % NU * UC + i) + 4 * g >= a.hd) kb[unit & 1][i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                }
                 // (two chains of sums: an instruction that waits for the one before it takes longer than its turn)
                 f32x4_t part[2] = {(f32x4_t){0.f, 0.f, 0.f, 0.f}, (f32x4_t){0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -925,11 +930,6 @@ struct F32Attention {
                     for (int i = 0; i < UC; ++i)
                         part[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[unit & 1][i][u], q[unit % NU * UC + i][u], part[i & 1], 0, 0, 0);
                 s[unit / NU] = unit % NU == 0 ? part[0] + part[1] : s[unit / NU] + (part[0] + part[1]);
-                if (a.hd < HDM) {      // numbers that the head does not have: zeros, for 0 (the query's) times infinity is none
-#pragma unroll
-                    for (int i = 0; i < UC; ++i)
-                        if (16 * (unit % NU * UC + i) + 4 * g >= a.hd) kb[unit & 1][i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-                }
             }
             float top = NEG_INF;
 #pragma unroll

@@ -824,8 +824,10 @@ struct WaveAttn {
 // values go from memory straight into operands, no LDS and no barrier.  A unit (16 keys x up to 128 numbers, or 32 value
 // rows x 64 keys) is on its way while the one before it is multiplied; page ids are asked for a tile ahead.
 // (A lane per key that reads its row number by number, as the kernels for any shape do, took 514 us a layer for 700
-// tokens of 16 heads and 124 us for four single queries at 1,030 keys; these take 111 and 30 us.  What bounds them now is
-// one wave's chain: 512 products of 32 cycles a tile of 64 keys x 128 numbers, 7 us, and few waves a SIMD to hide its waits.)
+// tokens of 16 heads and 124 us for four single queries at 1,030 keys; these take 95 and 25 us.  What bounds them now is
+// one wave's chain: 256 products of 32 cycles a tile of 64 keys x 128 numbers, 3.4 of the 7.2 us that a tile takes (5.0 with heads of 64,
+// 11.8 of 256: some 2.7 us a tile from scores to probabilities and for page ids, whatever the head, the rest waits for operands), and few
+// waves a SIMD to hide it.)
 // ---------------------------------------------------------------------------
 template <int HDM>
 struct F32Attention {
@@ -835,16 +837,20 @@ struct F32Attention {
     f32x4_t o[NC];     // the row's outputs 16 c + 4 g + u
     float m, l;
 
-    // `query`: the row's query or null (a row that does not exist)
-    __device__ __forceinline__ void begin(const AttnArgs& a, const float* query, int g) {
+    // `query`: the row's query, of a row that exists (`there`) or of any other.  The loads are unconditional, the choice comes after
+    // them: behind a branch each load was waited for before the next one, up to 64 waits in a row in front of the first key (a single
+    // query of 16 heads over 64 keys, merge included: heads of 64 12.8 -> 11.2 us, of 128 16.9 -> 14.2).
+    __device__ __forceinline__ void begin(const AttnArgs& a, const float* query, bool there, int g) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) q[c][u] = query[min(16 * c + 4 * g, a.hd - 4) + u];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
+            const bool real = there && 16 * c + 4 * g < a.hd;
             o[c] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int d = 16 * c + 4 * g + u;
-                q[c][u] = (query && d < a.hd) ? query[d] * a.scale : 0.f;
-            }
+            for (int u = 0; u < 4; ++u) q[c][u] = real ? q[c][u] * a.scale : 0.f;
         }
         m = NEG_INF;
         l = 0.f;
@@ -1001,7 +1007,7 @@ __global__ __launch_bounds__(256) void attn_f32_block_kernel(AttnArgs a) {
     const int pos = a.positions[tok], pmin = a.positions[tok0], pmax = a.positions[tok0 + n - 1];
     const KeySpan span = {first_visible(a, pmin), pmax + 1, a.keep_first};
     F32Attention<HDM> w;
-    w.begin(a, li < n ? (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd : nullptr, g);
+    w.begin(a, (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd, li < n, g);
     w.walk(a, bt, kvh, span, 0, pos, first_visible(a, pos), h);
     if (li >= n) return;
     const float fin = finish_row<false>(a, h, w.m, w.l);
@@ -1030,9 +1036,10 @@ __global__ __launch_bounds__(64) void attn_f32_decode_kernel(AttnArgs a) {
     const int p = a.positions[tok], s0 = split * a.chunk, lo = first_visible(a, p);
     const KeySpan span = {max(lo, s0), min(p + 1, s0 + a.chunk), a.keep_first};
     F32Attention<HDM> w;
-    w.begin(a, nullptr, g);
+    w.m = NEG_INF;
+    w.l = 0.f;
     if (s0 < span.end && (span.begin < span.end || s0 < span.keep)) {
-        w.begin(a, there ? (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd : nullptr, g);
+        w.begin(a, (const float*)a.q + (size_t)tok * a.ldq + (size_t)h * a.hd, there, g);
         w.walk(a, bt, kvh, span, s0, p, lo, h);
     }
     if (!there) return;

@@ -339,11 +339,11 @@ __global__ __launch_bounds__(64) void attn_tile_kernel(AttnArgs a) {
 // `chunk` positions; one wave per (sequence, head, chunk) writes a partial
 // (max, sum, output), and a second kernel merges the chunks in ascending order.
 // ---------------------------------------------------------------------------
-template <typename T, int HDM = HD_MAX>
-__global__ __launch_bounds__(64) void attn_decode_kernel(AttnArgs a) {
+template <typename T, int HDM>
+__device__ __forceinline__ void decode_head(const AttnArgs& a, int item, int h, int split) {
     __shared__ float Qs[HDM];
     __shared__ float Ps[64];
-    const int item = blockIdx.x, h = blockIdx.y, split = blockIdx.z, lane = threadIdx.x;
+    const int lane = threadIdx.x;
     const int kvh = h / (a.nh / a.nkv);
     const int tok = a.item_tok[item];
     const int* bt = a.block_table + (size_t)a.item_seq[item] * a.max_blocks;
@@ -410,6 +410,10 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(AttnArgs a) {
         pml[0] = m;
         pml[1] = l;
     }
+}
+template <typename T, int HDM = HD_MAX>
+__global__ __launch_bounds__(64) void attn_decode_kernel(AttnArgs a) {
+    decode_head<T, HDM>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Merges the chunks' partial results in ascending order.  One block per (token, head): first
@@ -1023,12 +1027,23 @@ __global__ __launch_bounds__(256) void attn_f32_block_kernel(AttnArgs a) {
         }
 }
 // decode: block = one wave = (item, kv head x block of 16 of its query heads, chunk of keys); results merge as those of
-// attn_decode_kernel do
+// attn_decode_kernel do.  Queries below position FEW_KEYS go a wave per head as in that kernel: it is through with so few keys before a
+// tile's chain of waits is (16 heads of 128, merge included: 5 keys 9.3 against 16.3 us, 16 keys 13.2 and 16.1, 24 the same, 32 19.5 and
+// 16.4; 16 of 64 in groups of four: 5 keys 7.3 against 12.1, 24 11.1 and 12.2, 32 12.6 and 12.2; 16 of 192 + 128 32 keys 20.4 against 26.2).
+// The waves for a group's other heads come behind the chunks' blocks (a wave per head in every chunk, most of which leave again: 16
+// sequences of 3,000 keys, heads of 64, 30 -> 42 us).  The choice is the position's alone, so a query's bits do not depend on the step.
 template <int HDM>
 __global__ __launch_bounds__(64) void attn_f32_decode_kernel(AttnArgs a) {
+    constexpr int FEW_KEYS = HDM == 128 ? 24 : 32;
     const int item = blockIdx.x, split = blockIdx.z, lane = threadIdx.x, li = lane & 15, g = lane >> 4;
     const int group = a.nh / a.nkv, group_blocks = (group + 15) / 16;
-    const int kvh = blockIdx.y / group_blocks, row = blockIdx.y % group_blocks * 16 + li;
+    const int kvh = blockIdx.y / group_blocks, first = blockIdx.y % group_blocks * 16, row = first + li;
+    if (split == 0 || split >= a.splits) {
+        const int own = split ? first + 1 + split - a.splits : first;
+        const bool few = a.positions[a.item_tok[item]] < FEW_KEYS;
+        if (few && own < group) decode_head<float, HDM>(a, item, kvh * group + own, 0);
+        if (few || split) return;
+    }
     const bool there = row < group;
     const int h = kvh * group + min(row, group - 1);
     const int tok = a.item_tok[item];
@@ -1867,7 +1882,8 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
     if (dtype == FX_F32) {
         if (f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
-            const dim3 gridf(n_items, nkv * ((nh / nkv + 15) / 16), splits);
+            const int group = nh / nkv;
+            const dim3 gridf(n_items, nkv * ((group + 15) / 16), splits + (group < 16 ? group : 16) - 1);
             if (hd <= 64 && vd <= 64) attn_f32_decode_kernel<64><<<gridf, 64, 0, s>>>(a);
             else if (hd <= 128 && vd <= 128) attn_f32_decode_kernel<128><<<gridf, 64, 0, s>>>(a);
             else attn_f32_decode_kernel<256><<<gridf, 64, 0, s>>>(a);

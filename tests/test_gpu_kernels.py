@@ -801,6 +801,34 @@ def test_a_float32_key_at_minus_infinity_is_not_attended_to(hd):
         assert torch.isfinite(a).all() and torch.allclose(a, b, rtol=2e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,vd", [(3, 3, 16, 16), (4, 1, 64, 64), (34, 2, 80, 48), (8, 4, 128, 128), (17, 1, 192, 256)])
+def test_float32_single_queries_at_the_first_positions(nh, nkv, hd, vd):
+    """Queries below position 24 (heads of 65 to 128) or 32 go a wave per head, the same bits as the kernel for any shape (pages of 7
+    keys), whatever the step holds beside them and under whatever bound; from there on 16 heads of a group in a wave, equal up to roundings."""
+    from ferrox_amd import ops
+    n, at, few = 140, [0, 7, 23, 24, 31, 32, 127, 128, 139], 24 if 64 < max(hd, vd) <= 128 else 32
+    q, k, v = rnd(n, nh * hd), rnd(n, nkv, hd, seed=1), rnd(n, nkv, vd, seed=2)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    pos = torch.arange(n, dtype=torch.int32, device=DEV)
+
+    def run(bs, toks, bound):
+        blocks = -(-n // bs)
+        kp, vp = torch.zeros(blocks, nkv, bs, hd, device=DEV), torch.zeros(blocks, nkv, vd, bs, device=DEV)
+        for t in range(blocks):
+            rows = slice(t * bs, min((t + 1) * bs, n))
+            kp[t, :, :rows.stop - rows.start], vp[t, :, :, :rows.stop - rows.start] = k[rows].transpose(0, 1), v[rows].permute(1, 2, 0)
+        y = torch.full((n, nh * vd), float("nan"), device=DEV)
+        ops.attention_decode(q, y, kp, vp, i32([list(range(blocks))]), pos, i32([0] * len(toks)), i32(toks), nh, nkv, hd, bs, 0, hd ** -0.5,
+                             max_kv_len=bound, v_dim=vd)
+        return y
+
+    both, any_shape = run(8, at, n), run(7, at, n)
+    for t in at:
+        alone = run(8, [t], 1000)
+        assert torch.equal(alone[t], both[t]), t
+        assert torch.equal(both[t], any_shape[t]) if t < few else torch.allclose(both[t], any_shape[t], rtol=2e-5, atol=2e-5), t
+
+
 @pytest.mark.parametrize("bs", [8, 7])
 @pytest.mark.parametrize("longest", [128 * 8192, 128 * 8192 + 1, 128 * 16384])
 def test_float32_single_queries_beside_a_very_long_sequence(bs, longest):

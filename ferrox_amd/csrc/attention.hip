@@ -421,7 +421,8 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(AttnArgs a) {
 // dimensions over the chunks with several loads in flight.
 #define MERGE_KEPT 8192        // weights that LDS holds
 #define MERGE_MOST 16384       // chunks that are merged: two million keys by 128
-template <typename T>
+template <typename T, bool BEYOND>      // BEYOND: more chunks than LDS holds the weights of (an instance of its own: its loops cost
+                                        // the others 0.05 to 0.15 us a launch)
 __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
     extern __shared__ float wsm[];   // the weights of up to MERGE_KEPT chunks
     __shared__ float red[2];
@@ -447,14 +448,16 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
         const float ms = pml[2 * s];
         return (ms == NEG_INF) ? 0.f : expf(ms - m);
     };
-    const int kept = min(S, MERGE_KEPT);
+    const int kept = BEYOND ? MERGE_KEPT : S;
     for (int s = tid; s < kept; s += 128) wsm[s] = weight_of(s);
     __syncthreads();
     float l = 0.f;
     for (int s = 0; s < kept; ++s) l += wsm[s] * ((wsm[s] > 0.f) ? pml[2 * s + 1] : 0.f);   // ascending, the same in every thread
-    for (int s = kept; s < S; ++s) {
-        const float w = weight_of(s);
-        l += w * ((w > 0.f) ? pml[2 * s + 1] : 0.f);
+    if constexpr (BEYOND) {
+        for (int s = kept; s < S; ++s) {
+            const float w = weight_of(s);
+            l += w * ((w > 0.f) ? pml[2 * s + 1] : 0.f);
+        }
     }
     const float fin = finish_row<false>(a, h, m, l);
     for (int d = tid; d < hd; d += 128) {
@@ -474,9 +477,11 @@ __global__ __launch_bounds__(128) void attn_decode_merge_kernel(AttnArgs a) {
             const float v = (w > 0.f) ? po[(size_t)s * hd + d] : 0.f;   // an empty chunk wrote nothing
             acc = fmaf(w, v, acc);
         }
-        for (int s = kept; s < S; ++s) {
-            const float w = weight_of(s);
-            acc = fmaf(w, (w > 0.f) ? po[(size_t)s * hd + d] : 0.f, acc);
+        if constexpr (BEYOND) {
+            for (int s = kept; s < S; ++s) {
+                const float w = weight_of(s);
+                acc = fmaf(w, (w > 0.f) ? po[(size_t)s * hd + d] : 0.f, acc);
+            }
         }
         store_lane<T>(a, tok, h, d, acc * fin);
     }
@@ -1856,6 +1861,12 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
 
 // Single queries.  part_o has n_items*nh*splits*hd floats, part_ml n_items*nh*splits*2;
 // splits * chunk must cover every position + 1.
+template <typename T>
+static void launch_merge(const AttnArgs& a, dim3 grid, hipStream_t s) {
+    if (a.splits > MERGE_KEPT) attn_decode_merge_kernel<T, true><<<grid, 128, MERGE_KEPT * sizeof(float), s>>>(a);
+    else attn_decode_merge_kernel<T, false><<<grid, 128, a.splits * sizeof(float), s>>>(a);
+}
+
 static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, void* out, long ldo,
                               const void* k_pages, const void* v_pages, const int* block_table, int max_blocks,
                               const int* positions, const int* item_seq, const int* item_tok, int n_items,
@@ -1878,7 +1889,6 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
     a.part_o = part_o; a.part_ml = part_ml; a.splits = splits; a.chunk = chunk;
     dim3 grid(n_items, nh, splits), grid2(n_items, nh);
     hipStream_t s = (hipStream_t)stream;
-    const size_t merge_lds = (splits < MERGE_KEPT ? splits : MERGE_KEPT) * sizeof(float);
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
     if (dtype == FX_F32) {
         if (f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
@@ -1889,10 +1899,10 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
             else attn_f32_decode_kernel<256><<<gridf, 64, 0, s>>>(a);
         } else if (beyond) attn_decode_kernel<float, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
         else attn_decode_kernel<float><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<float><<<grid2, 128, merge_lds, s>>>(a);
+        launch_merge<float>(a, grid2, s);
     } else if (beyond) {
         attn_decode_kernel<bf16, HD_MAX_ANY><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
+        launch_merge<bf16>(a, grid2, s);
     } else if (mfma_ok(dtype, hd, bs, q, ldq, k_pages, v_pages, vd)) {
         const int group = nh / nkv;
         dim3 gridm(nkv * ((group + 15) / 16), n_items, splits);
@@ -1922,10 +1932,10 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
             else if (hd <= 128) attn_mfma_decode_block_kernel<128, 512, SH><<<gridm, nw * 64, shm, s>>>(a);
             else attn_mfma_decode_block_kernel<256, 256, SH><<<gridm, nw * 64, shm, s>>>(a);
         });
-        if (splits > 1) attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
+        if (splits > 1) launch_merge<bf16>(a, grid2, s);
     } else {
         attn_decode_kernel<bf16><<<grid, 64, 0, s>>>(a);
-        attn_decode_merge_kernel<bf16><<<grid2, 128, merge_lds, s>>>(a);
+        launch_merge<bf16>(a, grid2, s);
     }
     FX_CHECK_LAUNCH("attn_decode");
     return 0;

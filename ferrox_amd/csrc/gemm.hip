@@ -1791,8 +1791,9 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // (the head's 151,936: 260 against 272 us at 4 rows, 240 the other way at one).  Tiles of 64 once they are two and
         // a half a CU (6,144 weight rows: 512 rows 121 against 139 us, 256 rows 76 against 71; 2,048 weight rows: 1,500
         // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: tiles of 32 up to 36 rows an expert (60 experts'
-        // gate/up product of 2,048: 4.3 rows 263 us against 277 for few rows and 428 with tiles of 64; 34 rows 396 and
-        // 437; 47 rows 496 and 424).
+        // gate/up product of 2,048: one row 173 us against 172 for few rows and 266 with tiles of 64, its down product 94 against 114
+        // and 136; 4.3 rows 255, 267 and 390; 36 rows 419, 618 and 427; 47 rows 496 and 424 with tiles of 64.  Steps of one and two
+        // tokens are behind the kernel for few rows with gate/up, 30 and 26, 43 and 37 us).
         int tile = 0, mt = 1, nw = 2;
         if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
         else if (expert_offsets) tile = group <= 36 ? 32 : 64;

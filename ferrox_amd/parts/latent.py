@@ -210,7 +210,7 @@ class LatentAttention(Mixer):
         debug.region("attention")
         out = torch.empty((T, H * R), dtype=q.dtype, device=q.device)
         # items of 128 queries where the kernel takes them (latents of 256 numbers) and a portion is longer: prompts of 1,337
-        # and 4,000 tokens 3.08 and 7.06 ms against 3.48 and 7.74 with items of 64, 200 tokens 1.52 and 1.61, 117 the same
+        # and 4,000 tokens 3.41 and 8.78 ms against 3.80 and 9.52 with items of 64, 200 tokens 1.33 and 1.39, 117 the same
         tile_q = 64 if longest_portion(ctx) <= 128 else ops.attention_tile_queries(q_lat.dtype, R + P, cache.block_size, v_dim=R)
         items = ctx.memo(f"attention_items {tile_q}", lambda: attention_items(ctx, tile_q))
         common = (H, 1, R + P, cache.block_size, self.window, self.scale)

@@ -450,8 +450,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// Many rows, K a multiple of 64: tiles of up to 256 rows x TN weight rows, eight
-// waves.  K advances in steps of 64 through a ring of NS stages in LDS; tiles
+// Many rows, K a multiple of 64, weights that are read about once or tiles of few
+// rows: tiles of up to 192 rows x TN weight rows, eight waves.  K advances in steps of 64 through a ring of NS stages in LDS; tiles
 // travel from global memory straight into LDS (no registers in between), NS-1
 // steps ahead of their use, and one barrier per step separates the waves that
 // still read a stage from the loads that refill it.  A wave-load fills 1 KB of
@@ -551,32 +551,22 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
     wait_loads_but<0>();                       // the loads past the end, before the block leaves
 }
 
-template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false>
-__global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
-    constexpr int TM = TMB * 16;
-    constexpr int MT = TMB / 2;            // row blocks per wave
-    constexpr int NT = TN / 64;            // 16-row blocks of W per wave
-    constexpr int WN = TN / 4;
-    constexpr int OUT_TN = DUAL ? TN / 2 : TN;
-    constexpr int NLA = TM / 64, NLB = TN / 64;   // wave-loads (8 rows each) per wave and K step
-    static_assert(TM % 64 == 0 && TN % 64 == 0, "eight waves load 64 rows at a time");
-    __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
-
+// Which tile of the output a block of the LDS-tiled kernels works on; false: none.
+__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& row_tile, int& col_tile) {
     // Blocks go to the 8 XCDs in turn (block b runs on XCD b % 8), each with an L2 of its own.  Plain: an XCD
     // works through a contiguous range of the tiles in an order that keeps neighbours in rows and columns
     // together, so the operands of the tiles it has at a time stay in its L2.  Grouped: XCD x takes the row tiles x, x + 8, ... and runs through the column tiles of each, so an
     // expert's rows are fetched once and stay in its L2 while its weights, which nothing reads twice, stream by
     // (the row tiles past the last expert are empty; dealing them out in turn spreads them over the XCDs).
-    int row_tile, col_tile;
     if (g.expert_offsets) {
         const int i = blockIdx.x / 8;
         row_tile = (i / g.n_col_tiles) * 8 + blockIdx.x % 8;
         col_tile = i % g.n_col_tiles;
-        if (row_tile >= g.n_row_tiles) return;
+        if (row_tile >= g.n_row_tiles) return false;
     } else {
         const int per_xcd = (g.n_col_tiles * g.n_row_tiles + 7) / 8;
         const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if (logical >= g.n_col_tiles * g.n_row_tiles) return;
+        if (logical >= g.n_col_tiles * g.n_row_tiles) return false;
         // bands of 8 row tiles, rows fastest inside a band: the 32 tiles that an XCD works on at a time are
         // 8 rows x 4 columns, so 12 operand tiles serve 32 products
         const int band = logical / (8 * g.n_col_tiles), rem = logical % (8 * g.n_col_tiles);
@@ -584,61 +574,13 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
         row_tile = band * 8 + rem % band_rows;
         col_tile = rem / band_rows;
     }
-    int r0, r_end, expert;
-    locate_rows<TM>(g, row_tile, r0, r_end, expert);
-    if (r0 < 0) return;
-    const int n0 = col_tile * OUT_TN;
-    const int rows_here = min(TM, r_end - r0);
-    const int nblk = (rows_here + 15) >> 4;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // waves w and w + 4 share a SIMD: one of each half of the rows, so that a tile with few rows loads the SIMDs evenly
-    const int wm = wave >> 2, wn = wave & 3;
-    const bf16* Wbase = (const bf16*)g.W + (size_t)expert * g.w_stride;
+    return true;
+}
 
-    // what this lane fetches in each of its wave-loads: row 8*j + lane/8 of the tile, chunk (lane%8) ^ ((row/2)%8)
-    const bf16* a_src[NLA];
-    const bf16* b_src[NLB];
-#pragma unroll
-    for (int i = 0; i < NLA; ++i) {
-        const int j = wave + 8 * i, row = 8 * j + (lane >> 3);
-        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
-        const int m = r0 + min(row, rows_here - 1);          // rows past the end repeat the last one, unused
-        a_src[i] = (const bf16*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + chunk * 8;
-    }
-#pragma unroll
-    for (int i = 0; i < NLB; ++i) {
-        const int j = wave + 8 * i, row = 8 * j + (lane >> 3);
-        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
-        int col = DUAL ? n0 + (row >> 5) * 16 + (row & 15) : n0 + row;
-        col = min(col, g.N - 1);
-        const bool up = DUAL && ((row >> 4) & 1);
-        b_src[i] = g.kb_stride ? Wbase + ((size_t)col + (up ? g.up_offset / g.K : 0)) * 64 + chunk * 8
-                               : Wbase + (size_t)col * g.K + (up ? g.up_offset : 0) + chunk * 8;
-    }
-
-    f32x4_t acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-    const int sw = (lane & 15) >> 1, kq = lane >> 4;
-    const int a_off = (wm * 16 + (lane & 15)) * 64, b_off = (wn * WN + (lane & 15)) * 64;
-    const int na = (nblk - wm + 1) >> 1;         // this wave's active row blocks
-#define FX_LOOP(NA) \
-    wide_k_loop<NA, MT, NT, TM, TN, NSA, NS, STREAM>(acc, a_src, b_src, stages, g.K, wave, a_off, b_off, sw, kq, g.kb_stride)
-    if constexpr (MT >= 4) {
-        if (na > 3 * MT / 4) FX_LOOP(MT);
-        else if (na > MT / 2) FX_LOOP(3 * MT / 4);
-        else if (na > MT / 4) FX_LOOP(MT / 2);
-        else FX_LOOP(MT / 4);
-    } else {
-        if (na > MT / 2) FX_LOOP(MT);
-        else FX_LOOP((MT + 1) / 2);
-    }
-#undef FX_LOOP
-
-    // epilogue: lane holds rows 4*(lane/16)+r, column lane%16 of each 16x16 tile
+// What the accumulators of a wave go through on their way to C: MT row blocks (2i + wm of the tile's), NT column blocks.
+template <int MT, int NT, int TM, int WN, bool DUAL, int EPI>
+__device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[MT][NT], int r0, int r_end, int n0, int wm, int wn, int lane) {
+    // lane holds rows 4*(lane/16)+r, column lane%16 of each 16x16 tile
     float bias_v[NT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) bias_v[j] = 0.f;
@@ -723,6 +665,318 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
         }
     }
     });
+}
+
+template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false>
+__global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
+    constexpr int TM = TMB * 16;
+    constexpr int MT = TMB / 2;            // row blocks per wave
+    constexpr int NT = TN / 64;            // 16-row blocks of W per wave
+    constexpr int WN = TN / 4;
+    constexpr int OUT_TN = DUAL ? TN / 2 : TN;
+    constexpr int NLA = TM / 64, NLB = TN / 64;   // wave-loads (8 rows each) per wave and K step
+    static_assert(TM % 64 == 0 && TN % 64 == 0, "eight waves load 64 rows at a time");
+    __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
+
+    int row_tile, col_tile;
+    if (!wide_tile(g, row_tile, col_tile)) return;
+    int r0, r_end, expert;
+    locate_rows<TM>(g, row_tile, r0, r_end, expert);
+    if (r0 < 0) return;
+    const int n0 = col_tile * OUT_TN;
+    const int rows_here = min(TM, r_end - r0);
+    const int nblk = (rows_here + 15) >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // waves w and w + 4 share a SIMD: one of each half of the rows, so that a tile with few rows loads the SIMDs evenly
+    const int wm = wave >> 2, wn = wave & 3;
+    const bf16* Wbase = (const bf16*)g.W + (size_t)expert * g.w_stride;
+
+    // what this lane fetches in each of its wave-loads: row 8*j + lane/8 of the tile, chunk (lane%8) ^ ((row/2)%8)
+    const bf16* a_src[NLA];
+    const bf16* b_src[NLB];
+#pragma unroll
+    for (int i = 0; i < NLA; ++i) {
+        const int j = wave + 8 * i, row = 8 * j + (lane >> 3);
+        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
+        const int m = r0 + min(row, rows_here - 1);          // rows past the end repeat the last one, unused
+        a_src[i] = (const bf16*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + chunk * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < NLB; ++i) {
+        const int j = wave + 8 * i, row = 8 * j + (lane >> 3);
+        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
+        int col = DUAL ? n0 + (row >> 5) * 16 + (row & 15) : n0 + row;
+        col = min(col, g.N - 1);
+        const bool up = DUAL && ((row >> 4) & 1);
+        b_src[i] = g.kb_stride ? Wbase + ((size_t)col + (up ? g.up_offset / g.K : 0)) * 64 + chunk * 8
+                               : Wbase + (size_t)col * g.K + (up ? g.up_offset : 0) + chunk * 8;
+    }
+
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+    const int sw = (lane & 15) >> 1, kq = lane >> 4;
+    const int a_off = (wm * 16 + (lane & 15)) * 64, b_off = (wn * WN + (lane & 15)) * 64;
+    const int na = (nblk - wm + 1) >> 1;         // this wave's active row blocks
+#define FX_LOOP(NA) \
+    wide_k_loop<NA, MT, NT, TM, TN, NSA, NS, STREAM>(acc, a_src, b_src, stages, g.K, wave, a_off, b_off, sw, kq, g.kb_stride)
+    if constexpr (MT >= 4) {
+        if (na > 3 * MT / 4) FX_LOOP(MT);
+        else if (na > MT / 2) FX_LOOP(3 * MT / 4);
+        else if (na > MT / 4) FX_LOOP(MT / 2);
+        else FX_LOOP(MT / 4);
+    } else {
+        if (na > MT / 2) FX_LOOP(MT);
+        else FX_LOOP((MT + 1) / 2);
+    }
+#undef FX_LOOP
+
+    wide_epilogue<MT, NT, TM, WN, DUAL, EPI>(g, acc, r0, r_end, n0, wm, wn, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Tiles in quarters, the products of prompts: the same blocks, tiles, waves and swizzled LDS rows as above, with two
+// stages only, but a step of 64 k is four phases, and the rows and the weights of a stage are two parts each, so that
+// a part is refilled for the step after the next as soon as every wave has read it.  Phase by phase a wave
+// multiplies part 0 of its rows with the step's first weights, then with its second, then part 1 of its rows with the second and
+// with the first; while it does, it reads from LDS what the next phases multiply, one operand between every few products:
+//     products              reads (this step's, ' the next one's)       refilled, for the step after the next
+//  1  rows 0 x first        second weights, rows 1 (first 32 k)         -
+//  2  rows 0 x second       rows 1 (second 32 k)                        rows 0, first weights
+//  3  rows 1 x second       rows 0' (first 32 k)                        second weights
+//  4  rows 1 x first        first weights', rows 0' (second 32 k)       rows 1
+// The next step's first weights are read into the registers of this step's second ones, which phase 4 no longer
+// needs, so first and second change places every step and 96 registers of operands suffice beside the 128 sums.
+// Barriers stand in front of phases 2, 3 and 4: what a phase refills every wave has read (it is multiplied, so waited for,
+// before the barrier), and what phases 3, 4 and 1' read has landed for every wave that waited in front of it.
+// The loop waits for loads a whole step old and never for the youngest, where the ring of two stages waited for all of them
+// every step: 8,192 x 8,192 x 8,192 878 -> 758 us (1,252 -> 1,450 TFLOP/s), 4,096 rows against 40,960 weight rows of 3,584 k
+// 1,047 -> 883 us, against 3,584 of 20,480 k 505 -> 432 us.  Neither a fourth barrier, nor the priority of waves that multiply, nor waves
+// of a SIMD taking turns (one group reads while the other multiplies, 786 us) is any better.  An element's products are
+// added in the order of k, as in every bf16 tile: the same bits.
+// ---------------------------------------------------------------------------
+template <int N>
+using fx_int = std::integral_constant<int, N>;
+
+// 16 bytes a lane from a base that all lanes share, `offset` bytes on, into 1 KB of LDS.
+__device__ __forceinline__ void load_lds16(const bf16* base, unsigned offset, bf16* to) {
+#ifdef __HIP_DEVICE_COMPILE__       // (the host's pass does not know the descriptor's type)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, -1, 0x00027000), (fx_lds_ptr)to, 16, offset, 0, 0, 0);
+#endif
+}
+
+// The K loop of one wave.  MA0, MA1: its row blocks in part 0 and 1 of the tile; NA0, NA1: those of them that exist.
+// NB0, NB1: its blocks of 16 weight rows in part 0 and 1.  a_src and b_base move along with the loads.
+template <int NA0, int NA1, int MA0, int MA1, int NB0, int NB1>
+__device__ __forceinline__ void quarters_k_loop(f32x4_t (&acc)[MA0 + MA1][NB0 + NB1], const bf16* (&a_src)[(MA0 + MA1) / 2],
+                                                const bf16* (&b_base)[2], const unsigned (&b_off)[NB0 + NB1], bf16* lds, int K,
+                                                int wave, int wm, int wn, int lane, long kb_stride) {
+    constexpr int LA0 = MA0 / 2, LA1 = MA1 / 2, TM = 32 * (MA0 + MA1), TN = 64 * (NB0 + NB1), STAGE = (TM + TN) * 64;
+    const int nk = K >> 6;
+    const long b_step = kb_stride ? kb_stride : 64;
+    // wave-loads FROM .. TO-1 of a step's rows or weights, steps in turn.  (The empty asm keeps the compiler from
+    // holding every address twice; the weights' are 32 bits beside a base that all lanes share.  With 64 bits each
+    // some of them lived in scratch memory, and the loop waited for those loads.)
+    auto load_a = [&](auto from, auto to, int kt) {
+        bf16* st = lds + (kt & 1) * STAGE;
+#pragma unroll
+        for (int i = decltype(from)::value; i < decltype(to)::value; ++i) {
+            __builtin_amdgcn_global_load_lds((fx_global_ptr)a_src[i], (fx_lds_ptr)(st + (wave + 8 * i) * 512), 16, 0, 0);
+            a_src[i] += 64;
+            asm volatile("" : "+v"(a_src[i]));
+        }
+    };
+    auto load_b = [&](auto from, auto to, auto part, int kt) {
+        bf16* st = lds + (kt & 1) * STAGE + TM * 64;
+#pragma unroll
+        for (int i = decltype(from)::value; i < decltype(to)::value; ++i)
+            load_lds16(b_base[decltype(part)::value], b_off[i], st + (wave + 8 * i) * 512);
+        b_base[decltype(part)::value] += b_step;
+    };
+    auto load_rows = [&](auto part, int kt) {
+        if constexpr (decltype(part)::value == 0) load_a(fx_int<0>{}, fx_int<LA0>{}, kt);
+        else load_a(fx_int<LA0>{}, fx_int<LA0 + LA1>{}, kt);
+    };
+    auto load_weights = [&](auto part, int kt) {
+        if constexpr (decltype(part)::value == 0) load_b(fx_int<0>{}, fx_int<NB0>{}, part, kt);
+        else load_b(fx_int<NB0>{}, fx_int<NB0 + NB1>{}, part, kt);
+    };
+
+    const int sw = (lane & 15) >> 1, kq = lane >> 4;
+    const int koff[2] = {(kq ^ sw) * 8, ((4 + kq) ^ sw) * 8};
+    const int a_off = (wm * 16 + (lane & 15)) * 64;
+    const int b_at[2] = {TM * 64 + (wn * 16 * NB0 + (lane & 15)) * 64, TM * 64 + (64 * NB0 + wn * 16 * NB1 + (lane & 15)) * 64};
+    constexpr int NBX = NB0 > NB1 ? NB0 : NB1;
+    bf16x8_t a[2][MA0][2], b[2][NBX][2];
+    // operand u of a part's rows (the existing blocks' first 32 k, then their second) and of a part's weights
+    auto read_rows = [&](auto part, auto uc, int st) {
+        constexpr int h = decltype(part)::value, u = decltype(uc)::value, na = h ? NA1 : NA0, kk = u / na, i = u % na;
+        a[h][i][kk] = *(const bf16x8_t*)(lds + st + a_off + koff[kk] + (h * MA0 + i) * 32 * 64);
+    };
+    auto read_weights = [&](auto part, auto uc, int st) {
+        constexpr int h = decltype(part)::value, u = decltype(uc)::value, nb = h ? NB1 : NB0, kk = u / nb, j = u % nb;
+        b[h][j][kk] = *(const bf16x8_t*)(lds + st + b_at[h] + koff[kk] + j * 16 * 64);
+    };
+    // a phase: the products of a part of the rows with a part of the weights, R reads spread over them
+    auto phase = [&](auto rows, auto weights, auto reads, auto&& read) {
+        constexpr int h = decltype(rows)::value, w = decltype(weights)::value, R = decltype(reads)::value;
+        constexpr int na = h ? NA1 : NA0, nb = w ? NB1 : NB0, P = 2 * na * nb;
+        if constexpr (P == 0) {
+            static_for(std::make_integer_sequence<int, R>{}, read);
+        } else {
+            static_for(std::make_integer_sequence<int, P>{}, [&](auto qc) {
+                constexpr int q = decltype(qc)::value, u0 = (q * R + P - 1) / P, u1 = ((q + 1) * R + P - 1) / P;
+                if constexpr (u1 > u0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    static_for(std::make_integer_sequence<int, u1 - u0>{}, [&](auto uc) { read(fx_int<u0 + decltype(uc)::value>{}); });
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                constexpr int kk = q / (na * nb), i = q / nb % na, j = q % nb;
+                acc[h * MA0 + i][w * NB0 + j] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i][kk], b[w][j][kk], acc[h * MA0 + i][w * NB0 + j], 0, 0, 0);
+            });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto barrier = [] {
+        asm volatile("" ::: "memory");       // (the barrier alone does not keep reads of LDS on their side of it)
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+    };
+    // one step; left: the steps behind it, as far as that matters (0, 1, or 2 for more)
+    auto step = [&](auto first, auto left, int kt) {
+        constexpr int f = decltype(first)::value, s = 1 - f, nb_s = s ? NB1 : NB0;
+        constexpr bool next = decltype(left)::value > 0, refill = decltype(left)::value > 1;
+        const int st = (kt & 1) * STAGE, sn = STAGE - st;
+        phase(fx_int<0>{}, fx_int<f>{}, fx_int<2 * nb_s + NA1>{}, [&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            if constexpr (u < 2 * nb_s) read_weights(fx_int<s>{}, uc, st);
+            else read_rows(fx_int<1>{}, fx_int<u - 2 * nb_s>{}, st);
+        });
+        if constexpr (refill) {
+            barrier();
+            load_rows(fx_int<0>{}, kt + 2);
+            load_weights(fx_int<f>{}, kt + 2);
+        }
+        phase(fx_int<0>{}, fx_int<s>{}, fx_int<NA1>{}, [&](auto uc) { read_rows(fx_int<1>{}, fx_int<decltype(uc)::value + NA1>{}, st); });
+        if constexpr (next) {
+            // rows 0 of the next step have landed: behind them may be its weights, its rows 1 and what phase 2 has asked for
+            wait_loads_but<refill ? NB0 + NB1 + LA1 + LA0 + (f ? NB1 : NB0) : 0>();
+            barrier();
+        }
+        if constexpr (refill) load_weights(fx_int<s>{}, kt + 2);
+        phase(fx_int<1>{}, fx_int<s>{}, fx_int<next ? NA0 : 0>{}, [&](auto uc) { read_rows(fx_int<0>{}, uc, sn); });
+        if constexpr (refill) {
+            wait_loads_but<LA0 + NB0 + NB1>();     // all of the next step has
+            barrier();
+            load_rows(fx_int<1>{}, kt + 2);
+        }
+        phase(fx_int<1>{}, fx_int<f>{}, fx_int<next ? 2 * nb_s + NA0 : 0>{}, [&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            if constexpr (u < 2 * nb_s) read_weights(fx_int<s>{}, uc, sn);
+            else read_rows(fx_int<0>{}, fx_int<u - 2 * nb_s + NA0>{}, sn);
+        });
+    };
+
+    // The last step's first weights are part 1, so the first step's are part 1 where the steps are an odd number.  The loads
+    // go out in the order in which the loop waits for them.
+    const bool odd = nk & 1;
+    load_rows(fx_int<0>{}, 0);
+    load_weights(fx_int<0>{}, 0);
+    load_weights(fx_int<1>{}, 0);
+    load_rows(fx_int<1>{}, 0);
+    if (nk > 1) {
+        load_rows(fx_int<0>{}, 1);
+        load_weights(fx_int<0>{}, 1);
+        load_weights(fx_int<1>{}, 1);
+        load_rows(fx_int<1>{}, 1);
+        wait_loads_but<LA0 + NB0 + NB1 + LA1>();
+    } else {
+        wait_loads_but<0>();
+    }
+    barrier();
+    static_for(std::make_integer_sequence<int, 2 * NA0>{}, [&](auto uc) { read_rows(fx_int<0>{}, uc, 0); });
+    int kt = 0;
+    if (odd) {
+        static_for(std::make_integer_sequence<int, 2 * NB1>{}, [&](auto uc) { read_weights(fx_int<1>{}, uc, 0); });
+        if (nk > 1) step(fx_int<1>{}, fx_int<2>{}, kt++);
+    } else {
+        static_for(std::make_integer_sequence<int, 2 * NB0>{}, [&](auto uc) { read_weights(fx_int<0>{}, uc, 0); });
+    }
+    for (; kt + 2 < nk; kt += 2) {
+        step(fx_int<0>{}, fx_int<2>{}, kt);
+        step(fx_int<1>{}, fx_int<2>{}, kt + 1);
+    }
+    if (nk > 1) step(fx_int<0>{}, fx_int<1>{}, kt++);
+    step(fx_int<1>{}, fx_int<0>{}, kt);
+}
+
+template <int TMB, int TN, bool DUAL, int EPI>
+__global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
+    constexpr int TM = TMB * 16, MT = TMB / 2, NT = TN / 64, WN = TN / 4, OUT_TN = DUAL ? TN / 2 : TN;
+    constexpr int MA0 = MT > 4 ? 4 : MT / 2, MA1 = MT - MA0, NB0 = (NT + 1) / 2, NB1 = NT - NB0;
+    constexpr int NLA = TM / 64, NLB = TN / 64;   // wave-loads (8 rows each) per wave and K step
+    static_assert(MA0 % 2 == 0 && MA1 % 2 == 0 && MA1 > 0 && NB1 > 0, "eight waves load 64 rows at a time, a part at a time");
+    __shared__ __attribute__((aligned(1024))) bf16 stages[2 * (TM + TN) * 64];
+
+    int row_tile, col_tile;
+    if (!wide_tile(g, row_tile, col_tile)) return;
+    int r0, r_end, expert;
+    locate_rows<TM>(g, row_tile, r0, r_end, expert);
+    if (r0 < 0) return;
+    const int n0 = col_tile * OUT_TN;
+    const int rows_here = min(TM, r_end - r0);
+    const int nblk = (rows_here + 15) >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 2, wn = wave & 3;
+    const bf16* Wbase = (const bf16*)g.W + (size_t)expert * g.w_stride;
+
+    const bf16* a_src[NLA];
+#pragma unroll
+    for (int i = 0; i < NLA; ++i) {
+        const int j = wave + 8 * i, row = 8 * j + (lane >> 3);
+        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
+        const int m = r0 + min(row, rows_here - 1);          // rows past the end repeat the last one, unused
+        a_src[i] = (const bf16*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + chunk * 8;
+    }
+    // part 0 of the weights holds the first 16*NB0 of every wave's weight rows, part 1 the others; all that a wave loads of a
+    // part are rows of one matrix where there are two (their blocks of 16 take turns)
+    const bf16* b_base[2];
+    unsigned b_off[NLB];
+    const long ldw = g.kb_stride ? 64 : g.K;
+#pragma unroll
+    for (int i = 0; i < NLB; ++i) {
+        const int j = wave + 8 * i, x = 8 * j + (lane >> 3);
+        const int chunk = (lane & 7) ^ (4 * (j & 1) + (lane >> 4));
+        const int row = i < NB0 ? x / (16 * NB0) * WN + x % (16 * NB0)
+                                : (x - 64 * NB0) / (16 * NB1) * WN + 16 * NB0 + (x - 64 * NB0) % (16 * NB1);
+        const int col = min(DUAL ? n0 + (row >> 5) * 16 + (row & 15) : n0 + row, g.N - 1);
+        b_off[i] = (unsigned)((col - n0) * ldw + chunk * 8) * 2;
+        if (i == 0 || i == NB0) {
+            const bool up = DUAL && __builtin_amdgcn_readfirstlane((row >> 4) & 1);
+            b_base[i != 0] = Wbase + n0 * ldw + (up ? (g.kb_stride ? g.up_offset / g.K * 64 : g.up_offset) : 0);
+        }
+    }
+
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+    const int na = (nblk - wm + 1) >> 1;         // this wave's row blocks that exist
+#define FX_LOOP(NA0_, NA1_) quarters_k_loop<NA0_, NA1_, MA0, MA1, NB0, NB1>(acc, a_src, b_base, b_off, stages, g.K, wave, wm, wn, lane, g.kb_stride)
+    if (na > (MA1 > 2 ? MA0 + MA1 / 2 : MA0)) FX_LOOP(MA0, MA1);
+    else if (MA1 > 2 && na > MA0) FX_LOOP(MA0, MA1 / 2);
+    else if (na > MA0 / 2) FX_LOOP(MA0, 0);
+    else FX_LOOP(MA0 / 2, 0);
+#undef FX_LOOP
+    wide_epilogue<MT, NT, TM, WN, DUAL, EPI>(g, acc, r0, r_end, n0, wm, wn, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -1507,7 +1761,7 @@ static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
 static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
-static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128) or 8128 (128 x 128 in two stages) picks that tile of the LDS-tiled kernel
+static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages) or 8256 (128 x 256) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "skinny_sets")) { g_skinny_nw = value; return 0; }
     if (!strcmp(key, "skinny_row_tiles")) { g_skinny_mt = value; return 0; }
@@ -1524,8 +1778,15 @@ FX_API int fx_debug_set(const char* key, int value) {
     return 1;
 }
 
+// The grid of the LDS-tiled kernels, which decode their block's tile themselves.
+static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles) {
+    g.n_col_tiles = ceil_div(g.N, epi == EPI_GATED ? tn / 2 : tn);
+    g.n_row_tiles = m_tiles;
+    return dim3(g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
+}
 template <int TMB, int TN, int NS, int NSA, bool STREAM>
-static void launch_wide_as(const GemmArgs& g, int epi, dim3 grid, hipStream_t s) {
+static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
     switch (epi) {
         case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
@@ -1535,21 +1796,29 @@ static void launch_wide_as(const GemmArgs& g, int epi, dim3 grid, hipStream_t s)
             break;
     }
 }
-template <int TMB, int TN, int NS, int NSA = NS>
-static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
-    g.n_col_tiles = ceil_div(g.N, epi == EPI_GATED ? TN / 2 : TN);
-    g.n_row_tiles = m_tiles;
-    dim3 grid(g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
-    // the streaming variant exists for the tiles that few rows take (up to 192 of them)
-    if constexpr (TMB <= 12) {
-        if (g.stream_w) {
-            launch_wide_as<TMB, TN, NS, NSA, true>(g, epi, grid, s);
-            return;
-        }
+template <int TMB, int TN>
+static void launch_quarters(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
+    switch (epi) {
+        case EPI_STORE: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE_F32: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE_F32><<<grid, 512, 0, s>>>(g); break;
+        case EPI_RESID: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_RESID><<<grid, 512, 0, s>>>(g); break;
+        default:
+            if constexpr (TN % 128 == 0) gemm_bf16_quarters_kernel<TMB, TN, true, EPI_GATED><<<grid, 512, 0, s>>>(g);
+            break;
     }
-    launch_wide_as<TMB, TN, NS, NSA, false>(g, epi, grid, s);
 }
-
+// Weights that are read about once go through the ring with the non-temporal hint, everything else in quarters.
+template <int TMB, int TN, int NS, int NSA = NS>
+static void launch_ring_or_quarters(const GemmArgs& g, int epi, int m_tiles, hipStream_t s) {
+    if (g.stream_w) launch_wide<TMB, TN, NS, NSA, true>(g, epi, m_tiles, s);
+    else launch_quarters<TMB, TN>(g, epi, m_tiles, s);
+}
+template <int TMB, int TN, int NS, int NSA = NS>
+static void launch_ring(const GemmArgs& g, int epi, int m_tiles, hipStream_t s) {
+    if (g.stream_w) launch_wide<TMB, TN, NS, NSA, true>(g, epi, m_tiles, s);
+    else launch_wide<TMB, TN, NS, NSA, false>(g, epi, m_tiles, s);
+}
 template <bool DUAL, int EPI, bool VEC>
 static void launch_f32(const GemmArgs& g, int tile, int mt, int nw, dim3 grid, hipStream_t s) {
     if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
@@ -1669,7 +1938,9 @@ FX_API int fx_gemm_row_tile_blocks(int M, int N, int cus) {
 }
 
 // The tile of the LDS-tiled kernel for plain rows, as the debug switch "wide" names them; all give the same bits.  `dual`: N
-// columns of two matrices.
+// columns of two matrices.  (The times beside the lines are those of tiles in rings of stages.  In quarters every tile from 128 x 128 on takes 7
+// to 18 % less and what is ahead stays ahead: 4,096 rows against 4,608 weight rows of 3,584 k 149.5 -> 129 us with 256 x 192, 157 with 256 x 256;
+// gate/up of 11,264, 2,048 rows 100 -> 91 with 192 x 256, 113 with 256 x 256; 2,048 rows against 2,048 of 5,632 k 55 -> 50 with 128 x 128, 62 with 128 x 256.)
 FX_API int fx_gemm_plain_tile(int M, int N, int K, int dual, int cus) {
     auto tiles = [&](int tm, int tn) { return (long)ceil_div(N, dual ? tn / 2 : tn) * ceil_div(M, tm); };
     // Fewer tiles of 128 x 128 than CUs: a block's chain of K steps takes the same 23-25 us (2,048 k) whatever the rows, so
@@ -1701,6 +1972,14 @@ FX_API int fx_gemm_plain_tile(int M, int N, int K, int dual, int cus) {
     // 88 -> 71 us; gate/up of 11,264, 1,337 rows 91 -> 79).  (Not ahead of the other tiles in general: four rounds' worth of tiles of 128 x 128,
     // 2,048 rows' gate/up of 8,192 73 against 67 us, 3,456 rows against 4,608 weight rows of 3,584 k 111 against 101.)
     return t128 > cus ? 8128 : 64;
+}
+// Plain products that take tiles of 128 x 128: whether 128 x 256 are ahead.  Two tiles of 128 x 128 on a CU take what one of twice the
+// width takes (2,048 k: 31 and 29 us), so while those are one round of the CUs, or their last round is nearly full (1,000 rows
+// against 6,144 weight rows 31.9 -> 30.0 us, gate/up of 11,264, 512 rows 32.1 -> 30.2 and 1,337 rows 67.9 -> 65.3, 3,001 rows against
+// 2,048 of 5,632 k 75 -> 65; the other way gate/up of 11,264, 1,000 rows, 1.4 rounds, 52 against 60).
+FX_API int fx_gemm_twice_as_wide(int M, int N, int dual, int cus) {
+    const long t = (long)ceil_div(N, dual ? 128 : 256) * ceil_div(M, 128), rounds = ceil_div(t, (long)cus);
+    return rounds == 1 || 10 * t >= 9 * rounds * cus;
 }
 // The same for rows sorted by expert.
 static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, int cus) {
@@ -1902,26 +2181,30 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     if (per_group <= 64 && !many_columns && !wide_ok) {
         const int m_tiles = M / 64 + (expert_offsets ? nonempty : (M % 64 != 0));
         launch_bf16<64, 64, 32, 32>(g, epi, m_tiles, s);
-    } else if (g.vec_ok && K % 64 == 0 && !g_no_wide) {
+    } else if (g.vec_ok && K % 64 == 0 && !g_no_wide && (g.kb_stride || K < (1 << 22))) {     // (32-bit offsets inside a tile of weights)
         const bool dual = epi == EPI_GATED;
         // weights that are read about once (an expert's rows fit one row tile on average; plain rows: one row tile)
         // are loaded with the non-temporal hint
         g.stream_w = g_stream_w >= 0 ? g_stream_w : (expert_offsets ? per_group <= 128 : M <= 128);
         int tile = expert_offsets && g_wide_grouped ? g_wide_grouped : g_wide_force;
         if (dual && (tile == 464 || tile == 192)) tile = 256;       // (no such tiles of two matrices)
-        if (!tile && !expert_offsets) tile = fx_gemm_plain_tile(M, N, K, dual, fx_compute_units());
+        if (!tile && !expert_offsets) {
+            tile = fx_gemm_plain_tile(M, N, K, dual, fx_compute_units());
+            if (tile == 8128 && !g.stream_w && fx_gemm_twice_as_wide(M, N, dual, fx_compute_units())) tile = 8256;
+        }
         else if (!tile) tile = small_groups ? 64 : grouped_tile(per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
         switch (tile) {
-            case 464: launch_wide<4, 64, 4>(g, epi, row_tiles(64), s); break;
-            case 4128: launch_wide<4, 128, 3>(g, epi, row_tiles(64), s); break;
-            case 8128: launch_wide<8, 128, 2>(g, epi, row_tiles(128), s); break;
-            case 4: launch_wide<4, 256, 4, 2>(g, epi, row_tiles(64), s); break;
-            case 12: launch_wide<12, 256, 3, 2>(g, epi, row_tiles(192), s); break;
-            case 192: launch_wide<16, 192, 2>(g, epi, row_tiles(256), s); break;
-            case 128: launch_wide<16, 128, 3>(g, epi, row_tiles(256), s); break;
-            case 64: launch_wide<8, 128, 4>(g, epi, row_tiles(128), s); break;
-            default: launch_wide<16, 256, 2>(g, epi, row_tiles(256), s); break;
+            case 464: launch_ring<4, 64, 4>(g, epi, row_tiles(64), s); break;
+            case 4128: launch_ring<4, 128, 3>(g, epi, row_tiles(64), s); break;
+            case 4: launch_ring<4, 256, 4, 2>(g, epi, row_tiles(64), s); break;
+            case 8128: launch_ring_or_quarters<8, 128, 2>(g, epi, row_tiles(128), s); break;
+            case 64: launch_ring_or_quarters<8, 128, 4>(g, epi, row_tiles(128), s); break;
+            case 12: launch_ring_or_quarters<12, 256, 3, 2>(g, epi, row_tiles(192), s); break;
+            case 8256: launch_quarters<8, 256>(g, epi, row_tiles(128), s); break;
+            case 192: launch_quarters<16, 192>(g, epi, row_tiles(256), s); break;
+            case 128: launch_quarters<16, 128>(g, epi, row_tiles(256), s); break;
+            default: launch_quarters<16, 256>(g, epi, row_tiles(256), s); break;
         }
     } else {
         const int m_tiles = M / 128 + (expert_offsets ? nonempty : (M % 128 != 0));

@@ -58,6 +58,14 @@ def test_tiles_of_plain_products():
     assert tile(4096, 2048, cus=128) == tile(8192, 2048)
 
 
+def test_tiles_twice_as_wide():
+    """128 x 256 in place of 128 x 128 while they are one round of the CUs, or nearly whole rounds."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, n, dual=0, cus=256: bool(load_library("gemm").fx_gemm_twice_as_wide(m, n, dual, cus))
+    assert rule(1000, 6144) and rule(3001, 2048) and rule(512, 5632, 1) and rule(1337, 5632, 1)
+    assert not rule(1000, 5632, 1) and rule(4096, 2048) and not rule(4097, 2048) and not rule(4096, 2048, cus=192)
+
+
 def test_the_chunk_rule_leaves_the_callers_arguments_alone():
     """The rule counts waves per block; it once did so in a variable named like the `waves` argument of
     `attention_decode`, which then reached the launch instead of the caller's value."""

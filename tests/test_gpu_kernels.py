@@ -185,6 +185,58 @@ def test_plain_products_have_the_same_bits_in_every_tile(M, N):
                 assert torch.equal(ops.gemm(a, w[:N // 2 * 2], epilogue=ops.EPI_GATED), gated), tile
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 576])      # one step of 64 k, an even and an odd number of them
+@pytest.mark.parametrize("M,N", [(129, 264), (500, 392)])
+def test_tiles_in_quarters_have_the_bits_of_the_ring(M, N, K):
+    """Every shape of tile that is worked on in quarters, rows and columns that end inside a tile, every epilogue."""
+    from ferrox_amd import debug, ops
+    dtype = torch.bfloat16
+    a, w, bias, w2 = rnd(M, K + 8, dtype=dtype)[:, :K], rnd(N, K, dtype=dtype, seed=1), rnd(N, dtype=dtype, seed=2), rnd(2 * N, K, dtype=dtype, seed=4, scale=0.5)
+    h, scale, blocked = rnd(M, N, seed=3), rnd(M, seed=5).abs(), ops.to_kblocked(w)
+
+    def products():
+        return (ops.gemm(a, w, bias=bias), ops.gemm(a, w, epilogue=ops.EPI_STORE_F32), ops.gemm(a, w, epilogue=ops.EPI_RESID, out=h.clone(), row_scale=scale),
+                ops.gemm(a, w2, epilogue=ops.EPI_GATED))
+
+    with debug.kernel_switch("gemm", "wide", 4):          # 64 x 256, whose stages go round in a ring
+        want = products()
+    close(want[1], a.double() @ w.double().T, dtype, "product")
+    for tile in (256, 192, 128, 12, 8256, 8128):
+        with debug.kernel_switch("gemm", "wide", tile):
+            for x, y, what in zip(products(), want, ("store + bias", "store float32", "residual", "gated")):
+                assert torch.equal(x, y), (tile, what)
+            assert torch.equal(ops.gemm(a, blocked, epilogue=ops.EPI_STORE_F32, w_kblocked=True), want[1]), (tile, "slabs")
+
+
+@pytest.mark.parametrize("blocked", [False, True])
+def test_grouped_tiles_in_quarters_at_every_number_of_row_blocks(blocked):
+    """Experts with 1 to 260 rows, so that tiles have every number of blocks of 16 rows, none included."""
+    from ferrox_amd import debug, ops
+    dtype, K, N = torch.bfloat16, 192, 136
+    sizes = [0, 1, 16, 17, 33, 64, 65, 96, 0, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 260, 0]
+    E, n = len(sizes), sum(sizes)
+    offsets = torch.tensor([sum(sizes[:i]) for i in range(E + 1)], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(3)
+    x, w, w2 = rnd(300, K, dtype=dtype), rnd(E, N, K, dtype=dtype, seed=1), rnd(E, 2 * N, K, dtype=dtype, seed=2, scale=0.5)
+    rows = torch.randint(0, 300, (n,), generator=g).to(torch.int32).to(DEV)
+    to = torch.randperm(n, generator=g).to(torch.int32).to(DEV)
+    kb = dict(w_kblocked=True) if blocked else {}
+    wb, w2b = (ops.to_kblocked(w), ops.to_kblocked(w2)) if blocked else (w, w2)
+    want = torch.zeros(n, N, dtype=torch.float64, device=DEV)
+    xs = x.double()[rows.long()]
+    for e in range(E):
+        r = slice(sum(sizes[:e]), sum(sizes[:e + 1]))
+        want[to[r].long()] = xs[r] @ w[e].double().T
+    first = None
+    for tile in (4, 256, 192, 128, 12, 8256, 8128):       # (4: the ring)
+        with debug.kernel_switch("gemm", "wide_grouped", tile), debug.kernel_switch("gemm", "stream_w", 0):
+            got = ops.gemm(x, wb, epilogue=ops.EPI_STORE_F32, a_rows=rows, c_rows=to, expert_offsets=offsets, n_rows=n, **kb)
+            act = ops.gemm(x, w2b, epilogue=ops.EPI_GATED, a_rows=rows, expert_offsets=offsets, n_rows=n, **kb)
+        first = first or (got, act)
+        close(got, want, dtype, f"tile {tile}")
+        assert torch.equal(got, first[0]) and torch.equal(act, first[1]), tile
+
+
 @pytest.mark.parametrize("T,E", [(2048, 65), (4096, 65), (4096, 128), (8065, 65)])
 def test_a_routers_logits_keep_their_order_of_sums(T, E):
     """Up to 524,288 logits come from the product for few rows, whose bits decide between experts that stand close."""

@@ -8,6 +8,7 @@
 #include "common.h"
 
 #include <type_traits>
+#include <utility>
 
 FX_DEFINE_LAST_ERROR()
 
@@ -295,6 +296,35 @@ __device__ __forceinline__ float column_sum(float v) {      // over the LPC lane
     return v;
 }
 
+// Two sums at once.  With 32 lanes to a column the first step is the exchange between neighbouring rows of 16, and of both sums: one
+// of a column's two rows goes on with a's and the other with b's, four rotations finish both, and a last exchange
+// hands each to the other row.  (One sum after the other is two chains of four rotations and an exchange.)
+template <int LPC>
+__device__ __forceinline__ void column_sums(float& a, float& b) {
+    if constexpr (LPC == 32) {
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        float v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        v += row_rotated<0x128>(v);
+        v += row_rotated<0x124>(v);
+        v += row_rotated<0x122>(v);
+        v += row_rotated<0x121>(v);
+        a = wave_partner_16(v, b);
+    } else {
+        a = column_sum<LPC>(a);
+        b = column_sum<LPC>(b);
+    }
+}
+
+// what lane p of a row of 16 lanes holds, in each of them
+template <int p>
+__device__ __forceinline__ float row_lane(float v) {
+    return row_rotated<0x150 + p>(v);      // row_newbcast:p
+}
+template <int... Is, typename F>
+__device__ __forceinline__ void tokens(std::integer_sequence<int, Is...>, F&& f) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+
 template <int DR, int LPC, bool VEC, int NW>
 __global__ __launch_bounds__(NW * 64) void channel_delta_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                                                                 const float* __restrict__ decay, const float* __restrict__ beta,
@@ -308,7 +338,7 @@ __global__ __launch_bounds__(NW * 64) void channel_delta_kernel(const float* __r
     constexpr int PIECES = 3 * DP / W;               // loads that bring one token's (k | q | decay)
     constexpr int NL = (P * PIECES + NT - 1) / NT;   // loads a thread makes per group
     constexpr int COLS = 64 / LPC;
-    static_assert(DR % 4 == 0, "a lane's rows are read from LDS in 16-byte pieces");
+    static_assert(DR % 4 == 0 && LPC >= P, "a lane's rows are read from LDS in 16-byte pieces; a group's numbers and outputs are a lane's each");
     __shared__ __attribute__((aligned(16))) float kqd[2][P][3][DP];      // two groups of P tokens x (k, q, decay)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane % LPC, j = (blockIdx.x * NW + wave) * COLS + lane / LPC;
@@ -330,64 +360,72 @@ __global__ __launch_bounds__(NW * 64) void channel_delta_kernel(const float* __r
         }
     }
     // a group's operands: piece number idx = n NT + tid of the group's P PIECES goes to kqd[.] at idx W, which is
-    // token idx / PIECES, then k, q or decay, then the row; pieces past D, past the group or past the sequence are zeros
-    float nxt[NL][W], v_nxt[P], b_nxt[P], kq_nxt[P];
-    auto fetch = [&](int first) {
+    // token idx / PIECES, then k, q or decay, then the row; pieces past D are zeros.  A token's beta and k.q, and its v for a
+    // column, lie in lane p of every row of 16 lanes, whence they are broadcast.  Nothing here is conditional (tokens past the
+    // sequence's are its last one, unused): behind branches the loads of both groups ahead would be waited for at once.
+    const float* src[NL];
+    long src_step[NL];
+    int src_token[NL];
+    bool src_in[NL];
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+        const int idx = min(n * NT + tid, P * PIECES - 1), p = idx / PIECES, e = (idx - p * PIECES) * W, which = e / DP, row = e - which * DP;
+        src_in[n] = row < D;
+        src_token[n] = p;
+        src_step[n] = which == 2 ? (long)H * D : (long)G * D;
+        src[n] = (which == 2 ? decay + (size_t)h * D : (which == 1 ? qn : kn) + (size_t)g * D) + (src_in[n] ? row : 0);
+    }
+    struct Group {
+        float piece[NL][W], v, beta, kq;
+    } ahead[2];
+    auto fetch = [&](Group& to, int first) {
 #pragma unroll
         for (int n = 0; n < NL; ++n) {
-            const int idx = n * NT + tid, p = idx / PIECES, e = (idx - p * PIECES) * W, which = e / DP, row = e - which * DP;
-            const int t = first + p;
-            const bool ok = idx < P * PIECES && t < t1 && row < D;
-            const float* src = which == 0 ? kn + ((size_t)t * G + g) * D : (which == 1 ? qn + ((size_t)t * G + g) * D
-                                                                                         : decay + ((size_t)t * H + h) * D);
+            const float* from = src[n] + min(first + src_token[n], t1 - 1) * src_step[n];
             if constexpr (VEC) {
-                const float4 x = ok ? *(const float4*)(src + row) : make_float4(0.f, 0.f, 0.f, 0.f);
-                nxt[n][0] = x.x; nxt[n][W - 3] = x.y; nxt[n][W - 2] = x.z; nxt[n][W - 1] = x.w;
+                const float4 x = *(const float4*)from;
+                to.piece[n][0] = x.x; to.piece[n][W - 3] = x.y; to.piece[n][W - 2] = x.z; to.piece[n][W - 1] = x.w;
             } else {
-                nxt[n][0] = ok ? src[row] : 0.f;
+                to.piece[n][0] = *from;
             }
         }
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const bool live = first + p < t1;
-            v_nxt[p] = (live && col) ? v[(size_t)(first + p) * ldv + (size_t)h * V + j] : 0.f;
-            b_nxt[p] = live ? beta[(size_t)(first + p) * H + h] : 0.f;
-            kq_nxt[p] = live ? kq_all[(size_t)(first + p) * G + g] : 0.f;
-        }
+        const size_t mine = min(first + lane % P, t1 - 1);
+        to.v = v[mine * ldv + (size_t)h * V + (col ? j : 0)];
+        to.beta = beta[mine * H + h];
+        to.kq = kq_all[mine * G + g];
     };
-    auto stage = [&](int slot) {
+    auto stage = [&](const Group& from, int slot) {
 #pragma unroll
         for (int n = 0; n < NL; ++n) {
             const int idx = n * NT + tid;
             if (idx < P * PIECES) {
                 float* dst = &kqd[slot][0][0][0] + (size_t)idx * W;
-                if constexpr (VEC) *(float4*)dst = make_float4(nxt[n][0], nxt[n][W - 3], nxt[n][W - 2], nxt[n][W - 1]);
-                else *dst = nxt[n][0];
+                const bool in = src_in[n];
+                if constexpr (VEC) *(float4*)dst = make_float4(in ? from.piece[n][0] : 0.f, in ? from.piece[n][W - 3] : 0.f, in ? from.piece[n][W - 2] : 0.f, in ? from.piece[n][W - 1] : 0.f);
+                else *dst = in ? from.piece[n][0] : 0.f;
             }
         }
     };
-    fetch(t0);
-    stage(0);
-    __syncthreads();
-    for (int first = t0, cur = 0; first < t1; first += P, cur ^= 1) {
-        float v_cur[P], b_cur[P], kq_cur[P];
+    // One group of tokens, staged in slot X and held in ahead[X]; the next one is in ahead[1 - X] or on its way there.
+    auto group = [&](auto slot, int first) {
+        constexpr int X = decltype(slot)::value;
+        const float v_now = ahead[X].v, beta_now = ahead[X].beta, kq_now = ahead[X].kq;
+        fetch(ahead[X], first + 2 * P);              // two groups ahead: a group's work is shorter than a trip to memory
+        float o_mine = 0.f;
+        float4 ops[2][3][DR / 4];                    // (k, q, decay) of this token and of the next, read while this one is worked on
+        auto read = [&](int p) {
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            v_cur[p] = v_nxt[p];
-            b_cur[p] = b_nxt[p];
-            kq_cur[p] = kq_nxt[p];
-        }
-        const bool more = first + P < t1;
-        if (more) fetch(first + P);                  // the next group's operands leave now and are staged after this group's work
-        auto token = [&](int p, int t) {
-            const float* kk = &kqd[cur][p][0][r * DR];
-            const float* qq = &kqd[cur][p][1][r * DR];
-            const float* dd = &kqd[cur][p][2][r * DR];
+            for (int w = 0; w < 3; ++w)
+#pragma unroll
+                for (int i = 0; i < DR / 4; ++i) ops[p & 1][w][i] = *(const float4*)&kqd[X][p][w][r * DR + 4 * i];
+        };
+        auto token = [&](auto pc) {
+            constexpr int p = decltype(pc)::value;
             float kv[DR];
             float sk = 0.f, sq = 0.f;
 #pragma unroll
             for (int i = 0; i < DR; i += 4) {
-                const float4 k4 = *(const float4*)(kk + i), q4 = *(const float4*)(qq + i), d4 = *(const float4*)(dd + i);
+                const float4 k4 = ops[p & 1][0][i / 4], q4 = ops[p & 1][1][i / 4], d4 = ops[p & 1][2][i / 4];
                 const float ka[4] = {k4.x, k4.y, k4.z, k4.w}, qa[4] = {q4.x, q4.y, q4.z, q4.w}, da[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -397,23 +435,39 @@ __global__ __launch_bounds__(NW * 64) void channel_delta_kernel(const float* __r
                     kv[i + e] = ka[e];
                 }
             }
-            sk = column_sum<LPC>(sk);
-            sq = column_sum<LPC>(sq);
-            const float u = b_cur[p] * (v_cur[p] - sk);
-            if (col && r == 0) out[(size_t)t * ldo + (size_t)h * V + j] = fmaf(u, kq_cur[p], sq);
+            column_sums<LPC>(sk, sq);
+            const float u = row_lane<p>(beta_now) * (row_lane<p>(v_now) - sk), o = fmaf(u, row_lane<p>(kq_now), sq);
+            o_mine = r == p ? o : o_mine;            // (every lane of the column has it: lane p keeps token p's for the store)
 #pragma unroll
             for (int i = 0; i < DR; ++i) S[i] = fmaf(kv[i], u, S[i]);
         };
-        if (first + P <= t1) {                       // a whole group: one stretch of code, so that a token's LDS reads leave
-#pragma unroll                                       // while the token before it is worked on
-            for (int p = 0; p < P; ++p) token(p, first + p);
+        if (first + P <= t1) {                       // a whole group: one stretch of code
+            read(0);
+            tokens(std::make_integer_sequence<int, P>{}, [&](auto pc) {
+                constexpr int p = decltype(pc)::value;
+                if (p + 1 < P) read(p + 1);
+                __builtin_amdgcn_sched_barrier(0);   // (the reads leave here, not where they are waited for)
+                token(pc);
+            });
         } else {
-#pragma unroll
-            for (int p = 0; p < P; ++p)
-                if (first + p < t1) token(p, first + p);
+            tokens(std::make_integer_sequence<int, P>{}, [&](auto pc) {
+                if (first + decltype(pc)::value < t1) {
+                    read(decltype(pc)::value);
+                    token(pc);
+                }
+            });
         }
-        if (more) stage(cur ^ 1);                    // (the buffer that every wave left before the last barrier)
+        if (col && r < P && first + r < t1) out[(size_t)(first + r) * ldo + (size_t)h * V + j] = o_mine;
+        stage(ahead[1 - X], 1 - X);                  // (the buffer that every wave left before the last barrier)
         __syncthreads();
+    };
+    fetch(ahead[0], t0);
+    fetch(ahead[1], t0 + P);
+    stage(ahead[0], 0);
+    __syncthreads();
+    for (int first = t0; first < t1; first += 2 * P) {
+        group(std::integral_constant<int, 0>{}, first);
+        if (first + P < t1) group(std::integral_constant<int, 1>{}, first + P);
     }
 #pragma unroll
     for (int i = 0; i < DR; i += 4) {

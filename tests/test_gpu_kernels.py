@@ -185,7 +185,7 @@ def test_plain_products_have_the_same_bits_in_every_tile(M, N):
                 assert torch.equal(ops.gemm(a, w[:N // 2 * 2], epilogue=ops.EPI_GATED), gated), tile
 
 
-@pytest.mark.parametrize("K", [64, 128, 192, 256, 576])      # one step of 64 k, an even and an odd number of them
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 576])      # steps of 64 k: fewer than stages, as many, one and more beyond
 @pytest.mark.parametrize("M,N", [(129, 264), (500, 392)])
 def test_tiles_in_quarters_have_the_bits_of_the_ring(M, N, K):
     """Every shape of tile that is worked on in quarters, rows and columns that end inside a tile, every epilogue."""
@@ -1283,3 +1283,42 @@ def test_sorted_experts_through_either_product(T, E, k, I, H):
         close(y, ref, dtype, f"sorted experts, few_rows {few}", k=I)
         outs.append(y)
     assert float((outs[0] - outs[1]).abs().max()) <= 2e-2 * float(ref.abs().max())
+
+
+# one case per instance of the kernel: 16 and 32 lanes a column, whole pieces of four rows and single ones, columns and rows past the end
+@pytest.mark.parametrize("D,V,H,G", [(64, 32, 2, 1), (64, 48, 2, 2), (33, 20, 2, 1), (30, 70, 1, 1), (128, 128, 4, 2), (100, 30, 2, 2), (66, 9, 2, 2),
+                                     (256, 24, 2, 1), (129, 17, 1, 1)])
+def test_delta_rule_at_every_length_of_a_group(D, V, H, G):
+    """Tokens travel in groups of eight, two groups ahead: lengths that end inside the first, second and third group, side by
+    side, and the same sequences cut in two.  Sums of up to 256 terms in float32: 1e-6 of a result's norm is ten times what is seen."""
+    from ferrox_amd import ops
+    lengths = [1, 7, 8, 9, 16, 17, 24, 31]
+    T, n = sum(lengths), len(lengths)
+    q, k = rnd(T, G, D), rnd(T, G, D, seed=1)
+    q, k = q / q.norm(dim=-1, keepdim=True), k / k.norm(dim=-1, keepdim=True)
+    decay, beta, v = torch.exp(-0.2 * rnd(T, H, D, seed=2).abs()), torch.sigmoid(rnd(T, H, seed=3)), rnd(T, H * V + 3, seed=4)[:, :H * V]
+    kq, before = (k * q).sum(-1), rnd(n, H, V, D, seed=5)
+    flat = lambda x, lo, hi: x[lo:hi].reshape(hi - lo, -1).contiguous()
+
+    def run(lo, hi, starts, slots, state):
+        return ops.channel_delta(flat(q, lo, hi), flat(k, lo, hi), flat(decay, lo, hi), flat(beta, lo, hi), flat(kq, lo, hi), v[lo:hi], state,
+                                 torch.tensor(starts, dtype=torch.int32, device=DEV), torch.tensor(slots, dtype=torch.int32, device=DEV), len(slots), H, G, D, V)
+
+    at = [sum(lengths[:i]) for i in range(n + 1)]
+    state = before.clone()
+    out = run(0, T, at, list(range(n)), state)
+    for i in range(n):
+        S = before[i].double().transpose(1, 2)
+        want = torch.empty(lengths[i], H, V, dtype=torch.float64, device=DEV)
+        for t in range(at[i], at[i + 1]):
+            kt, qt = (x[t].double().repeat_interleave(H // G, 0)[..., None] for x in (k, q))
+            S = decay[t].double()[..., None] * S
+            u = beta[t].double()[:, None] * (v[t].double().view(H, V) - (S * kt).sum(1))
+            S = S + kt * u[:, None]
+            want[t - at[i]] = (S * qt).sum(1)
+        got = out[at[i]:at[i + 1]].double().view(-1, H, V)
+        assert (got - want).norm() < 1e-6 * want.norm() and (state[i].double().transpose(1, 2) - S).norm() < 1e-6 * S.norm(), lengths[i]
+        # in two portions: the same bits
+        cut, part = lengths[i] // 2, before.clone()
+        halves = [run(lo, hi, [0, hi - lo], [i], part) for lo, hi in ((at[i], at[i] + cut), (at[i] + cut, at[i + 1])) if hi > lo]
+        assert torch.equal(torch.cat(halves), out[at[i]:at[i + 1]]) and torch.equal(part[i], state[i]), lengths[i]

@@ -1639,10 +1639,13 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(GemmArgs g) {
 }
 
 // Few rows: the weights go from memory straight into operands, every wave a part of K, 16 * MT rows and NW sets of 16
-// weight rows a block (DUAL: the sets alternate between the two matrices); 64 k a step, the next step's loads issued
-// before this step's products; the parts' sums meet in LDS.  Bound by the stream of the weights: 4 rows against 6,144 x
-// 2,048 17 us (3 TB/s, launch included; the FMA kernel's tile of 64 rows took 253).
-template <int MT, int NW, bool DUAL, int EPI, bool VEC>
+// weight rows a block (DUAL: the sets alternate between the two matrices); 32 k a step, the next step's loads issued
+// before this step's products; the parts' sums meet in LDS.  LINES (rows of whole 32 k): the weights come in whole lines of 128 bytes
+// with the non-temporal hint, the halves changing places before the products (`load_lines16`).  Bound by the stream of the weights: 4 rows
+// against 6,144 x 2,048 15.5 us, gate/up of 5,632 24.3, 15 experts' gate/up 63 (5.5 TB/s), the head of 151,936 235 (5.3 TB/s).  With half
+// lines and steps of 64 k these took 17.6, 30.0, 75 and 275: twice the registers a step leave half the waves, and it
+// is waves, not deeper loads, that keep memory busy (steps of 128 k: 19.9, 33.3, 95 and 329).
+template <int MT, int NW, bool DUAL, int EPI, bool VEC, bool LINES>
 __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
     __shared__ f32x4_t red[F32_PARTS][MT * NW][64];
@@ -1653,7 +1656,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
     const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
     const float* x_src[MT];
-    const float* w_src[NW];
+    const float* w_src[NW][LINES ? 2 : 1];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         int m = r0 + i * 16 + li;
@@ -1662,13 +1665,17 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     }
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
-        int n = n0 + (DUAL ? a >> 1 : a) * 16 + li;
-        n = n < g.N ? n : g.N - 1;
-        w_src[a] = Wbase + (size_t)n * g.K + (DUAL && (a & 1) ? g.up_offset : 0);
+#pragma unroll
+        for (int half = 0; half < (LINES ? 2 : 1); ++half) {
+            // LINES: what the lane loads is of row li % 8, and of row li % 8 + 8; else of row li
+            int n = n0 + (DUAL ? a >> 1 : a) * 16 + (LINES ? (li & 7) + 8 * half : li);
+            n = n < g.N ? n : g.N - 1;
+            w_src[a][half] = Wbase + (size_t)n * g.K + (DUAL && (a & 1) ? g.up_offset : 0) + (LINES ? (li >> 3) * 16 + gq * 4 : 0);
+        }
     }
     const int part = f32_part_length(g.K);
     const int k_first = wave * part, k_end = k_first + part < g.K ? k_first + part : g.K;
-    constexpr int STEP = MT > 1 ? 2 : 4;       // groups of 16 k that are on their way together
+    constexpr int STEP = 2;       // groups of 16 k that are on their way together
     f32x4_t w[2][STEP][NW], x[2][STEP][MT];
     const int k_full = k_first + (k_end - k_first) / 16 * 16;
     auto fetch = [&](int b, int k0) {
@@ -1676,7 +1683,14 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
         for (int c = 0; c < STEP; ++c) {
             const int kc = k0 + c * 16, k = (kc < k_full ? kc : k_full - 16) + gq * 4;
 #pragma unroll
-            for (int a = 0; a < NW; ++a) w[b][c][a] = f32_fetch<VEC>(w_src[a] + k);
+            for (int a = 0; a < NW; ++a) {
+                if constexpr (LINES) {
+                    const int pair = k0 + (c & ~1) * 16;        // 32 k, a line of each row
+                    w[b][c][a] = __builtin_bit_cast(f32x4_t, load_lines16(w_src[a][c & 1] + (pair < k_full ? pair : k_full - 32)));
+                } else {
+                    w[b][c][a] = f32_fetch<VEC>(w_src[a][0] + k);
+                }
+            }
 #pragma unroll
             for (int i = 0; i < MT; ++i) x[b][c][i] = f32_fetch<VEC>(x_src[i] + k);
         }
@@ -1695,13 +1709,25 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
                 fetch(b ^ 1, kb + STEP * 16);
 #pragma unroll
                 for (int c = 0; c < STEP; ++c)
-                    if (kb + c * 16 < k_full) f32_multiply(acc, w[b][c], x[b][c]);
+                    if (kb + c * 16 < k_full) {
+                        if constexpr (LINES) {
+                            f32x4_t own[NW];
+#pragma unroll
+                            for (int a = 0; a < NW; ++a) {
+                                const uint4 keep = __builtin_bit_cast(uint4, w[b][c][a]), other = __builtin_bit_cast(uint4, w[b][c ^ 1][a]);
+                                own[a] = __builtin_bit_cast(f32x4_t, c & 1 ? swap_halves<0x3>(keep, other) : swap_halves<0xC>(keep, other));
+                            }
+                            f32_multiply(acc, own, x[b][c]);
+                        } else {
+                            f32_multiply(acc, w[b][c], x[b][c]);
+                        }
+                    }
             }
         }
     }
-    if (k_first < k_end && k_full < k_end) {       // the last, partial group of K
+    if (!LINES && k_first < k_end && k_full < k_end) {       // the last, partial group of K
 #pragma unroll
-        for (int a = 0; a < NW; ++a) w[0][0][a] = f32_fetch_guarded<VEC>(w_src[a], k_full + gq * 4, k_end);
+        for (int a = 0; a < NW; ++a) w[0][0][a] = f32_fetch_guarded<VEC>(w_src[a][0], k_full + gq * 4, k_end);
 #pragma unroll
         for (int i = 0; i < MT; ++i) x[0][0][i] = f32_fetch_guarded<VEC>(x_src[i], k_full + gq * 4, k_end);
         f32_multiply(acc, w[0][0], x[0][0]);
@@ -1819,13 +1845,18 @@ static void launch_ring(const GemmArgs& g, int epi, int m_tiles, hipStream_t s) 
     if (g.stream_w) launch_wide<TMB, TN, NS, NSA, true>(g, epi, m_tiles, s);
     else launch_wide<TMB, TN, NS, NSA, false>(g, epi, m_tiles, s);
 }
+template <bool DUAL, int EPI, bool VEC, bool LINES>
+static void launch_f32_skinny(const GemmArgs& g, int mt, int nw, dim3 grid, hipStream_t s) {
+    if (mt == 2) gemm_f32_skinny_kernel<2, 2, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
+    else if (nw == 2 || DUAL) gemm_f32_skinny_kernel<1, 2, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
+    else gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
+}
 template <bool DUAL, int EPI, bool VEC>
 static void launch_f32(const GemmArgs& g, int tile, int mt, int nw, dim3 grid, hipStream_t s) {
     if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
     else if (tile == 32) gemm_f32_tiled_kernel<32, DUAL ? 64 : 32, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
-    else if (mt == 2) gemm_f32_skinny_kernel<2, 2, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
-    else if (nw == 2 || DUAL) gemm_f32_skinny_kernel<1, 2, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
-    else gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC><<<grid, 512, 0, s>>>(g);
+    else if (VEC && g.K % 32 == 0) launch_f32_skinny<DUAL, EPI, VEC, VEC>(g, mt, nw, grid, s);
+    else launch_f32_skinny<DUAL, EPI, VEC, false>(g, mt, nw, grid, s);
 }
 
 template <int MT, int WAVES, int NW>
@@ -2065,19 +2096,21 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         const bool dual = epi == EPI_GATED;
         const long group = expert_offsets ? (M + E - 1) / E : M, cus = fx_compute_units();
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
-        // Up to 32 plain rows: the kernel for few rows (2,048 x 2,048 weights, 4 rows: 10 us against 30 with tiles of 32 and 45
-        // of 64; 32 rows: 22, 30 and 47), but where the weight rows are so many that tiles of 32 fill the GPU many times
-        // (the head's 151,936: 260 against 272 us at 4 rows, 240 the other way at one).  Tiles of 64 once they are two and
+        // Up to 32 plain rows: the kernel for few rows (2,048 x 2,048 weights, 4 rows: 9 us against 24 with tiles of 32 and 45
+        // of 64; 6,144 weight rows, 30 rows: 21, 33 and 47).  Tiles of 64 once they are two and
         // a half a CU (6,144 weight rows: 512 rows 121 against 139 us, 256 rows 76 against 71; 2,048 weight rows: 1,500
-        // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: tiles of 32 up to 36 rows an expert (60 experts'
-        // gate/up product of 2,048: one row 173 us against 172 for few rows and 266 with tiles of 64, its down product 94 against 114
-        // and 136; 4.3 rows 255, 267 and 390; 36 rows 419, 618 and 427; 47 rows 496 and 424 with tiles of 64.  Steps of one and two
-        // tokens are behind the kernel for few rows with gate/up, 30 and 26, 43 and 37 us).
+        // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: the kernel for few rows up to five rows an expert (60 experts' gate/up
+        // products of 2,048, of 4, 16, 32 and 64 tokens: 64, 156, 197 and 220 us against 68, 173, 224 and 250 with tiles of 32, their down products 32,
+        // 83, 108 and 122 against 37, 90, 115 and 129; 64 tokens on 35 of the experts 163 and 91 against 169 and 86; 96 tokens there 188 and 104
+        // against 172 and 90), tiles of 32 up to 36 rows an expert (36 rows 419 us against 427 with tiles of 64; 47 rows 496 against 424).
+        // The head's 151,936 weight rows: the kernel for few rows up to eight rows (4 rows 235 against 254 us, 16 rows 277 against 258).
+        // Where it cannot take whole lines it stays behind tiles of 32 with sorted rows, and from three rows on with the head's.
+        const bool lines = g.vec_ok && K % 32 == 0;
         int tile = 0, mt = 1, nw = 2;
         if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
-        else if (expert_offsets) tile = group <= 36 ? 32 : 64;
+        else if (expert_offsets) tile = lines && group <= 5 ? 0 : (group <= 36 ? 32 : 64);
         else {
-            const bool many_columns = ceil_div(N, 32) >= 8 * cus && M > 2;
+            const bool many_columns = ceil_div(N, 32) >= 8 * cus && M > (lines ? 8 : 2);
             if (M > 32 || many_columns) tile = M > 32 && 2 * (long)ceil_div(N, 64) * ceil_div(M, 64) >= 5 * cus ? 64 : 32;
         }
         if (!tile) {

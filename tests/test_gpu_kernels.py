@@ -74,6 +74,19 @@ def test_float32_products_have_the_same_bits_in_every_kernel(N, K):
     assert torch.equal(ops.gemm(wide[:, 1:K + 1], w, bias=bias), whole)
 
 
+@pytest.mark.parametrize("N,K", [(16, 32), (40, 64), (33, 256), (72, 288), (50, 544), (24, 2080)])
+def test_float32_few_rows_in_whole_lines(N, K):
+    """Rows of whole 32 k: parts of K with one line, several, an odd number and none (the last parts), columns past the end, one and
+    two tiles of rows; against float64 and, bit for bit, against tiles of 32."""
+    from ferrox_amd import debug, ops
+    for rows in (1, 5, 16, 17, 32):
+        a, w, w2 = rnd(rows, K), rnd(N, K, seed=1), rnd(2 * N, K, seed=3, scale=0.3)
+        got, gated = ops.gemm(a, w), ops.gemm(a, w2, epilogue=ops.EPI_GATED)
+        close(got, a.double() @ w.double().T, torch.float32, f"{rows} rows")
+        with debug.kernel_switch("gemm", "f32_tile", 32):
+            assert torch.equal(got, ops.gemm(a, w)) and torch.equal(gated, ops.gemm(a, w2, epilogue=ops.EPI_GATED)), rows
+
+
 @pytest.mark.parametrize("T,E,k,I,H", [(1, 5, 2, 20, 36), (3, 60, 4, 96, 128), (90, 7, 3, 33, 50), (700, 4, 2, 64, 96)])
 def test_float32_grouped_products_have_the_same_bits_in_every_kernel(T, E, k, I, H):
     from ferrox_amd import debug, ops

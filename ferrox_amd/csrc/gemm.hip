@@ -551,30 +551,79 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
     wait_loads_but<0>();                       // the loads past the end, before the block leaves
 }
 
-// Which tile of the output a block of the LDS-tiled kernels works on; false: none.
-__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& row_tile, int& col_tile) {
-    // Blocks go to the 8 XCDs in turn (block b runs on XCD b % 8), each with an L2 of its own.  Plain: an XCD
-    // works through a contiguous range of the tiles in an order that keeps neighbours in rows and columns
-    // together, so the operands of the tiles it has at a time stay in its L2.  Grouped: XCD x takes the row tiles x, x + 8, ... and runs through the column tiles of each, so an
-    // expert's rows are fetched once and stay in its L2 while its weights, which nothing reads twice, stream by
-    // (the row tiles past the last expert are empty; dealing them out in turn spreads them over the XCDs).
-    if (g.expert_offsets) {
-        const int i = blockIdx.x / 8;
-        row_tile = (i / g.n_col_tiles) * 8 + blockIdx.x % 8;
-        col_tile = i % g.n_col_tiles;
-        if (row_tile >= g.n_row_tiles) return false;
-    } else {
-        const int per_xcd = (g.n_col_tiles * g.n_row_tiles + 7) / 8;
-        const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-        if (logical >= g.n_col_tiles * g.n_row_tiles) return false;
-        // bands of 8 row tiles, rows fastest inside a band: the 32 tiles that an XCD works on at a time are
-        // 8 rows x 4 columns, so 12 operand tiles serve 32 products
-        const int band = logical / (8 * g.n_col_tiles), rem = logical % (8 * g.n_col_tiles);
-        const int band_rows = min(8, g.n_row_tiles - band * 8);
-        row_tile = band * 8 + rem % band_rows;
-        col_tile = rem / band_rows;
+// Which tile of the output a block of the LDS-tiled kernels works on; false: none.  Blocks go to the 8 XCDs in turn (block
+// b runs on XCD b % 8), each with an L2 of its own: an XCD works through a contiguous eighth of the tiles in an order that keeps
+// neighbours in rows and columns together, so the operands of the tiles it has at a time stay in its L2.  That order is bands of
+// 8 row tiles, rows fastest inside a band: the 32 tiles that an XCD works on at a time are 8 rows x 4 columns, and 12 operand
+// tiles serve 32 products.
+// Rows sorted by expert, tiles in quarters: expert after expert, each in that order; how many tiles there are is counted from the
+// experts' shares (64 at a time, a lane each, as in `locate_rows`), blocks beyond them find none.  What an expert's row tiles have in
+// common, its weights, is then fetched by the one or two XCDs that its tiles fall to.  (BY_ROW_TILE, the rings: XCD x takes the row
+// tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles share are fetched by two XCDs, but no XCD has many
+// full tiles where another has nearly empty ones.  With that the tiles in quarters took 147 us instead of 139 for the gate/up product of 2,048
+// tokens on 30 of 60 experts, 236 instead of 195 for 3,500, 1,297 and 667 instead of 1,245 and 626 for both of 4,096 tokens of
+// the larger model; the rings the other way, 512 tokens on 40 experts 55 against 66 us for the down product.  Eighths of equal cost, a tile's
+// rows and a constant, instead of equal numbers of tiles: no better, 237 us for the 3,500.)
+template <int TM, bool BY_ROW_TILE>
+__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile) {
+    const int lane = threadIdx.x & 63, C = g.n_col_tiles;
+    if (BY_ROW_TILE && g.expert_offsets) {
+        const int i = blockIdx.x / 8, row_tile = (i / C) * 8 + blockIdx.x % 8;
+        col_tile = i % C;
+        locate_rows<TM>(g, row_tile, r0, r_end, expert);       // (r0 < 0: past the last one)
+        return r0 >= 0;
     }
-    return true;
+    auto share = [&](int base, int& b, int& en) {       // row tiles of expert base + lane
+        const int e = base + lane;
+        b = e < g.E ? g.expert_offsets[e] : 0;
+        en = e < g.E ? g.expert_offsets[e + 1] : 0;
+        return (en - b + TM - 1) / TM;
+    };
+    auto in_bands = [&](int t, int rows, int& row) {    // tile t of rows x C tiles
+        const int band = t / (8 * C), rem = t % (8 * C), band_rows = min(8, rows - band * 8);
+        row = band * 8 + rem % band_rows;
+        col_tile = rem / band_rows;
+    };
+    int rows = g.n_row_tiles, b = 0, en = 0, nt = 0, incl = 0;
+    if (g.expert_offsets) {
+        rows = 0;
+        for (int base = 0; base < g.E; base += 64) {
+            nt = share(base, b, en);
+            incl = wave_inclusive_sum(nt);
+            rows += __builtin_amdgcn_readlane(incl, 63);
+        }
+    }
+    const int per_xcd = (C * rows + 7) / 8, i = blockIdx.x / 8;
+    const int logical = (blockIdx.x % 8) * per_xcd + i;
+    if (i >= per_xcd || logical >= C * rows) return false;
+    if (!g.expert_offsets) {
+        int row;
+        in_bands(logical, rows, row);
+        r0 = row * TM;
+        r_end = g.M;
+        expert = 0;
+        return true;
+    }
+    int before = 0;
+    for (int base = 0; base < g.E; base += 64) {
+        if (g.E > 64) {
+            nt = share(base, b, en);
+            incl = wave_inclusive_sum(nt);
+        }
+        const int first = (before + incl - nt) * C;
+        const unsigned long long hit = __ballot(logical >= first && logical < first + nt * C);
+        if (hit) {
+            const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
+            int row;
+            in_bands(logical - __builtin_amdgcn_readlane(first, src), __builtin_amdgcn_readlane(nt, src), row);
+            r0 = __builtin_amdgcn_readlane(b, src) + row * TM;
+            r_end = __builtin_amdgcn_readlane(en, src);
+            expert = base + src;
+            return true;
+        }
+        before += __builtin_amdgcn_readlane(incl, 63);
+    }
+    return false;
 }
 
 // What the accumulators of a wave go through on their way to C: MT row blocks (2i + wm of the tile's), NT column blocks.
@@ -678,11 +727,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
     static_assert(TM % 64 == 0 && TN % 64 == 0, "eight waves load 64 rows at a time");
     __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
 
-    int row_tile, col_tile;
-    if (!wide_tile(g, row_tile, col_tile)) return;
-    int r0, r_end, expert;
-    locate_rows<TM>(g, row_tile, r0, r_end, expert);
-    if (r0 < 0) return;
+    int r0, r_end, expert, col_tile;
+    if (!wide_tile<TM, true>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -924,11 +970,8 @@ __global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
     static_assert(MA0 % 2 == 0 && MA1 % 2 == 0 && MA1 > 0 && NB1 > 0, "eight waves load 64 rows at a time, a part at a time");
     __shared__ __attribute__((aligned(1024))) bf16 stages[2 * (TM + TN) * 64];
 
-    int row_tile, col_tile;
-    if (!wide_tile(g, row_tile, col_tile)) return;
-    int r0, r_end, expert;
-    locate_rows<TM>(g, row_tile, r0, r_end, expert);
-    if (r0 < 0) return;
+    int r0, r_end, expert, col_tile;
+    if (!wide_tile<TM, false>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -1805,14 +1848,14 @@ FX_API int fx_debug_set(const char* key, int value) {
 }
 
 // The grid of the LDS-tiled kernels, which decode their block's tile themselves.
-static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles) {
+static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles, bool by_row_tile) {
     g.n_col_tiles = ceil_div(g.N, epi == EPI_GATED ? tn / 2 : tn);
     g.n_row_tiles = m_tiles;
-    return dim3(g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
+    return dim3(by_row_tile && g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
 }
 template <int TMB, int TN, int NS, int NSA, bool STREAM>
 static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
-    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles, true);
     switch (epi) {
         case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
@@ -1824,7 +1867,7 @@ static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
 }
 template <int TMB, int TN>
 static void launch_quarters(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
-    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles, false);
     switch (epi) {
         case EPI_STORE: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE_F32><<<grid, 512, 0, s>>>(g); break;

@@ -66,6 +66,15 @@ def test_tiles_twice_as_wide():
     assert not rule(1000, 5632, 1) and rule(4096, 2048) and not rule(4097, 2048) and not rule(4096, 2048, cus=192)
 
 
+def test_tiles_of_96_rows():
+    """In place of 128 rows while tiles of 96 are one round of the CUs too."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, n, tile, dual=0, cus=256: bool(load_library("gemm").fx_gemm_lower_tiles(m, n, tile, dual, cus))
+    assert rule(1337, 2048, 64) and rule(1536, 2048, 64) and not rule(1537, 2048, 64) and rule(1337, 4096, 8256)
+    assert not rule(1000, 6144, 8256) and rule(512, 2816, 8256, 1) and not rule(512, 5632, 8256, 1)
+    assert not rule(1337, 2048, 8128) and not rule(1337, 2048, 256) and not rule(1337, 2048, 64, cus=200)
+
+
 def test_the_chunk_rule_leaves_the_callers_arguments_alone():
     """The rule counts waves per block; it once did so in a variable named like the `waves` argument of
     `attention_decode`, which then reached the launch instead of the caller's value."""

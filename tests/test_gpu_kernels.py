@@ -214,7 +214,7 @@ def test_tiles_in_quarters_have_the_bits_of_the_ring(M, N, K):
     with debug.kernel_switch("gemm", "wide", 4):          # 64 x 256, whose stages go round in a ring
         want = products()
     close(want[1], a.double() @ w.double().T, dtype, "product")
-    for tile in (256, 192, 128, 12, 8256, 8128):
+    for tile in (256, 192, 128, 12, 8256, 8128, 6256, 6128):
         with debug.kernel_switch("gemm", "wide", tile):
             for x, y, what in zip(products(), want, ("store + bias", "store float32", "residual", "gated")):
                 assert torch.equal(x, y), (tile, what)

@@ -74,7 +74,7 @@ struct GemmArgs {
     int vec_ok;  // 16-byte loads are legal for A and W
     int c_vec;   // float32: so are 16-byte loads and stores of C
     int n_col_tiles, n_row_tiles;  // tiled kernels: the grid they decode block ids with
-    int tile_rows;  // tiles in quarters, plain rows: rows a tile takes, up to its height
+    int tile_rows;  // LDS-tiled kernels, plain rows: rows a tile takes, up to its height
 };
 
 // block -> (first logical row, end of rows, expert).  Plain: tiles of TM rows.
@@ -557,13 +557,13 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
 // neighbours in rows and columns together, so the operands of the tiles it has at a time stay in its L2.  That order is bands of
 // 8 row tiles, rows fastest inside a band: the 32 tiles that an XCD works on at a time are 8 rows x 4 columns, and 12 operand
 // tiles serve 32 products.
-// Rows sorted by expert, tiles in quarters: expert after expert, each in that order; how many tiles there are is counted from the
+// Rows sorted by expert: expert after expert, each in that order; how many tiles there are is counted from the
 // experts' shares (64 at a time, a lane each, as in `locate_rows`), blocks beyond them find none.  What an expert's row tiles have in
-// common, its weights, is then fetched by the one or two XCDs that its tiles fall to.  (BY_ROW_TILE, the rings: XCD x takes the row
+// common, its weights, is then fetched by the one or two XCDs that its tiles fall to.  (BY_ROW_TILE, the rings of 128 and 192 rows: XCD x takes the row
 // tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles share are fetched by two XCDs, but no XCD has many
 // full tiles where another has nearly empty ones.  With that the tiles in quarters took 147 us instead of 139 for the gate/up product of 2,048
 // tokens on 30 of 60 experts, 236 instead of 195 for 3,500, 1,297 and 667 instead of 1,245 and 626 for both of 4,096 tokens of
-// the larger model; the rings the other way, 512 tokens on 40 experts 55 against 66 us for the down product.  Eighths of equal cost, a tile's
+// the larger model; the ring of 192 rows the other way, 512 tokens on 40 experts 55 against 66 us for the down product.  Eighths of equal cost, a tile's
 // rows and a constant, instead of equal numbers of tiles: no better, 237 us for the 3,500.)
 template <int TM, bool BY_ROW_TILE>
 __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile) {
@@ -600,8 +600,8 @@ __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end
     if (!g.expert_offsets) {
         int row;
         in_bands(logical, rows, row);
-        r0 = row * (BY_ROW_TILE ? TM : g.tile_rows);
-        r_end = BY_ROW_TILE ? g.M : min(g.M, r0 + g.tile_rows);
+        r0 = row * g.tile_rows;
+        r_end = min(g.M, r0 + g.tile_rows);
         expert = 0;
         return true;
     }
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
 
     int r0, r_end, expert, col_tile;
-    if (!wide_tile<TM, true>(g, r0, r_end, expert, col_tile)) return;
+    if (!wide_tile<TM, (TMB > 4)>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -1825,7 +1825,7 @@ static int g_skinny_mt = 0;    // "skinny_row_tiles": 1, 2 or 4 tiles of 16 rows
 static int g_skinny_waves = 0; // "skinny_waves": 1, 2, 4 or 8 waves that split K in a block of that product (0: by the sizes)
 static int g_few_rows = 3;     // "few_rows": sorted by expert, up to this many rows an expert go to the product for few rows (at most 64)
 static int g_head_rows = 16;   // "head_rows": plain rows against very many weight rows go to the tiled kernel from more than this many on
-static int g_tile64_rows = 20; // "tile64_rows": experts with up to this many rows on average take tiles of 64 rows
+static int g_tile64_rows = 36; // "tile64_rows": experts with up to this many rows on average take tiles of 64 rows
 static int g_no_wide = 0;      // "wide": 0 sends many-row products to the register-staged tiled kernel, 1 (default) by the sizes,
 static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to the product for few rows whatever the weight rows (0: by the sizes)
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
@@ -1856,7 +1856,8 @@ static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles, bool by_row_til
 }
 template <int TMB, int TN, int NS, int NSA, bool STREAM>
 static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
-    const dim3 grid = wide_grid(g, epi, TN, m_tiles, true);
+    g.tile_rows = 16 * TMB;
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles, TMB > 4);
     switch (epi) {
         case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
@@ -2066,11 +2067,16 @@ FX_API int fx_gemm_lower_tiles(int M, int N, int tile, int dual, int cus) {
 }
 // The same for rows sorted by expert.
 static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, int cus) {
-    // an expert's share of up to 20 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
-    // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three, the same bits: decode
-    // at 64 sequences 11.2 -> 11.0 ms, a 192-token step 6.8 -> 6.4 ms; from 25 rows on average on, steps of 384
-    // tokens, more and more experts need a second tile and it falls behind)
+    // an expert's share of up to 36 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
+    // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three at up to 20 rows; with an XCD on a
+    // contiguous eighth of the tiles also beyond, where experts need a second tile: gate/up and down of 512 tokens on all of 60 experts 122 and 67 -> 116
+    // and 65 us, on 40 of them 104 and 55 -> 98 and 52; 200 tokens of the larger model on 40 of 64 experts 265 and 158 -> 244 and 144)
     if (per_group <= g_tile64_rows) return 4;
+    // up to 96 rows, a prompt's tokens, which crowd into some of the experts: tiles of 128 x 256 in quarters (700 tokens on 35 experts
+    // 94 and 57 -> 87 and 50 us, 1,000 on 30 experts 107 and 64 -> 85 and 50, 400 of the larger model on 40 experts 290 and 170 -> 271 and
+    // 159; spread evenly 127 and 71 -> 129 and 74, 136 and 75 -> 135 and 79, 376 and 224 -> 387 and 227).  From 113 rows on an even share spills into
+    // second tiles (900 tokens of the larger model 436 and 250 -> 478 and 274).
+    if (per_group <= 96) return 8256;
     // a share of up to 192 rows: the product streams the weights once and multiplies little, so it
     // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows
     // (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of

@@ -75,6 +75,7 @@ struct GemmArgs {
     int c_vec;   // float32: so are 16-byte loads and stores of C
     int n_col_tiles, n_row_tiles;  // tiled kernels: the grid they decode block ids with
     int tile_rows;  // LDS-tiled kernels, plain rows: rows a tile takes, up to its height
+    int by_row_tile;  // LDS-tiled kernels, rows sorted by expert: every eighth row tile to an XCD
 };
 
 // block -> (first logical row, end of rows, expert).  Plain: tiles of TM rows.
@@ -559,16 +560,16 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
 // tiles serve 32 products.
 // Rows sorted by expert: expert after expert, each in that order; how many tiles there are is counted from the
 // experts' shares (64 at a time, a lane each, as in `locate_rows`), blocks beyond them find none.  What an expert's row tiles have in
-// common, its weights, is then fetched by the one or two XCDs that its tiles fall to.  (BY_ROW_TILE, the rings of 128 and 192 rows: XCD x takes the row
+// common, its weights, is then fetched by the one or two XCDs that its tiles fall to.  (`by_row_tile`: XCD x takes the row
 // tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles share are fetched by two XCDs, but no XCD has many
 // full tiles where another has nearly empty ones.  With that the tiles in quarters took 147 us instead of 139 for the gate/up product of 2,048
 // tokens on 30 of 60 experts, 236 instead of 195 for 3,500, 1,297 and 667 instead of 1,245 and 626 for both of 4,096 tokens of
 // the larger model; the ring of 192 rows the other way, 512 tokens on 40 experts 55 against 66 us for the down product.  Eighths of equal cost, a tile's
 // rows and a constant, instead of equal numbers of tiles: no better, 237 us for the 3,500.)
-template <int TM, bool BY_ROW_TILE>
+template <int TM>
 __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile) {
     const int lane = threadIdx.x & 63, C = g.n_col_tiles;
-    if (BY_ROW_TILE && g.expert_offsets) {
+    if (g.by_row_tile && g.expert_offsets) {
         const int i = blockIdx.x / 8, row_tile = (i / C) * 8 + blockIdx.x % 8;
         col_tile = i % C;
         locate_rows<TM>(g, row_tile, r0, r_end, expert);       // (r0 < 0: past the last one)
@@ -729,7 +730,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
 
     int r0, r_end, expert, col_tile;
-    if (!wide_tile<TM, (TMB > 4)>(g, r0, r_end, expert, col_tile)) return;
+    if (!wide_tile<TM>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -972,7 +973,7 @@ __global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) bf16 stages[2 * (TM + TN) * 64];
 
     int r0, r_end, expert, col_tile;
-    if (!wide_tile<TM, false>(g, r0, r_end, expert, col_tile)) return;
+    if (!wide_tile<TM>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -1849,15 +1850,15 @@ FX_API int fx_debug_set(const char* key, int value) {
 }
 
 // The grid of the LDS-tiled kernels, which decode their block's tile themselves.
-static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles, bool by_row_tile) {
+static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles) {
     g.n_col_tiles = ceil_div(g.N, epi == EPI_GATED ? tn / 2 : tn);
     g.n_row_tiles = m_tiles;
-    return dim3(by_row_tile && g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
+    return dim3(g.by_row_tile && g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
 }
 template <int TMB, int TN, int NS, int NSA, bool STREAM>
 static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
     g.tile_rows = 16 * TMB;
-    const dim3 grid = wide_grid(g, epi, TN, m_tiles, TMB > 4);
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
     switch (epi) {
         case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
@@ -1870,7 +1871,7 @@ static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
 template <int TMB, int TN>
 static void launch_quarters(GemmArgs g, int epi, int m_tiles, hipStream_t s, int rows = 16 * TMB) {
     g.tile_rows = rows;
-    const dim3 grid = wide_grid(g, epi, TN, m_tiles, false);
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
     switch (epi) {
         case EPI_STORE: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE><<<grid, 512, 0, s>>>(g); break;
         case EPI_STORE_F32: gemm_bf16_quarters_kernel<TMB, TN, false, EPI_STORE_F32><<<grid, 512, 0, s>>>(g); break;
@@ -2157,16 +2158,16 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // Up to 32 plain rows: the kernel for few rows (2,048 x 2,048 weights, 4 rows: 9 us against 24 with tiles of 32 and 45
         // of 64; 6,144 weight rows, 30 rows: 21, 33 and 47).  Tiles of 64 once they are two and
         // a half a CU (6,144 weight rows: 512 rows 121 against 139 us, 256 rows 76 against 71; 2,048 weight rows: 1,500
-        // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: the kernel for few rows up to five rows an expert (60 experts' gate/up
+        // rows 112 against 129, 700 rows 74 against 67).  Sorted rows: the kernel for few rows up to two rows an expert (60 experts' gate/up
         // products of 2,048, of 4, 16, 32 and 64 tokens: 64, 156, 197 and 220 us against 68, 173, 224 and 250 with tiles of 32, their down products 32,
-        // 83, 108 and 122 against 37, 90, 115 and 129; 64 tokens on 35 of the experts 163 and 91 against 169 and 86; 96 tokens there 188 and 104
-        // against 172 and 90), tiles of 32 up to 36 rows an expert (36 rows 419 us against 427 with tiles of 64; 47 rows 496 against 424).
+        // 83, 108 and 122 against 37, 90, 115 and 129; but the tokens of one prompt crowd: 64 on 35 of the experts 163 and 91 against 169 and 86, 96 there 188 and 104
+        // against 172 and 90, a prompt of 60 tokens of six layers 2,631 against 2,512), tiles of 32 up to 36 rows an expert (36 rows 419 us against 427 with tiles of 64; 47 rows 496 against 424).
         // The head's 151,936 weight rows: the kernel for few rows up to eight rows (4 rows 235 against 254 us, 16 rows 277 against 258).
         // Where it cannot take whole lines it stays behind tiles of 32 with sorted rows, and from three rows on with the head's.
         const bool lines = g.vec_ok && K % 32 == 0;
         int tile = 0, mt = 1, nw = 2;
         if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
-        else if (expert_offsets) tile = lines && group <= 5 ? 0 : (group <= 36 ? 32 : 64);
+        else if (expert_offsets) tile = lines && group <= 2 ? 0 : (group <= 36 ? 32 : 64);
         else {
             const bool many_columns = ceil_div(N, 32) >= 8 * cus && M > (lines ? 8 : 2);
             if (M > 32 || many_columns) tile = M > 32 && 2 * (long)ceil_div(N, 64) * ceil_div(M, 64) >= 5 * cus ? 64 : 32;
@@ -2286,6 +2287,10 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         }
         else if (!tile) tile = small_groups ? 64 : grouped_tile(per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
+        // every eighth row tile to an XCD: the ring of 192 rows, and tiles of 64 for up to five rows an expert, which seldom need a second
+        // one (decoding 30 sequences of the larger model 2,902 us a step, 3,013 with contiguous eighths; a prompt of 117 tokens, eight an
+        // expert, the other way, 4,497 and 4,108)
+        g.by_row_tile = expert_offsets && (tile == 4 ? per_group <= 5 : tile == 12 && g.stream_w);
         switch (tile) {
             case 464: launch_ring<4, 64, 4>(g, epi, row_tiles(64), s); break;
             case 4128: launch_ring<4, 128, 3>(g, epi, row_tiles(64), s); break;

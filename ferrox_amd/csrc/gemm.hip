@@ -2079,8 +2079,8 @@ static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, i
     // second tiles (900 tokens of the larger model 436 and 250 -> 478 and 274).
     if (per_group <= 96) return 8256;
     // a share of up to 192 rows: the product streams the weights once and multiplies little, so it
-    // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows
-    // (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of
+    // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows, in quarters
+    // from 129 rows an expert on (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of
     // 256 do, 273 rows an expert as 2 x 192 instead of 2 x 256: the down product of a 4,096-token step 173
     // against 190 us)
     const long pad192 = ceil_div(per_group, 192) * 192L, pad256 = ceil_div(per_group, 256) * 256L;

@@ -2073,11 +2073,11 @@ static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, i
     // contiguous eighth of the tiles also beyond, where experts need a second tile: gate/up and down of 512 tokens on all of 60 experts 122 and 67 -> 116
     // and 65 us, on 40 of them 104 and 55 -> 98 and 52; 200 tokens of the larger model on 40 of 64 experts 265 and 158 -> 244 and 144)
     if (per_group <= g_tile64_rows) return 4;
-    // up to 96 rows, a prompt's tokens, which crowd into some of the experts: tiles of 128 x 256 in quarters (700 tokens on 35 experts
+    // up to 112 rows, a prompt's tokens, which crowd into some of the experts: tiles of 128 x 256 in quarters (700 tokens on 35 experts
     // 94 and 57 -> 87 and 50 us, 1,000 on 30 experts 107 and 64 -> 85 and 50, 400 of the larger model on 40 experts 290 and 170 -> 271 and
-    // 159; spread evenly 127 and 71 -> 129 and 74, 136 and 75 -> 135 and 79, 376 and 224 -> 387 and 227).  From 113 rows on an even share spills into
+    // 159; spread evenly 127 and 71 -> 129 and 74, 136 and 75 -> 135 and 79, 376 and 224 -> 387 and 227; a prompt of 1,500 tokens, 100 an expert, 12.30 -> 11.69 ms).  From 113 rows on an even share spills into
     // second tiles (900 tokens of the larger model 436 and 250 -> 478 and 274).
-    if (per_group <= 96) return 8256;
+    if (per_group <= 112) return 8256;
     // a share of up to 192 rows: the product streams the weights once and multiplies little, so it
     // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows, in quarters
     // from 129 rows an expert on (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of

@@ -274,10 +274,14 @@ FX_API int fx_small_rows_parts(void* stream, const float* x, long ldx, const flo
 // (k.q comes with the token, from the kernel above); the lanes of a column add theirs with four rotations inside their row of 16 lanes and, for 32 lanes, one
 // exchange between neighbouring rows (every lane gets the same bits: each step adds two sums of complementary
 // lanes, and a + b is b + a); then u and o = (dS)^T q + u (k.q) follow, and S takes k u^T.
+// (The two sums of a token are two such chains, side by side.  One chain for both, which adds a column's two rows first, one row
+// going on with either sum, is no faster at 128 x 128 and rounds otherwise: 193 against 188 us for 1,337 tokens of 16 heads, 293 against 285 for 2,048;
+// only at 256 x 128, two heads, it was ahead, 180 against 186 us for 700 tokens.)
 // A token's k, q and decay are the same for every column of a head, and reading them is most of the traffic: a
 // block of NW waves (NW 64 / LPC columns) brings them into LDS once for all its waves, a group of P tokens at a
-// time and a group ahead (memory is waited for once a group, not once a token; one barrier a group), and lanes
-// of one r read their rows as broadcasts.  (A wave that fetched for itself made a layer read 3 GB for a prompt of
+// time (memory is waited for once a group, not once a token; one barrier a group), and lanes
+// of one r read their rows as broadcasts.  A group is on its way in registers while the two groups before it are worked on,
+// and goes to LDS, which holds two groups, a group ahead of its work.  (A wave that fetched for itself made a layer read 3 GB for a prompt of
 // 2,048 tokens at 16 heads of 128 x 128, and more waves made it slower.)
 // The state is kept transposed, [slot][head][V][D]: a lane's rows of its column lie next to each other, and a
 // wave reads and writes contiguous floats (a decode step is little more than that read and write).
@@ -294,25 +298,6 @@ __device__ __forceinline__ float column_sum(float v) {      // over the LPC lane
         v = wave_partner_16(v, o) + o;      // rows 0 and 1, rows 2 and 3
     }
     return v;
-}
-
-// Two sums at once.  With 32 lanes to a column the first step is the exchange between neighbouring rows of 16, and of both sums: one
-// of a column's two rows goes on with a's and the other with b's, four rotations finish both, and a last exchange
-// hands each to the other row.  (One sum after the other is two chains of four rotations and an exchange.)
-template <int LPC>
-__device__ __forceinline__ void column_sums(float& a, float& b) {
-    if constexpr (LPC == 32) {
-        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        float v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
-        v += row_rotated<0x128>(v);
-        v += row_rotated<0x124>(v);
-        v += row_rotated<0x122>(v);
-        v += row_rotated<0x121>(v);
-        a = wave_partner_16(v, b);
-    } else {
-        a = column_sum<LPC>(a);
-        b = column_sum<LPC>(b);
-    }
 }
 
 // what lane p of a row of 16 lanes holds, in each of them
@@ -435,7 +420,8 @@ __global__ __launch_bounds__(NW * 64) void channel_delta_kernel(const float* __r
                     kv[i + e] = ka[e];
                 }
             }
-            column_sums<LPC>(sk, sq);
+            sk = column_sum<LPC>(sk);
+            sq = column_sum<LPC>(sq);
             const float u = row_lane<p>(beta_now) * (row_lane<p>(v_now) - sk), o = fmaf(u, row_lane<p>(kq_now), sq);
             o_mine = r == p ? o : o_mine;            // (every lane of the column has it: lane p keeps token p's for the store)
 #pragma unroll

@@ -1298,6 +1298,27 @@ def test_sorted_experts_through_either_product(T, E, k, I, H):
     assert float((outs[0] - outs[1]).abs().max()) <= 2e-2 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("D", [33, 64, 100, 128, 129, 256])
+def test_delta_rule_adds_a_column_in_one_order(D):
+    """One number per lane, queries of ones and nothing written: the output is the sum over a column's lanes alone.  Its bits are
+    those of the tree: four exchanges inside each row of 16 lanes, 8, 4, 2 and 1 apart, then the two rows of 32."""
+    from ferrox_amd import ops
+    V, lanes, per_lane = 40, 16 if D <= 64 else 32, 4 if D <= 128 else 8
+    one = lambda *s: torch.ones(s, device=DEV)
+    held = torch.zeros(1, 1, V, D, device=DEV)
+    held[..., ::per_lane] = rnd(1, 1, V, -(-D // per_lane), seed=6) * torch.exp(4 * rnd(1, 1, V, -(-D // per_lane), seed=7))
+    tree = torch.zeros(V, lanes)
+    tree[:, :-(-D // per_lane)] = held[0, 0, :, ::per_lane].cpu()
+    tree = tree.view(V, lanes // 16, 16)
+    for apart in (8, 4, 2, 1):
+        tree = tree[..., :apart] + tree[..., apart:2 * apart]
+    want = tree.sum(1)[:, 0] if lanes == 16 else tree[:, 0, 0] + tree[:, 1, 0]
+    state = held.clone()
+    out = ops.channel_delta(one(1, D), one(1, D), one(1, D), 0 * one(1, 1), 0 * one(1, 1), 0 * one(1, V), state,
+                            torch.tensor([0, 1], dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV), 1, 1, 1, D, V)
+    assert torch.equal(out.cpu().view(V), want) and torch.equal(state, held)
+
+
 # one case per instance of the kernel: 16 and 32 lanes a column, whole pieces of four rows and single ones, columns and rows past the end
 @pytest.mark.parametrize("D,V,H,G", [(64, 32, 2, 1), (64, 48, 2, 2), (33, 20, 2, 1), (30, 70, 1, 1), (128, 128, 4, 2), (100, 30, 2, 2), (66, 9, 2, 2),
                                      (256, 24, 2, 1), (129, 17, 1, 1)])

@@ -250,6 +250,44 @@ def test_grouped_tiles_in_quarters_at_every_number_of_row_blocks(blocked):
         assert torch.equal(got, first[0]) and torch.equal(act, first[1]), tile
 
 
+def grouped_products(sizes, N, K, seed):
+    """Rows sorted by expert with shares `sizes`: a stored product to scattered rows, in float64 too, and a gated one, as a call."""
+    from ferrox_amd import ops
+    E, n, dtype = len(sizes), sum(sizes), torch.bfloat16
+    offsets = torch.tensor([sum(sizes[:i]) for i in range(E + 1)], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(seed)
+    x, w, w2 = rnd(300, K, dtype=dtype, seed=seed), rnd(E, N, K, dtype=dtype, seed=seed + 1), rnd(E, 2 * N, K, dtype=dtype, seed=seed + 2, scale=0.5)
+    rows, to = torch.randint(0, 300, (n,), generator=g).to(torch.int32).to(DEV), torch.randperm(n, generator=g).to(torch.int32).to(DEV)
+    want, xs = torch.zeros(n, N, dtype=torch.float64, device=DEV), x.double()[rows.long()]
+    for e in range(E):
+        r = slice(sum(sizes[:e]), sum(sizes[:e + 1]))
+        want[to[r].long()] = xs[r] @ w[e].double().T
+    wb, w2b = ops.to_kblocked(w), ops.to_kblocked(w2)
+    return want, lambda: (ops.gemm(x, wb, epilogue=ops.EPI_STORE_F32, a_rows=rows, c_rows=to, expert_offsets=offsets, n_rows=n, w_kblocked=True),
+                          ops.gemm(x, w2b, epilogue=ops.EPI_GATED, a_rows=rows, expert_offsets=offsets, n_rows=n, w_kblocked=True))
+
+
+@pytest.mark.parametrize("most", [64, 65, 128, 129, 300])       # up to a tile of 64 and of 128 rows, one more, and beyond tiles of 256
+@pytest.mark.parametrize("E", [40, 72, 130])                    # tiles are found 64 experts at a time: one, two and three times
+def test_grouped_tiles_at_any_number_of_experts(E, most):
+    """Blocks find their tile among shares of 0 to `most` rows, the largest one in the first, a middle and the last expert, whether an XCD takes every
+    eighth row tile or an eighth of the tiles; with the hint on the weights that the shares call for and without."""
+    from ferrox_amd import debug
+    g = torch.Generator().manual_seed(E + most)
+    sizes = [int(s) for s in torch.randint(0, 24, (E,), generator=g)]
+    sizes[0] = sizes[E // 2 + 1] = sizes[E - 1] = most
+    sizes[1] = sizes[E // 2] = sizes[E - 3] = 0
+    want, products = grouped_products(sizes, 136, 192, E)
+    with debug.kernel_switch("gemm", "wide_grouped", 256), debug.kernel_switch("gemm", "stream_w", 0):
+        first = products()
+    close(first[0], want, torch.bfloat16, "256 x 256")
+    for tile in (4, 12, 64, 8128, 8256):
+        for hint in (-1, 0):
+            with debug.kernel_switch("gemm", "wide_grouped", tile), debug.kernel_switch("gemm", "stream_w", hint):
+                got = products()
+            assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), (tile, hint)
+
+
 @pytest.mark.parametrize("T,E", [(2048, 65), (4096, 65), (4096, 128), (8065, 65)])
 def test_a_routers_logits_keep_their_order_of_sums(T, E):
     """Up to 524,288 logits come from the product for few rows, whose bits decide between experts that stand close."""

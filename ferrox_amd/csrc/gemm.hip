@@ -569,11 +569,13 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
 // share are fetched by two XCDs, but no XCD has many full tiles where another has nearly empty ones (the ring of 192 rows, 512 tokens
 // on 40 experts, 55 against 66 us for the down product).  2: that where no expert has a second row tile, as when up to 64 sequences are decoded or shares
 // are even, and nothing is shared; else the contiguous eighths (both products of 64 decoded tokens of the larger model, tiles of 64 rows, 598 against 617 us,
-// of 128 tokens of the smaller one beside the shared expert's pieces, two tiles to a
-// piece, the other way, 221 against 194).
+// of 128 tokens beside the shared expert's pieces, which all lie at the end, tiles of 128, 637 against 682; of 128 tokens of the smaller one with tiles of
+// 64, two to a piece, the other way, 221 against 194).
+// `alone`: the expert's rows are one tile.
 template <int TM>
-__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile) {
+__device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile, bool* alone = nullptr) {
     const int lane = threadIdx.x & 63, C = g.n_col_tiles;
+    if (alone) *alone = true;
     if (g.by_row_tile == 1 && g.expert_offsets) {
         const int i = blockIdx.x / 8, row_tile = (i / C) * 8 + blockIdx.x % 8;
         col_tile = i % C;
@@ -637,6 +639,7 @@ __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end
             r0 = __builtin_amdgcn_readlane(b, src) + row * TM;
             r_end = __builtin_amdgcn_readlane(en, src);
             expert = base + src;
+            if (alone) *alone = __builtin_amdgcn_readlane(nt, src) == 1;
             return true;
         }
         before += __builtin_amdgcn_readlane(incl, 63);
@@ -734,8 +737,8 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[
     });
 }
 
-template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false>
-__global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
+template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA, bool STREAM>
+__device__ __forceinline__ void wide_block(const GemmArgs& g, bf16* stages, int r0, int r_end, int expert, int col_tile) {
     constexpr int TM = TMB * 16;
     constexpr int MT = TMB / 2;            // row blocks per wave
     constexpr int NT = TN / 64;            // 16-row blocks of W per wave
@@ -743,10 +746,6 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
     constexpr int OUT_TN = DUAL ? TN / 2 : TN;
     constexpr int NLA = TM / 64, NLB = TN / 64;   // wave-loads (8 rows each) per wave and K step
     static_assert(TM % 64 == 0 && TN % 64 == 0, "eight waves load 64 rows at a time");
-    __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * TM + NS * TN) * 64];    // the rows' ring, then the weights'
-
-    int r0, r_end, expert, col_tile;
-    if (!wide_tile<TM>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -799,6 +798,14 @@ __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
 #undef FX_LOOP
 
     wide_epilogue<MT, NT, TM, WN, DUAL, EPI>(g, acc, r0, r_end, n0, wm, wn, lane);
+}
+
+template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false>
+__global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * 16 * TMB + NS * TN) * 64];    // the rows' ring, then the weights'
+    int r0, r_end, expert, col_tile;
+    if (!wide_tile<16 * TMB>(g, r0, r_end, expert, col_tile)) return;
+    wide_block<TMB, TN, NS, DUAL, EPI, NSA, STREAM>(g, stages, r0, r_end, expert, col_tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -981,15 +988,11 @@ __device__ __forceinline__ void quarters_k_loop(f32x4_t (&acc)[MA0 + MA1][NB0 + 
 }
 
 template <int TMB, int TN, bool DUAL, int EPI>
-__global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
+__device__ __forceinline__ void quarters_block(const GemmArgs& g, bf16* stages, int r0, int r_end, int expert, int col_tile) {
     constexpr int TM = TMB * 16, MT = TMB / 2, NT = TN / 64, WN = TN / 4, OUT_TN = DUAL ? TN / 2 : TN;
     constexpr int MA0 = MT > 4 ? 4 : MT / 2, MA1 = MT - MA0, NB0 = (NT + 1) / 2, NB1 = NT - NB0;
     constexpr int NLA = TM / 64, NLB = TN / 64;   // wave-loads (8 rows each) per wave and K step
     static_assert(MA0 % 2 == 0 && MA1 % 2 == 0 && MA1 > 0 && NB1 > 0, "eight waves load 64 rows at a time, a part at a time");
-    __shared__ __attribute__((aligned(1024))) bf16 stages[2 * (TM + TN) * 64];
-
-    int r0, r_end, expert, col_tile;
-    if (!wide_tile<TM>(g, r0, r_end, expert, col_tile)) return;
     const int n0 = col_tile * OUT_TN;
     const int rows_here = min(TM, r_end - r0);
     const int nblk = (rows_here + 15) >> 4;
@@ -1038,6 +1041,33 @@ __global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
     else FX_LOOP(MA0 / 2, 0);
 #undef FX_LOOP
     wide_epilogue<MT, NT, TM, WN, DUAL, EPI>(g, acc, r0, r_end, n0, wm, wn, lane);
+}
+
+template <int TMB, int TN, bool DUAL, int EPI>
+__global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) bf16 stages[2 * (16 * TMB + TN) * 64];
+    int r0, r_end, expert, col_tile;
+    if (!wide_tile<16 * TMB>(g, r0, r_end, expert, col_tile)) return;
+    quarters_block<TMB, TN, DUAL, EPI>(g, stages, r0, r_end, expert, col_tile);
+}
+
+// Rows sorted by expert, tiles of 128 x 256, the loop by the expert's own share: one tile of rows reads its weights about once, so the ring with
+// the non-temporal hint streams them; an expert of more rows takes the tiles in quarters, whose weights its other tiles find in the cache.  Either
+// adds an element's products in the order of k.  Both products, us, even shares / crowded into half of the experts: tiles of 192 rows in a ring, these tiles in
+// quarters whatever the share, and by the share (60 experts of 1,408, then 64 of 2,560):
+//   560 tokens 194 137, 201 130, 189 128    700 203 160, 207 133, 198 139    1,000 214 181, 218 142, 211 140    1,400 235 217, 234 170, 229 171
+//   300 tokens 590 420, 601 340, 579 315    400 611 455, 614 401, 597 377    600 642 525, 642 460, 627 460
+// (One hot expert among many, 300 of the larger: 590, 663 and 620.)
+// (With four stages of weights, all of LDS, 1 to 2 % more.)
+template <int TMB, int TN, int NS, bool DUAL, int EPI>
+__global__ __launch_bounds__(512) void gemm_bf16_shares_kernel(GemmArgs g) {
+    constexpr int RING = 2 * 16 * TMB + NS * TN, QUARTERS = 2 * (16 * TMB + TN);
+    __shared__ __attribute__((aligned(1024))) bf16 stages[(RING > QUARTERS ? RING : QUARTERS) * 64];
+    int r0, r_end, expert, col_tile;
+    bool alone;
+    if (!wide_tile<16 * TMB>(g, r0, r_end, expert, col_tile, &alone)) return;
+    if (alone) wide_block<TMB, TN, NS, DUAL, EPI, 2, true>(g, stages, r0, r_end, expert, col_tile);
+    else quarters_block<TMB, TN, DUAL, EPI>(g, stages, r0, r_end, expert, col_tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -1848,7 +1878,7 @@ static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
 static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
-static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages), 8256 (128 x 256), 6128 or 6256 (96 rows) picks that tile of the LDS-tiled kernel
+static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages), 8256 (128 x 256), 6128 or 6256 (96 rows), or 1256 (sorted rows: 128 x 256 by the shares) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "skinny_sets")) { g_skinny_nw = value; return 0; }
     if (!strcmp(key, "skinny_row_tiles")) { g_skinny_mt = value; return 0; }
@@ -1898,6 +1928,17 @@ static void launch_quarters(GemmArgs g, int epi, int m_tiles, hipStream_t s, int
         default:
             if constexpr (TN % 128 == 0) gemm_bf16_quarters_kernel<TMB, TN, true, EPI_GATED><<<grid, 512, 0, s>>>(g);
             break;
+    }
+}
+template <int TMB, int TN, int NS>
+static void launch_shares(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
+    g.tile_rows = 16 * TMB;
+    const dim3 grid = wide_grid(g, epi, TN, m_tiles);
+    switch (epi) {
+        case EPI_STORE: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE_F32: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE_F32><<<grid, 512, 0, s>>>(g); break;
+        case EPI_RESID: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_RESID><<<grid, 512, 0, s>>>(g); break;
+        default: gemm_bf16_shares_kernel<TMB, TN, NS, true, EPI_GATED><<<grid, 512, 0, s>>>(g); break;
     }
 }
 // Weights that are read about once go through the ring with the non-temporal hint, everything else in quarters.
@@ -2086,17 +2127,16 @@ FX_API int fx_gemm_lower_tiles(int M, int N, int tile, int dual, int cus) {
     return tn && (long)ceil_div(N, dual ? tn / 2 : tn) * ceil_div(M, 96) <= cus;
 }
 // The same for rows sorted by expert.
-static int grouped_tile(long per_group, int M, int N, int nonempty, bool dual, int cus) {
+FX_API int fx_gemm_grouped_tile(int per_group, int M, int N, int nonempty, int dual, int cus) {
     // an expert's share of up to 36 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
     // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three at up to 20 rows; with an XCD on a
     // contiguous eighth of the tiles also beyond, where experts need a second tile: gate/up and down of 512 tokens on all of 60 experts 122 and 67 -> 116
     // and 65 us, on 40 of them 104 and 55 -> 98 and 52; 200 tokens of the larger model on 40 of 64 experts 265 and 158 -> 244 and 144)
     if (per_group <= g_tile64_rows) return 4;
-    // up to 112 rows, a prompt's tokens, which crowd into some of the experts: tiles of 128 x 256 in quarters (700 tokens on 35 experts
-    // 94 and 57 -> 87 and 50 us, 1,000 on 30 experts 107 and 64 -> 85 and 50, 400 of the larger model on 40 experts 290 and 170 -> 271 and
-    // 159; spread evenly 127 and 71 -> 129 and 74, 136 and 75 -> 135 and 79, 376 and 224 -> 387 and 227; a prompt of 1,500 tokens, 100 an expert, 12.30 -> 11.69 ms).  From 113 rows on an even share spills into
-    // second tiles (900 tokens of the larger model 436 and 250 -> 478 and 274).
-    if (per_group <= 112) return 8256;
+    // up to 104 rows: tiles of 128 x 256, streamed or in quarters by each expert's own share (`gemm_bf16_shares_kernel`).  Beyond 104 rows shares that are not quite
+    // even spill into second tiles (nearly even / crowded against tiles of 192 rows: 104 rows 245 220 -> 239 168, 106 235 224 -> 250 177, 110 236 237 -> 247 186; of the
+    // larger model 104 rows 678 577 -> 673 530, 109 674 625 -> 728 542).
+    if (per_group <= 104) return 1256;
     // a share of up to 192 rows: the product streams the weights once and multiplies little, so it
     // is bound by how many of them are on their way; a ring of three weight tiles beside two of the rows, in quarters
     // from 129 rows an expert on (beyond 192 rows: tiles of 192 rows too where they leave fewer empty rows than tiles of
@@ -2304,10 +2344,10 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
             if (tile == 8128 && !g.stream_w && fx_gemm_twice_as_wide(M, N, dual, fx_compute_units())) tile = 8256;
             if (!g.stream_w && fx_gemm_lower_tiles(M, N, tile, dual, fx_compute_units())) tile = tile == 64 ? 6128 : 6256;
         }
-        else if (!tile) tile = small_groups ? 64 : grouped_tile(per_group, M, N, nonempty, dual, fx_compute_units());
+        else if (!tile) tile = small_groups ? 64 : fx_gemm_grouped_tile((int)per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
         // (see `wide_tile`; tiles of 64 rows seldom are two to an expert at up to five rows each: nothing to count)
-        g.by_row_tile = !expert_offsets ? 0 : ((tile == 12 && g.stream_w) || (tile == 4 && per_group <= 5) ? 1 : (tile == 4 ? 2 : 0));
+        g.by_row_tile = !expert_offsets ? 0 : ((tile == 12 && g.stream_w) || (tile == 4 && per_group <= 5) ? 1 : (tile == 4 || tile == 1256 ? 2 : 0));
         switch (tile) {
             case 464: launch_ring<4, 64, 4>(g, epi, row_tiles(64), s); break;
             case 4128: launch_ring<4, 128, 3>(g, epi, row_tiles(64), s); break;
@@ -2318,6 +2358,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
             case 6128: launch_quarters<8, 128>(g, epi, row_tiles(96), s, 96); break;
             case 6256: launch_quarters<8, 256>(g, epi, row_tiles(96), s, 96); break;
             case 8256: launch_quarters<8, 256>(g, epi, row_tiles(128), s); break;
+            case 1256: launch_shares<8, 256, 3>(g, epi, row_tiles(128), s); break;
             case 192: launch_quarters<16, 192>(g, epi, row_tiles(256), s); break;
             case 128: launch_quarters<16, 128>(g, epi, row_tiles(256), s); break;
             default: launch_quarters<16, 256>(g, epi, row_tiles(256), s); break;

@@ -281,11 +281,28 @@ def test_grouped_tiles_at_any_number_of_experts(E, most):
     with debug.kernel_switch("gemm", "wide_grouped", 256), debug.kernel_switch("gemm", "stream_w", 0):
         first = products()
     close(first[0], want, torch.bfloat16, "256 x 256")
-    for tile in (4, 12, 64, 8128, 8256):
+    for tile in (4, 12, 64, 8128, 8256, 1256):
         for hint in (-1, 0):
             with debug.kernel_switch("gemm", "wide_grouped", tile), debug.kernel_switch("gemm", "stream_w", hint):
                 got = products()
             assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), (tile, hint)
+
+
+@pytest.mark.parametrize("average", [4, 5, 20, 21, 36, 37, 104, 105, 128, 129])
+@pytest.mark.parametrize("crowded", [False, True])
+def test_sorted_rows_as_the_sizes_choose(average, crowded):
+    """Both sides of every average share where the tiles change: even shares, and one expert with most of the rows."""
+    from ferrox_amd import debug
+    sizes = [average + d for d in (0, 3, -3, 2, -2, 1, -1, 0)]
+    if crowded:
+        sizes = [1, 0, average, 8 * average - 3 - 3 * (average // 2) - average, 2, average // 2, average // 2, average // 2]
+    assert sum(sizes) == 8 * average
+    want, products = grouped_products(sizes, 264, 320, average)
+    got = products()
+    close(got[0], want, torch.bfloat16, "chosen")
+    with debug.kernel_switch("gemm", "wide_grouped", 256), debug.kernel_switch("gemm", "stream_w", 0):
+        other = products()
+    assert torch.equal(got[0], other[0]) and torch.equal(got[1], other[1])
 
 
 @pytest.mark.parametrize("T,E", [(2048, 65), (4096, 65), (4096, 128), (8065, 65)])

@@ -1872,7 +1872,7 @@ static int g_skinny_mt = 0;    // "skinny_row_tiles": 1, 2 or 4 tiles of 16 rows
 static int g_skinny_waves = 0; // "skinny_waves": 1, 2, 4 or 8 waves that split K in a block of that product (0: by the sizes)
 static int g_few_rows = 3;     // "few_rows": sorted by expert, up to this many rows an expert go to the product for few rows (at most 64)
 static int g_head_rows = 16;   // "head_rows": plain rows against very many weight rows go to the tiled kernel from more than this many on
-static int g_tile64_rows = 36; // "tile64_rows": experts with up to this many rows on average take tiles of 64 rows
+static int g_tile64_rows = 20; // "tile64_rows": experts with up to this many rows on average take tiles of 64 rows
 static int g_no_wide = 0;      // "wide": 0 sends many-row products to the register-staged tiled kernel, 1 (default) by the sizes,
 static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to the product for few rows whatever the weight rows (0: by the sizes)
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
@@ -2128,12 +2128,12 @@ FX_API int fx_gemm_lower_tiles(int M, int N, int tile, int dual, int cus) {
 }
 // The same for rows sorted by expert.
 FX_API int fx_gemm_grouped_tile(int per_group, int M, int N, int nonempty, int dual, int cus) {
-    // an expert's share of up to 36 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
-    // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three at up to 20 rows; with an XCD on a
-    // contiguous eighth of the tiles also beyond, where experts need a second tile: gate/up and down of 512 tokens on all of 60 experts 122 and 67 -> 116
-    // and 65 us, on 40 of them 104 and 55 -> 98 and 52; 200 tokens of the larger model on 40 of 64 experts 265 and 158 -> 244 and 144)
+    // an expert's share of up to 20 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
+    // beside two of the rows (2-5 % less time than tiles of 192 rows with a ring of three)
     if (per_group <= g_tile64_rows) return 4;
-    // up to 104 rows: tiles of 128 x 256, streamed or in quarters by each expert's own share (`gemm_bf16_shares_kernel`).  Beyond 104 rows shares that are not quite
+    // up to 104 rows: tiles of 128 x 256, streamed or in quarters by each expert's own share (`gemm_bf16_shares_kernel`).  From 21 to 36 rows against tiles of 64,
+    // both products, even / crowded: 176 tokens beside the shared expert's pieces 217 123 -> 196 128, 256 222 146 -> 200 129, 400 178 114 -> 180 109, 512 184 118 -> 186 127; of the larger model
+    // 96 beside the pieces 662 394 -> 617 401, 200 557 353 -> 560 315, 256 569 364 -> 571 310.  Beyond 104 rows shares that are not quite
     // even spill into second tiles (nearly even / crowded against tiles of 192 rows: 104 rows 245 220 -> 239 168, 106 235 224 -> 250 177, 110 236 237 -> 247 186; of the
     // larger model 104 rows 678 577 -> 673 530, 109 674 625 -> 728 542).
     if (per_group <= 104) return 1256;

@@ -76,11 +76,11 @@ def test_tiles_of_96_rows():
 
 
 def test_tiles_of_sorted_rows():
-    """Average shares up to 36 rows go to tiles of 64, up to 104 to tiles whose loop an expert's own share decides (even shares lose
+    """Average shares up to 20 rows go to tiles of 64, up to 104 to tiles whose loop an expert's own share decides (even shares lose
     with tiles in quarters there, crowded ones with a ring), more to tiles of 192 or 256."""
     from ferrox_amd.csrc.build import load_library
     tile = lambda share, n=2816, experts=60, dual=1, cus=256: load_library("gemm").fx_gemm_grouped_tile(share, share * experts, n, experts, dual, cus)
-    assert tile(4) == tile(36) == 4 and tile(37) == tile(104) == tile(37, 2048, dual=0) == 1256
+    assert tile(4) == tile(20) == 4 and tile(21) == tile(37) == tile(104) == tile(37, 2048, dual=0) == 1256
     assert tile(105) == tile(113) == tile(128) == tile(176) == 12 and tile(193) == 256
 
 

@@ -1878,7 +1878,7 @@ static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
 static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
-static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages), 8256 (128 x 256), 6128 or 6256 (96 rows), or 1256 (sorted rows: 128 x 256 by the shares) picks that tile of the LDS-tiled kernel
+static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages), 8256 (128 x 256), 6128 or 6256 (96 rows), 1256 (sorted rows: 128 x 256 by the shares) or 1128 (128 x 128 in a ring) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "skinny_sets")) { g_skinny_nw = value; return 0; }
     if (!strcmp(key, "skinny_row_tiles")) { g_skinny_mt = value; return 0; }
@@ -2126,6 +2126,11 @@ FX_API int fx_gemm_lower_tiles(int M, int N, int tile, int dual, int cus) {
     const int tn = tile == 64 ? 128 : (tile == 8256 ? 256 : 0);
     return tn && (long)ceil_div(N, dual ? tn / 2 : tn) * ceil_div(M, 96) <= cus;
 }
+// Plain products that are one round of tiles of 128 x 128 (64): whether a ring of four stages is ahead of the tiles in quarters, whose two stages
+// do not reach as far: blocks that go through a long K drift apart, and find less of each other's operands in the caches (3,584 weight rows of 20,480 k, 800
+// rows 174 -> 167 us, 1,000 rows 190 -> 177, 1,100 rows 195 -> 181; 2,048 weight rows, 1,500 rows 172 -> 168. 14,336 k: 1,000 rows 132 -> 127 to 131, 600 and 700 rows
+// the other way, 116 against 121 and 118 against 120; 8,192 k: 800 rows 70 against 72; 3,584 k: 33 against 37).
+FX_API int fx_gemm_ring_of_four(int tile, int K) { return tile == 64 && K >= 16384; }
 // The same for rows sorted by expert.
 FX_API int fx_gemm_grouped_tile(int per_group, int M, int N, int nonempty, int dual, int cus) {
     // an expert's share of up to 20 rows on average: a tile of 64 rows leaves LDS for a ring of four weight tiles
@@ -2342,7 +2347,8 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         if (!tile && !expert_offsets) {
             tile = fx_gemm_plain_tile(M, N, K, dual, fx_compute_units());
             if (tile == 8128 && !g.stream_w && fx_gemm_twice_as_wide(M, N, dual, fx_compute_units())) tile = 8256;
-            if (!g.stream_w && fx_gemm_lower_tiles(M, N, tile, dual, fx_compute_units())) tile = tile == 64 ? 6128 : 6256;
+            if (!g.stream_w && fx_gemm_ring_of_four(tile, K)) tile = 1128;
+            else if (!g.stream_w && fx_gemm_lower_tiles(M, N, tile, dual, fx_compute_units())) tile = tile == 64 ? 6128 : 6256;
         }
         else if (!tile) tile = small_groups ? 64 : fx_gemm_grouped_tile((int)per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
@@ -2355,6 +2361,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
             case 8128: launch_ring_or_quarters<8, 128, 2>(g, epi, row_tiles(128), s); break;
             case 64: launch_ring_or_quarters<8, 128, 4>(g, epi, row_tiles(128), s); break;
             case 12: launch_ring_or_quarters<12, 256, 3, 2>(g, epi, row_tiles(192), s); break;
+            case 1128: launch_wide<8, 128, 4, 4, false>(g, epi, row_tiles(128), s); break;
             case 6128: launch_quarters<8, 128>(g, epi, row_tiles(96), s, 96); break;
             case 6256: launch_quarters<8, 256>(g, epi, row_tiles(96), s, 96); break;
             case 8256: launch_quarters<8, 256>(g, epi, row_tiles(128), s); break;

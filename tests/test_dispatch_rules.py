@@ -75,6 +75,15 @@ def test_tiles_of_96_rows():
     assert not rule(1337, 2048, 8128) and not rule(1337, 2048, 256) and not rule(1337, 2048, 64, cus=200)
 
 
+def test_long_sums_of_one_round_of_tiles_take_the_ring():
+    """128 x 128 tiles that are one round of the CUs: quarters, but the ring of four stages for a long K."""
+    from ferrox_amd.csrc.build import load_library
+    tile = lambda m, n, k: load_library("gemm").fx_gemm_plain_tile(m, n, k, 0, 256)
+    rule = lambda m, n, k: bool(load_library("gemm").fx_gemm_ring_of_four(tile(m, n, k), k))
+    assert rule(1000, 3584, 20480) and rule(800, 3584, 16384) and rule(1500, 2048, 20480)
+    assert not rule(1000, 3584, 14336) and not rule(300, 3584, 20480) and not rule(1500, 3584, 20480)
+
+
 def test_tiles_of_sorted_rows():
     """Average shares up to 20 rows go to tiles of 64, up to 104 to tiles whose loop an expert's own share decides (even shares lose
     with tiles in quarters there, crowded ones with a ring), more to tiles of 192 or 256."""

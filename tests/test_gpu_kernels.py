@@ -250,6 +250,18 @@ def test_grouped_tiles_in_quarters_at_every_number_of_row_blocks(blocked):
         assert torch.equal(got, first[0]) and torch.equal(act, first[1]), tile
 
 
+@pytest.mark.parametrize("K", [16320, 16384, 20480])        # both sides of the line
+def test_long_sums_have_the_bits_of_the_tiles_in_quarters(K):
+    from ferrox_amd import debug, ops
+    M, N = 1025, 2056
+    a, w = rnd(M, K, dtype=torch.bfloat16), rnd(N, K, dtype=torch.bfloat16, seed=1, scale=0.05)
+    got = ops.gemm(a, w, epilogue=ops.EPI_STORE_F32)
+    close(got, a.double() @ w.double().T, torch.bfloat16, "product")
+    for tile in (1128, 64, 6128):
+        with debug.kernel_switch("gemm", "wide", tile):
+            assert torch.equal(ops.gemm(a, w, epilogue=ops.EPI_STORE_F32), got), tile
+
+
 def grouped_products(sizes, N, K, seed):
     """Rows sorted by expert with shares `sizes`: a stored product to scattered rows, in float64 too, and a gated one, as a call."""
     from ferrox_amd import ops

@@ -25,6 +25,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ARCH = "gfx950"
 FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# A loop that is entered by a branch begins on a 32-byte boundary, what one instruction fetch brings: the small loops of the tiled products
+# otherwise take 3-4 % more or less whenever code in front of them changes (512 rows against 2,048 weight rows of 5,632 k 27.9 and 26.9 us,
+# 129 against 3,584 of 20,480 k 85.5 and 81.3).
+LIBRARY_FLAGS = {"gemm": ["-mllvm", "-align-all-nofallthru-blocks=5"]}
 HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC"]
 HOST_LIBRARIES = ("host_runtime",)
 KERNEL_LIBRARIES = ("elementwise", "gemm", "attention", "moe", "sampling", "recurrent")      # what parts of a model may name
@@ -69,7 +73,7 @@ def _sources(name: str) -> tuple:
 
 def _source_hash(name: str) -> str:
     h = hashlib.sha256()
-    h.update(" ".join(HOST_FLAGS if name in HOST_LIBRARIES else FLAGS).encode())
+    h.update(" ".join(HOST_FLAGS if name in HOST_LIBRARIES else FLAGS + LIBRARY_FLAGS.get(name, [])).encode())
     for f in _sources(name):
         with open(os.path.join(HERE, f), "rb") as fh:
             h.update(fh.read())
@@ -122,7 +126,7 @@ def compile_library(name: str, verbose: bool = True) -> str:
     out_dir = _writable_dir()
     so = os.path.join(out_dir, name + ".so")
     tmp = os.path.join(out_dir, f".{name}.{os.getpid()}.{threading.get_ident()}.so")
-    cmd = [compiler] + (HOST_FLAGS if host else FLAGS + ["-I", HERE]) + [os.path.join(HERE, _sources(name)[0]), "-o", tmp]
+    cmd = [compiler] + (HOST_FLAGS if host else FLAGS + LIBRARY_FLAGS.get(name, []) + ["-I", HERE]) + [os.path.join(HERE, _sources(name)[0]), "-o", tmp]
     env = dict(os.environ)
     env.setdefault("HOME", out_dir)   # hipcc wants a home for its temporary files
     t0 = time.time()

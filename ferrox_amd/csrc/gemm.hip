@@ -850,7 +850,8 @@ __device__ __forceinline__ void quarters_k_loop(f32x4_t (&acc)[MA0 + MA1][NB0 + 
     const long b_step = kb_stride ? kb_stride : 64;
     // wave-loads FROM .. TO-1 of a step's rows or weights, steps in turn.  (The empty asm keeps the compiler from
     // holding every address twice; the weights' are 32 bits beside a base that all lanes share.  With 64 bits each
-    // some of them lived in scratch memory, and the loop waited for those loads.)
+    // some of them lived in scratch memory, and the loop waited for those loads.  The tiles of 256 x 256 still keep 64 to 72 bytes a lane there, touched around
+    // the loop and in the first step of an odd number, not in the loop.)
     auto load_a = [&](auto from, auto to, int kt) {
         bf16* st = lds + (kt & 1) * STAGE;
 #pragma unroll
@@ -2076,20 +2077,23 @@ FX_API int fx_gemm_row_tile_blocks(int M, int N, int cus) {
 }
 
 // The tile of the LDS-tiled kernel for plain rows, as the debug switch "wide" names them; all give the same bits.  `dual`: N
-// columns of two matrices.  (The times beside the lines are those of tiles in rings of stages.  In quarters every tile from 128 x 128 on takes 7
-// to 18 % less and what is ahead stays ahead: 4,096 rows against 4,608 weight rows of 3,584 k 149.5 -> 129 us with 256 x 192, 157 with 256 x 256;
+// columns of two matrices.  (The times beside the lines, from 128 x 128 on, are those of tiles in rings of stages.  In quarters these take 7
+// to 18 % less and what is ahead of another of them stays ahead: 4,096 rows against 4,608 weight rows of 3,584 k 149.5 -> 129 us with 256 x 192, 157 with 256 x 256;
 // gate/up of 11,264, 2,048 rows 100 -> 91 with 192 x 256, 113 with 256 x 256; 2,048 rows against 2,048 of 5,632 k 55 -> 50 with 128 x 128, 62 with 128 x 256.)
 FX_API int fx_gemm_plain_tile(int M, int N, int K, int dual, int cus) {
     auto tiles = [&](int tm, int tn) { return (long)ceil_div(N, dual ? tn / 2 : tn) * ceil_div(M, tm); };
     // Fewer tiles of 128 x 128 than CUs: a block's chain of K steps takes the same 23-25 us (2,048 k) whatever the rows, so
     // smaller tiles on more CUs: 64 x 64 while they are one a CU (2,048 x 2,048 weights, 512 rows 23 -> 13 us; 5,632 k 55 -> 29;
-    // 6,144 weight rows, 128 rows 25 -> 14), then 64 x 128 (6,144 weight rows, 256 rows 25 -> 19; 2,048 x 5,632, 1,024 rows 56 -> 41).
+    // 6,144 weight rows, 128 rows 25 -> 14), then 64 x 128 (6,144 weight rows, 256 rows 25 -> 19; 2,048 x 5,632, 1,024 rows 56 -> 41).  Against 128 x 128 in
+    // quarters as well: 512 rows against 2,048 x 2,048 19 -> 14, 5,632 k 44 -> 28; 6,144 weight rows, 128 and 300 rows 25 -> 14 and 19.0 -> 17.5; 2,048 x 5,632, 1,024 rows 46 -> 39;
+    // gate/up of 11,264, 128 rows 27 -> 21, of 5,120 x 3,584, 384 rows 40 -> 30.
     if (!dual && tiles(64, 64) <= cus) return 464;
     if (tiles(64, 128) <= cus) return 4128;
     // One round of 128 x 128 in two stages, two blocks to a CU, whether half or all of it is there (2,048 k: 6,144 weight rows, 768 to
     // 1,280 rows 43 -> 34-36 us, gate/up of 11,264, 384 and 640 rows 40 -> 35 and 48 -> 38, 2,048 weight rows, 2,432 and 4,096 rows 49
     // -> 38 and 49 -> 42; 8,192 k: 3-24 % less).  But beyond 14,336 rows (of at most 512 weight rows then) of long K the
-    // tiles of 256 x 128 read the rows fewer times (16,384 rows: 4,096 k 79 against 86 us, 5,632 k 104 against 117; 3,584 k 67 and 66).
+    // tiles of 256 x 128 read the rows fewer times (16,384 rows, in quarters: 4,096 k 63 against 65 us, 5,632 k 83 against 91, 8,192 k 130 against 149; 3,584 k 57 and 58,
+    // where 128 x 256, which then take the place of 128 x 128, need 52).
     const long t128 = tiles(128, 128);
     if (t128 > cus && t128 <= 2L * cus && (M <= 14336 || K < 4096)) return 8128;
     // More: the widest tile that still gives the CUs (one block each) an even share of the work; a tile's score is the share of
@@ -2269,10 +2273,9 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
                               !g_no_wide && ceil_div(N, 128) >= 512;
     // Rows sorted by expert: the product for few rows only up to three rows an expert on average.  Its waves fetch
     // every row tile's operands themselves, so its time grows with the rows (512 tokens of the larger model, 64 rows
-    // an expert: 1,107 us for the gate/up product at 2.1 TB/s), while the tiled product, whose tile of 192 rows
-    // holds an expert's share, streams the weights at the same speed whatever the rows (400 us at 5.9 TB/s); decode
-    // steps of 48 and 64 sequences 10.3 -> 10.0 and 12.0 -> 11.4 ms, of 17 to 64 of the larger model's sizes 8-24 %
-    // less; with three rows an expert the product for few rows is still 1-2 % ahead of the tiles of 64 rows.
+    // an expert: 1,100 us for the gate/up product), while tiles of an expert's rows stream the weights at the same speed
+    // whatever the rows (128 x 256: 384 us at 6.1 TB/s).  Both products at three rows an expert 144 against 152 us with tiles of 64 rows (60 experts), 469 against 493
+    // (64 of the larger model); at four rows 164 against 162 and 564 against 513.
     // 65 to 128 plain rows against few weight rows (the attention's output product): the product for few rows, 32 or 64 rows
     // a block, still streams the weights faster than tiles of 64 x 64 (2,048 x 2,048 weights 12 against 13 us, 2,048 x 5,632
     // 25 against 28-30; 3,584 x 3,584 the other way, 31 against 20)

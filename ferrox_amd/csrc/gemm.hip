@@ -14,7 +14,6 @@
 // Dual mode: two weight matrices (gate, up) are multiplied at once and the
 // epilogue stores silu(gate) * up  (ferrox-moe/src/lib.rs:655-658).
 #include "common.h"
-#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -76,7 +75,7 @@ struct GemmArgs {
     int c_vec;   // float32: so are 16-byte loads and stores of C
     int n_col_tiles, n_row_tiles;  // tiled kernels: the grid they decode block ids with
     int tile_rows;  // LDS-tiled kernels, plain rows: rows a tile takes, up to its height
-    int by_row_tile;  // LDS-tiled kernels, rows sorted by expert: every eighth row tile to an XCD (2: where no expert has two)
+    int by_row_tile;  // LDS-tiled kernels, rows sorted by expert: every eighth row tile to an XCD
 };
 
 // block -> (first logical row, end of rows, expert).  Plain: tiles of TM rows.
@@ -565,18 +564,17 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
 // tokens on 30 of 60 experts, 236 instead of 195 for 3,500, 1,297 and 667 instead of 1,245 and 626 for both of 4,096 tokens of
 // the larger model.  Eighths of equal cost, a tile's
 // rows and a constant, instead of equal numbers of tiles: no better, 237 us for the 3,500.)
-// `by_row_tile` 1: XCD x takes the row tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles
-// share are fetched by two XCDs, but no XCD has many full tiles where another has nearly empty ones (the ring of 192 rows, 512 tokens
-// on 40 experts, 55 against 66 us for the down product).  2: that where no expert has a second row tile, as when up to 64 sequences are decoded or shares
-// are even, and nothing is shared; else the contiguous eighths (both products of 64 decoded tokens of the larger model, tiles of 64 rows, 598 against 617 us,
-// of 128 tokens beside the shared expert's pieces, which all lie at the end, tiles of 128, 637 against 682; of 128 tokens of the smaller one with tiles of
-// 64, two to a piece, the other way, 221 against 194).
-// `alone`: the expert's rows are one tile.
+// `by_row_tile`: XCD x takes the row tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles
+// share are fetched by two XCDs, but no XCD has many full tiles where another has nearly empty ones, and nothing is counted: for the ring of 192 rows (512 tokens
+// on 40 experts, 55 against 66 us for the down product), and where the caller knows that no expert has a second row tile (both products of 64 decoded tokens
+// of the larger model, tiles of 64 rows, 598 against 617 us, of 128 tokens beside the shared expert's pieces, which all lie at the end, tiles of 128, 637 against
+// 682; of 128 tokens of the smaller one with tiles of 64, two to a piece, the other way, 221 against 194).
+// `alone`: the expert's rows are one tile (so they are taken to be with `by_row_tile`; either answer gives the same sums).
 template <int TM>
 __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile, bool* alone = nullptr) {
     const int lane = threadIdx.x & 63, C = g.n_col_tiles;
     if (alone) *alone = true;
-    if (g.by_row_tile == 1 && g.expert_offsets) {
+    if (g.by_row_tile && g.expert_offsets) {
         const int i = blockIdx.x / 8, row_tile = (i / C) * 8 + blockIdx.x % 8;
         col_tile = i % C;
         locate_rows<TM>(g, row_tile, r0, r_end, expert);       // (r0 < 0: past the last one)
@@ -594,27 +592,17 @@ __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end
         col_tile = rem / band_rows;
     };
     int rows = g.n_row_tiles, b = 0, en = 0, nt = 0, incl = 0;
-    int used = 0;                            // experts that have rows
     if (g.expert_offsets) {
         rows = 0;
         for (int base = 0; base < g.E; base += 64) {
             nt = share(base, b, en);
             incl = wave_inclusive_sum(nt);
             rows += __builtin_amdgcn_readlane(incl, 63);
-            used += __popcll(__ballot(nt > 0));
         }
     }
-    const bool two = !g.by_row_tile || rows != used;       // an expert has a second row tile (or it does not matter)
     const int per_xcd = (C * rows + 7) / 8, i = blockIdx.x / 8;
-    // logical: a tile in the order above, or, where an XCD takes every eighth row tile, a row tile
-    int logical = (blockIdx.x % 8) * per_xcd + i, per_row = C;
-    if (g.expert_offsets && !two) {
-        logical = (i / C) * 8 + blockIdx.x % 8;
-        per_row = 1;
-        if (logical >= rows) return false;
-    } else if (i >= per_xcd || logical >= C * rows) {
-        return false;
-    }
+    const int logical = (blockIdx.x % 8) * per_xcd + i;
+    if (i >= per_xcd || logical >= C * rows) return false;
     if (!g.expert_offsets) {
         int row;
         in_bands(logical, rows, row);
@@ -629,13 +617,12 @@ __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end
             nt = share(base, b, en);
             incl = wave_inclusive_sum(nt);
         }
-        const int first = (before + incl - nt) * per_row;
-        const unsigned long long hit = __ballot(logical >= first && logical < first + nt * per_row);
+        const int first = (before + incl - nt) * C;
+        const unsigned long long hit = __ballot(logical >= first && logical < first + nt * C);
         if (hit) {
             const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)hit) - 1);
-            int row = 0;
-            if (two) in_bands(logical - __builtin_amdgcn_readlane(first, src), __builtin_amdgcn_readlane(nt, src), row);
-            else col_tile = i % C;
+            int row;
+            in_bands(logical - __builtin_amdgcn_readlane(first, src), __builtin_amdgcn_readlane(nt, src), row);
             r0 = __builtin_amdgcn_readlane(b, src) + row * TM;
             r_end = __builtin_amdgcn_readlane(en, src);
             expert = base + src;
@@ -1900,10 +1887,7 @@ FX_API int fx_debug_set(const char* key, int value) {
 static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles) {
     g.n_col_tiles = ceil_div(g.N, epi == EPI_GATED ? tn / 2 : tn);
     g.n_row_tiles = m_tiles;
-    const long eighths = 8L * ceil_div((long)g.n_col_tiles * m_tiles, 8);
-    if (!g.by_row_tile || !g.expert_offsets) return dim3(eighths);
-    const long row_tiles = g.by_row_tile == 2 ? std::min(std::min(g.E, g.M), m_tiles) : m_tiles;      // (2: there are no more than experts where it matters)
-    return dim3(std::max(eighths, 8L * ceil_div(row_tiles, 8L) * g.n_col_tiles));
+    return dim3(g.by_row_tile && g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
 }
 template <int TMB, int TN, int NS, int NSA, bool STREAM>
 static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
@@ -2162,14 +2146,14 @@ FX_API int fx_gemm_grouped_tile(int per_group, int M, int N, int nonempty, int d
 }
 
 // dtype: type of A and W.  C is: T for EPI_STORE and EPI_GATED, float32 otherwise.
-// rows_hint: in grouped mode, the expected number of rows per expert (chooses the tile).
+// max_share: rows sorted by expert, a number that no expert's rows exceed (0: none is known); the order of tiles depends on it, no result does.
 FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, const void* W, long w_stride,
                    long up_offset, const void* bias, int bias_dtype, void* C, long ldc,
                    const float* row_scale, const int* a_rows, const int* c_rows, const int* expert_offsets,
                    int E, int M, int N, int K, const void* norm_w, int norm_dtype, float norm_eps,
                    const int* pair_ids, int pair_div, int n_always, int always_rows, int always_from_a, long kb_rows,
                    const float* row_ss, int row_ss_n, int act, int store_act, float act_limit, float act_alpha,
-                   const float* pre_scale, const int* pre_scale_rows, const float* out_gate, long ld_gate, int gate_div) {
+                   const float* pre_scale, const int* pre_scale_rows, const float* out_gate, long ld_gate, int gate_div, int max_share) {
     FX_REQUIRE((store_act == SACT_GATE) == (out_gate != nullptr) && (!out_gate || (gate_div >= 1 && ld_gate >= (long)gate_div * N)),
                "gemm: gated outputs need gate rows of %d x %d columns, got a row distance of %ld", gate_div, N, ld_gate);
     FX_REQUIRE(store_act >= 0 && store_act < SACT_COUNT && (store_act == 0 || ((epi == EPI_STORE || epi == EPI_STORE_F32) && !bias)),
@@ -2355,8 +2339,9 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         }
         else if (!tile) tile = small_groups ? 64 : fx_gemm_grouped_tile((int)per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
-        // (see `wide_tile`; tiles of 64 rows seldom are two to an expert at up to five rows each: nothing to count)
-        g.by_row_tile = !expert_offsets ? 0 : ((tile == 12 && g.stream_w) || (tile == 4 && per_group <= 5) ? 1 : (tile == 4 || tile == 1256 ? 2 : 0));
+        // (see `wide_tile`; tiles of 64 rows seldom are two to an expert at up to five rows each)
+        g.by_row_tile = expert_offsets && (tile == 12 ? g.stream_w : tile == 4 ? per_group <= 5 || (max_share > 0 && max_share <= 64)
+                                                                            : tile == 1256 && max_share > 0 && max_share <= 128);
         switch (tile) {
             case 464: launch_ring<4, 64, 4>(g, epi, row_tiles(64), s); break;
             case 4128: launch_ring<4, 128, 3>(g, epi, row_tiles(64), s); break;

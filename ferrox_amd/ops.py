@@ -129,7 +129,7 @@ _sigs = {
     ("gemm", "fx_gemm"): [c_void_p, c_int, c_int, c_void_p, c_long, c_void_p, c_long, c_long, c_void_p, c_int,
                           c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_int, c_long, c_void_p, c_int, c_int, c_int,
-                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int],
+                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int],
     ("gemm", "fx_qkv_rope"): [c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_void_p, c_long, c_int, c_int,
                               c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
@@ -664,7 +664,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
          always: tuple | None = None, w_kblocked: bool = False, row_ss: tuple | None = None,
          activation: str = "silu", store_activation: str | None = None, activation_params: tuple = (0.0, 0.0),
          pre_scale: torch.Tensor | None = None, pre_scale_rows: torch.Tensor | None = None,
-         out_gate: tuple | None = None) -> torch.Tensor:
+         out_gate: tuple | None = None, max_share: int = 0) -> torch.Tensor:
     """C[m, n] = sum_k a[m, k] * w[n, k] with an epilogue.
 
     `w` is [N, K], or [E, N, K] with `expert_offsets` [E+1] (rows sorted by expert).
@@ -694,6 +694,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
     scaled by that number.
     `out_gate` = (logits float32 [rows, >= div * N], div) (EPI_STORE or EPI_STORE_F32 without bias): element n of output row m
     is multiplied by sigmoid(logits[m // div, (m % div) * N + n]); div > 1 where the output's rows are parts of the gate's.
+    `max_share` (with `expert_offsets`): a number of rows that no expert's share exceeds, if the caller knows one (a step's tokens, each
+    of which takes an expert once): the order in which tiles are worked on depends on it, no result does.
     """
     gate_logits, gate_div = out_gate if out_gate is not None else (None, 0)
     if gate_logits is not None and (store_activation is not None or epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None
@@ -780,7 +782,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
           _p(row_ss[0]) if row_ss is not None else None, row_ss[0].shape[1] if row_ss is not None else 0,
           ACTIVATIONS[activation], STORED_ACTIVATIONS[store_activation] if gate_logits is None else _SACT_GATE,
           float(activation_params[0]), float(activation_params[1]), _p(pre_scale), _p(_i32(pre_scale_rows, "pre_scale_rows")),
-          _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div))
+          _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share))
     return out
 
 

@@ -194,9 +194,9 @@ class SparseMoE(FeedForward):
             kb = dict(w_kblocked=True) if self.kblocked else {}
             debug.region("experts gate/up")
             act = matmul(x, self.w_gate_up_all, epilogue=ops.EPI_GATED, a_rows=sorted_token, expert_offsets=offsets,
-                         n_rows=n + S * T, **self._gated(weights, sorted_pair), **kb)
+                         n_rows=n + S * T, max_share=T, **self._gated(weights, sorted_pair), **kb)
             debug.region("experts down")
-            y = matmul(act, self.w_down_all, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, **kb)
+            y = matmul(act, self.w_down_all, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, max_share=T, **kb)
             debug.region("combine")
             ctx.carry = ops.moe_combine(residual, y[:n], None, weights, self.top_k, shared=y[n:].view(S, T, -1), gate=gate,
                                         **then)
@@ -267,10 +267,10 @@ class SparseMoE(FeedForward):
             y = ops.gemm(act, self.w_down, epilogue=ops.EPI_STORE_F32, pair_ids=ids, **kb)
         else:
             act = matmul(x, self.w_gate_up, epilogue=ops.EPI_GATED, a_rows=sorted_token,
-                         expert_offsets=offsets, n_rows=T * self.top_k, **self._gated(weights, sorted_pair), **kb)
+                         expert_offsets=offsets, n_rows=T * self.top_k, max_share=T, **self._gated(weights, sorted_pair), **kb)
             debug.region("experts down")
             # each expert's rows go back to the place of their (token, slot) pair
-            y = matmul(act, self.w_down, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, **kb)
+            y = matmul(act, self.w_down, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, max_share=T, **kb)
         debug.region("combine")
         if overlap:
             main.wait_event(join)
@@ -360,9 +360,9 @@ class RoutedExperts(FeedForward):
                 offsets, sorted_token, sorted_pair, _ = ops.moe_align(ids, E + self.n_identity)
                 debug.region("experts up")
                 act = matmul(x, self.w_up, epilogue=ops.EPI_STORE, store_activation=self.activation, a_rows=sorted_token,
-                             expert_offsets=offsets, n_rows=T * k, **kb)
+                             expert_offsets=offsets, n_rows=T * k, max_share=T, **kb)
                 debug.region("experts down")
-                y = matmul(act, self.w_down, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, **kb)
+                y = matmul(act, self.w_down, epilogue=ops.EPI_STORE_F32, expert_offsets=offsets, c_rows=sorted_pair, max_share=T, **kb)
         else:
             y = torch.empty((T * k, self.hidden_size), dtype=torch.float32, device=x.device)
         debug.region("combine")

@@ -275,15 +275,16 @@ def grouped_products(sizes, N, K, seed):
         r = slice(sum(sizes[:e]), sum(sizes[:e + 1]))
         want[to[r].long()] = xs[r] @ w[e].double().T
     wb, w2b = ops.to_kblocked(w), ops.to_kblocked(w2)
-    return want, lambda: (ops.gemm(x, wb, epilogue=ops.EPI_STORE_F32, a_rows=rows, c_rows=to, expert_offsets=offsets, n_rows=n, w_kblocked=True),
-                          ops.gemm(x, w2b, epilogue=ops.EPI_GATED, a_rows=rows, expert_offsets=offsets, n_rows=n, w_kblocked=True))
+    kb = dict(expert_offsets=offsets, n_rows=n, w_kblocked=True)
+    return want, lambda most=0: (ops.gemm(x, wb, epilogue=ops.EPI_STORE_F32, a_rows=rows, c_rows=to, max_share=most, **kb),
+                                 ops.gemm(x, w2b, epilogue=ops.EPI_GATED, a_rows=rows, max_share=most, **kb))
 
 
 @pytest.mark.parametrize("most", [64, 65, 128, 129, 300])       # up to a tile of 64 and of 128 rows, one more, and beyond tiles of 256
 @pytest.mark.parametrize("E", [40, 72, 130])                    # tiles are found 64 experts at a time: one, two and three times
 def test_grouped_tiles_at_any_number_of_experts(E, most):
     """Blocks find their tile among shares of 0 to `most` rows, the largest one in the first, a middle and the last expert, whether an XCD takes every
-    eighth row tile or an eighth of the tiles; with the hint on the weights that the shares call for and without."""
+    eighth row tile or an eighth of the tiles (the largest share known, too small a number and unknown); with the hint on the weights that the shares call for and without."""
     from ferrox_amd import debug
     g = torch.Generator().manual_seed(E + most)
     sizes = [int(s) for s in torch.randint(0, 24, (E,), generator=g)]
@@ -295,9 +296,10 @@ def test_grouped_tiles_at_any_number_of_experts(E, most):
     close(first[0], want, torch.bfloat16, "256 x 256")
     for tile in (4, 12, 64, 8128, 8256, 1256):
         for hint in (-1, 0):
-            with debug.kernel_switch("gemm", "wide_grouped", tile), debug.kernel_switch("gemm", "stream_w", hint):
-                got = products()
-            assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), (tile, hint)
+            for known in (0, 1, most):
+                with debug.kernel_switch("gemm", "wide_grouped", tile), debug.kernel_switch("gemm", "stream_w", hint):
+                    got = products(known)
+                assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), (tile, hint, known)
 
 
 @pytest.mark.parametrize("average", [4, 5, 20, 21, 36, 37, 104, 105, 128, 129])

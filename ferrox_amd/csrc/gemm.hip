@@ -565,16 +565,19 @@ __device__ __forceinline__ void wide_k_loop(f32x4_t (&acc)[MT][NT], const bf16* 
 // the larger model.  Eighths of equal cost, a tile's
 // rows and a constant, instead of equal numbers of tiles: no better, 237 us for the 3,500.)
 // `by_row_tile`: XCD x takes the row tiles x, x + 8, ... and runs through the columns of each, so weights that two row tiles
-// share are fetched by two XCDs, but no XCD has many full tiles where another has nearly empty ones, and nothing is counted: for the ring of 192 rows (512 tokens
-// on 40 experts, 55 against 66 us for the down product), and where the caller knows that no expert has a second row tile (both products of 64 decoded tokens
-// of the larger model, tiles of 64 rows, 598 against 617 us, of 128 tokens beside the shared expert's pieces, which all lie at the end, tiles of 128, 637 against
-// 682; of 128 tokens of the smaller one with tiles of 64, two to a piece, the other way, 221 against 194).
-// `alone`: the expert's rows are one tile (so they are taken to be with `by_row_tile`; either answer gives the same sums).
-template <int TM>
+// share are fetched by two XCDs, but no XCD has many full tiles where another has nearly empty ones, and nothing is counted (the ring of 192 rows, 512 tokens
+// on 40 experts, 55 against 66 us for the down product).
+// SPREAD, where the caller knows that no expert has a second row tile and nothing is shared: eighths of the tiles again, equal to one, but of the row tiles in
+// the order 0, 8, 16, .., 1, 9, .., so that full and nearly empty ones are dealt out (both products of 64 decoded tokens of the larger model, tiles of 64
+// rows, in order 617 us, dealt out 600, of 128 tokens beside the shared expert's pieces, which all lie at the end, tiles of 128, 673 in order with tiles of 64, 635; a prompt of 64
+// tokens, which takes some of the experts only, 3,550 a step either way, 3,910 with every eighth row tile, which are not equally many).  Not a flag tested here: the
+// step of 117 tokens, which has second row tiles, took 0.5-1 % more for it.
+// `alone`: the expert's rows are one tile (so they are taken to be with `by_row_tile` and SPREAD; either answer gives the same sums).
+template <int TM, bool SPREAD = false>
 __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end, int& expert, int& col_tile, bool* alone = nullptr) {
     const int lane = threadIdx.x & 63, C = g.n_col_tiles;
     if (alone) *alone = true;
-    if (g.by_row_tile && g.expert_offsets) {
+    if (!SPREAD && g.by_row_tile && g.expert_offsets) {
         const int i = blockIdx.x / 8, row_tile = (i / C) * 8 + blockIdx.x % 8;
         col_tile = i % C;
         locate_rows<TM>(g, row_tile, r0, r_end, expert);       // (r0 < 0: past the last one)
@@ -603,6 +606,13 @@ __device__ __forceinline__ bool wide_tile(const GemmArgs& g, int& r0, int& r_end
     const int per_xcd = (C * rows + 7) / 8, i = blockIdx.x / 8;
     const int logical = (blockIdx.x % 8) * per_xcd + i;
     if (i >= per_xcd || logical >= C * rows) return false;
+    if constexpr (SPREAD) {          // (rows sorted by expert)
+        const int s = logical / C, q = rows >> 3, m = rows & 7, longer = m * (q + 1);     // the first m of the eight have q + 1 row tiles
+        const int nth = s < longer ? s / (q + 1) : m + (s - longer) / max(q, 1), in = s < longer ? s % (q + 1) : (s - longer) % max(q, 1);
+        col_tile = logical % C;
+        locate_rows<TM>(g, in * 8 + nth, r0, r_end, expert);
+        return r0 >= 0;
+    }
     if (!g.expert_offsets) {
         int row;
         in_bands(logical, rows, row);
@@ -787,11 +797,11 @@ __device__ __forceinline__ void wide_block(const GemmArgs& g, bf16* stages, int 
     wide_epilogue<MT, NT, TM, WN, DUAL, EPI>(g, acc, r0, r_end, n0, wm, wn, lane);
 }
 
-template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false>
+template <int TMB, int TN, int NS, bool DUAL, int EPI, int NSA = NS, bool STREAM = false, bool SPREAD = false>
 __global__ __launch_bounds__(512) void gemm_bf16_wide_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) bf16 stages[(NSA * 16 * TMB + NS * TN) * 64];    // the rows' ring, then the weights'
     int r0, r_end, expert, col_tile;
-    if (!wide_tile<16 * TMB>(g, r0, r_end, expert, col_tile)) return;
+    if (!wide_tile<16 * TMB, SPREAD>(g, r0, r_end, expert, col_tile)) return;
     wide_block<TMB, TN, NS, DUAL, EPI, NSA, STREAM>(g, stages, r0, r_end, expert, col_tile);
 }
 
@@ -1047,13 +1057,13 @@ __global__ __launch_bounds__(512) void gemm_bf16_quarters_kernel(GemmArgs g) {
 //   300 tokens 590 420, 601 340, 579 315    400 611 455, 614 401, 597 377    600 642 525, 642 460, 627 460
 // (One hot expert among many, 300 of the larger: 590, 663 and 620.)
 // (With four stages of weights, all of LDS, 1 to 2 % more.)
-template <int TMB, int TN, int NS, bool DUAL, int EPI>
+template <int TMB, int TN, int NS, bool DUAL, int EPI, bool SPREAD>
 __global__ __launch_bounds__(512) void gemm_bf16_shares_kernel(GemmArgs g) {
     constexpr int RING = 2 * 16 * TMB + NS * TN, QUARTERS = 2 * (16 * TMB + TN);
     __shared__ __attribute__((aligned(1024))) bf16 stages[(RING > QUARTERS ? RING : QUARTERS) * 64];
     int r0, r_end, expert, col_tile;
     bool alone;
-    if (!wide_tile<16 * TMB>(g, r0, r_end, expert, col_tile, &alone)) return;
+    if (!wide_tile<16 * TMB, SPREAD>(g, r0, r_end, expert, col_tile, &alone)) return;
     if (alone) wide_block<TMB, TN, NS, DUAL, EPI, 2, true>(g, stages, r0, r_end, expert, col_tile);
     else quarters_block<TMB, TN, DUAL, EPI>(g, stages, r0, r_end, expert, col_tile);
 }
@@ -1889,16 +1899,16 @@ static dim3 wide_grid(GemmArgs& g, int epi, int tn, int m_tiles) {
     g.n_row_tiles = m_tiles;
     return dim3(g.by_row_tile && g.expert_offsets ? 8 * ceil_div(m_tiles, 8) * g.n_col_tiles : 8 * ceil_div((long)g.n_col_tiles * m_tiles, 8));
 }
-template <int TMB, int TN, int NS, int NSA, bool STREAM>
+template <int TMB, int TN, int NS, int NSA, bool STREAM, bool SPREAD = false>
 static void launch_wide(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
     g.tile_rows = 16 * TMB;
     const dim3 grid = wide_grid(g, epi, TN, m_tiles);
     switch (epi) {
-        case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
-        case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
-        case EPI_RESID: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_RESID, NSA, STREAM><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE, NSA, STREAM, SPREAD><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE_F32: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_STORE_F32, NSA, STREAM, SPREAD><<<grid, 512, 0, s>>>(g); break;
+        case EPI_RESID: gemm_bf16_wide_kernel<TMB, TN, NS, false, EPI_RESID, NSA, STREAM, SPREAD><<<grid, 512, 0, s>>>(g); break;
         default:
-            if constexpr (TN % 128 == 0) gemm_bf16_wide_kernel<TMB, TN, NS, true, EPI_GATED, NSA, STREAM><<<grid, 512, 0, s>>>(g);
+            if constexpr (TN % 128 == 0) gemm_bf16_wide_kernel<TMB, TN, NS, true, EPI_GATED, NSA, STREAM, SPREAD><<<grid, 512, 0, s>>>(g);
             break;
     }
 }
@@ -1915,15 +1925,15 @@ static void launch_quarters(GemmArgs g, int epi, int m_tiles, hipStream_t s, int
             break;
     }
 }
-template <int TMB, int TN, int NS>
+template <int TMB, int TN, int NS, bool SPREAD>
 static void launch_shares(GemmArgs g, int epi, int m_tiles, hipStream_t s) {
     g.tile_rows = 16 * TMB;
     const dim3 grid = wide_grid(g, epi, TN, m_tiles);
     switch (epi) {
-        case EPI_STORE: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE><<<grid, 512, 0, s>>>(g); break;
-        case EPI_STORE_F32: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE_F32><<<grid, 512, 0, s>>>(g); break;
-        case EPI_RESID: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_RESID><<<grid, 512, 0, s>>>(g); break;
-        default: gemm_bf16_shares_kernel<TMB, TN, NS, true, EPI_GATED><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE, SPREAD><<<grid, 512, 0, s>>>(g); break;
+        case EPI_STORE_F32: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_STORE_F32, SPREAD><<<grid, 512, 0, s>>>(g); break;
+        case EPI_RESID: gemm_bf16_shares_kernel<TMB, TN, NS, false, EPI_RESID, SPREAD><<<grid, 512, 0, s>>>(g); break;
+        default: gemm_bf16_shares_kernel<TMB, TN, NS, true, EPI_GATED, SPREAD><<<grid, 512, 0, s>>>(g); break;
     }
 }
 // Weights that are read about once go through the ring with the non-temporal hint, everything else in quarters.
@@ -2340,12 +2350,15 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         else if (!tile) tile = small_groups ? 64 : fx_gemm_grouped_tile((int)per_group, M, N, nonempty, dual, fx_compute_units());
         auto row_tiles = [&](int tm) { return M / tm + (expert_offsets ? nonempty : (M % tm != 0)); };
         // (see `wide_tile`; tiles of 64 rows seldom are two to an expert at up to five rows each)
-        g.by_row_tile = expert_offsets && (tile == 12 ? g.stream_w : tile == 4 ? per_group <= 5 || (max_share > 0 && max_share <= 64)
-                                                                            : tile == 1256 && max_share > 0 && max_share <= 128);
+        const bool one_tile = expert_offsets && max_share > 0 && max_share <= (tile == 4 ? 64 : tile == 1256 ? 128 : 0);
+        g.by_row_tile = expert_offsets && ((tile == 12 && g.stream_w) || (tile == 4 && per_group <= 5));
         switch (tile) {
             case 464: launch_ring<4, 64, 4>(g, epi, row_tiles(64), s); break;
             case 4128: launch_ring<4, 128, 3>(g, epi, row_tiles(64), s); break;
-            case 4: launch_ring<4, 256, 4, 2>(g, epi, row_tiles(64), s); break;
+            case 4:
+                if (one_tile && g.stream_w && !g.by_row_tile) launch_wide<4, 256, 4, 2, true, true>(g, epi, row_tiles(64), s);
+                else launch_ring<4, 256, 4, 2>(g, epi, row_tiles(64), s);
+                break;
             case 8128: launch_ring_or_quarters<8, 128, 2>(g, epi, row_tiles(128), s); break;
             case 64: launch_ring_or_quarters<8, 128, 4>(g, epi, row_tiles(128), s); break;
             case 12: launch_ring_or_quarters<12, 256, 3, 2>(g, epi, row_tiles(192), s); break;
@@ -2353,7 +2366,10 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
             case 6128: launch_quarters<8, 128>(g, epi, row_tiles(96), s, 96); break;
             case 6256: launch_quarters<8, 256>(g, epi, row_tiles(96), s, 96); break;
             case 8256: launch_quarters<8, 256>(g, epi, row_tiles(128), s); break;
-            case 1256: launch_shares<8, 256, 3>(g, epi, row_tiles(128), s); break;
+            case 1256:
+                if (one_tile) launch_shares<8, 256, 3, true>(g, epi, row_tiles(128), s);
+                else launch_shares<8, 256, 3, false>(g, epi, row_tiles(128), s);
+                break;
             case 192: launch_quarters<16, 192>(g, epi, row_tiles(256), s); break;
             case 128: launch_quarters<16, 128>(g, epi, row_tiles(256), s); break;
             default: launch_quarters<16, 256>(g, epi, row_tiles(256), s); break;

@@ -190,14 +190,14 @@ __device__ __forceinline__ bool locate_pairs(const GemmArgs& g, int tile, int& e
 enum { ACT_SILU = 0, ACT_GELU_TANH = 1, ACT_GELU = 2, ACT_RELU = 3, ACT_SWIGLU_CLAMP = 4, ACT_COUNT = 5 };
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 // The same for several elements at once: the quotient by a reciprocal, one step of refinement and no scaling, which the divisor, 1 to
-// e^80, does not need; beyond, and for NaN, as above.  The same bits for every float of either sign from 1e-30 to 80 (checked against
-// the division and against 64 bits), four instructions instead of eleven an element: the epilogue of a gate/up tile is bound by them.
+// e^80, does not need; where one of them is beyond that or infinite (inf / 1 has no remainder to refine with), as above.  The same bits for every float of either sign from
+// 1e-30 to 80 (checked against the division and against 64 bits), four instructions instead of eleven an element: the epilogue of a gate/up tile is bound by them.
 template <int N>
 __device__ __forceinline__ void silu_n(float (&x)[N]) {
-    bool plain = true;
+    float low = x[0], high = x[0];      // (a NaN among them is passed over and comes out of either path as one)
 #pragma unroll
-    for (int i = 0; i < N; ++i) plain = plain && x[i] > -80.0f;
-    if (plain) {
+    for (int i = 1; i < N; ++i) low = fminf(low, x[i]), high = fmaxf(high, x[i]);
+    if (low > -80.0f && high < INFINITY) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const float d = 1.0f + expf(-x[i]), r = __builtin_amdgcn_rcpf(d), q = x[i] * r;

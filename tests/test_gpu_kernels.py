@@ -272,6 +272,35 @@ def test_tiled_silu_at_the_ends_of_its_range():
     assert torch.equal(got[finite], want[finite]) and bool(torch.isnan(got[~finite]).all())
 
 
+@pytest.mark.parametrize("tile", [256, 128, 64, 12, 4, 4128, 8128, 8256, 1128, 6128, 6256])
+@pytest.mark.parametrize("N", [48, 200, 61])
+def test_a_gate_that_overflows_stays_infinite(tile, N):
+    """Two finite numbers whose product float32 does not hold, in the gates of every third column and the first row of every four, negative ones in
+    the second: an infinite gate times up is infinite with the sign of up (and NaN for minus infinity, whose quotient is inf / inf), in every tile as in
+    the kernel for few rows; the columns and rows beside it stay what they are."""
+    from ferrox_amd import debug, ops
+    a = torch.zeros(40, 64, dtype=torch.bfloat16)
+    a[:, 0] = torch.tensor([3e38, -3e38, 1e38, 0.0]).repeat(10)
+    a[:, 1] = torch.tensor([1.0, -1.0, 0.5, -2.0, 1.5]).repeat(8)
+    w = torch.zeros(2 * N, 64, dtype=torch.bfloat16)
+    w[:N, 0] = torch.tensor([2.0, 2.0 ** -125, 2.0 ** -126])[torch.arange(N) % 3]
+    w[N:, 1] = torch.tensor([1.0, -1.0])[torch.arange(N) % 2]
+    gate = a[:, :1].float() * w[:N, 0].float()          # (one product of each sum is not zero)
+    up = a[:, 1:2].float() * w[N:, 1].float()
+    want = (gate / (1.0 + torch.exp(-gate)) * up).to(torch.bfloat16)
+    assert bool((want == math.inf).any()) and bool((want == -math.inf).any()) and bool(torch.isnan(want).any())
+    a, w, want = a.to(DEV), w.to(DEV), want.to(DEV)
+    few = ops.gemm(a[:16], w, epilogue=ops.EPI_GATED)
+    with debug.kernel_switch("gemm", "wide", tile), debug.kernel_switch("gemm", "plain_rows", 1):
+        got = ops.gemm(a, w, epilogue=ops.EPI_GATED)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got, nan=0.0, posinf=1e38, neginf=-1e38)[:16],
+                                                                            torch.nan_to_num(few, nan=0.0, posinf=1e38, neginf=-1e38))
+    infinite = torch.isinf(want)
+    assert torch.equal(got[infinite], want[infinite])
+    finite = torch.isfinite(want)
+    assert torch.allclose(got[finite].float(), want[finite].float(), rtol=2.0 ** -7, atol=1e-30)      # (a rounding to bfloat16 either way)
+
+
 @pytest.mark.parametrize("M,N", [(33, 4096), (64, 8200), (129, 64), (257, 1000), (513, 2048), (700, 3000)])
 def test_plain_products_have_the_same_bits_in_every_tile(M, N):
     """The tile that the sizes choose (64 x 64 to 256 x 256, edges inside tiles) against one that is forced: every tile adds an

@@ -952,7 +952,7 @@ def decode_attention_chunk(n_items: int, n_heads: int, n_kv_heads: int, max_kv_l
         # a wave of the widest heads has a SIMD to itself and its tile's chain of waits is what takes the time: as many chunks as
         # one round of the SIMDs holds, down to one tile each (latent heads of 256 and 192, us, eight waves' worth a CU as below / so: 8 sequences of
         # 2,060 keys 20.6 / 17.3, 16 26.6 / 19.4, 32 of 1,030 26.8 / 19.3, of 2,060 34.9 / 26.9)
-        return -(-(-(-max_kv_len // 64)) // max(1, 4 * cus // pairs)) * 64
+        return max(64, -(-(-(-max_kv_len // 64)) // max(1, 4 * cus // max(1, pairs))) * 64)
     want = max(1, 8 * cus // max(1, pairs * 8))
     # More (sequence, kv head) pairs than CUs: a CU holds eight waves of this kernel, which the launch groups
     # into blocks of eight or four (one chunk a sequence), so the waves run in rounds, and a last round that

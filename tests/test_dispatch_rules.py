@@ -41,6 +41,12 @@ def test_chunks_of_the_widest_heads_are_one_round_of_the_simds():
             assert c % 64 == 0 and c >= 64 and (c == 64 or n * -(-kv // c) <= 1024 or c >= kv)
 
 
+def test_chunks_of_the_widest_heads_without_items_or_keys():
+    for hd in (64, 128, 192, 256):
+        assert ops.decode_attention_chunk(0, 16, 1, 2060, 256, hd) >= 64 and ops.decode_attention_chunk(0, 16, 1, 0, 256, hd) == 64
+        assert ops.decode_attention_chunk(8, 16, 1, 0, 256, hd) == 64 and ops.decode_attention_chunk(8, 16, 16, 0, 256, hd) == 64
+
+
 def test_half_sets_of_weight_rows_where_the_busiest_cu_fetches_less():
     from ferrox_amd.csrc.build import load_library
     rule = lambda m, n, dual=0, sets=None, cus=256: bool(load_library("gemm").fx_gemm_half_sets(

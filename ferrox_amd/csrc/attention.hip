@@ -1879,10 +1879,16 @@ __global__ __launch_bounds__(256 * G, 2) void attn_mfma_rows32_kernel(AttnArgs a
     const int tok = tok_first + min(32 * wave + li, n_all - 1);
     int hi = a.positions[tok], lo = first_visible(a, hi);
     if (li >= n) lo = 1, hi = 0;
-    int w_lo_max = 0x7fffffff, w_hi_min = -1;       // keys that all rows of the wave see
-    if (n == 32) {
-        w_hi_min = a.positions[tok0];
-        w_lo_max = first_visible(a, a.positions[tok0 + 31]);
+    int w_lo = 0x7fffffff, w_hi = -1;               // keys any row of the wave can see (the same in every lane, and kept as such)
+    int w_lo_max = 0x7fffffff, w_hi_min = -1;       // keys that all of them see
+    if (n > 0) {
+        const int first_pos = __builtin_amdgcn_readfirstlane(a.positions[tok0]), last_pos = __builtin_amdgcn_readfirstlane(a.positions[tok0 + n - 1]);
+        w_hi = last_pos;
+        w_lo = first_visible(a, first_pos);
+        if (n == 32) {
+            w_lo_max = first_visible(a, last_pos);
+            w_hi_min = first_pos;
+        }
     }
     const float cs = a.scale * LOG2E;
     float m = NEG_INF, l = 0.f;
@@ -2052,7 +2058,9 @@ __global__ __launch_bounds__(256 * G, 2) void attn_mfma_rows32_kernel(AttnArgs a
             weight(qc);
         });
         fence();
-        if (kt0 >= kv_end) return;             // (no such tile: its weights are zeros, but what the stage holds need not be numbers)
+        // Nothing in this tile for this wave's rows, or no such tile (which begins at kv_end): the weights are zeros and nothing would change, but values need not be
+        // numbers, and a product with them would be none either (an infinite value of a later token then reached every query of the item).
+        if (kt0 > w_hi || (kt0 + 64 <= w_lo && kt0 >= span.keep)) return;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
             for (int db = 0; db < 4; ++db)

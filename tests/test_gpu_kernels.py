@@ -959,6 +959,30 @@ def test_waves_of_32_queries(form, bs):
         assert bool((room[T] == 7).all()) and bool((room[:, :odd] == 7).all())
 
 
+@pytest.mark.parametrize("window,keep,broken,clean", [(0, 0, 100, [(0, 64)]), (0, 0, 200, [(0, 192)]), (0, 0, 300, [(0, 256)]),
+                                                      (64, 0, 70, [(0, 64), (192, 330)]), (64, 10, 70, [(0, 64), (192, 330)]), (64, 10, 5, [])])
+def test_a_value_that_is_not_a_number_reaches_no_wave_of_queries_that_sees_none_of_its_tile(window, keep, broken, clean):
+    """Infinite values of one key (a later one, one before the window, a kept one): queries in waves of 32 that see no key of its 64 have the bits that they have
+    without it, whatever the other waves of their item see; the queries that do see the key are not finite."""
+    from ferrox_amd import debug, ops
+    nh, nkv, hd, bs, n = 4, 2, 128, 64, 330
+    q, k, v, q_rot, k_pages, v_pages, table, pos, seq, toks = paged_setup(torch.bfloat16, nh, nkv, hd, bs, [n], 1e4, hd, 64)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    cols = [i32([0, 0, 0]), i32([0, 128, 256]), i32([128, 128, n - 256])]
+    bad = v_pages.clone()
+    bad[int(table[0, broken // bs]), :, :, broken % bs] = math.inf
+    sees = torch.arange(n)
+    sees = (sees >= broken) & ((sees - broken < window) | (broken < keep) if window else True)
+    for groups in (1, 2):
+        out = [torch.zeros(n, nh * hd, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        with debug.kernel_switch("attention", "rows32", 2), debug.kernel_switch("attention", "direct_groups", groups):
+            for y, vp in zip(out, (v_pages, bad)):
+                ops.attention_tiles(q_rot, y, k_pages, vp, table, pos, *cols, nh, nkv, hd, bs, window, hd ** -0.5, tile_q=128, keep_first=keep)
+        for b, e in clean:
+            assert torch.equal(out[0][b:e], out[1][b:e]), (groups, b, e)
+        assert not bool(torch.isfinite(out[1][sees.to(DEV)]).any()) and bool(torch.isfinite(out[0]).all())
+
+
 @pytest.mark.parametrize("form", ["plain", "window", "window_keep", "shaped", "chunked"])
 @pytest.mark.parametrize("vd,bs", [(192, 64), (256, 64), (16, 128)])
 def test_attention_of_the_widest_heads_in_blocks_of_64_queries(vd, bs, form):

@@ -943,11 +943,22 @@ def _check_attention_shapes(q, out, k_pages, v_pages, n_heads, n_kv_heads, head_
 SPLIT_PARTIAL_ROUNDS = True      # decode attention: more chunks where the blocks' last round over the CUs would be far from full
 
 
-def decode_attention_chunk(n_items: int, n_heads: int, n_kv_heads: int, max_kv_len: int, cus: int, head_dim: int = 128) -> int:
+def decode_attention_chunk(n_items: int, n_heads: int, n_kv_heads: int, max_kv_len: int, cus: int, head_dim: int = 128,
+                           span: int = 0, any_shape: bool = False) -> int:
     """Keys per chunk of the bfloat16 decode attention, where the caller names none: the fewest chunks that still put
     about eight waves on every CU (one chunk, and no merge launch, from as many (sequence, kv head) pairs as CUs
-    on), unless the waves' last round over the CUs would be far from full."""
+    on), unless the waves' last round over the CUs would be far from full.  `span`: the keys a mask lets a query see (0: all);
+    `any_shape`: the heads go to the kernel for any shape, which has a wave per head."""
     pairs = n_items * n_kv_heads * (-(-(n_heads // n_kv_heads) // 16))
+    if head_dim > 128 and any_shape:
+        # The same eight waves a CU, counted as this kernel has them, and an eighth more, so that a length just past whole chunks does not lengthen them all (us by pairs as below / by pairs with the line for matrix units / so: 16 heads of 512 on one kv
+        # head, 32 sequences of 2,060 keys 1,694 / 2,200 / 1,311, 8 of 8,200 2,194 / 2,287 / 2,142; of 200, 32 of 2,060 682 / 786 / 644; 16 of 168 on 16, 8 of 2,060 725 / 235 /
+        # 206; four or sixteen waves a CU up to 1.9 times that).  Its chunks lie at multiples of their length, so a span needs short ones wherever it begins: no
+        # more of them in all than one round of the SIMDs has pairs (16 of 512, 8 of 30,000 with a window of 1,024 1,616 / 461 / 463).
+        tiles = -(-max_kv_len // 64)
+        seen = min(tiles, (span + 126) // 64) if span else tiles      # (a span's first tile can begin up to 63 keys before it)
+        want, most = 9 * cus // max(1, n_items * n_heads), 4 * cus // max(1, pairs)
+        return max(1, -(-seen // max(1, want)), -(-tiles // max(1, want, most))) * 64
     if head_dim > 128:
         # a wave of the widest heads has a SIMD to itself and its tile's chain of waits is what takes the time: as many chunks as
         # one round of the SIMDs holds, down to one tile each (latent heads of 256 and 192, us, eight waves' worth a CU as below / so: 8 sequences of
@@ -989,7 +1000,10 @@ def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq,
     if chunk is None:
         chunk = 128 if q.dtype == torch.float32 else 256
         if q.dtype == torch.bfloat16:
-            chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device), head_dim)
+            any_shape = head_dim > 128 and (head_dim > 256 or head_dim % 16 or block_size % 16 or v_dim > head_dim or v_dim % 16 or q.stride(0) % 8
+                                            or (q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16)      # (as fx_attn_decode decides it)
+            span = int(window or mask_chunk or 0) if any_shape else 0
+            chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device), head_dim, span, bool(any_shape))
     splits = max(1, -(-max_kv_len // chunk))
     part_o = torch.empty((n, n_heads, splits, v_dim), dtype=torch.float32, device=q.device)
     part_ml = torch.empty((n, n_heads, splits, 2), dtype=torch.float32, device=q.device)

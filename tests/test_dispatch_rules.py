@@ -47,6 +47,19 @@ def test_chunks_of_the_widest_heads_without_items_or_keys():
         assert ops.decode_attention_chunk(8, 16, 1, 0, 256, hd) == 64 and ops.decode_attention_chunk(8, 16, 16, 0, 256, hd) == 64
 
 
+def test_chunks_of_wide_heads_on_the_kernel_for_any_shape():
+    """A wave per head there: eight or nine waves a CU, however few kv heads there are."""
+    rule = lambda n, nh, nkv, kv, span=0: ops.decode_attention_chunk(n, nh, nkv, kv, 256, 512, span, True)
+    assert rule(32, 16, 1, 2060) == rule(32, 16, 16, 2060) == 576 and rule(8, 16, 1, 8200) == 512 and rule(8, 16, 16, 2060) == 128
+    assert rule(1, 16, 1, 2060) == 64 and rule(5000, 16, 1, 100) == 128 and rule(0, 16, 1, 0) == rule(0, 16, 1, 500) == rule(8, 16, 1, 0) == 64
+    assert rule(1, 16, 1, 30000, 1024) == 64 and rule(8, 16, 1, 30000, 1024) == 256 and rule(8, 16, 1, 500, 1024) == rule(8, 16, 1, 500)
+    for n in (1, 8, 100):
+        for kv in (500, 8200, 30000):
+            for span in (0, 64, 1024):
+                c = rule(n, 16, 4, kv, span)
+                assert c % 64 == 0 and -(-kv // c) <= max(1, 2304 // (16 * n), 1024 // (4 * n))
+
+
 def test_half_sets_of_weight_rows_where_the_busiest_cu_fetches_less():
     from ferrox_amd.csrc.build import load_library
     rule = lambda m, n, dual=0, sets=None, cus=256: bool(load_library("gemm").fx_gemm_half_sets(

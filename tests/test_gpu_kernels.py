@@ -1037,6 +1037,36 @@ def test_attention_of_the_widest_heads_in_blocks_of_64_queries(vd, bs, form):
         assert torch.equal(out, got[128, 2]), key
 
 
+@pytest.mark.parametrize("form", ["plain", "window", "window_keep", "chunked"])
+@pytest.mark.parametrize("nh,nkv,hd,vd", [(16, 1, 256, 192), (32, 1, 256, 256), (8, 4, 256, 256), (28, 4, 192, 192), (4, 1, 320, 320), (3, 3, 200, 136)])
+def test_single_queries_of_wide_heads_far_into_a_sequence(nh, nkv, hd, vd, form):
+    """Chunks as the sizes and the mask choose them: sequences deep behind a mask's first key, at both ends of a tile and shorter than the mask, beside each other."""
+    from ferrox_amd import ops
+    bs, seq_lens = 64, [2100, 1, 64, 65, 700, 2047]
+    q, k, v, q_rot, k_pages, v_pages, table, pos, seq, toks = paged_setup(torch.bfloat16, nh, nkv, hd, bs, seq_lens, 1e4, min(hd, 256), 96)
+    v_pages = v_pages[:, :, :vd].contiguous()
+    window, mask_chunk = 130 if "window" in form else 0, 200 if form == "chunked" else 0
+    keep, scale = 20 if form == "window_keep" else 0, hd ** -0.5
+    kp, vp, tab = k_pages.double().cpu(), v_pages.double().cpu(), table.cpu().long()
+    last = [sum(seq_lens[:i + 1]) - 1 for i in range(len(seq_lens))]
+    want = torch.zeros(len(seq_lens), nh, vd, dtype=torch.float64)
+    for s, L in enumerate(seq_lens):
+        pages = tab[s, :-(-L // bs)]
+        ks = kp[pages].permute(0, 2, 1, 3).reshape(-1, nkv, hd)[:L].repeat_interleave(nh // nkv, 1)
+        vs = vp[pages].permute(0, 3, 1, 2).reshape(-1, nkv, vd)[:L].repeat_interleave(nh // nkv, 1)
+        t = torch.arange(L)
+        seen = (L - 1 - t < window) | (t < keep) if window else t >= ((L - 1) // mask_chunk * mask_chunk if mask_chunk else 0)
+        sc = (torch.einsum("hd,khd->hk", q_rot[last[s]].double().cpu().view(nh, hd), ks) * scale).masked_fill(~seen, -math.inf)
+        want[s] = torch.einsum("hk,khd->hd", torch.softmax(sc, -1), vs)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    for bound in (max(seq_lens), 30000):        # (what a recorded step is told is more than the sequences have)
+        out = torch.full((len(toks), nh * vd), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.attention_decode(q_rot, out, k_pages, v_pages, table, pos, i32(range(len(seq_lens))), i32(last), nh, nkv, hd, bs, window, scale,
+                             max_kv_len=bound, v_dim=vd, mask_chunk=mask_chunk, keep_first=keep)
+        close(out[last], want.reshape(len(seq_lens), nh * vd), torch.bfloat16, f"{form}, {bound} keys at most")
+        assert bool((out[:last[0]] == 7).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,bs,window", [(4, 4, 16, 16, 0), (3, 1, 32, 8, 16), (6, 3, 48, 4, 40), (2, 2, 128, 64, 0),
                                                  (8, 2, 80, 16, 7), (4, 1, 256, 32, 100), (4, 2, 64, 64, 50), (3, 1, 128, 128, 90),

@@ -2347,7 +2347,11 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
         // 14.3 and 16.1 ms with two waves a block, 11.9, 13.5 and 15.9 with four, 11.7, 13.3 and 15.6 with one).
         const long slots = 8L * fx_compute_units();
         const int nw_min = splits > 1 ? 1 : 4;
-        while (nw > 1 && ((size_t)nw * rows * (hdc + 2) * 4 > 48 * 1024 || nw * 64 >= 2 * chunk)) nw >>= 1;
+        // (wide heads under a mask: a sequence's own chunks hold its span's tiles, however long the sequences are.  17 chunks of one tile, 16 sequences of 16 heads on one
+        // kv head: a second wave that has nothing to do 22.6 us, without it 20.1)
+        const long span = hd > 128 ? (window > 0 ? window : mask_chunk) : 0;
+        const long own = span > 0 ? std::min<long>(chunk, ((span + 63 + splits - 1) / splits + 63) / 64 * 64 + (keep_first + 63L) / 64 * 64) : chunk;
+        while (nw > 1 && ((size_t)nw * rows * (hdc + 2) * 4 > 48 * 1024 || nw * 64 >= 2 * own)) nw >>= 1;
         while (nw > nw_min && n_blocks * (nw / 2) >= slots) nw >>= 1;
         if (splits == 1 && 2 * n_blocks >= slots) nw = 1;
         // heads wider than 128: a wave has a SIMD to itself, and waves beyond one round of the SIMDs cost a whole one more

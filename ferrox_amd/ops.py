@@ -949,21 +949,17 @@ def decode_attention_chunk(n_items: int, n_heads: int, n_kv_heads: int, max_kv_l
     about eight waves on every CU (one chunk, and no merge launch, from as many (sequence, kv head) pairs as CUs
     on), unless the waves' last round over the CUs would be far from full.  `span`: the keys a mask lets a query see (0: all);
     `any_shape`: the heads go to the kernel for any shape, which has a wave per head."""
-    pairs = n_items * n_kv_heads * (-(-(n_heads // n_kv_heads) // 16))
+    group = n_heads // n_kv_heads
+    pairs = n_items * n_kv_heads * (-(-group // 16))
+    tiles = -(-max_kv_len // 64)
+    seen = min(tiles, (span + 126) // 64) if span else tiles      # (a span's first tile can begin up to 63 keys before it)
     if head_dim > 128 and any_shape:
         # The same eight waves a CU, counted as this kernel has them, and an eighth more, so that a length just past whole chunks does not lengthen them all (us by pairs as below / by pairs with the line for matrix units / so: 16 heads of 512 on one kv
         # head, 32 sequences of 2,060 keys 1,694 / 2,200 / 1,311, 8 of 8,200 2,194 / 2,287 / 2,142; of 200, 32 of 2,060 682 / 786 / 644; 16 of 168 on 16, 8 of 2,060 725 / 235 /
         # 206; four or sixteen waves a CU up to 1.9 times that).  Its chunks lie at multiples of their length, so a span needs short ones wherever it begins: no
         # more of them in all than one round of the SIMDs has pairs (16 of 512, 8 of 30,000 with a window of 1,024 1,616 / 461 / 463).
-        tiles = -(-max_kv_len // 64)
-        seen = min(tiles, (span + 126) // 64) if span else tiles      # (a span's first tile can begin up to 63 keys before it)
         want, most = 9 * cus // max(1, n_items * n_heads), 4 * cus // max(1, pairs)
         return max(1, -(-seen // max(1, want)), -(-tiles // max(1, want, most))) * 64
-    if head_dim > 128:
-        # a wave of the widest heads has a SIMD to itself and its tile's chain of waits is what takes the time: as many chunks as
-        # one round of the SIMDs holds, down to one tile each (latent heads of 256 and 192, us, eight waves' worth a CU as below / so: 8 sequences of
-        # 2,060 keys 20.6 / 17.3, 16 26.6 / 19.4, 32 of 1,030 26.8 / 19.3, of 2,060 34.9 / 26.9)
-        return max(64, -(-(-(-max_kv_len // 64)) // max(1, 4 * cus // max(1, pairs))) * 64)
     want = max(1, 8 * cus // max(1, pairs * 8))
     # More (sequence, kv head) pairs than CUs: a CU holds eight waves of this kernel, which the launch groups
     # into blocks of eight or four (one chunk a sequence), so the waves run in rounds, and a last round that
@@ -979,7 +975,19 @@ def decode_attention_chunk(n_items: int, n_heads: int, n_kv_heads: int, max_kv_l
         rounds = pairs * per_block / (8 * cus)
         if (math.ceil(rounds) - rounds) / math.ceil(rounds) >= 0.10:
             want = 8
-    return max(64, -(-(-(-max_kv_len // want)) // 64) * 64)
+    chunk = max(64, -(-(-(-max_kv_len // want)) // 64) * 64)
+    if head_dim <= 128:
+        return chunk
+    # A wave of the widest heads has a SIMD to itself and its tile's chain of waits is what takes the time: as many chunks as one round of the SIMDs
+    # holds, down to one tile each of the keys that a query sees (us with the merge, as above / so; 16 heads on one kv head, latents of 256 and 192: 8 sequences of
+    # 2,060 keys 20.4 / 16.8, 16 26.3 / 19.1, 32 of 1,030 26.5 / 18.8, of 2,060 33.8 / 25.7; one of 30,000 with a window of 1,024 27.1 / 15.0, and 34.5 with a chunk for each
+    # of the sequence's tiles; 16 heads of 256 on 16 kv heads: 9 of 2,060 80.6 / 55.6, 20 of 500 48.5 / 36.5; on 4: 14 of 1,030 27.0 / 22.6, 36 of 8,200 276 / 188).
+    # As above it stays where a block's LDS holds the results of four waves, which then share a chunk of three tiles or more, and such blocks fill nine tenths of the CUs
+    # (16 heads on 4: one of 8,200 19.9 / 23.5, 5 of 2,060 19.3 / 21.2, 10 39.0 / 41.4 at 8,200; 28 heads of 192 on 4, 12 of 8,200 62.3 / 63.6; with one, two or eight
+    # query heads a kv head it is as often behind), and where one chunk, which no launch merges, fills seven eighths (16 heads on 4, 64 of 500 28.7 / 33.7; on 16, 14 of 2,060 83.2 / 84.5).
+    if pairs <= cus and ((3 <= group <= 7 and seen > 2 * want and 10 * pairs * want >= 9 * cus) or (group <= 7 and want == 1 and 8 * pairs >= 7 * cus)):
+        return chunk
+    return max(64, -(-tiles // max(1, min(seen, 4 * cus // max(1, pairs)))) * 64)
 
 
 def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq, item_tok,
@@ -1002,8 +1010,7 @@ def attention_decode(q, out, k_pages, v_pages, block_table, positions, item_seq,
         if q.dtype == torch.bfloat16:
             any_shape = head_dim > 128 and (head_dim > 256 or head_dim % 16 or block_size % 16 or v_dim > head_dim or v_dim % 16 or q.stride(0) % 8
                                             or (q.data_ptr() | k_pages.data_ptr() | v_pages.data_ptr()) % 16)      # (as fx_attn_decode decides it)
-            span = int(window or mask_chunk or 0) if any_shape else 0
-            chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device), head_dim, span, bool(any_shape))
+            chunk = decode_attention_chunk(n, n_heads, n_kv_heads, max_kv_len, compute_units(q.device), head_dim, int(window or mask_chunk or 0), bool(any_shape))
     splits = max(1, -(-max_kv_len // chunk))
     part_o = torch.empty((n, n_heads, splits, v_dim), dtype=torch.float32, device=q.device)
     part_ml = torch.empty((n, n_heads, splits, 2), dtype=torch.float32, device=q.device)

@@ -60,6 +60,31 @@ def test_chunks_of_wide_heads_on_the_kernel_for_any_shape():
                 assert c % 64 == 0 and -(-kv // c) <= max(1, 2304 // (16 * n), 1024 // (4 * n))
 
 
+def test_chunks_of_the_widest_heads_by_the_keys_that_a_query_sees():
+    """No more chunks than a span of keys touches tiles, wherever it begins, and chunks that cover the sequence; the same without a span that is shorter."""
+    rule = ops.decode_attention_chunk
+    for n in (1, 8, 16, 100, 1024):
+        for kv in (1, 64, 500, 2060, 30000):
+            for span in (1, 2, 64, 65, 66, 128, 1024, 5000, 50000):
+                c, whole = rule(n, 16, 1, kv, 256, 256, span), rule(n, 16, 1, kv, 256, 256)
+                chunks = -(-kv // c)
+                touched = max(-(-(first % 64 + span) // 64) for first in range(64))
+                assert c % 64 == 0 and c >= whole and chunks <= max(1, min(touched, -(-kv // whole))) and chunks * c >= kv
+                assert span < kv or c == whole
+    assert -(-30000 // rule(8, 16, 1, 30000, 256, 256, 1024)) == 17 and rule(8, 16, 1, 30000, 256, 256) == 256
+
+
+def test_chunks_of_wide_heads_with_few_query_heads_a_kv_head():
+    """3 to 7 query heads a kv head take the chunks of narrower heads where those hold three tiles or more and fill the CUs, and so does one chunk a sequence."""
+    wide = lambda n, nh, nkv, kv, span=0: ops.decode_attention_chunk(n, nh, nkv, kv, 256, 256, span)
+    narrow = lambda n, nh, nkv, kv: ops.decode_attention_chunk(n, nh, nkv, kv, 256)
+    for n, nh, nkv, kv in ((1, 16, 4, 8200), (5, 16, 4, 2060), (10, 16, 4, 8200), (12, 28, 4, 8200), (64, 16, 4, 500), (32, 16, 8, 2060), (14, 16, 16, 2060)):
+        assert wide(n, nh, nkv, kv) == narrow(n, nh, nkv, kv) >= 192
+    assert wide(1, 16, 4, 2060) == wide(4, 16, 4, 1030) == wide(14, 16, 4, 1030) == 64      # two tiles or fewer; blocks for 7/8 of the CUs
+    assert wide(36, 16, 4, 8200) == 1216 and wide(9, 16, 16, 2060) == 320 and wide(33, 16, 8, 500) == 192 and wide(1, 16, 16, 8200) == 192
+    assert wide(1, 16, 4, 30000, 1024) == 1792 and wide(8, 16, 4, 30000, 1024) == narrow(8, 16, 4, 30000)
+
+
 def test_half_sets_of_weight_rows_where_the_busiest_cu_fetches_less():
     from ferrox_amd.csrc.build import load_library
     rule = lambda m, n, dual=0, sets=None, cus=256: bool(load_library("gemm").fx_gemm_half_sets(

@@ -88,7 +88,8 @@ def test_float32_few_rows_in_whole_lines(N, K):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("N,K", [(8, 64), (61, 72), (61, 288), (100, 520), (256, 2048), (40, 4168), (2048, 1024)])
+@pytest.mark.parametrize("N,K", [(8, 64), (61, 72), (61, 288), (100, 520), (256, 2048), (40, 4168), (2048, 1024),
+                                 (24, 2560), (24, 3072), (24, 3584), (24, 4608), (24, 5120), (40, 5632), (24, 6144)])       # (5, 6, 7, 9, 10, 11 and 12 whole pieces a wave: every remainder of four)
 def test_half_sets_of_weight_rows_have_the_bits_of_whole_sets(dtype, N, K):
     """Up to 16 rows: blocks of eight weight rows (of each matrix), with two and with four pieces of K on their way, fewer pieces than that, the piece
     that K ends in, columns past the end; every epilogue, rows and slabs of weights; the sums of whole sets bit for bit."""
@@ -254,7 +255,8 @@ def test_wide_tiles_store_the_same_at_any_columns_and_alignment(tile, M, N):
 
 def test_tiled_silu_at_the_ends_of_its_range():
     """Gates that reach the activation exactly (one product of each sum is not zero), on both sides of where the quotient is scaled, and
-    beyond what the exponential holds: what 32-bit division gives, rounded to bfloat16."""
+    beyond what the exponential holds: what 32-bit division gives, rounded to bfloat16.  Operands that are no finite numbers stay in their rows (an
+    infinite gate beside a finite up is `test_a_gate_that_overflows_stays_infinite`)."""
     from ferrox_amd import debug, ops
     x = torch.tensor([0.0, -0.0, 1e-3, -1e-3, 1.0, -1.0, 20.0, -20.0, 79.5, -79.5, 80.0, -80.0, 80.5, -80.5, 87.0, -87.0, -88.5, 89.0, -103.0, 1e4, -1e4,
                       3e38, -3e38, math.inf, math.nan] * 8, dtype=torch.bfloat16, device=DEV)[:, None]
@@ -266,7 +268,7 @@ def test_tiled_silu_at_the_ends_of_its_range():
     want = (f / (1.0 + torch.exp(-f))).to(torch.bfloat16).expand(-1, 16)
     with debug.kernel_switch("gemm", "wide", 8128):
         assert torch.equal(ops.gemm(a, w, epilogue=ops.EPI_GATED), want)
-        a[:, :1] = x                                    # (infinities and NaN stay in their rows; 0 * inf in the other column is NaN too)
+        a[:, :1] = x                                    # (0 * inf in the up column: NaN, whatever the gate becomes)
         got = ops.gemm(a, w, epilogue=ops.EPI_GATED)
     finite = torch.isfinite(x[:, 0])
     assert torch.equal(got[finite], want[finite]) and bool(torch.isnan(got[~finite]).all())
@@ -1240,10 +1242,10 @@ def test_float32_single_queries_at_the_first_positions(nh, nkv, hd, vd):
 
 
 @pytest.mark.parametrize("bs", [8, 7])
-@pytest.mark.parametrize("longest", [128 * 8192, 128 * 8192 + 1, 128 * 16384])
+@pytest.mark.parametrize("longest", [128 * 7936, 128 * 7936 + 1, 128 * 8192, 128 * 8192 + 1, 128 * 16384])
 def test_float32_single_queries_beside_a_very_long_sequence(bs, longest):
     """The chunks of a float32 sequence, hence its bits, do not depend on the longest sequence that a launch is told of: up to
-    the most chunks that are merged, of which LDS holds the weights of 8,192.  (bs 8: the matrix units; 7: any shape)"""
+    the most chunks that are merged, of which LDS holds the weights and sums of 7,936.  (bs 8: the matrix units; 7: any shape)"""
     from ferrox_amd import ops
     nh, hd, n = 2, 16, 700
     q, k, v = rnd(1, nh * hd), rnd(n, 1, hd, seed=1), rnd(n, 1, hd, seed=2)
@@ -1261,6 +1263,29 @@ def test_float32_single_queries_beside_a_very_long_sequence(bs, longest):
     assert torch.equal(out[0], out[1])
     with pytest.raises(ops.KernelError):
         ops.attention_decode(q, y, kp, vp, table, i32([n - 1]), i32([0]), i32([0]), nh, 1, hd, bs, 0, hd ** -0.5, max_kv_len=128 * 16384 + 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("chunks", [7921, 7936, 7937, 7960])
+def test_merge_of_more_chunks_than_lds_holds(dtype, chunks):
+    """A sequence of that many chunks of 64 keys, every one of them with a weight: the first, the last and one in the middle of those that LDS holds
+    with the largest, so that chunks on both sides of what it holds decide the result."""
+    from ferrox_amd import ops
+    nh, hd, bs = 2, 16, 64
+    n = 64 * chunks - 5
+    q, k, v = rnd(1, hd, dtype=dtype).repeat(1, nh), rnd(chunks * bs, hd, dtype=dtype, seed=1), rnd(chunks * bs, hd, dtype=dtype, seed=2)
+    for at, score in ((3, 15.0), (64 * 4000 + 7, 16.0), (n - 70, 15.5), (n - 10, 14.5), (n - 1, 16.0)):      # (the others' weights: the size of one of e^13.5)
+        k[at] = (q[0, :hd].float() * (score * hd ** 0.5 / float((q[0, :hd].float() ** 2).sum()))).to(dtype)
+    q[0, hd:] *= 0.95
+    kp, vp = k.view(chunks, bs, hd)[:, None].contiguous(), v.view(chunks, bs, hd).transpose(1, 2)[:, None].contiguous()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    y = torch.zeros(1, nh * hd, dtype=dtype, device=DEV)
+    ops.attention_decode(q, y, kp, vp, i32([list(range(chunks))]), i32([n - 1]), i32([0]), i32([0]), nh, 1, hd, bs, 0, hd ** -0.5, max_kv_len=n, chunk=64)
+    sc = q.double().view(nh, hd) @ k[:n].double().T.contiguous() * hd ** -0.5
+    p = torch.softmax(sc, -1)
+    inside, beyond = p[:, :64 * 7900].sum(-1), p[:, n - 64:].sum(-1)
+    assert bool((inside > 0.05).all()) and bool((beyond > 0.05).all())
+    close(y.view(nh, hd), p @ v[:n].double(), dtype, f"{chunks} chunks")
 
 
 @pytest.mark.parametrize("hd,bs,window", [(64, 16, 0), (64, 64, 0), (128, 64, 40000), (32, 16, 9000)])
@@ -1293,6 +1318,29 @@ def test_attention_over_more_pages_than_a_block_copies(hd, bs, window):
         ops.attention_decode(q_rot, out2, k_pages, v_pages, table, pos, i32([0]), i32([L - 1]), nh, nkv, hd, bs, window, scale,
                              max_kv_len=L, chunk=chunk)
         close(out2[L - 1], ref[63], dtype, f"decode attention chunk {chunk}")
+
+
+@pytest.mark.parametrize("window", [0, 64 * 1027])
+def test_waves_of_32_queries_over_more_pages_than_a_block_copies(window):
+    """The last 131 tokens of a sequence of more than 1024 pages, in items of 128 on waves of 32 queries: the first pages' ids come from LDS, the last ones' from the table."""
+    from ferrox_amd import debug, ops
+    nh, nkv, hd, bs, n = 2, 1, 128, 64, 131
+    L = bs * 1030 + 5
+    q, k, v, q_rot, k_pages, v_pages, table, pos, seq, toks = paged_setup(torch.bfloat16, nh, nkv, hd, bs, [L], 1e6, hd, 1040)
+    pages = table[0].long()
+    ks, vs = k_pages[pages].permute(0, 2, 1, 3).reshape(-1, hd)[:L].double(), v_pages[pages].permute(0, 3, 1, 2).reshape(-1, hd)[:L].double()
+    back = pos[L - n:, None] - pos[None]
+    seen = (back >= 0) & (back < window) if window else back >= 0
+    want = torch.zeros(n, nh, hd, dtype=torch.float64, device=DEV)
+    for h in range(nh):
+        sc = q_rot[L - n:, h * hd:(h + 1) * hd].double() @ ks.T.contiguous() * hd ** -0.5
+        want[:, h] = torch.softmax(sc.masked_fill(~seen, -math.inf), -1) @ vs
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    for groups in (1, 2):
+        out = torch.zeros(L, nh * hd, dtype=torch.bfloat16, device=DEV)
+        with debug.kernel_switch("attention", "rows32", 2), debug.kernel_switch("attention", "direct_groups", groups):
+            ops.attention_tiles(q_rot, out, k_pages, v_pages, table, pos, i32([0, 0]), i32([L - n, L - 3]), i32([128, 3]), nh, nkv, hd, bs, window, hd ** -0.5, tile_q=128)
+        close(out[L - n:], want.reshape(n, nh * hd), torch.bfloat16, f"{groups} group(s)")
 
 
 def test_decode_attention_of_a_short_sequence_beside_a_very_long_one():

@@ -1315,7 +1315,7 @@ static size_t bias_lds_bytes(const AttnArgs& a) { return a.bias ? (size_t)bias_r
 
 // Which item and head a block of a prompt takes.  Blocks go to the 8 XCDs in turn, each with an L2 of its own: block b runs on XCD b % 8, as number j = b / 8 there.
 // Later items of a prompt see more keys, so every XCD takes the items from the last to the first, each for the heads that are its own: an eighth of them, so
-// that their keys and values stay in its L2.  Where that is no whole number, the lines between the XCDs shift from item to item, through the eighths of a
+// that their keys and values stay in its L2 (the eight, and the 32 CUs below, are this GPU's; another would lose balance, no item).  Where that is no whole number, the lines between the XCDs shift from item to item, through the eighths of a
 // head in turn, and eight items make nh blocks for each.  PAIRED: two blocks fit a CU, and as the first 64 of an XCD are handed out to its 32 CUs in turn the
 // second half of them runs the other way, so that a CU's two have the same work together.  (Before, an XCD took an eighth of the pairs, heads outermost: with 28 heads half of an XCD's
 // last head was the long half, 7 % more than its share, and every other head's longest item came last.)
@@ -1553,7 +1553,9 @@ __global__ __launch_bounds__(256, HD > 128 ? 2 : 1) void attn_mfma_block_kernel(
 // Prefill when head_dim is exactly 64 or 128 and a page holds a multiple of 64 keys: a tile of 64
 // keys then lies in one page, 64 * HD contiguous elements of keys and as many of transposed values,
 // and travels from global memory straight into LDS (no registers in between, nothing to unpack),
-// two stages, the next tile's loads in flight while this one is multiplied, one barrier per tile.
+// two stages, one barrier per tile.  (The next tile's loads are asked for in front of this one's products, but not in flight
+// beside them: the compiler cannot tell the reads of LDS from what these loads write there, and waits for all of them, s_waitcnt
+// vmcnt(0), in front of the first read behind them.  What a second stage hides is the way to that read, and other waves.)
 // A wave-load fills 1 KB: 1024 / (2 HD) key rows, or eight value rows of 64 keys.  Key row
 // 16 kb + 4 a + b of LDS holds key 16 a + 4 kb + b (what the MFMA operands want, see above; four
 // such keys follow each other in memory and in LDS alike), and inside a row the 16-byte chunks
@@ -1596,7 +1598,7 @@ __device__ __forceinline__ void each(F&& f) {
 // four column blocks ahead (values).  us left to the compiler / so / with value_turn and the pairs of keys that an edge masks, 16 heads of 256 and 192 numbers: 1,337
 // tokens 69 / 53 / 51, 2,048 104 / 83 / 82, at 4,096 keys 295 / 233 / 229, 4,000 210 / 171 / 166; left to the compiler / all of it, items of 64 of 16 heads of 128: 497
 // tokens 16.7 / 16.1, at 2,048 keys 51.5 / 49.1, 28 heads over 4, 60 tokens at 2,048 43.4 / 42.0; without read-ahead, items of 128 of 16 heads of 128, 1,000 tokens 33.5 / 31.0.
-// What is left of a tile (2.2 us at 256) is neither LDS (1.3 us) nor the matrix units (0.8) but a wave's own chain and its tile's way into LDS.
+// What is left of a tile (2.2 us at 256) is neither LDS (1.3 us) nor the matrix units (0.8) but a wave's own chain, in which the next tile's way into LDS is waited for (above).
 template <int HD, int NS, int W, int G, int SHAPE>
 __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : W / 2) void attn_mfma_direct_kernel(AttnArgs a) {      // two blocks on a CU, or one of two groups
     const int vd = HD > 128 ? a.vd : HD;
@@ -1854,10 +1856,11 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : W / 2) void attn_mfm
 // one exchange between the halves of the wave.  The accumulator of lane (q, h = lane / 32) holds rows 8 (i / 4) + 4 h + i % 4; key row 16 s + 8 a + 4 h + b of LDS
 // (within 32) holds key 16 s + 8 h + 4 a + b, so that a lane's scores 8 s .. 8 s + 7 are of the eight keys 16 s + 8 h .. that it supplies to
 // the second product, whose other operand is then 16 bytes of a value row.
-// 256 registers, two waves a SIMD: two blocks of four waves on a CU, or one whose two groups take the tiles in turn (fx_attn_rows32 has the line and its
-// figures).  us, waves of 16 / of 32 queries: 28 heads over 4, 4,096 queries at 0 165 / 140, at 4,096 453 / 380, at 12,288 1,070 / 857 (787 / 982 TFLOP/s), 12,000 at 0
-// 1,200 / 1,035; 16 heads, 2,048 at 0 56 / 47, 8,000 335 / 310.  What is left of a round are waits in a wave's own chain (a wave alone on its SIMD takes 1.9 us a tile, two
-// take 2.3).  A register more a tile to touch lines two and three rounds ahead: slower (907 -> 1,082).
+// 250 registers (256 and 36 bytes a lane in scratch memory with two groups, of which an edge tile reloads some), two waves a SIMD: two blocks of four waves on a CU, or one
+// whose two groups take the tiles in turn (fx_attn_rows32 has the line and its figures).  us, waves of 16 / of 32 queries: 28 heads over 4, 4,096 queries at 0 168 / 140, at 4,096
+// 456 / 379, at 12,288 1,070 / 857 (787 / 982 TFLOP/s), 12,000 at 0 1,213 / 1,028; 16 heads, 2,048 at 0 51 / 47, 8,000 337 / 278.  What is left of a round are waits in a wave's own chain (a wave
+// alone on its SIMD takes 1.9 us a tile, two take 2.3), a whole trip of the loads for the next two tiles among them, which are waited for in front of the round's first read of LDS as in the kernel
+// above.  A register more a tile to touch lines two and three rounds ahead: slower (907 -> 1,082).
 template <int G>
 __global__ __launch_bounds__(256 * G, 2) void attn_mfma_rows32_kernel(AttnArgs a) {
     constexpr int HD = 128, W = 4, NS = 2, NLOAD = 4, TILE = 2 * 64 * HD;
@@ -1970,7 +1973,8 @@ __global__ __launch_bounds__(256 * G, 2) void attn_mfma_rows32_kernel(AttnArgs a
     issue_values(first, 0);
     f32x16_t sc[2], next[2];
     scores(sc, 0);
-    // A round: the products of the next tile's keys run under this tile's softmax, then come its values.  What a round waits for was asked for a round ago.
+    // A round: the products of the next tile's keys run under this tile's softmax, then come its values.  Both were asked for a round ago and landed then; what this
+    // round asks for has landed before its first product too (see above).
     auto one = [&](auto sg, int round, f32x16_t (&now)[2], f32x16_t (&then)[2]) {
         constexpr int stage = decltype(sg)::value;
         const int kt0 = start(round + grp);
@@ -2196,10 +2200,11 @@ FX_API int fx_attn_block_place(int b, int nh, int n_items, int paired) {
 }
 
 // Groups of waves of 32 queries for that many blocks, or 0: waves of 16.  us with 16 (the better of one and two groups) / 32 one group / 32 two groups, 28 heads over 4 and
-// (*) 16 heads: 160 blocks* 35 / 46 / 37, 168 24 / 30 / 27, 176* 37 / 50 / 40, at 8,192 keys 199 / 292 / 207; 192* 47 / 57 / 44, 196 at 8,192 191 / 277 / 192, 224 36 / 42 / 34, 256* 56 / 53 / 47,
-// 336 50 / 59 / 46, 448 63 / 76 / 56, at 8,192 350 / 368 / 330, 512* 111 / 134 / 106, 640* 158 / 182 / 149, at 8,192 637 / 579 / 549, 752* 194 / 225 / 194; 784 129 / 111 / 134, at 8,192
-// 681 / 565 / 675, 896 165 / 140 / 165, at 12,288 1,070 / 857 / 980, 1,008* 335 / 310 / 329.  So two blocks of one group on a CU from three a CU on, where
-// they even out; before, two groups; and with a quarter of the CUs idle four waves a SIMD hide more than two do.
+// (*) 16 heads: 160 blocks* 36 / 36 / 31, 168 25 / 25 / 24, 176* 37 / 38 / 33, at 8,192 keys 215 / 233 / 175; 192* 40 / 41 / 35, 196 at 8,192 206 / 221 / 166, 224 30 / 31 / 28, 256* 51 / 54 / 47,
+// 336 41 / 44 / 38, 448 59 / 59 / 55, at 8,192 353 / 289 / 334, 512* 111 / 111 / 96, 640* 166 / 145 / 154, at 8,192 676 / 558 / 562, 752* 200 / 177 / 199; 784 133 / 111 / 137, at 8,192
+// 718 / 574 / 686, 896 168 / 140 / 167, at 12,288 1,070 / 855 / 987, 1,008* 337 / 279 / 323.  So two blocks of one group on a CU from three a CU on, where
+// they even out, and before, two groups.  The line was drawn when a wave still multiplied tiles that it does not see, at 3/4 of a block a CU for waves of 16 queries and three a CU for one
+// group: since then the columns say two groups from 160 blocks on and one from some 600, which is not done yet.
 FX_API int fx_attn_rows32(long blocks, int cus) { return 4 * blocks < 3L * cus ? 0 : blocks <= 3L * cus ? 2 : 1; }
 
 // Queries in blocks: item i covers item_n[i] <= tile_q consecutive tokens of one sequence; tile_q is 64, or what

@@ -377,13 +377,18 @@ class PagedAttention(Mixer):
 
     def tile_queries(self, ctx, dtype, block_size: int) -> int:
         """Queries per work item of this step's prompt portions: 64, or 128 where the kernel takes that many (a block
-        of eight waves then shares every tile of keys it brings in between twice as many queries).  The kernel gives
+        then shares every tile of keys it brings in between twice as many queries).  The kernels give
         a launch of no more blocks than the GPU has CUs (256) two groups of waves per block, which halves a block's chain of
-        tiles; so: items of 64 while they number no more than the CUs; else items of 128 if those do (a 2,048-token
-        portion deep in a prompt: 603 against 784 us at 16 heads); else items of 128 if they still number about
+        tiles; so: items of 64 while they number no more than the CUs; else items of 128 if those do (16 heads, a 2,048-token
+        portion at depth 24,576: heads of 64 412 against 467 us; of 128, whose waves then take 32 queries, 465 against 623, at
+        depth 0 47 against 52); else items of 128 if they still number about
         one evenly loaded block per CU (blocks of a portion that starts a prompt differ in work up to the portion's
-        length in keys and count by their mean share of the longest; +8-26 % from 448 such blocks on); else 64.
-        Measured with heads of 64 and 128.  Heads of 256 take items of 64: their block of 128 queries is alone on its CU
+        length in keys and count by their mean share of the longest; 16 heads of 128, 4,096 tokens 97 against 120 us, 8,000
+        278 against 405; 28 heads over 4, 4,096 at depth 12,288 858 against 1,344); else 64.
+        The last line is that of blocks of eight waves of 16 queries, which heads of 64 and shaped scores still take (heads of 64, 2,500
+        tokens 64 against 57 us with items of 64); waves of 32 queries would pay in front of it too (16 heads of 128, 2,049 tokens
+        56 against 59 us, 3,000 78 against 88, 3,900 99 against 112), which is not done yet.
+        Heads of 256 take items of 64: their block of 128 queries is alone on its CU
         and has no second group of waves, so none of the above holds for it (latents, one key head for all, have a
         rule of their own)."""
         if ctx.recorded or self.v_dim != self.head_dim or self.head_dim > 128 or \

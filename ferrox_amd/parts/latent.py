@@ -210,7 +210,7 @@ class LatentAttention(Mixer):
         debug.region("attention")
         out = torch.empty((T, H * R), dtype=q.dtype, device=q.device)
         # items of 128 queries where the kernel takes them (latents of 256 numbers) and a portion is longer: one launch over 16 heads of 256 and
-        # 192 numbers 53 us for 1,337 tokens against 60 with blocks of 64, 4,000 173 against 307, 300 17.5 against 20.4, 200 the same
+        # 192 numbers 51 us for 1,337 tokens against 62 with blocks of 64, 4,000 167 against 305, 300 17.6 against 21.0, 200 the same
         tile_q = 64 if longest_portion(ctx) <= 128 else ops.attention_tile_queries(q_lat.dtype, R + P, cache.block_size, v_dim=R)
         items = ctx.memo(f"attention_items {tile_q}", lambda: attention_items(ctx, tile_q))
         common = (H, 1, R + P, cache.block_size, self.window, self.scale)

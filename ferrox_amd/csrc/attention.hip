@@ -1718,12 +1718,36 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : W / 2) void attn_mfm
             any_edge = any_edge || (round + q < walk.n && !span.holds_tile(walk.start(round + q)));
         if (any_edge) {
             if (kt0 < kv_end && !span.holds_tile(kt0)) {
-                uint32_t* v = (uint32_t*)(st + 64 * HD);
-                const int pair = tid & 31;                 // of keys, the same in all rows that this thread takes
-                uint32_t kept[1] = {0xffffffffu};
-                key_masks(kept, kt0 + 2 * pair, span);
-                if (kept[0] != 0xffffffffu)
-                    for (int d = tid >> 5; d < vd; d += 2 * W) v[d * 32 + ((pair >> 2) ^ value_turn(d)) * 4 + (pair & 3)] &= kept[0];
+                if constexpr (W == 8 && G == 1 && HD <= 128) {
+                    // (two such blocks on a CU fill LDS with their reads: stores alone, a key at a time.  16 heads of 128 over 4 with biases, 4,096 tokens 145 us with pairs read and
+                    // written, 134 so; capped, 4,096 175 and 168, 8,000 450 and 438; two groups on a CU 46 and 49 for 1,337, one block of heads of 256 31.8 and 32.9 for 700)
+                    for (int idx = tid; idx < vd * 64; idx += W * 64) {
+                        const int d = idx >> 6, key = idx & 63;
+                        if (!span.has(kt0 + key)) st[64 * HD + d * 64 + (((key >> 3) ^ value_turn(d)) * 8) + (key & 7)].bits = 0;
+                    }
+                } else {
+                    uint32_t* v = (uint32_t*)(st + 64 * HD);
+                    const int pair = tid & 31;                 // of keys, the same in all rows that this thread takes
+                    uint32_t kept[1] = {0xffffffffu};
+                    key_masks(kept, kt0 + 2 * pair, span);
+                    if (kept[0] != 0xffffffffu) {
+                        // (with few waves beside it a wave has eight reads on their way at once: one after the other 16 of them took a microsecond of a launch, 16 heads of 128,
+                        // 60 tokens 9.6 us, so 8.1, with a window of 256 at 2,048 keys 15.7 and 12.5; items of 128, whose waves hide each other's reads, are behind with several)
+                        constexpr int B = W == 4 ? 8 : 1;
+                        for (int r = 0; r < vd; r += 2 * W * B) {
+                            uint32_t was[B], *at[B];
+#pragma unroll
+                            for (int i = 0; i < B; ++i) {
+                                const int d = r + 2 * W * i + (tid >> 5);
+                                at[i] = v + d * 32 + ((pair >> 2) ^ value_turn(d)) * 4 + (pair & 3);
+                                if (r + 2 * W * i < vd) was[i] = *at[i];
+                            }
+#pragma unroll
+                            for (int i = 0; i < B; ++i)
+                                if (r + 2 * W * i < vd) *at[i] = was[i] & kept[0];
+                        }
+                    }
+                }
             }
             lds_barrier();      // the zeros are in LDS (a bare s_barrier does not wait for this wave's stores) before any wave reads values
         }

@@ -1600,9 +1600,9 @@ __device__ __forceinline__ void each(F&& f) {
 // tokens 16.7 / 16.1, at 2,048 keys 51.5 / 49.1, 28 heads over 4, 60 tokens at 2,048 43.4 / 42.0; without read-ahead, items of 128 of 16 heads of 128, 1,000 tokens 33.5 / 31.0.
 // What is left of a tile (2.2 us at 256) is neither LDS (1.3 us) nor the matrix units (0.8) but a wave's own chain, in which the next tile's way into LDS is waited for (above).
 template <int HD, int NS, int W, int G, int SHAPE>
-__global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : W / 2) void attn_mfma_direct_kernel(AttnArgs a) {      // two blocks on a CU, or one of two groups
+__global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ? 4 : W / 2) void attn_mfma_direct_kernel(AttnArgs a) {      // two blocks on a CU (heads of 64: four), or one of two groups
     const int vd = HD > 128 ? a.vd : HD;
-    constexpr bool AHEAD = HD > 128 || W == 4;      // no more than two waves on a SIMD
+    constexpr bool AHEAD = HD > 128 || W == 4;      // no more than two waves on a SIMD (heads of 64, whose four blocks fit a CU: up to four, but few where it counts)
     static_assert(G == 1 || (G == 2 && NS == 2), "one group, or two with two stages each");
     constexpr int KS = HD / 32, CB = HD / 16;
     constexpr int NCH = HD / 8;                 // 16-byte chunks of a key row
@@ -1760,7 +1760,8 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : W / 2) void attn_mfm
         };
         auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
         if constexpr (AHEAD) {
-            constexpr int D = 6, N = 4 * KS;
+            // (heads of 64, one group: four, in 128 registers.  With 131 three blocks fitted a CU instead of four, 32 heads over 8, 2,048 tokens at 8,192 keys 295 us, so 260; a window of 1,024 46 and 40)
+            constexpr int D = HD == 64 && G == 1 ? 4 : 6, N = 4 * KS;
             bf16x8_t ring[D + 1];
             auto read_key = [&](auto qc) {
                 constexpr int q = decltype(qc)::value;

@@ -1604,6 +1604,8 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
     const int vd = HD > 128 ? a.vd : HD;
     constexpr bool AHEAD = HD > 128 || W == 4;      // no more than two waves on a SIMD (heads of 64, whose four blocks fit a CU: up to four, but few where it counts)
     static_assert(G == 1 || (G == 2 && NS == 2), "one group, or two with two stages each");
+    // (heads of 64 in items of 128 keep the plain order: 16 over 4, 1,500 tokens at 8,192 keys 176 us with value_turn, 170 so; in items of 64 value_turn is ahead, 90 -> 78)
+    auto turn_of = [](int d) { return HD == 64 && W == 8 ? (d >> 1) & 7 : value_turn(d); };
     constexpr int KS = HD / 32, CB = HD / 16;
     constexpr int NCH = HD / 8;                 // 16-byte chunks of a key row
     constexpr int KROWS = 1024 / (2 * HD);      // key rows of a wave-load
@@ -1673,7 +1675,7 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
         const int key = 16 * ((row >> 2) & 3) + 4 * (row >> 4) + (row & 3);
         k_src[i] = key * HD + (((lane % NCH) ^ (NCH >= 16 ? (row & 15) : ((row >> 1) & 7))) * 8);
         const int d = 8 * j + (lane >> 3);                   // value row
-        v_src[i] = d * bs + (((lane & 7) ^ value_turn(d)) * 8);
+        v_src[i] = d * bs + (((lane & 7) ^ turn_of(d)) * 8);
     }
     auto issue = [&](int kt0, int stage) {
         int blk, slot;
@@ -1693,7 +1695,7 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
     };
     // operands: key row 16 kb + li, chunk 4 u + g; value row 16 cb + li, chunks 2 g and 2 g + 1
     const int k_at = li * HD, v_at = 64 * HD + li * 64;
-    const int ksw = NCH >= 16 ? li : (li >> 1) & 7, vsw = value_turn(li);
+    const int ksw = NCH >= 16 ? li : (li >> 1) & 7, vsw = turn_of(li);
 
     // Every wave of the block goes through the same barriers: the loop runs over rounds of G tiles, of which group
     // grp takes tile grp (a round's last tiles may not exist: that group then only keeps step).
@@ -1723,7 +1725,7 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
                     // written, 134 so; capped, 4,096 175 and 168, 8,000 450 and 438; two groups on a CU 46 and 49 for 1,337, one block of heads of 256 31.8 and 32.9 for 700)
                     for (int idx = tid; idx < vd * 64; idx += W * 64) {
                         const int d = idx >> 6, key = idx & 63;
-                        if (!span.has(kt0 + key)) st[64 * HD + d * 64 + (((key >> 3) ^ value_turn(d)) * 8) + (key & 7)].bits = 0;
+                        if (!span.has(kt0 + key)) st[64 * HD + d * 64 + (((key >> 3) ^ turn_of(d)) * 8) + (key & 7)].bits = 0;
                     }
                 } else {
                     uint32_t* v = (uint32_t*)(st + 64 * HD);
@@ -1739,7 +1741,7 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
 #pragma unroll
                             for (int i = 0; i < B; ++i) {
                                 const int d = r + 2 * W * i + (tid >> 5);
-                                at[i] = v + d * 32 + ((pair >> 2) ^ value_turn(d)) * 4 + (pair & 3);
+                                at[i] = v + d * 32 + ((pair >> 2) ^ turn_of(d)) * 4 + (pair & 3);
                                 if (r + 2 * W * i < vd) was[i] = *at[i];
                             }
 #pragma unroll

@@ -2232,6 +2232,19 @@ FX_API int fx_attn_block_place(int b, int nh, int n_items, int paired) {
 // group: since then the columns say two groups from 160 blocks on and one from some 600, which is not done yet.
 FX_API int fx_attn_rows32(long blocks, int cus) { return 4 * blocks < 3L * cus ? 0 : blocks <= 3L * cus ? 2 : 1; }
 
+// The same where a mask, a window of `span` keys or chunks of that many, bounds the keys that a query sees.  Items of a few tiles are what the longer start and end of waves of 32 queries take; and behind
+// the first span all items of a window have the same work, so from a block a CU on one group, which leaves no wave without a tile.  us with 16 (one group; up to a block a CU two) / 32 one / 32 two, at
+// 8,192 keys: 16 heads, 2,048 tokens (256 blocks), a window of 256 19 / 23 / 22, 1,024 36 / 40 / 36, 2,048 60 / 65 / 56; 4,096 (512) 256 30 / 31 / 42, 512 39 / 40 / 50, 1,024 60 / 57 / 68, 4,096 187 / 160 / 175;
+// 6,000 (752) 512 57 / 60 / 73, 700 70 / 72 / 88, 1,024 89 / 86 / 99; 28 heads over 4, 1,500 (336) 256 26 / 26 / 38, 1,024 53 / 49 / 63, 4,096 167 / 145 / 164; 4,096 (896) 256 47 / 53 / 73.  Chunks, whose
+// items see from none to all of one, at 9,000 keys: 2,048 tokens, chunks of 2,048 59 / 77 / 61, 4,096 72 / 79 / 66; 4,096 (512) 1,024 54 / 54 / 73, 1,536 69 / 70 / 85, 4,096 140 / 149 / 121; 1,500 (336) 1,024 45 / 49 / 54,
+// 1,536 72 / 72 / 70; 3,000 (672) 2,048 93 / 94 / 112, 8,192 152 / 134 / 159.  Two groups where most of the launch's tokens can lie in front of the span, as in a prompt without a mask (4,096 tokens at 0, a window
+// of 4,096 129 / 111 / 96, chunks 125 / 114 / 101), up to 5/2 blocks a CU (5,000 at 0 143 / 132 / 143); with windows and fewer than two, only portions behind a long context come in items of 128.
+FX_API int fx_attn_rows32_masked(long blocks, int cus, long span, int chunked, long tokens) {
+    if (4 * blocks < 3L * cus || span <= (chunked ? 1024 : 768)) return 0;
+    if (blocks <= cus) return span > (chunked ? 2048 : 1024) ? 2 : 0;
+    return 2 * blocks < 5L * cus && 4 * span > 3 * tokens && (chunked || blocks >= 2L * cus) ? 2 : 1;
+}
+
 // Queries in blocks: item i covers item_n[i] <= tile_q consecutive tokens of one sequence; tile_q is 64, or what
 // fx_attn_tile_queries gives for these sizes.
 FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void* out, long ldo,
@@ -2269,6 +2282,8 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
     // (measured: 512-token portions at depth 8k-24k 130 and 360 us against 214 and 616 us; from 448 blocks on, one
     // group and two blocks to a CU are as fast or faster)
     const bool two_groups = g_groups ? g_groups == 2 : (long)n_items * nh <= fx_compute_units();
+    const long span = window > 0 ? window : mask_chunk, blocks = (long)n_items * nh;
+    const int rows32 = span > 0 ? fx_attn_rows32_masked(blocks, fx_compute_units(), span, window <= 0, 128L * n_items) : fx_attn_rows32(blocks, fx_compute_units());
     const bool beyond = hd > HD_MAX || vd > HD_MAX;      // heads wider than the matrix-unit kernels take
     if (dtype == FX_F32 && f32_mfma_ok(hd, vd, bs, k_pages, v_pages)) {
         const dim3 grid_items(n_items, nh);
@@ -2292,8 +2307,8 @@ FX_API int fx_attn_tiles(void* stream, int dtype, const void* q, long ldq, void*
         else if (vd != hd && hd <= 64) attn_mfma_tile_kernel<64, SH><<<grid, 64, 0, s>>>(a);
         else if (vd != hd) attn_mfma_tile_kernel<128, SH><<<grid, 64, 0, s>>>(a);
         else if (SH == SHAPE_NONE && tile_q == 128 && hd == 128 && !turns &&
-                 (g_rows32 == 2 || (g_rows32 && fx_attn_rows32((long)n_items * nh, fx_compute_units())))) {
-            if (g_groups ? g_groups == 2 : fx_attn_rows32((long)n_items * nh, fx_compute_units()) != 1) attn_mfma_rows32_kernel<2><<<grid_blocks, 512, 0, s>>>(a);
+                 (g_rows32 == 2 || (g_rows32 && rows32))) {
+            if (g_groups ? g_groups == 2 : rows32 != 1) attn_mfma_rows32_kernel<2><<<grid_blocks, 512, 0, s>>>(a);
             else attn_mfma_rows32_kernel<1><<<grid_blocks, 256, 0, s>>>(a);
         }
         else if (tile_q == 128 && hd == 128 && two_groups) attn_mfma_direct_kernel<128, 2, 8, 2, SH><<<grid_blocks, 1024, shm, s>>>(a);

@@ -155,6 +155,19 @@ def test_items_on_waves_of_32_queries():
     assert rule(95, 128) == 0 and rule(192, 128) == 2 and rule(385, 128) == 1
 
 
+def test_items_on_waves_of_32_queries_under_a_mask():
+    """Short spans stay on waves of 16; even work takes one group from a block a CU on."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda blocks, span, tokens, cus=256, chunked=0: load_library("attention").fx_attn_rows32_masked(blocks, cus, span, chunked, tokens)
+    for blocks, tokens in ((1, 128), (191, 1536), (192, 1536), (256, 2048), (336, 1536), (512, 4096), (896, 4096), (5000, 20000)):
+        assert rule(blocks, 1, tokens) == rule(blocks, 768, tokens) == rule(blocks, 1024, tokens, chunked=1) == 0
+    assert rule(191, 4096, 1536) == 0 and rule(192, 1024, 1536) == rule(256, 1024, 2048) == 0 and rule(256, 1025, 2048) == rule(256, 40000, 2048) == 2
+    assert rule(257, 769, 2112) == rule(511, 40000, 4096) == rule(512, 1024, 4096) == rule(512, 3072, 4096) == rule(640, 40000, 5120) == rule(769, 40000, 6000) == 1
+    assert rule(512, 3073, 4096) == rule(639, 40000, 5120) == 2 and rule(400, 2049, 4096, cus=128) == 1 and rule(256, 3073, 4096, cus=128) == 2
+    assert rule(256, 2048, 2048, chunked=1) == 0 and rule(256, 2049, 2048, chunked=1) == rule(336, 1536, 1536, chunked=1) == rule(512, 4096, 4096, chunked=1) == 2
+    assert rule(512, 1536, 4096, chunked=1) == rule(640, 8192, 4096, chunked=1) == rule(900, 8192, 4096, chunked=1) == 1
+
+
 def test_every_item_and_head_of_a_prompt_has_its_block():
     """Numbers of heads that eight XCDs share evenly and not, of items on both sides of eight: every pair once, last items first, an XCD's share of
     the work of a causal prompt within a row of its heads' mean."""

@@ -72,7 +72,7 @@ struct GemmArgs {
     long ld_gate;            //   (m % gate_div) * N + n
     int gate_div;
     int vec_ok;  // 16-byte loads are legal for A and W
-    int c_vec;   // 16-byte loads and stores of C are legal at columns that are a multiple of 16 bytes
+    int c_vec;   // float32: so are 16-byte loads and stores of C
     int n_col_tiles, n_row_tiles;  // tiled kernels: the grid they decode block ids with
     int tile_rows;  // LDS-tiled kernels, plain rows: rows a tile takes, up to its height
     int by_row_tile;  // LDS-tiled kernels, rows sorted by expert: every eighth row tile to an XCD
@@ -675,19 +675,45 @@ __device__ __forceinline__ int wide_column(int row) {
     return wn * 16 * NC + (PAIRED && j < (NC & ~1) ? (j >> 1) * 32 + (i >> 2) * 8 + (j & 1) * 4 + (i & 3) : j * 16 + i);
 }
 
-// N values to C[at .. at + N), as far as they are columns below `left`; vec: 16-byte accesses are legal where N values are whole.
+// N values to C[at .. at + N), as far as they are columns below `left`.  Whole runs are one store (float32: one a 16 bytes) wherever the row begins, for global accesses need no
+// more alignment than an element's here; rows of bfloat16 that begin between two words take three, words in the middle (one store there: 4,096 rows against 2,049 weight rows of 2,048 k
+// 51 us, three 44).  A store an element touched 64 places with two bytes each: 62 us there, 2,048 rows against 50,257 532 us, now 388.
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
 template <int N, typename T>
-__device__ __forceinline__ void store_columns(T* to, const float (&v)[N], int left, bool vec) {
-    if (vec && left >= N) {
+__device__ __forceinline__ void store_columns(T* to, const float (&v)[N], int left) {
+    if (left >= N) {
         if constexpr (sizeof(T) == 4) {
+            if constexpr (N % 4 == 0) {
 #pragma unroll
-            for (int r = 0; r < N; r += 4) *(f32x4_t*)(to + r) = (f32x4_t){v[r], v[r + 1], v[r + 2], v[r + 3]};
+                for (int r = 0; r < N; r += 4) *(f32x4_any_t*)(to + r) = (f32x4_t){v[r], v[r + 1], v[r + 2], v[r + 3]};
+            } else {
+                typedef __attribute__((ext_vector_type(N))) float run_t;
+                typedef run_t run_any_t __attribute__((aligned(4)));
+                run_t p;
+#pragma unroll
+                for (int r = 0; r < N; ++r) p[r] = v[r];
+                *(run_any_t*)to = p;
+            }
         } else {
             typedef __attribute__((ext_vector_type(N / 2))) uint32_t packed_t;
+            typedef packed_t packed_any_t __attribute__((aligned(2)));
             packed_t p;
 #pragma unroll
             for (int r = 0; r < N; r += 2) p[r / 2] = pack_bf16(v[r], v[r + 1]);
-            *(packed_t*)to = p;
+            if constexpr (N >= 4) {
+                if ((uintptr_t)to & 2) {
+                    typedef __attribute__((ext_vector_type(N / 2 - 1))) uint32_t inner_t;
+                    typedef inner_t inner_any_t __attribute__((aligned(4)));
+                    inner_t in;
+#pragma unroll
+                    for (int r = 0; r < N / 2 - 1; ++r) in[r] = __builtin_amdgcn_alignbit(p[r + 1], p[r], 16);
+                    to[0].bits = (uint16_t)p[0];
+                    *(inner_any_t*)(to + 1) = in;
+                    to[N - 1].bits = (uint16_t)(p[N / 2 - 1] >> 16);
+                    return;
+                }
+            }
+            *(packed_any_t*)to = p;
         }
         return;
     }
@@ -711,7 +737,6 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[
     wm = __builtin_amdgcn_readfirstlane(wm);
     wn = __builtin_amdgcn_readfirstlane(wn);
     const int last = min(r_end, r0 + TM), q = lane >> 4;
-    const bool vec = g.c_vec;
     // Where each of this lane's rows goes (and its scale) is fetched for all rows at once: a load inside the loops below
     // would be waited for before the next leaves.
     int m_of[MT];
@@ -755,7 +780,7 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[
                             y[r] = gated_c<decltype(ac)::value>(acc[i][2 * (b + r / 4)][r & 3] * ps, acc[i][2 * (b + r / 4) + 1][r & 3] * ps, g.act_limit, g.act_alpha);
                     }
                     const int n = column(u);
-                    if (first + (lane & 15) < last) store_columns<N>(to + n, y, g.N - n, vec);
+                    if (first + (lane & 15) < last) store_columns<N>(to + n, y, g.N - n);
                 });
             });
         });
@@ -780,10 +805,10 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[
             each_run([&](auto uc, auto cc, auto bc) {
                 constexpr int u = decltype(uc)::value, N = decltype(cc)::value, b = decltype(bc)::value;
                 const int n = column(u);
-                if (vec && n + N <= g.N) {
+                if (n + N <= g.N) {
 #pragma unroll
                     for (int r = 0; r < N; r += 4) {
-                        const f32x4_t v = *(const f32x4_t*)(from + n + r);
+                        const f32x4_t v = *(const f32x4_any_t*)(from + n + r);
 #pragma unroll
                         for (int t = 0; t < 4; ++t) old[i][4 * b + r + t] = v[t];
                     }
@@ -833,8 +858,8 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& g, f32x4_t (&acc)[
                     }
                 }
                 if (first + (lane & 15) < last) {
-                    if constexpr (EPI == EPI_STORE) store_columns<N>((bf16*)g.C + (size_t)m * g.ldc + n, y, g.N - n, vec);
-                    else store_columns<N>((float*)g.C + (size_t)m * g.ldc + n, y, g.N - n, vec);
+                    if constexpr (EPI == EPI_STORE) store_columns<N>((bf16*)g.C + (size_t)m * g.ldc + n, y, g.N - n);
+                    else store_columns<N>((float*)g.C + (size_t)m * g.ldc + n, y, g.N - n);
                 }
             });
         });
@@ -2494,7 +2519,6 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     g.vec_ok = norm_w != nullptr ||
                ((K % 8 == 0) && (lda % 8 == 0) && (w_stride % 8 == 0) && (up_offset % 8 == 0) &&
                 (((uintptr_t)A | (uintptr_t)W) % 16 == 0));
-    g.c_vec = ldc % (epi == EPI_STORE || epi == EPI_GATED ? 8 : 4) == 0 && ((uintptr_t)C % 16) == 0;
     const long per_group = expert_offsets ? (M + E - 1) / E : M;
     const bool wide_ok = g.vec_ok && K % 64 == 0 && !g_no_wide;
     FX_REQUIRE(!pair_ids || g.vec_ok, "gemm: unsorted pairs need K a multiple of 8 and 16-byte aligned rows");

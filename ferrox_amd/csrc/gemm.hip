@@ -1433,29 +1433,52 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         }
     };
     if constexpr (!ROPE) first_pieces();
-    // The outputs of a thread: element idx = tid + i * threads of the block's OUTS tiles of 16 rows x CW columns, so that a row's
-    // columns go out together and all waves work.  (dual: a tile of gates and one of ups make one of outputs)
+    // The outputs of a thread: runs of V columns of a row, run tid + i * threads of the block's OUTS tiles of 16 rows x CW columns, so that all waves work and none has more
+    // to keep, read and store than it must: where a block has one tile a thread has one element and a row's columns go out together, where it has four or more the run is what a lane
+    // of the accumulators holds (in elements, eight of them a thread, 64 rows against 5,632 weight rows of 2,048 k took 18.3 us, so 16.5; 32 rows added into 2,048
+    // columns 8.9, 8.2).  (dual: a tile of gates and one of ups make one of outputs)
     constexpr int SETS = DUAL ? NW / 2 : NW;      // column groups of a block
-    constexpr int OUTS = MT * SETS, THREADS = WAVES * 64, PER = 16 * CW, IT = (OUTS * PER + THREADS - 1) / THREADS;
+    constexpr int OUTS = MT * SETS, THREADS = WAVES * 64, PER = 16 * CW;
+    constexpr int V = OUTS * PER >= 4 * THREADS ? 4 : (OUTS * PER >= 2 * THREADS ? 2 : 1), RUNS = PER / V, IT = (OUTS * RUNS + THREADS - 1) / THREADS;
+    static_assert(V == 1 || CW == 16, "runs of several columns are of whole sets");
+    typedef __attribute__((ext_vector_type(V == 1 ? 2 : V))) float run_t;
+    typedef run_t run_any_t __attribute__((aligned(4)));
     int m_of[IT];                                 // row of C, or -1
-    float old[IT], scale_of[IT], gate[IT];
-    RawElement bias_of[IT];
-    auto tile_of = [&](int i) { return OUTS == 1 ? 0 : (tid + i * THREADS) / PER; };
-    auto row_in_tile = [&](int i) { return (tid + i * THREADS) / CW % 16; };
-    auto column_of = [&](int i) { return n0 + (tile_of(i) % SETS) * CW + tid % CW; };
+    float old[IT][V], scale_of[IT], gate[IT][V];
+    RawElement bias_of[IT][V];
+    auto tile_of = [&](int i) { return OUTS == 1 && V == 1 ? 0 : (tid + i * THREADS) / RUNS; };
+    auto row_in_tile = [&](int i) { return V == 1 ? (tid + i * THREADS) / CW % 16 : (tid + i * THREADS) % RUNS / (4 / V) % 16; };
+    auto column_in_tile = [&](int i) { return V == 1 ? tid % CW : (tid + i * THREADS) % RUNS / (RUNS / 4) * 4 + (V == 2 ? (tid & 1) * 2 : 0); };
+    auto column_of = [&](int i) { return n0 + (tile_of(i) % SETS) * CW + column_in_tile(i); };
     if constexpr (!ROPE) {
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
-            const int row = row_in_tile(i);
+            const int row = row_in_tile(i), first = column_of(i);
             const int ml = pairs ? __shfl(pair_c, row) : r0 + (tile_of(i) / SETS) * 16 + row;
-            const bool live = (pairs ? ml >= 0 : ml < r_end) && column_of(i) < g.N && (OUTS * PER % THREADS == 0 || tid + i * THREADS < OUTS * PER);
-            const int safe = live ? ml : (pairs ? 0 : r0), n = min(column_of(i), g.N - 1);
+            const bool live = (pairs ? ml >= 0 : ml < r_end) && first < g.N && (OUTS * RUNS % THREADS == 0 || tid + i * THREADS < OUTS * RUNS);
+            const int safe = live ? ml : (pairs ? 0 : r0);
             const int m = (g.c_rows && !pairs) ? g.c_rows[safe] : safe;
             m_of[i] = live ? m : -1;
             scale_of[i] = DUAL ? FX_PRE_SCALE(g, safe) : (EPI == EPI_RESID && g.row_scale ? g.row_scale[safe] : 1.f);
-            if constexpr (EPI == EPI_RESID) old[i] = ((const float*)g.C)[(size_t)m * g.ldc + n];
-            if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_F32) gate[i] = gate_of(g, m, n);
-            if (!DUAL && g.bias) bias_of[i] = fetch_element(g.bias, g.bias_dtype, n);
+            if constexpr (EPI == EPI_RESID) {
+                const float* from = (const float*)g.C + (size_t)m * g.ldc;
+                if (V > 1 && first + V <= g.N) {
+                    const run_t was = *(const run_any_t*)(from + first);
+#pragma unroll
+                    for (int r = 0; r < V; ++r) old[i][r] = was[r];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < V; ++r) old[i][r] = from[min(first + r, g.N - 1)];
+                }
+            }
+            if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_F32) {
+#pragma unroll
+                for (int r = 0; r < V; ++r) gate[i][r] = gate_of(g, m, min(first + r, g.N - 1));
+            }
+            if (!DUAL && g.bias) {
+#pragma unroll
+                for (int r = 0; r < V; ++r) bias_of[i][r] = fetch_element(g.bias, g.bias_dtype, min(first + r, g.N - 1));
+            }
         }
     }
     // rope epilogue: what thread (lane, wave) needs for its pairs of outputs, rows 16 mt + lane % 16, column
@@ -1638,24 +1661,35 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         return;
     }
     // parts in their order; lane 16 (column / 4) + row of an accumulator holds columns 4 (column / 4) ..
-    const float* sums = (const float*)red + (size_t)((tid % CW >> 2) * 16) * 4 + (tid & 3);
-    auto sum_of = [&](int acc_tile, int row) {
-        float v = 0.f;
+    auto sum_of = [&](int acc_tile, int row, int column, float (&v)[V]) {
+        const float* at = (const float*)red + ((size_t)acc_tile * 64 + (column >> 2) * 16 + row) * 4 + (column & 3);
 #pragma unroll
-        for (int w = 0; w < PARTS; ++w) v += sums[((size_t)(w * NACC + acc_tile) * 64 + row) * 4];
-        return v;
+        for (int r = 0; r < V; ++r) v[r] = 0.f;
+#pragma unroll
+        for (int w = 0; w < PARTS; ++w) {
+            if constexpr (V == 1) {
+                v[0] += at[(size_t)w * NACC * 256];
+            } else {
+                const run_t part = *(const run_t*)(at + (size_t)w * NACC * 256);
+#pragma unroll
+                for (int r = 0; r < V; ++r) v[r] += part[r];
+            }
+        }
     };
     auto finish = [&](auto kind) {
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
             const int m = m_of[i];
             if (m < 0) continue;
-            const int t = tile_of(i), mt = t / SETS, a = t % SETS, row = row_in_tile(i);
+            const int t = tile_of(i), mt = t / SETS, a = t % SETS, row = row_in_tile(i), column = column_in_tile(i);
             const int n = column_of(i);
-            float o = sum_of(mt * NW + (DUAL ? 2 * a : a), row);
+            float o[V];
+            sum_of(mt * NW + (DUAL ? 2 * a : a), row, column, o);
             if constexpr (DUAL) {
-                const float up = sum_of(mt * NW + 2 * a + 1, row);
-                from_float((bf16*)g.C + (size_t)m * g.ldc + n, gated_c<decltype(kind)::value>(o * scale_of[i], up * scale_of[i], g.act_limit, g.act_alpha));
+                float up[V];
+                sum_of(mt * NW + 2 * a + 1, row, column, up);
+#pragma unroll
+                for (int r = 0; r < V; ++r) o[r] = gated_c<decltype(kind)::value>(o[r] * scale_of[i], up[r] * scale_of[i], g.act_limit, g.act_alpha);
             } else {
                 float rstd = 1.f;
                 if (!NORM && g.row_ss) rstd = row_rstd(sum_in_order(g.row_ss + (size_t)m * g.row_ss_n, g.row_ss_n), g.K, g.norm_eps);
@@ -1667,21 +1701,26 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
                         for (int q = 0; q < 4; ++q) total += red_ss[w][mt][row + 16 * q];
                     rstd = row_rstd(total, g.K, g.norm_eps);
                 }
-                o *= rstd;
-                asm volatile("" : "+v"(o));          // the product is rounded before the bias is added (no fused multiply-add)
-                if (g.bias) o += element_as_float(bias_of[i]);
-                if constexpr (EPI == EPI_STORE) {
-                    from_float((bf16*)g.C + (size_t)m * g.ldc + n, stored_c<decltype(kind)::value>(g, o, gate[i]));
-                } else if constexpr (EPI == EPI_STORE_F32) {
-                    ((float*)g.C)[(size_t)m * g.ldc + n] = stored_c<decltype(kind)::value>(g, o, gate[i]);
-                } else {
-                    if (g.row_scale) {
-                        o *= scale_of[i];
-                        asm volatile("" : "+v"(o));
+#pragma unroll
+                for (int r = 0; r < V; ++r) {
+                    o[r] *= rstd;
+                    asm volatile("" : "+v"(o[r]));          // the product is rounded before the bias is added (no fused multiply-add)
+                    if (g.bias) o[r] += element_as_float(bias_of[i][r]);
+                    if constexpr (EPI == EPI_RESID) {
+                        if (g.row_scale) {
+                            o[r] *= scale_of[i];
+                            asm volatile("" : "+v"(o[r]));
+                        }
+                        o[r] = old[i][r] + o[r];
+                    } else {
+                        o[r] = stored_c<decltype(kind)::value>(g, o[r], gate[i][r]);
                     }
-                    ((float*)g.C)[(size_t)m * g.ldc + n] = old[i] + o;
                 }
             }
+            typedef std::conditional_t<EPI == EPI_STORE || EPI == EPI_GATED, bf16, float> out_t;
+            out_t* to = (out_t*)g.C + (size_t)m * g.ldc + n;
+            if constexpr (V == 1) from_float(to, o[0]);
+            else store_columns<V>(to, o, g.N - n);
         }
     };
     if constexpr (DUAL) with_activation(g.act, finish);

@@ -114,6 +114,36 @@ def test_half_sets_of_weight_rows_have_the_bits_of_whole_sets(dtype, N, K):
         close(whole[0], h0.double() + (a.double() @ w.double().T) * scale.double()[:, None], dtype, "residual")
 
 
+@pytest.mark.parametrize("N,K", [(33, 128), (46, 520), (71, 640), (128, 256)])
+@pytest.mark.parametrize("waves", [1, 2, 4, 8])
+def test_few_rows_store_runs_of_one_two_and_four_columns(waves, N, K):
+    """What a thread finishes of a block's outputs depends on the row tiles, sets and waves of a block: runs that begin and end anywhere, rows and columns past the end, outputs in
+    whole rows and in a view that begins and steps at odd places; near float64 whatever the block, the bits of one wave count, and nothing written beside."""
+    from ferrox_amd import debug, ops
+    for M in (1, 15, 17, 33, 50, 64):
+        a, w, w2 = (rnd(r, K, dtype=torch.bfloat16, seed=s, scale=0.3) for r, s in ((M, 0), (N, 1), (2 * N, 2)))
+        bias, scale, logits, h0 = rnd(N, seed=3), rnd(M, seed=4), rnd(M, N, seed=5), rnd(M, N, seed=6)
+        ref, ref2 = a.double() @ w.double().T, a.double() @ w2.double().T
+        cases = [(dict(bias=bias), w, ref + bias.double(), torch.bfloat16), (dict(epilogue=ops.EPI_STORE_F32, out_gate=(logits, 1)), w, ref * torch.sigmoid(logits.double()), torch.float32),
+                 (dict(epilogue=ops.EPI_RESID, row_scale=scale, bias=bias), w, h0.double() + (ref + bias.double()) * scale.double()[:, None], torch.float32),
+                 (dict(epilogue=ops.EPI_GATED), w2, plain.silu(ref2[:, :N]) * ref2[:, N:], torch.bfloat16)]
+        got = {}
+        for tiles in (1, 2) if waves == 8 else (1, 2, 4):          # (four tiles of two sets take four waves, whose sums are of other parts)
+            for sets in (1, 2):
+                with debug.kernel_switch("gemm", "skinny_row_tiles", tiles), debug.kernel_switch("gemm", "skinny_sets", sets), \
+                        debug.kernel_switch("gemm", "skinny_waves", waves), debug.kernel_switch("gemm", "skinny_half", 0), debug.kernel_switch("gemm", "plain_rows", 64):
+                    for i, (kw, weights, want, dtype) in enumerate(cases):
+                        odd = torch.full((M, N + 5), 7.0, device=DEV, dtype=dtype)
+                        whole = torch.full((M, -(-N // 8) * 8), 7.0, device=DEV, dtype=dtype)
+                        for out in (whole[:, :N], odd[:, 3:3 + N]):
+                            if kw.get("epilogue") == ops.EPI_RESID:
+                                out.copy_(h0)
+                            ops.gemm(a, weights, out=out, **kw)
+                            close(out, want, torch.bfloat16, f"{M} rows, {tiles} tiles, {sets} sets, case {i}")
+                        assert torch.equal(whole[:, :N], odd[:, 3:3 + N]) and torch.equal(whole[:, :N], got.setdefault(i, whole)[:, :N]), (M, tiles, sets, i)
+                        assert bool((whole[:, N:] == 7).all()) and bool((odd[:, :3] == 7).all()) and bool((odd[:, 3 + N:] == 7).all()), (M, tiles, sets, i)
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 48, 49, 64, 65, 81])
 def test_float32_tiles_leave_out_row_blocks_that_they_do_not_have(rows):
     """Tiles of 64 and of 32 rows with one to four blocks of 16 rows, steps of K odd and even in number and a partial one: the bits of the product

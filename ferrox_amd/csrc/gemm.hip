@@ -2362,7 +2362,12 @@ FX_API int fx_gemm_row_tile_blocks(int M, int N, int cus) {
 //   2,048 x 2,048 5.3 4.4, 5.8 5.0, 6.3 5.7     2,048 x 5,632 10.4 7.9, 10.8 8.8, 12.6 10.4     1,024 x 2,048 5.0 3.8, 5.5 4.5, 6.0 5.3
 //   gate/up of 1,408 x 2,048 6.8 5.1, 7.4 5.8, 7.9 6.5, of 5,632 12.4 11.2, 13.6 12.0, 14.3 14.0     6,144 x 2,048 7.9 7.0, 8.1 8.7, 8.6 10.3
 //   the other way 2,560 x 2,048 5.3 5.3, 5.8 6.5, 6.3 8.0     3,584 x 3,584 7.7 8.0, 8.3 10.2, 9.4 12.9     4,096 x 1,024 3.9 4.1, 4.4 4.6, 4.5 5.7
+// That holds where blocks of half sets are one round of the CUs.  Beyond, more blocks pay each block's start and end more often, and the rule is only taken where it was measured ahead: up
+// to 24 columns a CU with two matrices, up to 40 for one or two rows of one, sums of 2,048 and more in both (`fx_gemm`: a wave's part is four pieces or more then).  Elsewhere, at 1 and 4 rows:
+//   4,608 x 1,024 4.5 4.8, 4.8 5.3     5,632 x 5,632 16.9 16.6, 15.2 17.0     12,288 x 3,584 19.0 20.2, 20.1 21.1     20,480 x 1,024 10.1 12.2, 9.8 13.5     50,257 x 2,048 35.0 39.6, 35.7 44.5
+//   gate/up of 4,608 x 1,024 6.6 7.5, 7.0 8.0, of 9,216 x 1,024 8.6 10.8, 9.2 11.5, x 5,632 40.4 39.1, 41.8 42.1, of 18,432 x 2,048 26.0 27.5, 25.7 28.0
 FX_API int fx_gemm_half_sets(int M, int N, int dual, int sets, int cus) {
+    if (ceil_div(N, 8) > cus && (dual ? N > 24 * cus : M > 2 || N > 40 * cus)) return 0;
     auto cost = [&](int columns, int weight_rows) { return ceil_div(ceil_div(N, columns), cus) * (2L * weight_rows + M); };
     return M <= 16 && (dual ? cost(8, 16) < cost(8 * sets, 16 * sets) : cost(8, 8) < cost(16 * sets, 16 * sets));
 }
@@ -2629,7 +2634,8 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         if (expert_offsets && mt == 1) waves = 2;      // sorted, up to 16 rows per expert: 152 against 159 us at 64 tokens
         if (g_skinny_waves == 8 || g_skinny_waves == 4 || g_skinny_waves == 2 || g_skinny_waves == 1) waves = g_skinny_waves;
         const bool half = g_skinny_half >= 0 ? g_skinny_half && M <= 16 && !expert_offsets && !pair_ids && !norm_w && waves == 4 && mt == 1
-                                             : !expert_offsets && !pair_ids && !norm_w && waves == 4 && mt == 1 && fx_gemm_half_sets(M, N, dual, nw, fx_compute_units());
+                                             : !expert_offsets && !pair_ids && !norm_w && waves == 4 && mt == 1 && (K >= 2048 || ceil_div(N, 8) <= fx_compute_units()) &&
+                                                   fx_gemm_half_sets(M, N, dual, nw, fx_compute_units());
         launch_skinny(g, epi, mt, nw, waves, half, m_tiles, s);
         FX_CHECK_LAUNCH("gemm_bf16_skinny");
         return 0;

@@ -95,6 +95,18 @@ def test_half_sets_of_weight_rows_where_the_busiest_cu_fetches_less():
     assert rule(1, 6144) and not rule(8, 6144) and not rule(16, 6144) and not rule(17, 2048)
 
 
+def test_half_sets_beyond_one_round_of_the_cus_only_where_they_were_ahead():
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, n, dual=0, cus=256: bool(load_library("gemm").fx_gemm_half_sets(m, n, dual, 2 if dual or -(-n // 32) >= 160 else 1, cus))
+    for m in (1, 2):
+        assert rule(m, 6144) and rule(m, 9216) and not any(rule(m, n) for n in (12288, 18432, 20480, 50257, 151936))
+    for m in (3, 5, 16):
+        assert not any(rule(m, n) for n in (4608, 5632, 9216, 12288, 50257)) and rule(m, 2048)
+    for m in (1, 4, 16):
+        assert rule(m, 4608, 1) and rule(m, 6144, 1) and not any(rule(m, n, 1) for n in (9216, 18432, 50257))
+    assert rule(1, 5120, cus=128) and not rule(1, 6144, cus=128) and not rule(1, 6144, 1, cus=128)
+
+
 def test_a_block_per_row_tile_while_such_blocks_are_one_a_cu():
     """The product of 33 to 128 plain rows: beyond 64 rows a second round of blocks is behind two row tiles a block."""
     from ferrox_amd.csrc.build import load_library

@@ -1245,9 +1245,10 @@ FX_API int fx_cast(void* stream, int src_dtype, const void* src, int dst_dtype, 
 // VEC = 4: a thread takes four neighbouring columns with 16-byte loads (H % 4 == 0, aligned rows); a block then
 // covers 1024 columns, and each of its waves one group of 256 for the sums of squares.
 // KB terms and SB slabs are asked for together and added in order: the sums are those of a plain loop.  What depends on nothing is asked for in front of
-// the terms, whose places must arrive first (one after the other these were up to five waits for memory: 8 tokens of 2,048 with four slabs 2.7 -> 2.4 us), and
-// no more of either than most launches have (512 tokens, four terms and one slab 5.4 -> 4.0; many tokens are bound by the memory's rate: 4,096 of 3,584, eight
-// terms and one slab, 128 us for 0.6 GB either way).
+// the terms, whose places must arrive first (one after the other these were up to five waits for memory: 8 tokens of 2,048 with four slabs 2.7 -> 2.4 us), but for the
+// slabs of many tokens (VEC = 4), whose registers cost waves that are needed then (asked for first / so: 512 tokens of 2,048, ten terms and six slabs 13.6 / 12.4, 1,000 wide with
+// six and eight 6.0 / 5.5); and no more of either than most launches have (512 tokens, four terms and one slab 5.3 -> 3.7; many more are bound by the memory's rate: 4,096 of 3,584,
+// eight terms and one slab, 131 us for 0.6 GB either way).  Whether there are places is asked once: a branch a term cost 0.1 to 0.3 us.
 template <typename T, int VEC, int KB, int SB>
 __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                           const int* __restrict__ inv, const float* __restrict__ w,
@@ -1275,8 +1276,12 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ h,
 #pragma unroll
             for (int u = 0; u < KB; ++u) {
                 const int j = min(j0 + u, k - 1);
-                from[u] = inv ? inv[t * k + j] : t * k + j;
+                from[u] = t * k + j;
                 wv[u] = w[t * k + j];
+            }
+            if (inv) {
+#pragma unroll
+                for (int u = 0; u < KB; ++u) from[u] = inv[from[u]];
             }
         };
         auto fetch_slabs = [&](int s0) {
@@ -1291,7 +1296,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ h,
 #pragma unroll
             for (int i = 0; i < VEC; ++i) raw[i] = fetch_element(norm_w, norm_dtype, c + i);
         }
-        if (shared) fetch_slabs(0);
+        if (VEC == 1 && shared) fetch_slabs(0);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
         for (int j0 = 0; j0 < k; j0 += KB) {
@@ -1314,7 +1319,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ h,
 #pragma unroll
             for (int i = 0; i < VEC; ++i) sh[i] = 0.f;
             for (int s0 = 0; s0 < slabs; s0 += SB) {
-                if (s0) fetch_slabs(s0);
+                if (VEC == 4 || s0) fetch_slabs(s0);
 #pragma unroll
                 for (int u = 0; u < SB; ++u)
                     if (s0 + u < slabs) {

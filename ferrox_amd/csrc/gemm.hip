@@ -1254,13 +1254,14 @@ __device__ __forceinline__ void load8f(const float* p, bool ok, float* v) {
 // down product 36.6 -> 32.7 us, the head 132 -> 101 us (4.7 -> 6.2 TB/s).
 // NW: sets of 16 weight rows per wave; in dual mode set a is the gate (a even) or up (a odd) rows of
 // column group a / 2.
-template <int MT, int WAVES, int NW, bool DUAL, int EPI, bool NORM = false, bool ROPE = false, bool HALF = false, int DEPTH = 2>
+template <int MT, int WAVES, int NW, bool DUAL, int EPI, bool NORM = false, bool ROPE = false, bool HALF = false, int DEPTH = 2, bool WEIGHTS_FIRST = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g) {
     static_assert(!HALF || (MT == 1 && WAVES == 4 && !NORM && !ROPE), "sets of eight weight rows are for few plain rows");
     constexpr int CW = HALF ? 8 : 16;               // weight rows of a set, output columns of a tile
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
     static_assert(!ROPE || (NW == 2 && !DUAL && !NORM && EPI == EPI_STORE), "the rope epilogue pairs two sets of columns");
     static_assert(!NORM || (!DUAL && EPI == EPI_STORE), "the fused norm feeds a plain product");
+    static_assert(!WEIGHTS_FIRST || ROPE, "only the rope epilogue's operands have an order to choose");
     __shared__ float red_ss[NORM ? WAVES : 1][MT][64];
     float ss[MT];
 #pragma unroll
@@ -1507,23 +1508,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         const int p = rope_rotated ? 16 * rope_j + cc : 0;
         const float freq = g.rope_inv_freq[p];
         const float freq_div = g.rope_freq_factors ? g.rope_freq_factors[p] : 1.f;
-        float squares[MT][8];      // (of the first eight parts; summed where they are needed)
-        if (g.row_ss) {
+        if constexpr (WEIGHTS_FIRST) {      // (sums of squares of one batch: asked for in front of the first weights, summed behind them)
+            float squares[MT][8];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int u = 0; u < 8; ++u) squares[mt][u] = g.row_ss[(size_t)row_of[mt] * g.row_ss_n + min(u, g.row_ss_n - 1)];
-        }
-        first_pieces();      // (behind the short loads and in front of what waits for them)
+            first_pieces();
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            total[mt] = 0.f;
-            if (g.row_ss && g.row_ss_n <= 8) {
+            for (int mt = 0; mt < MT; ++mt) {
+                total[mt] = 0.f;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) total[mt] = u < g.row_ss_n ? total[mt] + squares[mt][u] : total[mt];
-            } else if (g.row_ss) {
-                total[mt] = sum_in_order(g.row_ss + (size_t)row_of[mt] * g.row_ss_n, g.row_ss_n);
             }
+        } else {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                total[mt] = g.row_ss ? sum_in_order(g.row_ss + (size_t)row_of[mt] * g.row_ss_n, g.row_ss_n) : 0.f;
         }
         rope_b0 = element_as_float(e0);
         rope_b1 = element_as_float(e1);
@@ -1547,6 +1548,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
                 sincosf(angle, &rope_sn[mt], &rope_cs[mt]);
             }
         }
+        // (what the epilogue needs first: behind the weights those short loads would wait for them)
+        if constexpr (!WEIGHTS_FIRST) first_pieces();
     }
     // Few accumulators leave registers for two pieces: the loads of the next piece are then issued before the
     // products of this one, so a wave always has a piece on its way from memory.  Each product follows the
@@ -2302,6 +2305,11 @@ static void launch_skinny(const GemmArgs& g, int epi, int mt, int nw, int waves,
 #undef FX_SK
 }
 
+// Whether the first weights of the rotating product leave before the sums of squares of its rows have arrived.  What else its epilogue needs then waits for the weights, so it pays
+// with sums of one batch and rows enough (us, weights behind / first; 2,048 k and 6,144 columns, 8 rows 9.9 9.4, 13 10.7 10.3, 16 11.1 10.6; 1,024 k, 16 rows 6.9 6.5; but without sums 16
+// rows 10.4 10.7, 2 rows of 1,024 k 6.3 6.8; sums of two batches, 3,584 k, 2 rows 12.0 12.7, 17 rows 16.8 18.0; two row tiles of 2,048 k with sums 13.1 13.5).
+FX_API int fx_qkv_rope_weights_first(int M, int K, int sums) { return M <= 16 && sums >= 1 && sums <= 8 && (long)M * K >= 16384; }
+
 // The q/k/v product of up to 64 tokens with the rotation and the cache write in its epilogue (see GemmArgs):
 // bfloat16, C [M, (nh + 2 nkv) hd], bias [N] or null, row_ss as in fx_gemm.  head_dim and the rotary dimension
 // are multiples of 32.  k_pages [pages][nkv][bs][hd] and v_pages [pages][nkv][hd][bs], or both null.
@@ -2331,7 +2339,9 @@ FX_API int fx_qkv_rope(void* stream, const void* A, long lda, const void* W, lon
     g.rope_inv_freq = inv_freq ? inv_freq : (const float*)positions;      // (rot == 0: read, never used)
     g.rope_freq_factors = freq_factors;
     dim3 grid((nh + 2 * nkv) * (hd / 32), 1);
-    if (M <= 16) gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
+    if (row_ss && fx_qkv_rope_weights_first(M, K, row_ss_n))
+        gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true, false, 2, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
+    else if (M <= 16) gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
     else if (M <= 32) gemm_bf16_skinny_kernel<2, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
     else {
         // 33..64 rows: two blocks of 32 rows a column group rather than one of 64 (a wave fetches the operands of

@@ -885,6 +885,14 @@ def test_qkv_product_that_rotates_and_writes_the_cache(later, T, H, nh, nkv, hd,
     assert not ops.can_qkv_rope(x, w, 65, hd, rot, False) and not ops.can_qkv_rope(x, w, T, hd, rot, True)
 
 
+@pytest.mark.parametrize("T,H", [(16, 1032), (13, 1384), (9, 2000), (16, 2048)])
+def test_rotating_product_whose_weights_leave_before_the_sums(T, H):
+    """Sums of one batch and rows enough for it, K with and without a last part of a piece: the bits of the product and the rotation."""
+    from ferrox_amd.csrc.build import load_library
+    assert load_library("gemm").fx_qkv_rope_weights_first(T, H, -(-H // 256))
+    test_qkv_product_that_rotates_and_writes_the_cache(True, T, H, 6, 2, 64, 16, 32, True)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nh,nkv,hd,bs,rot,interleaved", [(3, 1, 32, 8, 32, False), (2, 2, 64, 16, 32, False),
                                                           (2, 1, 48, 8, 24, True), (4, 2, 128, 64, 128, False)])

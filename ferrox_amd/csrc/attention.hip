@@ -1730,12 +1730,11 @@ __global__ __launch_bounds__(W * G * 64, HD > 128 ? W / 4 : HD == 64 && G == 1 ?
         if (any_edge) {
             if (kt0 < kv_end && !span.holds_tile(kt0)) {
                 if constexpr (W == 8 && G == 1 && HD <= 128) {
-                    // (two such blocks on a CU fill LDS with their reads: stores alone, a key at a time.  16 heads of 128 over 4 with biases, 4,096 tokens 145 us with pairs read and
+                    // (two such blocks on a CU fill LDS with their reads: stores alone, of one key in all rows that a thread takes.  16 heads of 128 over 4 with biases, 4,096 tokens 145 us with pairs read and
                     // written, 134 so; capped, 4,096 175 and 168, 8,000 450 and 438; two groups on a CU 46 and 49 for 1,337, one block of heads of 256 31.8 and 32.9 for 700)
-                    for (int idx = tid; idx < vd * 64; idx += W * 64) {
-                        const int d = idx >> 6, key = idx & 63;
-                        if (!span.has(kt0 + key)) st[64 * HD + d * 64 + (((key >> 3) ^ turn_of(d)) * 8) + (key & 7)].bits = 0;
-                    }
+                    const int key = tid & 63;                  // the same in all rows that this thread takes
+                    if (!span.has(kt0 + key))
+                        for (int d = tid >> 6; d < vd; d += W) st[64 * HD + d * 64 + (((key >> 3) ^ turn_of(d)) * 8) + (key & 7)].bits = 0;
                 } else {
                     uint32_t* v = (uint32_t*)(st + 64 * HD);
                     const int pair = tid & 31;                 // of keys, the same in all rows that this thread takes

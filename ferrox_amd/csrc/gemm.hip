@@ -1434,13 +1434,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         }
     };
     if constexpr (!ROPE) first_pieces();
-    // The outputs of a thread: runs of V columns of a row, run tid + i * threads of the block's OUTS tiles of 16 rows x CW columns, so that all waves work and none has more
-    // to keep, read and store than it must: where a block has one tile a thread has one element and a row's columns go out together, where it has four or more the run is what a lane
-    // of the accumulators holds (in elements, eight of them a thread, 64 rows against 5,632 weight rows of 2,048 k took 18.3 us, so 16.5; 32 rows added into 2,048
-    // columns 8.9, 8.2).  (dual: a tile of gates and one of ups make one of outputs)
+    // The outputs of a thread: runs of V columns of a row, run tid + i * threads of the block's OUTS tiles of 16 rows x CW columns, so that all waves work.  Single elements, whose
+    // rows' columns go out together, but where a thread adds to what is there, or has several row tiles of plain outputs, for what it keeps of each through the loop: as many then as
+    // leave every wave its share, up to the four that a lane of the accumulators holds.  us, elements / runs: 32 rows added into 2,048 columns 8.9 / 8.2, 64 rows against 5,632
+    // weight rows of 2,048 k 18.3 / 17.5, against 2,560 with a bias 13.5 / 12.6; the other way an expert's down product of one token 7.1 / 7.5, of 8 tokens 21.6 / 22.8, gate/up of
+    // 1,408 and 64 rows 16.3 / 17.3.  (dual: a tile of gates and one of ups make one of outputs)
     constexpr int SETS = DUAL ? NW / 2 : NW;      // column groups of a block
-    constexpr int OUTS = MT * SETS, THREADS = WAVES * 64, PER = 16 * CW;
-    constexpr int V = OUTS * PER >= 4 * THREADS ? 4 : (OUTS * PER >= 2 * THREADS ? 2 : 1), RUNS = PER / V, IT = (OUTS * RUNS + THREADS - 1) / THREADS;
+    constexpr int OUTS = MT * SETS, THREADS = WAVES * 64, PER = 16 * CW, SHARE = OUTS * PER / THREADS;
+    constexpr int V = EPI != EPI_RESID && (DUAL || MT == 1) ? 1 : (SHARE >= 4 ? 4 : (SHARE >= 2 ? 2 : 1)), RUNS = PER / V, IT = (OUTS * RUNS + THREADS - 1) / THREADS;
     static_assert(V == 1 || CW == 16, "runs of several columns are of whole sets");
     typedef __attribute__((ext_vector_type(V == 1 ? 2 : V))) float run_t;
     typedef run_t run_any_t __attribute__((aligned(4)));
@@ -1449,8 +1450,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
     RawElement bias_of[IT][V];
     auto tile_of = [&](int i) { return OUTS == 1 && V == 1 ? 0 : (tid + i * THREADS) / RUNS; };
     auto row_in_tile = [&](int i) { return V == 1 ? (tid + i * THREADS) / CW % 16 : (tid + i * THREADS) % RUNS / (4 / V) % 16; };
-    auto column_in_tile = [&](int i) { return V == 1 ? tid % CW : (tid + i * THREADS) % RUNS / (RUNS / 4) * 4 + (V == 2 ? (tid & 1) * 2 : 0); };
-    auto column_of = [&](int i) { return n0 + (tile_of(i) % SETS) * CW + column_in_tile(i); };
+    static_assert(V == 1 || THREADS % RUNS == 0, "the runs of a thread begin at one column");
+    const int column_in_tile = V == 1 ? tid % CW : tid % RUNS / (RUNS / 4) * 4 + (V == 2 ? (tid & 1) * 2 : 0);
+    auto column_of = [&](int i) { return n0 + (tile_of(i) % SETS) * CW + column_in_tile; };
     if constexpr (!ROPE) {
 #pragma unroll
         for (int i = 0; i < IT; ++i) {
@@ -1664,16 +1666,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         return;
     }
     // parts in their order; lane 16 (column / 4) + row of an accumulator holds columns 4 (column / 4) ..
-    auto sum_of = [&](int acc_tile, int row, int column, float (&v)[V]) {
-        const float* at = (const float*)red + ((size_t)acc_tile * 64 + (column >> 2) * 16 + row) * 4 + (column & 3);
+    const float* sums = (const float*)red + (size_t)((column_in_tile >> 2) * 16) * 4 + (column_in_tile & 3);
+    auto sum_of = [&](int acc_tile, int row, float (&v)[V]) {
 #pragma unroll
         for (int r = 0; r < V; ++r) v[r] = 0.f;
 #pragma unroll
         for (int w = 0; w < PARTS; ++w) {
             if constexpr (V == 1) {
-                v[0] += at[(size_t)w * NACC * 256];
+                v[0] += sums[((size_t)(w * NACC + acc_tile) * 64 + row) * 4];
             } else {
-                const run_t part = *(const run_t*)(at + (size_t)w * NACC * 256);
+                const run_t part = *(const run_t*)(sums + ((size_t)(w * NACC + acc_tile) * 64 + row) * 4);
 #pragma unroll
                 for (int r = 0; r < V; ++r) v[r] += part[r];
             }
@@ -1684,13 +1686,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
         for (int i = 0; i < IT; ++i) {
             const int m = m_of[i];
             if (m < 0) continue;
-            const int t = tile_of(i), mt = t / SETS, a = t % SETS, row = row_in_tile(i), column = column_in_tile(i);
+            const int t = tile_of(i), mt = t / SETS, a = t % SETS, row = row_in_tile(i);
             const int n = column_of(i);
             float o[V];
-            sum_of(mt * NW + (DUAL ? 2 * a : a), row, column, o);
+            sum_of(mt * NW + (DUAL ? 2 * a : a), row, o);
             if constexpr (DUAL) {
                 float up[V];
-                sum_of(mt * NW + 2 * a + 1, row, column, up);
+                sum_of(mt * NW + 2 * a + 1, row, up);
 #pragma unroll
                 for (int r = 0; r < V; ++r) o[r] = gated_c<decltype(kind)::value>(o[r] * scale_of[i], up[r] * scale_of[i], g.act_limit, g.act_alpha);
             } else {

@@ -2308,9 +2308,10 @@ static void launch_skinny(const GemmArgs& g, int epi, int mt, int nw, int waves,
 }
 
 // Whether the first weights of the rotating product leave before the sums of squares of its rows have arrived.  What else its epilogue needs then waits for the weights, so it pays
-// with sums of one batch and rows enough (us, weights behind / first; 2,048 k and 6,144 columns, 8 rows 9.9 9.4, 13 10.7 10.3, 16 11.1 10.6; 1,024 k, 16 rows 6.9 6.5; but without sums 16
-// rows 10.4 10.7, 2 rows of 1,024 k 6.3 6.8; sums of two batches, 3,584 k, 2 rows 12.0 12.7, 17 rows 16.8 18.0; two row tiles of 2,048 k with sums 13.1 13.5).
-FX_API int fx_qkv_rope_weights_first(int M, int K, int sums) { return M <= 16 && sums >= 1 && sums <= 8 && (long)M * K >= 16384; }
+// with sums of one batch and k enough, or rows (us, weights behind / first; 2,048 k and 6,144 columns, 1 row 9.1 8.7, 8 9.9 9.3, 16 11.2 10.4; 1,024 k, 16 rows 6.9 6.4; in a step of one
+// sequence, where the kernel before has just written the sums, 24 layers take 1,781 us with the weights behind, so 1,763; but without sums 16 rows 10.4 10.7, 2 rows of 1,024 k 6.5
+// 6.7; sums of two batches, 3,584 k, 2 rows 12.0 12.7, 17 rows 16.8 18.0; two row tiles of 2,048 k with sums 13.1 13.5).
+FX_API int fx_qkv_rope_weights_first(int M, int K, int sums) { return M <= 16 && sums >= 1 && sums <= 8 && (K > 1024 || (long)M * K >= 16384); }
 
 // The q/k/v product of up to 64 tokens with the rotation and the cache write in its epilogue (see GemmArgs):
 // bfloat16, C [M, (nh + 2 nkv) hd], bias [N] or null, row_ss as in fx_gemm.  head_dim and the rotary dimension

@@ -107,10 +107,10 @@ def test_half_sets_beyond_one_round_of_the_cus_only_where_they_were_ahead():
     assert rule(1, 5120, cus=128) and not rule(1, 6144, cus=128) and not rule(1, 6144, 1, cus=128)
 
 
-def test_weights_of_the_rotating_product_leave_first_with_sums_of_one_batch_and_rows_enough():
+def test_weights_of_the_rotating_product_leave_first_with_sums_of_one_batch_and_k_or_rows_enough():
     from ferrox_amd.csrc.build import load_library
     rule = lambda m, k, sums=None: bool(load_library("gemm").fx_qkv_rope_weights_first(m, k, -(-k // 256) if sums is None else sums))
-    assert rule(8, 2048) and rule(16, 2048) and rule(16, 1024) and not rule(17, 2048) and not rule(7, 2048) and not rule(15, 1024)
+    assert rule(1, 2048) and rule(16, 2048) and rule(1, 1032) and rule(16, 1024) and not rule(17, 2048) and not rule(15, 1024) and not rule(16, 768)
     assert not rule(16, 2048, 0) and not rule(16, 2056) and not rule(16, 3584) and rule(16, 3584, 8)
 
 

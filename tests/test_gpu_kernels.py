@@ -885,7 +885,7 @@ def test_qkv_product_that_rotates_and_writes_the_cache(later, T, H, nh, nkv, hd,
     assert not ops.can_qkv_rope(x, w, 65, hd, rot, False) and not ops.can_qkv_rope(x, w, T, hd, rot, True)
 
 
-@pytest.mark.parametrize("T,H", [(16, 1032), (13, 1384), (9, 2000), (16, 2048)])
+@pytest.mark.parametrize("T,H", [(16, 1032), (13, 1384), (9, 2000), (16, 2048), (1, 1032), (3, 2000), (16, 1024)])
 def test_rotating_product_whose_weights_leave_before_the_sums(T, H):
     """Sums of one batch and rows enough for it, K with and without a last part of a piece: the bits of the product and the rotation."""
     from ferrox_amd.csrc.build import load_library

@@ -3,7 +3,8 @@
 // for plain and for expert-grouped rows.
 //
 //  * bfloat16: MFMA 16x16x32 tiles, float32 accumulators.
-//  * float32 : MFMA 16x16x4 in float32 (no reduced-precision matrix mode).
+//  * float32 : MFMA 16x16x4 in float32, or every operand as the sum of three bfloat16
+//    numbers on the bfloat16 instruction, with no larger error (see `f32_split8`).
 //
 // In both, one output element's products are added in an order that the sizes of the
 // weights fix, whatever the tile shape and whatever else is in the batch, so a float32
@@ -1772,6 +1773,93 @@ __device__ __forceinline__ f32x4_t f32_fetch_guarded(const float* row, int k, in
     }
     return v;
 }
+// ---------------------------------------------------------------------------
+// float32 products as bfloat16 ones
+// ---------------------------------------------------------------------------
+// A float32 is the sum of three bfloat16 numbers h + m + l, each the rest of the ones before it rounded to nearest (8 + 8 + 8 bits and two signs hold
+// its 24 bits), and a product of two such sums has six terms down to 2^-18 of it: hh, hm, mh, mm, hl, lh; what is left out, ml, lm and ll, is
+// 2^-26 of the product or less and of either sign (6e-9 of a sum's norm, where rounding a float32 product takes 3e-8).  The matrix instruction adds 32 bfloat16 products in 16 cycles where the float32 one adds
+// four in 32, so six terms take 96 cycles instead of 256.
+// The instruction cuts a sum off below instead of rounding it, so a step's 32 k start from zero, small terms first, and are added to the sums so far with an add that rounds; and every second step works
+// out the negative and subtracts it, so that what is cut off has either sign: else outputs are low by 5e-8 of their size, which the mean over a thousand keys brings out (decoded logits at 1,030 keys: 1.3e-6
+// off 64 bits instead of 0.8e-6).  Error against 64 bits, float32 instruction / taken apart: 2,048 k 2.9e-7 / 7.5e-8, 5,632 k 4.8e-7 / 7.3e-8, terms of one sign 8.9e-8 / 4.5e-8.
+// Parts of K (F32_PARTS, of whole pairs of steps) are added in their order, in the kernel for few rows and in tiles alike: a row's bits do not depend on which of them computes it.
+// Four columns of a row that hold an infinity, a NaN or a sum beyond float32 are worked out again on the float32 instruction: an infinity has no rest.
+__host__ __device__ __forceinline__ int f32_split_part_length(int K) { return ((K + F32_PARTS - 1) / F32_PARTS + 63) / 64 * 64; }
+typedef __attribute__((ext_vector_type(8))) __bf16 f32_part8_t;
+typedef __attribute__((ext_vector_type(2))) __bf16 f32_part2_t;
+struct F32Split {
+    f32_part8_t h, m, l;
+};
+// (a, b) as packed bfloat16, and what is left of both, which is exact.  A dot product with (-1, 0) or (0, -1) takes the place of moving a half into place and
+// subtracting it; the two constants pass through an empty statement, in the form of inline constants the instruction reads them otherwise.  (700 x 2,048 x 5,632 160 -> 143 us.)
+template <bool NEG>
+__device__ __forceinline__ uint32_t f32_peel(float& a, float& b) {
+    const uint32_t p = pack_bf16(NEG ? -a : a, NEG ? -b : b);
+    uint32_t first = NEG ? 0x00003f80u : 0x0000bf80u, second = first << 16;
+    asm("" : "+v"(first), "+v"(second));
+    a = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(f32_part2_t, p), __builtin_bit_cast(f32_part2_t, first), a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(f32_part2_t, p), __builtin_bit_cast(f32_part2_t, second), b, false);
+    return p;
+}
+template <bool NEG>      // NEG: of -v
+__device__ __forceinline__ void f32_split4(f32x4_t v, uint2& h, uint2& m, uint2& l) {
+    float a = v[0], b = v[1], c = v[2], d = v[3];
+    h.x = f32_peel<NEG>(a, b); h.y = f32_peel<NEG>(c, d);
+    m.x = f32_peel<NEG>(a, b); m.y = f32_peel<NEG>(c, d);
+    l.x = NEG ? pack_bf16(-a, -b) : pack_bf16(a, b); l.y = NEG ? pack_bf16(-c, -d) : pack_bf16(c, d);
+}
+template <bool NEG>
+__device__ __forceinline__ F32Split f32_split8(f32x4_t lo, f32x4_t hi) {
+    uint2 h0, m0, l0, h1, m1, l1;
+    f32_split4<NEG>(lo, h0, m0, l0);
+    f32_split4<NEG>(hi, h1, m1, l1);
+    F32Split s;
+    s.h = __builtin_bit_cast(f32_part8_t, make_uint4(h0.x, h0.y, h1.x, h1.y));
+    s.m = __builtin_bit_cast(f32_part8_t, make_uint4(m0.x, m0.y, m1.x, m1.y));
+    s.l = __builtin_bit_cast(f32_part8_t, make_uint4(l0.x, l0.y, l1.x, l1.y));
+    return s;
+}
+// 32 k of a tile: the small terms first
+#define FX_MFMA32(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
+template <bool NEG, int MT, int NT>
+__device__ __forceinline__ void f32_split_multiply(f32x4_t (&acc)[MT][NT], const F32Split (&w)[NT], const F32Split (&x)[MT]) {
+    f32x4_t t[MT][NT];
+#define FX_TERM(W, X, C)                       \
+    _Pragma("unroll") for (int i = 0; i < MT; ++i) \
+        _Pragma("unroll") for (int j = 0; j < NT; ++j) t[i][j] = FX_MFMA32(w[j].W, x[i].X, C)
+    FX_TERM(l, h, ((f32x4_t){0.f, 0.f, 0.f, 0.f}));
+    FX_TERM(h, l, t[i][j]);
+    FX_TERM(m, m, t[i][j]);
+    FX_TERM(m, h, t[i][j]);
+    FX_TERM(h, m, t[i][j]);
+    FX_TERM(h, h, t[i][j]);
+#undef FX_TERM
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = NEG ? acc[i][j] - t[i][j] : acc[i][j] + t[i][j];
+}
+// one tile's sums on the float32 instruction, K a multiple of 32, rows from memory
+template <bool VEC>
+__device__ __forceinline__ f32x4_t f32_whole_sum(int K, const float* w_row, const float* x_row, int gq) {
+    const int part = f32_part_length(K);
+    f32x4_t acc[1][1] = {{(f32x4_t){0.f, 0.f, 0.f, 0.f}}}, total = acc[0][0];
+    for (int k = 0, end = part; k < K; k += 16) {
+        if (k == end) {
+            total += acc[0][0];
+            acc[0][0] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            end += part;
+        }
+        const f32x4_t w[1] = {f32_fetch<VEC>(w_row + k + gq * 4)}, x[1] = {f32_fetch<VEC>(x_row + k + gq * 4)};
+        f32_multiply(acc, w, x);
+    }
+    return total + acc[0][0];
+}
+__device__ __forceinline__ bool f32_all_finite(f32x4_t v) {
+    return fabsf(v[0]) < INFINITY && fabsf(v[1]) < INFINITY && fabsf(v[2]) < INFINITY && fabsf(v[3]) < INFINITY;
+}
+
 // What columns n .. n + 3 of logical row ml need on their way out besides the product: a kernel whose last wait is for its operands
 // asks for it in front of them.
 template <int EPI>
@@ -1987,6 +2075,213 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(GemmArgs g) {
     }
 }
 
+// Many rows, taken apart: up to TM rows x 64 NT columns a block (DUAL: 32 NT of both matrices, in each wave's blocks in turn or, ROLES, one matrix to a pair of waves), four waves that
+// take 16 NT weight rows each and all the rows.  A weight row goes from memory into its wave's registers and is taken apart there, once; the rows are taken apart on their way into LDS, whose
+// planes every wave reads in 16-byte pieces (swizzled by pairs of rows); two steps of 32 k between barriers, the loads of the next DEPTH such stages on their way.  LINES: the weights in whole
+// lines with the non-temporal hint, where they are read about once.
+// Bound by issue: of a step of 32 k of 64 x 128 outputs a wave issues 48 products of 16 cycles (23 at the clock that random values leave) and some 180 vector instructions, 84 of
+// them the splitting, 32 the sums, and of these a SIMD hides up to four behind a product.  us, float32 instruction / taken apart: 700 x 6,144 x 2,048 190 / 130, 700 x 2,048 x 5,632
+// 181 / 132, gate/up of 5,632 x 2,048 for 700 rows 287 / 196; both products of 700 tokens on 60 experts of 1,408, even shares 416 + 208 / 346 + 169, crowded 432 + 223 / 354 + 187;
+// 1,500 x 6,144 x 2,048 321 / 230 (164 TFLOP/s; the instruction itself 153).  With a barrier a step of 32 k the tiles of few blocks took a third longer (64 x 2,048 x 2,048
+// in 32 x 64 36 -> 25); the next step's splitting between this step's products 155 instead of 149 (700 x 6,144); tiles of 64 x 256 and 128 x 128 leave one wave a SIMD (214, 161).
+template <int TM, int NT, int DEPTH, bool DUAL, int EPI, bool VEC, bool LINES>
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(GemmArgs g) {
+    constexpr bool ROLES = DUAL && NT == 1;           // waves 0 and 1 take gate's rows and store, 2 and 3 up's
+    constexpr int MB = TM / 16, AR = TM / 32, PER = DUAL && !ROLES ? 2 : 1;
+    __shared__ uint2 Xs[2][2][3][TM][8];        // two steps of 32 k to a stage, two stages
+    int r0, r_end, expert;
+    if (g.expert_offsets) {
+        locate_rows<TM>(g, blockIdx.y, r0, r_end, expert);
+    } else {
+        r0 = blockIdx.y * g.tile_rows;
+        r_end = min(r0 + g.tile_rows, g.M);
+        expert = 0;
+    }
+    if (r0 < 0) return;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
+    const int n0 = ROLES ? blockIdx.x * 32 + (wave & 1) * 16 : (blockIdx.x * 4 + wave) * (16 * NT / PER);
+    const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
+    const int piece = tid & 7, x_row = tid >> 3;
+    const float* a_src[AR];
+    const float* b_src[NT][LINES ? 2 : 1];      // LINES: of row li % 8, and of row li % 8 + 8
+    auto a_row = [&](int i) {
+        const int m = min(r0 + i, r_end - 1);
+        return (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda;
+    };
+    auto b_row = [&](int t, int m, int row) {
+        return Wbase + (size_t)min(n0 + t * 16 + row, g.N - 1) * g.K + (m ? g.up_offset : 0);
+    };
+#pragma unroll
+    for (int i = 0; i < AR; ++i) a_src[i] = a_row(x_row + 32 * i) + piece * 4;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int h = 0; h < (LINES ? 2 : 1); ++h)
+            b_src[j][h] = b_row(j / PER, ROLES ? wave >> 1 : DUAL ? j & 1 : 0, LINES ? (li & 7) + 8 * h : li) + (LINES ? (li >> 3) * 16 : 0) + gq * 4;
+    f32x4_t rx[2 * DEPTH][AR], rw[2 * DEPTH][NT][2];
+    const int n_steps = g.K / 32;
+    auto fetch_x = [&](auto some, int set, int step) {
+        const int k = min(step, n_steps - 1) * 32;
+#pragma unroll
+        for (int i = 0; i < decltype(some)::value; ++i) rx[set][i] = f32_fetch<VEC>(a_src[i] + k);
+    };
+    auto fetch_w = [&](int set, int step) {
+        const int k = min(step, n_steps - 1) * 32;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            if constexpr (LINES) {
+                rw[set][j][0] = __builtin_bit_cast(f32x4_t, load_lines16(b_src[j][0] + k));
+                rw[set][j][1] = __builtin_bit_cast(f32x4_t, load_lines16(b_src[j][1] + k));
+            } else {
+                rw[set][j][0] = f32_fetch<VEC>(b_src[j][0] + k);
+                rw[set][j][1] = f32_fetch<VEC>(b_src[j][0] + k + 16);
+            }
+        }
+    };
+    // k = 4 p .. 4 p + 3 of a row are the half p >> 2 of what a lane of group p & 3 takes; 16-byte pieces swizzled by pairs of rows
+    const int x_at = ((piece & 3) ^ ((x_row >> 1) & 3)) * 2 + (piece >> 2);
+    auto keep = [&](auto some, auto setc, int buf) {          // (the operands of odd steps with the other sign)
+        constexpr int set = decltype(setc)::value;
+#pragma unroll
+        for (int i = 0; i < decltype(some)::value; ++i) {
+            uint2 h, m, l;
+            f32_split4<(set & 1) == 1>(rx[set][i], h, m, l);
+            Xs[buf][set & 1][0][x_row + 32 * i][x_at] = h;
+            Xs[buf][set & 1][1][x_row + 32 * i][x_at] = m;
+            Xs[buf][set & 1][2][x_row + 32 * i][x_at] = l;
+        }
+    };
+    f32x4_t acc[MB][NT], total[MB][NT];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = total[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int part = f32_split_part_length(g.K) / 32;
+    int next_end = part;
+    const int at16 = (gq ^ ((li >> 1) & 3)) * 2;
+    auto multiply = [&](auto blocks, auto setc, int buf, int step) {
+        constexpr int NA = decltype(blocks)::value, set = decltype(setc)::value;
+        constexpr bool NEG = (set & 1) == 1;
+        if (!NEG && step == next_end) {         // (a part is an even number of steps)
+            next_end += part;
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    total[i][j] += acc[i][j];
+                    acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        F32Split w[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            if constexpr (LINES) {
+                const uint4 one = __builtin_bit_cast(uint4, rw[set][j][0]), two = __builtin_bit_cast(uint4, rw[set][j][1]);
+                w[j] = f32_split8<false>(__builtin_bit_cast(f32x4_t, swap_halves<0xC>(one, two)), __builtin_bit_cast(f32x4_t, swap_halves<0x3>(two, one)));
+            } else {
+                w[j] = f32_split8<false>(rw[set][j][0], rw[set][j][1]);
+            }
+        }
+        fetch_w(set, step + 2 * DEPTH);
+        auto operand = [&](int i) {
+            F32Split x;
+            x.h = *(const f32_part8_t*)&Xs[buf][set & 1][0][i * 16 + li][at16];
+            x.m = *(const f32_part8_t*)&Xs[buf][set & 1][1][i * 16 + li][at16];
+            x.l = *(const f32_part8_t*)&Xs[buf][set & 1][2][i * 16 + li][at16];
+            return x;
+        };
+#pragma unroll
+        for (int i = 0; i + 1 < NA; i += 2) {
+            const F32Split x[2] = {operand(i), operand(i + 1)};
+            f32_split_multiply<NEG, 2, NT>(*(f32x4_t(*)[2][NT])&acc[i], w, x);
+        }
+        if constexpr (NA % 2) {
+            const F32Split x[1] = {operand(NA - 1)};
+            f32_split_multiply<NEG, 1, NT>(*(f32x4_t(*)[1][NT])&acc[NA - 1], w, x);
+        }
+    };
+    auto loop = [&](auto blocks) {
+        const fx_int<(decltype(blocks)::value + 1) / 2> some;
+#pragma unroll
+        for (int d = 0; d < 2 * DEPTH; ++d) fetch_x(some, d, d), fetch_w(d, d);
+        keep(some, fx_int<0>{}, 0);
+        keep(some, fx_int<1>{}, 0);
+        fetch_x(some, 0, 2 * DEPTH);
+        fetch_x(some, 1, 2 * DEPTH + 1);
+        int buf = 0;
+        auto two = [&](auto setc, int step, auto odd_too) {
+            constexpr int set = decltype(setc)::value, next = (set + 2) % (2 * DEPTH);
+            lds_barrier();
+            multiply(blocks, setc, buf, step);
+            if constexpr (decltype(odd_too)::value) {
+                multiply(blocks, fx_int<set + 1>{}, buf, step + 1);
+                buf ^= 1;
+                keep(some, fx_int<next>{}, buf);
+                keep(some, fx_int<next + 1>{}, buf);
+                fetch_x(some, next, step + 2 + 2 * DEPTH);
+                fetch_x(some, next + 1, step + 3 + 2 * DEPTH);
+            }
+        };
+        int step = 0;
+        for (; step + 2 * DEPTH <= n_steps; step += 2 * DEPTH)
+            static_for(std::make_integer_sequence<int, DEPTH>{}, [&](auto u) { two(fx_int<2 * decltype(u)::value>{}, step + 2 * decltype(u)::value, fx_int<1>{}); });
+        if (DEPTH == 2 && step + 2 <= n_steps) {
+            two(fx_int<0>{}, step, fx_int<1>{});
+            if (n_steps & 1) two(fx_int<2 * (DEPTH - 1)>{}, step + 2, fx_int<0>{});
+        } else if (n_steps & 1) {
+            two(fx_int<0>{}, step, fx_int<0>{});
+        }
+    };
+    const int n_blocks = (min(TM, r_end - r0) + 15) >> 4;
+    if constexpr (MB == 8) {
+        if (n_blocks <= 2) loop(fx_int<2>{});
+        else if (n_blocks <= 4) loop(fx_int<4>{});
+        else if (n_blocks <= 6) loop(fx_int<6>{});
+        else loop(fx_int<8>{});
+    } else {
+        if (n_blocks == 1) loop(fx_int<1>{});
+        else if (MB == 2 || n_blocks == 2) loop(fx_int<2>{});
+        else if constexpr (MB > 2) {
+            if (n_blocks == 3) loop(fx_int<3>{});
+            else loop(fx_int<4>{});
+        }
+    }
+    f32x4_t(*other)[64] = (f32x4_t(*)[64]) & Xs[0][0][0][0][0];       // ROLES: up's sums, MB blocks of each of two waves
+    if constexpr (ROLES) {
+        __syncthreads();
+        if (wave >= 2) {
+#pragma unroll
+            for (int i = 0; i < MB; ++i) other[(wave & 1) * MB + i][lane] = total[i][0] + acc[i][0];
+        }
+        __syncthreads();
+        if (wave >= 2) return;
+    }
+    unsigned odd = 0;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        const int ml = r0 + i * 16 + li;
+        if (ml >= r_end) continue;
+#pragma unroll
+        for (int j = 0; j < NT; j += PER) {
+            const int n = n0 + j / PER * 16 + 4 * gq;
+            const f32x4_t v = total[i][j] + acc[i][j], v2 = ROLES ? other[wave * MB + i][lane] : DUAL ? total[i][j + PER - 1] + acc[i][j + PER - 1] : v;
+            if (!(f32_all_finite(v) && f32_all_finite(v2))) odd |= 1u << (i * (NT / PER) + j / PER);
+            else f32_store4<DUAL, EPI>(g, f32_ask<DUAL, EPI>(g, ml, min(n, g.N - 1)), n, v, v2);
+        }
+    }
+    if (__ballot(odd != 0) == 0) return;
+#pragma unroll 1
+    for (int i = 0; i < n_blocks; ++i)
+#pragma unroll 1
+        for (int t = 0; t < NT / PER; ++t) {
+            if (__ballot(odd >> (i * (NT / PER) + t) & 1) == 0) continue;
+            const float* x = a_row(i * 16 + li);
+            const f32x4_t v = f32_whole_sum<VEC>(g.K, b_row(t, 0, li), x, gq), v2 = DUAL ? f32_whole_sum<VEC>(g.K, b_row(t, 1, li), x, gq) : v;
+            const int n = n0 + t * 16 + 4 * gq;
+            if (odd >> (i * (NT / PER) + t) & 1) f32_store4<DUAL, EPI>(g, f32_ask<DUAL, EPI>(g, r0 + i * 16 + li, min(n, g.N - 1)), n, v, v2);
+        }
+}
+
 // Few rows: the weights go from memory straight into operands, every wave a part of K, 16 * MT rows and NW sets of 16
 // weight rows a block (DUAL: the sets alternate between the two matrices); 32 k a step, the next step's loads issued
 // before this step's products; the parts' sums meet in LDS.  LINES (rows of whole 32 k): the weights come in whole lines of 128 bytes
@@ -1994,7 +2289,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(GemmArgs g) {
 // against 6,144 x 2,048 15.5 us, gate/up of 5,632 24.3, 15 experts' gate/up 63 (5.5 TB/s), the head of 151,936 235 (5.3 TB/s).  With half
 // lines and steps of 64 k these took 17.6, 30.0, 75 and 275: twice the registers a step leave half the waves, and it
 // is waves, not deeper loads, that keep memory busy (steps of 128 k: 19.9, 33.3, 95 and 329).
-template <int MT, int NW, bool DUAL, int EPI, bool VEC, bool LINES, bool HALF = false>
+template <int MT, int NW, bool DUAL, int EPI, bool VEC, bool LINES, bool HALF = false, bool SPLIT = false>
 __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
     static_assert(!HALF || (LINES && MT == 1), "sets of eight weight rows come in whole lines, for few rows");
@@ -2025,7 +2320,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
             w_src[a][half] = Wbase + (size_t)n * g.K + (DUAL && (a & 1) ? g.up_offset : 0) + (LINES ? (li >> 3) * 16 + gq * 4 : 0);
         }
     }
-    const int part = f32_part_length(g.K);
+    const int part = SPLIT ? f32_split_part_length(g.K) : f32_part_length(g.K);
     const int k_first = wave * part, k_end = k_first + part < g.K ? k_first + part : g.K;
     constexpr int STEP = 2;       // groups of 16 k that are on their way together
     f32x4_t w[2][STEP][NW], x[2][STEP][MT];
@@ -2067,27 +2362,43 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
             for (int b = 0; b < 2; ++b) {
                 const int kb = k0 + b * STEP * 16;
                 fetch(b ^ 1, kb + STEP * 16);
+                // what the lane multiplies of weight set a in group c of 16 k
+                auto own = [&](int c, int a) -> f32x4_t {
+                    if constexpr (!LINES) return w[b][c][a];
+                    const uint4 keep = __builtin_bit_cast(uint4, w[b][HALF ? c & ~1 : c][a]), other = __builtin_bit_cast(uint4, w[b][HALF ? c & ~1 : c ^ 1][a]);
+                    // (HALF: rows 8 .. 15 of the operand are the other k of rows 0 .. 7, and what they give is dropped)
+                    if constexpr (HALF) return __builtin_bit_cast(f32x4_t, c & 1 ? swap_halves<0x3>(keep, other) : keep);
+                    else return __builtin_bit_cast(f32x4_t, c & 1 ? swap_halves<0x3>(keep, other) : swap_halves<0xC>(keep, other));
+                };
+                if constexpr (SPLIT) {
+                    if (kb < k_full) {          // (whole steps of 32 k)
+                        F32Split ws[NW], xs[MT];
+#pragma unroll
+                        for (int a = 0; a < NW; ++a) ws[a] = f32_split8<false>(own(0, a), own(1, a));
+                        if (b & 1) {
+#pragma unroll
+                            for (int i = 0; i < MT; ++i) xs[i] = f32_split8<true>(x[b][0][i], x[b][1][i]);
+                            f32_split_multiply<true>(acc, ws, xs);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < MT; ++i) xs[i] = f32_split8<false>(x[b][0][i], x[b][1][i]);
+                            f32_split_multiply<false>(acc, ws, xs);
+                        }
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int c = 0; c < STEP; ++c)
                     if (kb + c * 16 < k_full) {
-                        if constexpr (LINES) {
-                            f32x4_t own[NW];
+                        f32x4_t ws[NW];
 #pragma unroll
-                            for (int a = 0; a < NW; ++a) {
-                                const uint4 keep = __builtin_bit_cast(uint4, w[b][HALF ? c & ~1 : c][a]), other = __builtin_bit_cast(uint4, w[b][HALF ? c & ~1 : c ^ 1][a]);
-                                // (HALF: rows 8 .. 15 of the operand are the other k of rows 0 .. 7, and what they give is dropped)
-                                if constexpr (HALF) own[a] = __builtin_bit_cast(f32x4_t, c & 1 ? swap_halves<0x3>(keep, other) : keep);
-                                else own[a] = __builtin_bit_cast(f32x4_t, c & 1 ? swap_halves<0x3>(keep, other) : swap_halves<0xC>(keep, other));
-                            }
-                            f32_multiply(acc, own, x[b][c]);
-                        } else {
-                            f32_multiply(acc, w[b][c], x[b][c]);
-                        }
+                        for (int a = 0; a < NW; ++a) ws[a] = own(c, a);
+                        f32_multiply(acc, ws, x[b][c]);
                     }
             }
         }
     }
-    if (!LINES && k_first < k_end && k_full < k_end) {       // the last, partial group of K
+    if (!LINES && !SPLIT && k_first < k_end && k_full < k_end) {       // the last, partial group of K
 #pragma unroll
         for (int a = 0; a < NW; ++a) w[0][0][a] = f32_fetch_guarded<VEC>(w_src[a][0], k_full + gq * 4, k_end);
 #pragma unroll
@@ -2099,7 +2410,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
 #pragma unroll
         for (int a = 0; a < NW; ++a) red[wave][i * NW + a][lane] = acc[i][a];
     __syncthreads();
-    if (!finishes) return;
+    if (SPLIT ? wave >= MT * NW / PER : !finishes) return;
     f32x4_t v = red[0][ti * NW + ta][lane], v2 = v;
 #pragma unroll
     for (int p = 1; p < F32_PARTS; ++p) v += red[p][ti * NW + ta][lane];
@@ -2107,6 +2418,16 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
         v2 = red[0][ti * NW + ta + PER - 1][lane];
 #pragma unroll
         for (int p = 1; p < F32_PARTS; ++p) v2 += red[p][ti * NW + ta + PER - 1][lane];
+    }
+    if constexpr (SPLIT) {
+        const bool odd = finishes && !(f32_all_finite(v) && f32_all_finite(v2));
+        if (__ballot(odd)) {            // (the whole wave: the products take all its lanes)
+            const int m = min(r0 + ti * 16 + li, r_end - 1), n = min(n0 + (DUAL ? ta >> 1 : ta) * CW + (HALF ? li & 7 : li), g.N - 1);
+            const float *x_row = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda, *w_row = Wbase + (size_t)n * g.K;
+            const f32x4_t whole = f32_whole_sum<VEC>(g.K, w_row, x_row, gq), whole2 = DUAL ? f32_whole_sum<VEC>(g.K, w_row + g.up_offset, x_row, gq) : whole;
+            if (odd) v = whole, v2 = whole2;
+        }
+        if (!finishes) return;
     }
     f32_store4<DUAL, EPI>(g, ask, out_col, v, v2);
 }
@@ -2144,7 +2465,8 @@ static int g_tile64_rows = 20; // "tile64_rows": experts with up to this many ro
 static int g_no_wide = 0;      // "wide": 0 sends many-row products to the register-staged tiled kernel, 1 (default) by the sizes,
 static int g_plain_rows = 0;   // "plain_rows": plain rows up to this many go to the product for few rows whatever the weight rows (0: by the sizes)
 static int g_stream_w = -1;    // "stream_w": 1 / 0 forces the non-temporal hint on the tiled kernel's weight loads on / off; -1: by the shape
-static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 to tiles of that size (0: by the sizes)
+static int g_f32_split = -1;   // "f32_split": 1 / 0 works float32 products of whole 32 k out as bfloat16 ones or on the float32 instruction (-1: by the weights' size)
+static int g_f32_tile = 0;     // "f32_tile": 1 sends float32 products to the kernel for few rows, 32 or 64 (taken apart also 48, 128, 144 and 160, see fx_gemm_f32_split_tile) to those tiles (0: by the sizes)
 static int g_wide_grouped = 0; // "wide_grouped": as "wide", for products whose rows are sorted by expert only
 static int g_wide_force = 0;   //         256, 192, 128, 64, 12 or 4 (tiles of 64 rows), 464, 4128 (64 x 64, 64 x 128), 8128 (128 x 128 in two stages), 8256 (128 x 256), 6128 or 6256 (96 rows), 1256 (sorted rows: 128 x 256 by the shares) or 1128 (128 x 128 in a ring) picks that tile of the LDS-tiled kernel
 FX_API int fx_debug_set(const char* key, int value) {
@@ -2159,8 +2481,9 @@ FX_API int fx_debug_set(const char* key, int value) {
     if (!strcmp(key, "wide_grouped")) { g_wide_grouped = value > 1 ? value : 0; return 0; }
     if (!strcmp(key, "stream_w")) { g_stream_w = value; return 0; }
     if (!strcmp(key, "f32_tile")) { g_f32_tile = value; return 0; }
+    if (!strcmp(key, "f32_split")) { g_f32_split = value; return 0; }
     if (!strcmp(key, "plain_rows")) { g_plain_rows = value; return 0; }
-    FX_REQUIRE(false, "gemm: no debug switch '%s' (skinny_sets, skinny_row_tiles, skinny_waves, skinny_half, few_rows, head_rows, tile64_rows, wide, wide_grouped, stream_w, plain_rows, f32_tile)", key);
+    FX_REQUIRE(false, "gemm: no debug switch '%s' (skinny_sets, skinny_row_tiles, skinny_waves, skinny_half, few_rows, head_rows, tile64_rows, wide, wide_grouped, stream_w, plain_rows, f32_tile, f32_split)", key);
     return 1;
 }
 
@@ -2218,24 +2541,35 @@ static void launch_ring(const GemmArgs& g, int epi, int m_tiles, hipStream_t s) 
     if (g.stream_w) launch_wide<TMB, TN, NS, NSA, true>(g, epi, m_tiles, s);
     else launch_wide<TMB, TN, NS, NSA, false>(g, epi, m_tiles, s);
 }
-template <bool DUAL, int EPI, bool VEC, bool LINES>
+template <bool DUAL, int EPI, bool VEC, bool LINES, bool SPLIT>
 static void launch_f32_skinny(const GemmArgs& g, int mt, int nw, bool half, dim3 grid, hipStream_t s) {
     if constexpr (LINES) {
         if (half) {
-            gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC, LINES, true><<<grid, 512, 0, s>>>(g);
+            gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC, LINES, true, SPLIT><<<grid, 512, 0, s>>>(g);
             return;
         }
     }
-    if (mt == 2) gemm_f32_skinny_kernel<2, 2, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
-    else if (nw == 2 || DUAL) gemm_f32_skinny_kernel<1, 2, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
-    else gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC, LINES><<<grid, 512, 0, s>>>(g);
+    if (mt == 2) gemm_f32_skinny_kernel<2, 2, DUAL, EPI, VEC, LINES, false, SPLIT><<<grid, 512, 0, s>>>(g);
+    else if (nw == 2 || DUAL) gemm_f32_skinny_kernel<1, 2, DUAL, EPI, VEC, LINES, false, SPLIT><<<grid, 512, 0, s>>>(g);
+    else gemm_f32_skinny_kernel<1, DUAL ? 2 : 1, DUAL, EPI, VEC, LINES, false, SPLIT><<<grid, 512, 0, s>>>(g);
 }
 template <bool DUAL, int EPI, bool VEC>
-static void launch_f32(const GemmArgs& g, int tile, int mt, int nw, bool half, dim3 grid, hipStream_t s) {
-    if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
+static void launch_f32(const GemmArgs& g, bool split, int tile, int stream, int mt, int nw, bool half, dim3 grid, hipStream_t s) {
+    if (tile && split) {
+        if (tile >= 128) gemm_f32_split_kernel<64, 2, 1, DUAL, EPI, VEC, false><<<grid, 256, 0, s>>>(g);
+        else if (tile == 32) {
+            if (VEC && stream) gemm_f32_split_kernel<32, 1, 2, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
+            else gemm_f32_split_kernel<32, 1, 2, DUAL, EPI, VEC, false><<<grid, 256, 0, s>>>(g);
+        } else if (VEC && stream == 2) gemm_f32_split_kernel<64, 1, 2, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
+        else if (VEC && stream) gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
+        else gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, VEC, false><<<grid, 256, 0, s>>>(g);
+    } else if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
     else if (tile == 32) gemm_f32_tiled_kernel<32, DUAL ? 64 : 32, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
-    else if (VEC && g.K % 32 == 0) launch_f32_skinny<DUAL, EPI, VEC, VEC>(g, mt, nw, half, grid, s);
-    else launch_f32_skinny<DUAL, EPI, VEC, false>(g, mt, nw, false, grid, s);
+    else if (VEC && g.K % 32 == 0) {
+        if (split) launch_f32_skinny<DUAL, EPI, VEC, VEC, true>(g, mt, nw, half, grid, s);
+        else launch_f32_skinny<DUAL, EPI, VEC, VEC, false>(g, mt, nw, half, grid, s);
+    } else if (split) launch_f32_skinny<DUAL, EPI, VEC, false, true>(g, mt, nw, false, grid, s);
+    else launch_f32_skinny<DUAL, EPI, VEC, false, false>(g, mt, nw, false, grid, s);
 }
 
 template <int MT, int WAVES, int NW, bool HALF = false, int DEPTH = 2>
@@ -2383,6 +2717,28 @@ FX_API int fx_gemm_half_sets(int M, int N, int dual, int sets, int cus) {
     if (ceil_div(N, 8) > cus && (dual ? N > 24 * cus : M > 2 || N > 40 * cus)) return 0;
     auto cost = [&](int columns, int weight_rows) { return ceil_div(ceil_div(N, columns), cus) * (2L * weight_rows + M); };
     return M <= 16 && (dual ? cost(8, 16) < cost(8 * sets, 16 * sets) : cost(8, 8) < cost(16 * sets, 16 * sets));
+}
+
+// Whether a float32 product is worked out from operands taken apart into bfloat16 ones (gemm_f32_split_kernel, and in the kernel for few rows): by the weights alone, so that the bits of a row
+// do not depend on the rows beside it.  Whole steps of 32 k; sums of 1,024 and more, where the error is a third of the float32 instruction's (it is level around 256); and weights of a million numbers, below which the
+// products are a few microseconds either way and some have their sums repeated elsewhere in the float32 order (`f32_ordered_dot`).
+FX_API int fx_gemm_f32_split(int N, int K) { return K % 32 == 0 && K >= 1024 && (long)N * K >= 1L << 20; }
+
+// The tile of such a product of plain rows, more than a few: its rows (32, 48 or 64) by 64 columns, or, as 128, 144 and 160, 64, 48 or 32 rows by 128
+// columns (dual: half as many of both matrices).  The time goes with how many blocks the busiest CU gets: us of a first block, of each further one and beside them, of 2,048 k
+// (1 to 6 blocks; up to 32 rows 32 x 64, one reading of the weights: 32 x 64 25 40 60 76 93 115; 48 x 64 34 50 70 88 104 131; 64 x 64 42 57 85 113 131 172; 32 x 128 49 70 107 137; 48 x 128 51 83 127 154 205 248; 64 x 128 59 92 141 184 229); other k in proportion.
+FX_API int fx_gemm_f32_split_tile(int M, int N, int dual, int cus) {
+    static const struct { int code, rows, columns; float first, each, beside; } kinds[] = {
+        {32, 32, 64, 25, 18.5f, 4}, {48, 48, 64, 34, 20.5f, 8}, {64, 64, 64, 42, 28.3f, 0}, {160, 32, 128, 49, 33, 5}, {144, 48, 128, 51, 41, 3}, {128, 64, 128, 59, 46, 2}};
+    if (M <= 32) return 32;
+    int best = 128;
+    float least = INFINITY;
+    for (const auto& k : kinds) {
+        const int blocks = ceil_div((long)ceil_div(N, dual ? k.columns / 2 : k.columns) * ceil_div(M, k.rows), cus);
+        const float us = blocks == 1 ? k.first : k.each * blocks + k.beside;
+        if (us < least) least = us, best = k.code;
+    }
+    return best;
 }
 
 // The tile of the LDS-tiled kernel for plain rows, as the debug switch "wide" names them; all give the same bits.  `dual`: N
@@ -2544,25 +2900,42 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // x 5,632 18.5 -> 16.1, gate/up of 1,408 12.8 -> 9.1, a router of 61 8.2 -> 6.2; of 6,144 x 2,048, 768 of them, 15.9 -> 17.1).
         // Where it cannot take whole lines it stays behind tiles of 32 with sorted rows, and from three rows on with the head's.
         const bool lines = g.vec_ok && K % 32 == 0;
+        const bool split = g_f32_split >= 0 ? g_f32_split && K % 32 == 0 : fx_gemm_f32_split(N, K);
         int tile = 0, mt = 1, nw = 2;
         if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
-        else if (expert_offsets) tile = lines && group <= 2 ? 0 : (group <= 36 ? 32 : 64);
+        else if (expert_offsets) tile = lines && group <= 2 ? 0 : (group <= 36 && !split ? 32 : 64);
         else {
             const bool many_columns = ceil_div(N, 32) >= 8 * cus && M > (lines ? 8 : 2);
-            if (M > 32 || many_columns) tile = M > 32 && 2 * (long)ceil_div(N, 64) * ceil_div(M, 64) >= 5 * cus ? 64 : 32;
+            if (M > 32 || many_columns) tile = split ? fx_gemm_f32_split_tile(M, N, dual, (int)cus) : M > 32 && 2 * (long)ceil_div(N, 64) * ceil_div(M, 64) >= 5 * cus ? 64 : 32;
+        }
+        // Sorted rows taken apart, 64 rows a tile: up to 24 an expert 64 columns (of one matrix, or 32 of both) a block and whole lines with the non-temporal hint, up to 12 with the weights
+        // two stages ahead, beyond 128 columns (both products, float32 instruction / those three ways; tokens of 60 experts of 1,408: 45 373 / 374 349 407, 150 402 / 382 381 430, 300
+        // 432 / 411 418 441, crowded 414 / 387 403 390, 450 crowded 507 / 470 476 431, 700 624 / 519 549 514, crowded 655 / 612 622 541).
+        int stream = 0;
+        if (tile) {
+            if (split && expert_offsets) {
+                if (!g_f32_tile) tile = group <= 24 ? 64 : 128;
+                if (tile != 64) tile = 128;
+                else stream = group <= 12 ? 2 : (group <= 24 ? 1 : 0);
+            } else if (!(tile == 32 || (split && (tile == 48 || tile == 128 || tile == 144 || tile == 160)))) tile = 64;
+            if (split && tile == 32 && M <= 32) stream = 1;
         }
         if (!tile) {
             mt = group <= 16 ? 1 : 2;
-            if (mt == 1 && !dual && (long)ceil_div(N, 32) * row_tiles(16) < cus) nw = 1;
+            // one set of weight rows a block where two give fewer blocks than CUs; taken apart, where a block has its rows to split besides, fewer than five eighths of them
+            // (2,048 k, 4 rows: 3,072 weight rows 9.8 us with one and 12.9 with two, 4,096 10.1 and 14.4, 5,120 15.7 and 15.3, 6,144 15.6 and 13.8)
+            if (mt == 1 && !dual && (long)ceil_div(N, 32) * row_tiles(16) < (split ? 5 * cus / 8 : cus)) nw = 1;
         }
         const bool half = !tile && lines && mt == 1 && !expert_offsets && M <= 16 &&
                           (g_skinny_half >= 0 ? g_skinny_half != 0 : ceil_div(N, 8) <= cus);
         if (half) nw = dual ? 2 : 1;
-        const int tm = tile ? tile : 16 * mt, tn = tile ? (tile == 32 && dual ? 64 : tile) : (half ? 8 : 16) * nw;
-        dim3 grid(ceil_div(N, dual ? tn / 2 : tn), row_tiles(tm));
+        if (tile && split) g.tile_rows = tile >= 128 ? 192 - tile : tile;
+        const int tm = !tile ? 16 * mt : split ? g.tile_rows : tile;
+        const int columns = !tile ? (half ? 8 : 16) * nw / (dual ? 2 : 1) : split ? (tile >= 128 ? 128 : 64) / (dual ? 2 : 1) : dual ? 32 : tile;
+        dim3 grid(ceil_div(N, columns), row_tiles(tm));
 #define FX_F32(DUAL_, EPI_)                                                            \
-    if (g.vec_ok) launch_f32<DUAL_, EPI_, true>(g, tile, mt, nw, half, grid, s);             \
-    else launch_f32<DUAL_, EPI_, false>(g, tile, mt, nw, false, grid, s)
+    if (g.vec_ok) launch_f32<DUAL_, EPI_, true>(g, split, tile, stream, mt, nw, half, grid, s);             \
+    else launch_f32<DUAL_, EPI_, false>(g, split, tile, 0, mt, nw, false, grid, s)
         switch (epi) {
             case EPI_STORE:
             case EPI_STORE_F32: FX_F32(false, EPI_STORE_F32); break;

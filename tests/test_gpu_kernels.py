@@ -163,6 +163,61 @@ def test_float32_tiles_leave_out_row_blocks_that_they_do_not_have(rows):
                 assert torch.equal(x, y), (tile, K)
 
 
+@pytest.mark.parametrize("N,K", [(33, 32), (40, 96), (130, 64), (70, 1056), (200, 2080), (257, 5632)])
+def test_float32_products_from_bfloat16_parts(N, K):
+    """Every tile and the kernel for few rows, at the edges of row blocks, with an odd and an even number of steps, plain, sorted by expert and from rows that
+    begin at odd multiples of four bytes: the same bits row for row, and an error against float64 of at most a float32 sum's (sqrt(K / 32) roundings of a sum, 2^-24 each, a factor of two on top)."""
+    from ferrox_amd import debug, ops
+    M = 130
+    a, w, w2 = rnd(M, K), rnd(N, K, seed=1), rnd(2 * N, K, seed=3, scale=0.3)
+    bias, scale, h0 = rnd(N, seed=2), rnd(M, seed=4), rnd(M, N, seed=5)
+    ref, ref2 = a.double() @ w.double().T, a.double() @ w2.double().T
+    wide = rnd(M, K + 3, seed=6)
+    wide[:, 1:K + 1] = a
+    we, we2 = torch.stack([rnd(N, K, seed=7), w]), torch.stack([rnd(2 * N, K, seed=8), w2])
+    with debug.kernel_switch("gemm", "f32_split", 1):
+        whole, gated = ops.gemm(a, w, bias=bias), ops.gemm(a, w2, epilogue=ops.EPI_GATED)
+        err = (whole.double() - ref - bias.double()).norm() / ref.norm()
+        assert float(err) <= 2 * (K / 32 + 1) ** 0.5 * 2.0 ** -24 + 2.0 ** -24, float(err)
+        close(gated, plain.silu(ref2[:, :N]) * ref2[:, N:], torch.float32, "silu(gate)*up")
+        for tile in (1, 32, 48, 64, 128, 144, 160, 0):
+            with debug.kernel_switch("gemm", "f32_tile", tile):
+                for rows in (1, 16, 17, 31, 33, 47, 48, 49, 63, 64, 65, M):
+                    assert torch.equal(ops.gemm(a[:rows], w, bias=bias), whole[:rows]), (tile, rows)
+                    assert torch.equal(ops.gemm(a[:rows], w2, epilogue=ops.EPI_GATED), gated[:rows]), (tile, rows)
+                h = h0.clone()
+                ops.gemm(a, w, epilogue=ops.EPI_RESID, out=h, row_scale=scale)
+                close(h, h0.double() + ref * scale.double()[:, None], torch.float32, "residual")
+                assert torch.equal(ops.gemm(wide[:, 1:K + 1], w, bias=bias), whole), tile
+                for first in (1, 40, 66, 0):                  # (shares of 1 to 130 rows: the second expert's are the plain product's)
+                    offsets = torch.tensor([0, first, M], dtype=torch.int32, device=DEV)
+                    assert torch.equal(ops.gemm(a, we, expert_offsets=offsets, n_rows=M, bias=None, epilogue=ops.EPI_STORE_F32)[first:], ops.gemm(a[first:], w, epilogue=ops.EPI_STORE_F32)), (tile, first)
+                    assert torch.equal(ops.gemm(a, we2, epilogue=ops.EPI_GATED, expert_offsets=offsets, n_rows=M)[first:], gated[first:]), (tile, first)
+
+
+@pytest.mark.parametrize("tile", [1, 32, 48, 128])
+def test_float32_parts_leave_what_is_not_finite_to_the_float32_instruction(tile):
+    """Infinities, NaN and values that round to infinity as bfloat16: what has one of them in its four columns is what the float32 instruction gives, and everything else is as without them."""
+    from ferrox_amd import debug, ops
+    M, N, K = 70, 72, 96
+    a, w = rnd(M, K), rnd(N, K, seed=1)
+    w2 = torch.cat([w, rnd(N, K, seed=2)])
+    bad_a, bad_w2 = a.clone(), w2.clone()
+    bad_a[3, 5], bad_a[9, 7], bad_a[20, 3], bad_a[66, 95], bad_w2[17, 90], bad_w2[N + 30, 0] = math.inf, math.nan, 3.4e38, -math.inf, -math.inf, math.nan
+    for kw, weights in ((dict(epilogue=ops.EPI_STORE_F32), lambda x: x[:N].contiguous()), (dict(epilogue=ops.EPI_GATED), lambda x: x)):
+        clean_w, bad_w = weights(w2), weights(bad_w2)
+        with debug.kernel_switch("gemm", "f32_tile", tile):
+            with debug.kernel_switch("gemm", "f32_split", 1):
+                clean, got = ops.gemm(a, clean_w, **kw), ops.gemm(bad_a, bad_w, **kw)
+            with debug.kernel_switch("gemm", "f32_split", 0):
+                want = ops.gemm(bad_a, bad_w, **kw)
+        sums = bad_a @ bad_w[:N].T, bad_a @ bad_w[-N:].T
+        odd = ~(torch.isfinite(sums[0]) & torch.isfinite(sums[1])).view(M, N // 4, 4).all(-1, keepdim=True).expand(M, N // 4, 4).reshape(M, N)
+        odd[20] = True                                       # (finite as float32 there, not as bfloat16)
+        assert torch.equal(torch.isnan(got[odd]), torch.isnan(want[odd])) and torch.equal(torch.nan_to_num(got[odd], nan=7.0), torch.nan_to_num(want[odd], nan=7.0))
+        assert torch.equal(got[~odd], clean[~odd]) and bool(odd.any()) and not bool(odd.all())
+
+
 @pytest.mark.parametrize("T,E,k,I,H", [(1, 5, 2, 20, 36), (3, 60, 4, 96, 128), (90, 7, 3, 33, 50), (700, 4, 2, 64, 96)])
 def test_float32_grouped_products_have_the_same_bits_in_every_kernel(T, E, k, I, H):
     from ferrox_amd import debug, ops

@@ -61,6 +61,8 @@ struct GemmArgs {
     void* rope_k_pages;     // null: nothing is written to pages (a layer that reads another's cache)
     void* rope_v_pages;
     int rope_nh, rope_nkv, rope_hd, rope_bs, rope_rot;
+    // TURN (few rows, stored): columns come in heads of rope_hd (0: nothing is turned), and of each the rope_rot dimensions from rope_nh on are turned in pairs
+    // (2i, 2i + 1), row m by rope_positions[m] * rope_inv_freq[i], and stretched by act_alpha
     const float* rope_inv_freq;       // rot/2 floats: pair i turns by (float)pos * rope_inv_freq[i]
     const float* rope_freq_factors;   // rot/2 floats or null: the angle of pair i is divided by rope_freq_factors[i]
     int stream_w;  // tiled kernel: the weights are read about once (one row tile a weight matrix): load them non-temporal
@@ -1255,8 +1257,10 @@ __device__ __forceinline__ void load8f(const float* p, bool ok, float* v) {
 // down product 36.6 -> 32.7 us, the head 132 -> 101 us (4.7 -> 6.2 TB/s).
 // NW: sets of 16 weight rows per wave; in dual mode set a is the gate (a even) or up (a odd) rows of
 // column group a / 2.
-template <int MT, int WAVES, int NW, bool DUAL, int EPI, bool NORM = false, bool ROPE = false, bool HALF = false, int DEPTH = 2, bool WEIGHTS_FIRST = false>
-__global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g) {
+// TURN: some outputs of each head are turned in pairs of neighbours (see GemmArgs).
+template <int MT, int WAVES, int NW, bool DUAL, int EPI, bool NORM, bool ROPE, bool HALF, int DEPTH, bool WEIGHTS_FIRST, bool TURN>
+__device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned block_x, const unsigned block_y) {
+    static_assert(!TURN || (EPI == EPI_STORE && MT == 1 && !NORM && !ROPE), "turned outputs are a few plain stored rows");
     static_assert(!HALF || (MT == 1 && WAVES == 4 && !NORM && !ROPE), "sets of eight weight rows are for few plain rows");
     constexpr int CW = HALF ? 8 : 16;               // weight rows of a set, output columns of a tile
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
@@ -1277,12 +1281,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
     int r0 = 0, r_end = 0, expert = 0, pair_a = -1, pair_c = -1;
     const bool pairs = MT == 1 && g.pair_ids != nullptr;
     if (pairs) {
-        if (!locate_pairs(g, blockIdx.y, expert, pair_a, pair_c)) return;
+        if (!locate_pairs(g, block_y, expert, pair_a, pair_c)) return;
     } else {
-        locate_rows<16 * MT>(g, blockIdx.y, r0, r_end, expert);
+        locate_rows<16 * MT>(g, block_y, r0, r_end, expert);
         if (r0 < 0) return;
     }
-    const int n0 = blockIdx.x * COLS;
+    const int n0 = block_x * COLS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, grp = lane >> 4;
     const bf16* Wbase = (const bf16*)g.W + (size_t)expert * g.w_stride;
@@ -1292,8 +1296,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
     bool rope_rotated = false;
     if constexpr (ROPE) {
         const int per_head = g.rope_hd >> 5;
-        rope_head = blockIdx.x / per_head;
-        rope_j = blockIdx.x - rope_head * per_head;
+        rope_head = block_x / per_head;
+        rope_j = block_x - rope_head * per_head;
         const bool is_v = rope_head >= g.rope_nh + g.rope_nkv;
         const int n_rot = is_v ? 0 : g.rope_rot >> 5;          // blocks of this head whose columns are rotated
         rope_rotated = rope_j < n_rot;
@@ -1482,6 +1486,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
             if (!DUAL && g.bias) {
 #pragma unroll
                 for (int r = 0; r < V; ++r) bias_of[i][r] = fetch_element(g.bias, g.bias_dtype, min(first + r, g.N - 1));
+            }
+        }
+    }
+    // (the angle of the pair that a thread's output belongs to, worked out while the weights are on their way; 0 where it is not turned)
+    float turn_cs[TURN ? IT : 1], turn_sn[TURN ? IT : 1];
+    bool turned[TURN ? IT : 1];
+    if constexpr (TURN) {
+        static_assert(V == 1, "a lane's neighbour holds the other number of its pair");
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int c = g.rope_hd ? column_of(i) % g.rope_hd - g.rope_nh : -1;
+            turned[i] = m_of[i] >= 0 && c >= 0 && c < g.rope_rot;
+            if (turned[i]) {
+                sincosf((float)g.rope_positions[m_of[i]] * g.rope_inv_freq[c >> 1], &turn_sn[i], &turn_cs[i]);
+                turn_cs[i] *= g.act_alpha;
+                turn_sn[i] *= g.act_alpha;
             }
         }
     }
@@ -1723,6 +1743,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
                     }
                 }
             }
+            if constexpr (TURN) {
+                if (turned[i]) {      // (rounded before it is turned, as when the rotation is a kernel of its own; a pair's two lanes are here together)
+                    const float own = bf16_to_float(float_to_bf16(o[0])), other = lane_pair_other(own);
+                    float y0, y1;
+                    rotate_pair(n & 1 ? other : own, n & 1 ? own : other, turn_cs[i], turn_sn[i], y0, y1);
+                    o[0] = n & 1 ? y1 : y0;
+                }
+            }
             typedef std::conditional_t<EPI == EPI_STORE || EPI == EPI_GATED, bf16, float> out_t;
             out_t* to = (out_t*)g.C + (size_t)m * g.ldc + n;
             if constexpr (V == 1) from_float(to, o[0]);
@@ -1731,6 +1759,24 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
     };
     if constexpr (DUAL) with_activation(g.act, finish);
     else with_stored<EPI == EPI_STORE || EPI == EPI_STORE_F32>(g.store_act, finish);
+}
+
+template <int MT, int WAVES, int NW, bool DUAL, int EPI, bool NORM = false, bool ROPE = false, bool HALF = false, int DEPTH = 2, bool WEIGHTS_FIRST = false>
+__global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g) {
+    skinny_block<MT, WAVES, NW, DUAL, EPI, NORM, ROPE, HALF, DEPTH, WEIGHTS_FIRST, false>(g, blockIdx.x, blockIdx.y);
+}
+
+// Two products of up to 16 plain rows that do not need each other, one launch: the first's blocks (gate/up, or a product that is added, in half sets of
+// weight rows), then the second's (stored; in half or whole sets).  A step of few tokens is a chain of launches of 3 us and more that each wait for memory alone;
+// side by side they wait together, and the streams of the larger one go on meanwhile.  The same blocks, so the same bits.  us apart -> together: gate/up of 5,632 x 2,048 and
+// 1,024 x 2,048 1 row 14.6 -> 11.2, 8 rows 16.1 -> 13.2, 16 rows 18.6 -> 16.6; 2,048 x 5,632 added and 4,096 x 512 with its heads turned (a launch of its own before)
+// 13.5 -> 8.0, 14.1 -> 8.9, 16.3 -> 10.9.
+template <bool GATED, int DEPTH, int NW2, int EPI2, bool HALF2>
+__global__ __launch_bounds__(256) void gemm_bf16_skinny_pair_kernel(GemmArgs a, GemmArgs b, int first) {
+    if ((int)blockIdx.x < first)
+        skinny_block<1, 4, GATED ? 2 : 1, GATED, GATED ? EPI_GATED : EPI_RESID, false, false, true, DEPTH, false, false>(a, blockIdx.x, 0);
+    else
+        skinny_block<1, 4, NW2, false, EPI2, false, false, HALF2, HALF2 ? 4 : 2, false, EPI2 == EPI_STORE>(b, blockIdx.x - first, 0);
 }
 
 // ===========================================================================
@@ -2739,6 +2785,79 @@ FX_API int fx_gemm_f32_split_tile(int M, int N, int dual, int cus) {
         if (us < least) least = us, best = k.code;
     }
     return best;
+}
+
+// How the product for few rows takes up to 16 plain rows: sets of weight rows a wave has, half sets or whole ones, pieces of K on their way.
+struct FewRows {
+    int sets;
+    bool half, deep;
+};
+static FewRows few_plain_rows(int M, int N, int K, bool dual, int cus) {
+    FewRows f;
+    f.sets = dual || ceil_div(N, 32) >= 160 ? 2 : 1;
+    if (!dual && M <= 2 && ceil_div(N, 16) >= 4096) f.sets = 1;
+    f.half = (K >= 2048 || ceil_div(N, 8) <= cus) && fx_gemm_half_sets(M, N, dual, f.sets, cus);
+    f.deep = K <= 2048 || M <= 4;
+    return f;
+}
+
+// A product of up to 16 plain bfloat16 rows for `fx_gemm_pair`.
+struct FxProduct {
+    const void *A, *W;
+    void* C;
+    const float* row_scale;
+    const int* turn_positions;
+    const float* turn_inv_freq;
+    long lda, ldc, up_offset;
+    int epi, M, N, K, act, turn_width, turn_from, turn_dims;
+    float act_limit, act_alpha, turn_magnitude;
+};
+// Whether two such products go out in one launch: the first one's kernel is the one for half sets of weight rows (gate/up with four pieces on their way).
+FX_API int fx_gemm_pairs(int M, int epi, int N, int K, int epi2, int N2, int K2, int cus) {
+    const FewRows f = few_plain_rows(M, N, K, epi == EPI_GATED, cus);
+    return M >= 1 && M <= 16 && K % 8 == 0 && K2 % 8 == 0 && N2 < 65536 && N < 65536 && (epi2 == EPI_STORE || epi2 == EPI_STORE_F32) &&
+           f.half && (epi == EPI_RESID || (epi == EPI_GATED && f.deep));
+}
+FX_API int fx_gemm_pair(void* stream, const FxProduct* first, const FxProduct* second) {
+    const int cus = fx_compute_units();
+    const FxProduct* products[2] = {first, second};
+    FX_REQUIRE(first && second && first->M == second->M && fx_gemm_pairs(first->M, first->epi, first->N, first->K, second->epi, second->N, second->K, cus),
+               "gemm_pair: up to 16 rows of a product in half sets of weight rows and of one that is stored");
+    GemmArgs g[2] = {};
+    for (int i = 0; i < 2; ++i) {
+        const FxProduct& p = *products[i];
+        FX_REQUIRE(p.A && p.W && p.C && p.N > 0 && p.K > 0 && p.lda >= p.K && p.ldc >= p.N && p.lda % 8 == 0 && p.up_offset % 8 == 0 && (((uintptr_t)p.A | (uintptr_t)p.W) % 16) == 0,
+                   "gemm_pair: operands of product %d are not aligned rows", i);
+        FX_REQUIRE(p.act >= 0 && p.act < ACT_COUNT && (p.act != ACT_SWIGLU_CLAMP || p.act_limit > 0.f), "gemm_pair: activation %d", p.act);
+        FX_REQUIRE(p.turn_width == 0 || (i == 1 && p.epi == EPI_STORE && p.turn_positions && p.turn_inv_freq && p.turn_from >= 0 && p.turn_dims >= 0 && p.turn_from % 2 == 0 &&
+                                         p.turn_dims % 2 == 0 && p.turn_width % 2 == 0 && p.turn_from + p.turn_dims <= p.turn_width && p.N % p.turn_width == 0),
+                   "gemm_pair: %d turned dimensions from %d on of heads of %d", p.turn_dims, p.turn_from, p.turn_width);
+        g[i].A = p.A; g[i].lda = p.lda; g[i].W = p.W; g[i].C = p.C; g[i].ldc = p.ldc; g[i].up_offset = p.up_offset; g[i].row_scale = p.row_scale;
+        g[i].M = p.M; g[i].N = p.N; g[i].K = p.K; g[i].act = p.act; g[i].act_limit = p.act_limit; g[i].act_alpha = p.act_alpha; g[i].vec_ok = 1;
+        if (p.turn_width) {
+            g[i].rope_positions = p.turn_positions; g[i].rope_inv_freq = p.turn_inv_freq; g[i].act_alpha = p.turn_magnitude;
+            g[i].rope_hd = p.turn_width; g[i].rope_nh = p.turn_from; g[i].rope_rot = p.turn_dims;
+        }
+    }
+    FX_REQUIRE(first->turn_width == 0, "gemm_pair: the first product is not turned");
+    const FewRows f = few_plain_rows(first->M, first->N, first->K, first->epi == EPI_GATED, cus), f2 = few_plain_rows(second->M, second->N, second->K, false, cus);
+    const int blocks = ceil_div(first->N, 8), blocks2 = ceil_div(second->N, f2.half ? 8 : 16 * f2.sets);
+    const dim3 grid(blocks + blocks2);
+    hipStream_t s = (hipStream_t)stream;
+    auto go = [&](auto gated, auto depth, auto sets, auto half) {
+        if (second->epi == EPI_STORE) gemm_bf16_skinny_pair_kernel<decltype(gated)::value, decltype(depth)::value, decltype(sets)::value, EPI_STORE, decltype(half)::value><<<grid, 256, 0, s>>>(g[0], g[1], blocks);
+        else gemm_bf16_skinny_pair_kernel<decltype(gated)::value, decltype(depth)::value, decltype(sets)::value, EPI_STORE_F32, decltype(half)::value><<<grid, 256, 0, s>>>(g[0], g[1], blocks);
+    };
+    auto with_second = [&](auto gated, auto depth) {
+        if (f2.half) go(gated, depth, fx_int<1>{}, std::true_type{});
+        else if (f2.sets == 1) go(gated, depth, fx_int<1>{}, std::false_type{});
+        else go(gated, depth, fx_int<2>{}, std::false_type{});
+    };
+    if (first->epi == EPI_GATED) with_second(std::true_type{}, fx_int<4>{});
+    else if (f.deep) with_second(std::false_type{}, fx_int<4>{});
+    else with_second(std::false_type{}, fx_int<2>{});
+    FX_CHECK_LAUNCH("gemm_pair");
+    return 0;
 }
 
 // The tile of the LDS-tiled kernel for plain rows, as the debug switch "wide" names them; all give the same bits.  `dual`: N

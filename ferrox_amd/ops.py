@@ -7,7 +7,8 @@ library, raises.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_float, c_int, c_long, c_void_p
+from ctypes import Structure, byref, c_float, c_int, c_long, c_void_p
+from dataclasses import dataclass
 
 import math
 
@@ -149,6 +150,8 @@ _sigs = {
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     ("moe", "fx_moe_front"): [c_void_p, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_int,
                               c_int, c_int, c_int, c_int, c_float, c_float, c_int] + [c_void_p] * 9 + [c_int],
+    ("gemm", "fx_gemm_pairs"): [c_int] * 8,
+    ("gemm", "fx_gemm_pair"): [c_void_p, c_void_p, c_void_p],
     ("moe", "fx_moe_align"): [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int],
     ("sampling", "fx_sample_greedy"): [c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_void_p, c_void_p],
     ("sampling", "fx_sample"): [c_void_p, c_void_p, c_long, c_void_p, c_int, c_int] + [c_void_p] * 10,
@@ -784,6 +787,77 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
           float(activation_params[0]), float(activation_params[1]), _p(pre_scale), _p(_i32(pre_scale_rows, "pre_scale_rows")),
           _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share))
     return out
+
+
+PAIR_MAX_ROWS = 16
+
+
+@dataclass
+class Product:
+    """A product of plain rows that is yet to be launched: arguments of `gemm`, and `turn` = (positions, inv_freq, head width, first and
+    number of the turned dimensions of a head, magnitude): outputs turned as `latent_q_rot` turns them (a stored product in `gemm_pair`)."""
+    a: torch.Tensor
+    w: torch.Tensor
+    out: torch.Tensor
+    epilogue: int = EPI_STORE
+    activation: str = "silu"
+    activation_params: tuple = (0.0, 0.0)
+    row_scale: torch.Tensor | None = None
+    turn: tuple | None = None
+
+    def columns(self) -> int:
+        return self.w.shape[0] // 2 if self.epilogue == EPI_GATED else self.w.shape[0]
+
+    def launch(self) -> None:
+        """By itself (without `turn`)."""
+        gemm(self.a, self.w, epilogue=self.epilogue, out=self.out, activation=self.activation, activation_params=self.activation_params,
+             row_scale=self.row_scale)
+
+
+class _ProductArgs(Structure):
+    _fields_ = [(n, c_void_p) for n in ("A", "W", "C", "row_scale", "turn_positions", "turn_inv_freq")] + \
+               [(n, c_long) for n in ("lda", "ldc", "up_offset")] + \
+               [(n, c_int) for n in ("epi", "M", "N", "K", "act", "turn_width", "turn_from", "turn_dims")] + \
+               [(n, c_float) for n in ("act_limit", "act_alpha", "turn_magnitude")]
+
+
+def can_pair(first: Product, second: Product) -> bool:
+    """Whether `gemm_pair` takes the two: up to 16 rows of bfloat16, the first gated or added in blocks of half sets of weight rows, the second stored."""
+    M = first.a.shape[0]
+    if not 1 <= M <= PAIR_MAX_ROWS or second.a.shape[0] != M:
+        return False
+    for p in (first, second):
+        if p.a.dtype != torch.bfloat16 or p.w.dtype != torch.bfloat16 or p.w.dim() != 2 or not p.w.is_contiguous() or p.a.dim() != 2 or p.a.stride(1) != 1 \
+                or p.a.stride(0) % 8 or p.a.shape[1] != p.w.shape[1] or p.a.data_ptr() % 16 or p.w.data_ptr() % 16 or p.columns() * p.w.shape[1] % 8:
+            return False
+    fn, _ = _fn("gemm", "fx_gemm_pairs")
+    return bool(fn(M, first.epilogue, first.columns(), first.w.shape[1], second.epilogue, second.columns(), second.w.shape[1], compute_units(first.a.device)))
+
+
+def gemm_pair(first: Product, second: Product) -> None:
+    """Both products in one launch, each with the bits of a launch of its own.  Neither may read or add to what the other writes."""
+    if not can_pair(first, second):
+        raise KernelError("gemm_pair: these products do not go out together")
+    args = []
+    for p in (first, second):
+        M, N, K = p.a.shape[0], p.columns(), p.w.shape[1]
+        dtype = p.w.dtype if p.epilogue in (EPI_STORE, EPI_GATED) else torch.float32
+        if p.out.dtype != dtype or p.out.dim() != 2 or p.out.stride(1) != 1 or p.out.shape[0] < M or p.out.shape[1] < N:
+            raise KernelError(f"gemm_pair: output {tuple(p.out.shape)} {p.out.dtype} does not fit [{M},{N}] {dtype}")
+        if p.activation not in ACTIVATIONS:
+            raise KernelError(f"gemm_pair: activation '{p.activation}' is not one of {sorted(ACTIVATIONS)}")
+        if p.row_scale is not None and (p.epilogue != EPI_RESID or p.row_scale.dtype != torch.float32 or p.row_scale.numel() < M):
+            raise KernelError("gemm_pair: a row scale is float32, a number per row of a product that is added")
+        g = _ProductArgs(A=_p(p.a), W=_p(p.w), C=_p(p.out), row_scale=_p(p.row_scale), lda=p.a.stride(0), ldc=p.out.stride(0),
+                         up_offset=N * K if p.epilogue == EPI_GATED else 0, epi=p.epilogue, M=M, N=N, K=K, act=ACTIVATIONS[p.activation],
+                         act_limit=float(p.activation_params[0]), act_alpha=float(p.activation_params[1]))
+        if p.turn is not None:
+            positions, inv_freq, g.turn_width, g.turn_from, g.turn_dims, g.turn_magnitude = p.turn
+            if positions.numel() < M or inv_freq.dtype != torch.float32 or 2 * inv_freq.numel() < g.turn_dims:
+                raise KernelError("gemm_pair: a position per row and a float32 frequency per turned pair")
+            g.turn_positions, g.turn_inv_freq = _p(_i32(positions, "positions")), _p(inv_freq)
+        args.append(g)
+    _call("gemm", "fx_gemm_pair", _stream(), byref(args[0]), byref(args[1]))
 
 
 def can_qkv_rope(x, w, n_rows: int, head_dim: int, rotary_dim: int, interleaved: bool) -> bool:

@@ -18,7 +18,7 @@ import torch
 
 from .. import debug, limits, ops
 from .base import MIXERS, NORMS, POSITION_ENCODINGS, Mixer, ParamSpec, PartSpec, Rotary
-from .linear import Linear, matmul, same_dtype
+from .linear import Linear, matmul, matmul_with, same_dtype
 
 NO_ROTATION = Rotary(0, 1.0)
 FUSE_HEAD_NORMS = True      # (a switch for tests: the norms of q's and k's heads and the cache write as one launch)
@@ -332,8 +332,8 @@ class PagedAttention(Mixer):
         wq, eps = self.q_norm.rms_params()
         w = self.qkv.weight
         cut = self.qw + self.kvw + self.vw
-        qk = matmul(x, w[:cut], epilogue=ops.EPI_STORE_F32)
-        rest = matmul(x, w[cut:]) if w.shape[0] > cut else None
+        qk, _ = matmul_with(ctx, x, w[:cut], epilogue=ops.EPI_STORE_F32)
+        rest = matmul_with(ctx, x, w[cut:])[0] if w.shape[0] > cut else None
         q = torch.empty((ctx.n_tokens, self.qw), dtype=ctx.act_dtype, device=qk.device)
         writes = self.own_kv and cache.writes
         debug.region("rope + cache write")

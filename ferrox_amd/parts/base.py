@@ -152,6 +152,7 @@ class StepContext:
     recorded: bool = False
     kv_bound: int = 0
     carry: object = None               # what a feed-forward hands on to the next block (its rows, normed), see PreNormBlock
+    waiting: list = field(default_factory=list)      # products (ops.Product) that a block has left for its mixer's launches, see `linear.matmul_with`
     _memo: dict = field(default_factory=dict)
 
     def memo(self, key, make: Callable):

@@ -3,7 +3,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import debug
+from .. import debug, ops
 from .base import BLOCKS, FEED_FORWARDS, MIXERS, NORMS, Block, ParamSpec, PartSpec
 from .linear import Linear
 
@@ -107,7 +107,8 @@ class SandwichBlock(Block):
 class ParallelBlock(Block):
     """h += mixer(norm1(h)) + ffn(norm1(h)): one norm, and both sublayers read its output.  A layer without a
     feed-forward has the mixer only.  Both sublayers end with a product that adds into the float32 stream; the
-    normed rows are made before either has added, so the order of the two additions changes rounding alone."""
+    normed rows are made before either has added, so the order of the two additions changes rounding alone.
+    For a few bfloat16 rows the feed-forward's products go out in the launches of products of the mixer that do not need them (Fokinex, 8 layers, a decode step of 8 sequences: 673 -> 609 us)."""
     slots = {"norm1": NORMS, "mixer": MIXERS, "ffn": FEED_FORWARDS}
     optional_slots = ("ffn",)
 
@@ -121,15 +122,20 @@ class ParallelBlock(Block):
     def forward(self, h, ctx, cache):
         debug.region("norm")
         x = self.norm1.forward(h, ctx)
+        few = x.dtype == torch.bfloat16 and x.shape[0] <= ops.PAIR_MAX_ROWS and hasattr(self.ffn, "products")
+        products = self.ffn.products(x, h) if few else []
+        ctx.waiting = list(products)
         self.mixer.forward(x, ctx, cache, h)
-        if self.ffn is not None:
+        rest, ctx.waiting = ctx.waiting, []
+        for product in rest:
+            product.launch()
+        if self.ffn is not None and not products:
             self.ffn.forward(x, ctx, h)
 
 
 def sublayer_rows(part, out, x, ctx, *cache):
     """The sublayer's output rows in `out`: a part that says `takes_fresh` stores them with its last product,
     any other adds them into a zeroed buffer."""
-    from .. import ops
     if getattr(part, "takes_fresh", False):
         part.forward(x, ctx, *cache, out, fresh=True)
     else:

@@ -28,7 +28,7 @@ import torch
 from .. import debug, limits, ops
 from .attention import attention_items
 from .base import MIXERS, NORMS, POSITION_ENCODINGS, Mixer, ParamSpec, PartSpec
-from .linear import Linear, matmul, same_dtype
+from .linear import Linear, matmul, matmul_with, same_dtype
 from .recurrent import longest_portion
 
 _head_groups: dict = {}
@@ -176,7 +176,7 @@ class LatentAttention(Mixer):
         table = ctx.block_tables[cache.group]
         k_pages, v_pages = cache.pages["k"], cache.pages["v"]
         debug.region("latent down")
-        down = matmul(x, self.down, epilogue=ops.EPI_STORE_F32)          # float32: the norms read it
+        down, _ = matmul_with(ctx, x, self.down, epilogue=ops.EPI_STORE_F32)          # float32: the norms read it
         wq, eps = self.q_norm.rms_params() if self.q_norm is not None else (None, 0.0)
         kv_at = self.front
         gate = down[:, down.shape[1] - self.gate_width:] if self.out_gate else None       # (float32 logits)
@@ -203,8 +203,10 @@ class LatentAttention(Mixer):
             c_q = ops.rmsnorm(down, wq, eps, ctx.act_dtype, width=self.q_rank)
         if self.q_rank is not None:
             debug.region("latent up")
-            q_lat = self.up_q(c_q)                                        # [T, H * (R + P)]: absorbed parts, parts to rotate
-            if self.rot.rotary_dim:                                       # (in place: a pair is read and written by one thread)
+            # [T, H * (R + P)]: absorbed parts, parts to rotate
+            turn = (ctx.positions, self.inv_freq, R + P, R, self.rot.rotary_dim, self.rot.magnitude) if self.rot.rotary_dim else None
+            q_lat, turned = matmul_with(ctx, c_q, self.up_q.weight, turn=turn)
+            if self.rot.rotary_dim and not turned:                        # (in place: a pair is read and written by one thread)
                 ops.latent_q_rot(q_lat, q_lat, ctx.positions, H, R, P, self.rot.rotary_dim, R, self.inv_freq, self.rot.magnitude)
         q = q_lat
         debug.region("attention")

@@ -45,6 +45,14 @@ class GatedMLP(FeedForward):
 
     takes_fresh = True       # forward(..., fresh=True): `residual` holds nothing yet, the output is stored into it
 
+    def products(self, x, residual) -> list:
+        """What `forward` launches, in its order, for a caller that launches it beside other products (none where a weight is of another type than the rows)."""
+        if not x.dtype == self.gate_up.weight.dtype == self.down.weight.dtype:
+            return []
+        act = torch.empty((x.shape[0], self.intermediate_size), dtype=self.gate_up.weight.dtype, device=x.device)
+        return [ops.Product(x, self.gate_up.weight, act, ops.EPI_GATED, self.activation, self.activation_params),
+                ops.Product(act, self.down.weight, residual, ops.EPI_RESID)]
+
     def forward(self, x, ctx, residual, row_scale=None, fresh: bool = False) -> None:
         debug.region("mlp gate/up")
         act = self._act(x)

@@ -21,7 +21,7 @@ import torch
 
 from .. import debug, ops
 from .base import MIXERS, Mixer, ParamSpec
-from .linear import Linear, matmul, same_dtype
+from .linear import Linear, matmul, matmul_with, same_dtype
 
 _aranges: dict = {}
 
@@ -176,7 +176,7 @@ class HeadDelta(ChannelDelta):
         H, G, D, V = self.n_heads, self.n_kv_heads, self.key_dim, self.v_dim
         C, QK = self.conv_channels, self.qk_width
         debug.region("delta in")
-        proj = matmul(x, self.w_in, epilogue=ops.EPI_STORE_F32)
+        proj, _ = matmul_with(ctx, x, self.w_in, epilogue=ops.EPI_STORE_F32)
         starts = sequence_starts(ctx)
         o1 = C + H          # beta ends
         o2 = o1 + H         # decay ends; the gate's rows follow

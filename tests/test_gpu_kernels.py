@@ -1842,3 +1842,37 @@ def test_delta_rule_at_every_length_of_a_group(D, V, H, G):
         cut, part = lengths[i] // 2, before.clone()
         halves = [run(lo, hi, [0, hi - lo], [i], part) for lo, hi in ((at[i], at[i] + cut), (at[i] + cut, at[i + 1])) if hi > lo]
         assert torch.equal(torch.cat(halves), out[at[i]:at[i + 1]]) and torch.equal(part[i], state[i]), lengths[i]
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("N2,K2,epi2", [(256, 128, 0), (1024, 2048, 1), (4096, 512, 0), (5120, 512, 1), (24, 64, 0)])
+def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2):
+    """Gate/up and an added product, each beside a stored one in half sets, whole sets and two of them, with the pairs of its heads turned and without."""
+    from ferrox_amd import ops
+    x, w_gu, w_down = rnd(M, 2048, dtype=torch.bfloat16), rnd(2 * 5632, 2048, dtype=torch.bfloat16, seed=1, scale=0.02), rnd(2048, 5632, dtype=torch.bfloat16, seed=2, scale=0.02)
+    y, w2 = rnd(M, K2, dtype=torch.bfloat16, seed=3), rnd(N2, K2, dtype=torch.bfloat16, seed=4, scale=0.1)
+    h0, scale = rnd(M, 2048, seed=5), rnd(M, seed=6)
+    heads = 4
+    width = N2 // heads
+    first_dim = width // 4 * 2
+    n_dims = min(first_dim, 64)             # (the rotation by itself takes up to 256)
+    positions, inv_freq = torch.randint(0, 30000, (M,), device=DEV, dtype=torch.int32), torch.rand(n_dims // 2, device=DEV)
+    def stored():
+        return torch.full((M, N2 + 8), 7.0, dtype=torch.bfloat16 if epi2 == 0 else torch.float32, device=DEV)
+    act, h = ops.gemm(x, w_gu, epilogue=ops.EPI_GATED, activation="gelu_tanh"), h0.clone()
+    ops.gemm(act, w_down, epilogue=ops.EPI_RESID, out=h, row_scale=scale)
+    plain2 = ops.gemm(y, w2, epilogue=epi2)
+    for turn in (None, (positions, inv_freq, width, first_dim, n_dims, 1.25)) if epi2 == 0 else (None,):
+        want = plain2.clone()
+        if turn is not None:
+            ops.latent_q_rot(want, want, positions, heads, first_dim, width - first_dim, n_dims, first_dim, inv_freq, 1.25)
+        got_act, got_h, one, two = torch.full((M, 5632), 7.0, dtype=torch.bfloat16, device=DEV), h0.clone(), stored(), stored()
+        first = ops.Product(x, w_gu, got_act, ops.EPI_GATED, "gelu_tanh")
+        ops.gemm_pair(first, ops.Product(y, w2, one[:, :N2], epi2, turn=turn))
+        ops.gemm_pair(ops.Product(got_act, w_down, got_h, ops.EPI_RESID, row_scale=scale), ops.Product(y, w2, two[:, :N2], epi2, turn=turn))
+        assert torch.equal(got_act, act) and torch.equal(got_h, h)
+        for out in (one, two):
+            assert torch.equal(out[:, :N2], want) and bool((out[:, N2:] == 7).all()), turn is not None
+    assert not ops.can_pair(first, ops.Product(y[:, 1:], w2[:, 1:], one, epi2)) and not ops.can_pair(first, ops.Product(y.float(), w2.float(), one, epi2))
+    with pytest.raises(ops.KernelError):
+        ops.gemm_pair(first, ops.Product(y, w2, h0, ops.EPI_RESID))

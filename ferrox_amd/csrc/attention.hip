@@ -866,10 +866,10 @@ struct WaveAttn {
 // values go from memory straight into operands, no LDS and no barrier.  A unit (16 keys x up to 128 numbers, or 32 value
 // rows x 64 keys) is on its way while the one before it is multiplied; page ids are asked for a tile ahead.
 // (A lane per key that reads its row number by number, as the kernels for any shape do, took 514 us a layer for 700
-// tokens of 16 heads and 124 us for four single queries at 1,030 keys; these take 95 and 25 us.  What bounds them now is
-// one wave's chain: 256 products of 32 cycles a tile of 64 keys x 128 numbers, 3.4 of the 7.2 us that a tile takes (5.0 with heads of 64,
-// 11.8 of 256: some 2.7 us a tile from scores to probabilities and for page ids, whatever the head, the rest waits for operands), and few
-// waves a SIMD to hide it.)
+// tokens of 16 heads and 124 us for four single queries at 1,030 keys; these take 88 and 22 us.  What bounds them now is
+// one wave's chain: 256 products of 32 cycles a tile of 64 keys x 128 numbers, 3.4 of the 5.8 us that a tile takes where the other SIMDs are idle, and where four waves
+// of a block read the same tile, 8 us, the CU's L1: half lines, 64 KB a tile and wave.  Masks and pages without branches: 700 tokens 94.5 -> 88.2 us, 300 46.9 -> 38.7,
+// 64 17.9 -> 16.1, 20 at 3,000 keys 345 -> 271, 1,500 under a window of 128 74.5 -> 62.0; four single queries at 1,030 keys 24.9 -> 21.7; heads of 64, 700 tokens 64.7 -> 47.2, single queries 17.3 -> 13.7.)
 // ---------------------------------------------------------------------------
 template <int HDM>
 struct F32Attention {
@@ -910,30 +910,42 @@ struct F32Attention {
         const int safe = span.begin < span.end ? span.end - 1 : min(span.keep, span.end) - 1;
         const float* kp[4];       // the tile's key rows of this lane, from number 4 g on
         const float* vp[4];       // row li of the values, at keys 16 c + 4 g
-        int kpage[4], kslot[4], vpage[4], vslot[4];
+        int page_ids[8], page_slots[8];      // of the keys, then of the values
         auto ask_pages = [&](int kt0) {
+            int t[8], blk[8];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                int t = kt0 + 16 * c + li, blk;
-                t = span.has(t) ? t : safe;
-                page_slot(a, t, blk, kslot[c]);
-                kpage[c] = bt[blk];
-                t = kt0 + 16 * c + 4 * g;
+                const int k = kt0 + 16 * c + li, v = kt0 + 16 * c + 4 * g;
+                t[c] = (k < span.end) & ((k >= span.begin) | (k < span.keep)) ? k : safe;
                 // (four keys of one page: the page is there if any of them is in the span)
-                t = span.touches(t, 4) ? t : (safe & ~3);
-                page_slot(a, t, blk, vslot[c]);
-                vpage[c] = bt[blk];
+                t[4 + c] = (v < span.end) & ((v + 4 > span.begin) | (v < span.keep)) ? v : safe & ~3;
             }
+            int (&slot)[8] = page_slots;
+            if (a.bs_shift >= 0) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    blk[c] = t[c] >> a.bs_shift;
+                    slot[c] = t[c] & (a.bs - 1);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    blk[c] = t[c] / a.bs;
+                    slot[c] = t[c] - blk[c] * a.bs;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) page_ids[c] = bt[blk[c]];
         };
         auto point_keys = [&]() {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                kp[c] = (const float*)a.k_pages + (((size_t)kpage[c] * a.nkv + kvh) * a.bs + kslot[c]) * a.hd + min(4 * g, a.hd - 4);
+                kp[c] = (const float*)a.k_pages + (((size_t)page_ids[c] * a.nkv + kvh) * a.bs + page_slots[c]) * a.hd + min(4 * g, a.hd - 4);
         };
         auto point_values = [&]() {
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                vp[c] = (const float*)a.v_pages + (((size_t)vpage[c] * a.nkv + kvh) * a.vd + min(li, a.vd - 1)) * a.bs + vslot[c];
+                vp[c] = (const float*)a.v_pages + (((size_t)page_ids[4 + c] * a.nkv + kvh) * a.vd + min(li, a.vd - 1)) * a.bs + page_slots[4 + c];
         };
         f32x4_t kb[2][UC];
         auto fetch_keys = [&](int set, int unit) {       // unit: key block, then the part of its numbers
@@ -979,31 +991,51 @@ struct F32Attention {
                         part[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[unit & 1][i][u], q[unit % NU * UC + i][u], part[i & 1], 0, 0, 0);
                 s[unit / NU] = unit % NU == 0 ? part[0] + part[1] : s[unit / NU] + (part[0] + part[1]);
             }
+            if (shaped) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[c][r] = shaped_score(a, h, slope, s[c][r], pos - (kt0 + 16 * c + 4 * g + r));
+            }
+            // (masks as one number each, and none for a tile that all rows see whole: in `&&` and `||` a score's was up to four branches of some 35 ns)
+            const bool whole = span.holds_tile(kt0);
+            if (!whole || !__all((kt0 >= lo) & (kt0 + 63 <= pos))) {
+                const int from = max(lo, span.begin), to = min(pos, span.end - 1);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int t = kt0 + 16 * c + 4 * g + r;
+                        s[c][r] = (t <= to) & ((t >= from) | (t < a.keep_first)) ? s[c][r] : NEG_INF;
+                    }
+            }
             float top = NEG_INF;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int t = kt0 + 16 * c + 4 * g + r;
-                    const bool sees = t <= pos && span.has(t) && (t >= lo || t < a.keep_first);
-                    float v = s[c][r];
-                    if (shaped) v = shaped_score(a, h, slope, v, pos - t);
-                    s[c][r] = sees ? v : NEG_INF;
-                    top = fmaxf(top, s[c][r]);
-                }
+                for (int r = 0; r < 4; ++r) top = fmaxf(top, s[c][r]);
             const float m_new = fmaxf(m, quad_max(top));
-            const float al = m_new == NEG_INF ? 1.f : expf(m - m_new);
+            const float al = m_new == NEG_INF ? 1.f : expf(m - m_new), from_m = m_new == NEG_INF ? 0.f : m_new;
             float sum = 0.f;
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    s[c][r] = s[c][r] == NEG_INF ? 0.f : expf(s[c][r] - m_new);
+                    s[c][r] = expf(s[c][r] - from_m);       // (minus infinity: 0)
                     sum += s[c][r];
                 }
             l = l * al + quad_sum(sum);
             m = m_new;
-            const bool whole = span.holds_tile(kt0);
+            int inside = 0;      // bit 4 c + r: key 16 c + 4 g + r of the tile is in the span
+            if (!whole) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int t = kt0 + 16 * c + 4 * g + r;
+                        inside |= ((t < span.end) & ((t >= span.begin) | (t < span.keep)) ? 1 : 0) << (4 * c + r);
+                    }
+            }
 #pragma unroll
             for (int pair = 0; pair < (NC + 1) / 2; ++pair) {
                 if (pair + 1 < (NC + 1) / 2) fetch_values((pair + 1) & 1, pair + 1);
@@ -1013,7 +1045,7 @@ struct F32Attention {
                     for (int c = 0; c < 4; ++c)
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            if (!span.has(kt0 + 16 * c + 4 * g + r)) v[c][r] = v[4 + c][r] = 0.f;
+                            if (!(inside >> (4 * c + r) & 1)) v[c][r] = v[4 + c][r] = 0.f;
                 }
                 o[2 * pair] *= al;
                 o[2 * pair + 1] *= al;
@@ -1066,8 +1098,9 @@ __global__ __launch_bounds__(256) void attn_f32_block_kernel(AttnArgs a) {
 }
 // decode: block = one wave = (item, kv head x block of 16 of its query heads, chunk of keys); results merge as those of
 // attn_decode_kernel do.  Queries below position FEW_KEYS go a wave per head as in that kernel: it is through with so few keys before a
-// tile's chain of waits is (16 heads of 128, merge included: 5 keys 9.3 against 16.3 us, 16 keys 13.2 and 16.1, 24 the same, 32 19.5 and
-// 16.4; 16 of 64 in groups of four: 5 keys 7.3 against 12.1, 24 11.1 and 12.2, 32 12.6 and 12.2; 16 of 192 + 128 32 keys 20.4 against 26.2).
+// tile's chain of waits is, which takes the same for any number of keys (merge included, 16 heads of 128: 5 keys 10.0 against 14.0 us, 12 12.4, 16 13.9, 20 15.4; 16 of 64 in groups
+// of four: 5 keys 8.0 against 11.0, 16 10.1, 20 10.8, 24 11.6; 16 of 256 in groups of eight: 5 keys 14.1 against 20.5, 12 19.4, 14 20.9.  By time
+// alone the line would be at 20, 16 and 12 keys for heads of 64, 128 and 256; it is where these positions have had the bits of the kernels for any shape).
 // The waves for a group's other heads come behind the chunks' blocks (a wave per head in every chunk, most of which leave again: 16
 // sequences of 3,000 keys, heads of 64, 30 -> 42 us).  The choice is the position's alone, so a query's bits do not depend on the step.
 template <int HDM>

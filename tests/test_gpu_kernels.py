@@ -1281,6 +1281,40 @@ def test_float32_attention_on_the_matrix_units_against_the_kernels_for_any_shape
         assert torch.allclose(a, b, rtol=2e-5, atol=2e-5), float((a - b).abs().max())
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("window,keep", [(0, 0), (50, 0), (130, 20), (300, 70)])
+def test_float32_prompt_queries_have_the_same_bits_wherever_items_start(hd, window, keep):
+    """Items that start at multiples of 64 and items that start anywhere give a query the same bits: tiles of 64 keys that all of a wave's rows
+    see whole, which go without masks, beside tiles that some rows see in part or not at all, and tiles left out between kept keys and the
+    window.  Against 64 bits: errors of sums of float32 products of up to `hd` and 512 terms."""
+    from ferrox_amd import ops
+    nh, nkv, n, bs = 4, 2, 512, 16
+    q, k, v = rnd(n, nh * hd), rnd(n, nkv, hd, seed=1), rnd(n, nkv, hd, seed=2)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    kp = k.view(n // bs, bs, nkv, hd).transpose(1, 2).contiguous()
+    vp = v.view(n // bs, bs, nkv, hd).permute(0, 2, 3, 1).contiguous()
+    pos, table = torch.arange(n, dtype=torch.int32, device=DEV), i32([list(range(n // bs))])
+    got = []
+    for edges in (list(range(0, n + 1, 64)), [0, 1, 6, 63, 66, 128, 145, 209, 257, 321, 380, 444, 508, 512]):
+        out = torch.zeros(n, nh * hd, device=DEV)
+        starts, sizes = edges[:-1], [b - a for a, b in zip(edges, edges[1:])]
+        ops.attention_tiles(q, out, kp, vp, table, pos, i32([0] * len(starts)), i32(starts), i32(sizes), nh, nkv, hd, bs, window,
+                            hd ** -0.5, keep_first=keep)
+        got.append(out)
+    assert torch.equal(got[0], got[1])
+    t = torch.arange(n, device=DEV)
+    sees = t[None] <= t[:, None]
+    if window:
+        sees &= (t[:, None] - t[None] < window) | (t[None] < keep)
+    qd, kd, vd = q.double().view(n, nh, hd), k.double().repeat_interleave(nh // nkv, 1), v.double().repeat_interleave(nh // nkv, 1)
+    for h in range(nh):
+        scores = (qd[:, h] @ kd[:, h].T * hd ** -0.5).masked_fill(~sees, -float("inf"))
+        want = torch.softmax(scores, -1) @ vd[:, h]
+        # a score's error, at most 2^-24 times a few of its roundings times |q||k| / sqrt(hd) < 2 sqrt(hd): 5e-6 of a probability, and
+        # as much again for the sums, times values below 6
+        assert float((got[0].view(n, nh, hd)[:, h].double() - want).abs().max()) < 6 * 1e-5
+
+
 @pytest.mark.parametrize("hd", [20, 64, 80, 132])
 def test_a_float32_key_at_minus_infinity_is_not_attended_to(hd):
     """A key whose last four numbers (the ones that stand in for numbers that a narrow head does not have) are minus infinity scores

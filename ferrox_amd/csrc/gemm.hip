@@ -1266,7 +1266,7 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
     static_assert(!ROPE || (NW == 2 && !DUAL && !NORM && EPI == EPI_STORE), "the rope epilogue pairs two sets of columns");
     static_assert(!NORM || (!DUAL && EPI == EPI_STORE), "the fused norm feeds a plain product");
-    static_assert(!WEIGHTS_FIRST || ROPE, "only the rope epilogue's operands have an order to choose");
+    static_assert(!WEIGHTS_FIRST || (ROPE && MT == 1), "only the rope epilogue's operands of one row tile have an order to choose");
     __shared__ float red_ss[NORM ? WAVES : 1][MT][64];
     float ss[MT];
 #pragma unroll
@@ -1425,7 +1425,7 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
     int sp = wave * VW * per;
     // Few accumulators leave registers for two pieces or more (see the loop below).  The first loads leave here,
     // and so do the old values that a block adds its product to: nothing of the epilogue waits for memory then.
-    constexpr bool TWO = MT * NW <= 4 && !NORM;
+    constexpr bool TWO = MT * NW <= (ROPE ? 8 : 4) && !NORM;
     uint4 w0[TWO ? DEPTH : 1][TWO ? NW : 1][WL], x0[TWO ? DEPTH : 1][TWO ? MT : 1][4];
     const bool deep = DEPTH > 2 && s_whole - sp >= DEPTH;
     auto first_pieces = [&]() {
@@ -1507,6 +1507,14 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
     }
     // rope epilogue: what thread (lane, wave) needs for its pairs of outputs, rows 16 mt + lane % 16, column
     // 4 (lane / 16) + wave of the two sets, is fetched and worked out here, while the weights are on their way
+    // More than two row tiles: what a row has of its own, its scale and its place in the pages, is found by one lane, asked for in front of the first weights and handed
+    // to the others in LDS (a lane that finds it for all of its rows reads eight sums for each: 64 rows of 2,048 k with sums 24.0 us, so 21.4; of two tiles 32 rows 15.8
+    // and 15.7, but without sums 14.3 and 15.3).
+    constexpr bool LANE_PER_ROW = ROPE && MT > 2;
+    __shared__ float row_scale_of[LANE_PER_ROW ? 16 * MT : 1];
+    __shared__ int row_place_of[LANE_PER_ROW ? 2 : 1][LANE_PER_ROW ? 16 * MT : 1];
+    float rstd_of_lane = 1.f;
+    int page_of_lane = 0, slot_of_lane = 0;
     float rope_sn[MT], rope_cs[MT], rope_rstd[MT], rope_b0 = 0.f, rope_b1 = 0.f;
     size_t rope_page[MT];
     int rope_slot[MT];
@@ -1516,11 +1524,23 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
         // first every load that depends on nothing, then the page ids, which need position and sequence
         int row_of[MT], pos[MT], seq[MT];
         float total[MT];
+        float squares_of_lane[8];
+        int pos_of_lane = 0, seq_of_lane = 0;
+        if constexpr (LANE_PER_ROW) {
+            const int row = min(r0 + min(lane, 16 * MT - 1), r_end - 1), n = g.row_ss ? g.row_ss_n : 1;
+            const float* ss = g.row_ss ? g.row_ss + (size_t)row * n : g.rope_inv_freq;      // (without sums the same load, not used)
+            pos_of_lane = g.rope_positions[row];
+            seq_of_lane = to_pages ? g.rope_token_seq[row] : 0;
+            if (n > 8) squares_of_lane[0] = sum_in_order(ss, n);
+            else
+#pragma unroll
+                for (int u = 0; u < 8; ++u) squares_of_lane[u] = ss[min(u, n - 1)];
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             row_of[mt] = min(r0 + 16 * mt + li, r_end - 1);
             pos[mt] = g.rope_positions[row_of[mt]];
-            seq[mt] = to_pages ? g.rope_token_seq[row_of[mt]] : 0;
+            if constexpr (!LANE_PER_ROW) seq[mt] = to_pages ? g.rope_token_seq[row_of[mt]] : 0;
         }
         // (without a bias the same loads read the positions instead: a branch around them would wait for them)
         const void* bias_or = g.bias ? g.bias : (const void*)g.rope_positions;
@@ -1544,6 +1564,17 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
 #pragma unroll
                 for (int u = 0; u < 8; ++u) total[mt] = u < g.row_ss_n ? total[mt] + squares[mt][u] : total[mt];
             }
+        } else if constexpr (LANE_PER_ROW) {
+            first_pieces();
+            float sum = squares_of_lane[0];
+            if (g.row_ss && g.row_ss_n <= 8) {
+                sum = 0.f;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum = u < g.row_ss_n ? sum + squares_of_lane[u] : sum;
+            }
+            rstd_of_lane = g.row_ss ? row_rstd(sum, g.K, g.norm_eps) : 1.f;
+            slot_of_lane = pos_of_lane % g.rope_bs;
+            if (to_pages) page_of_lane = g.rope_table[(size_t)seq_of_lane * g.rope_max_blocks + pos_of_lane / g.rope_bs];
         } else {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
@@ -1555,14 +1586,14 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
         for (int mt = 0; mt < MT; ++mt) {
             rope_page[mt] = 0;
             rope_slot[mt] = 0;
-            if (to_pages) {
+            if (!LANE_PER_ROW && to_pages) {
                 rope_page[mt] = (size_t)g.rope_table[(size_t)seq[mt] * g.rope_max_blocks + pos[mt] / g.rope_bs];
                 rope_slot[mt] = pos[mt] % g.rope_bs;
             }
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            rope_rstd[mt] = g.row_ss ? row_rstd(total[mt], g.K, g.norm_eps) : 1.f;
+            if constexpr (!LANE_PER_ROW) rope_rstd[mt] = g.row_ss ? row_rstd(total[mt], g.K, g.norm_eps) : 1.f;
             rope_sn[mt] = 0.f;
             rope_cs[mt] = 1.f;
             if (rope_rotated) {
@@ -1572,7 +1603,7 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
             }
         }
         // (what the epilogue needs first: behind the weights those short loads would wait for them)
-        if constexpr (!WEIGHTS_FIRST) first_pieces();
+        if constexpr (!WEIGHTS_FIRST && !LANE_PER_ROW) first_pieces();
     }
     // Few accumulators leave registers for two pieces: the loads of the next piece are then issued before the
     // products of this one, so a wave always has a piece on its way from memory.  Each product follows the
@@ -1641,6 +1672,13 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) red_ss[wave][mt][lane] = ss[mt];
     }
+    if constexpr (LANE_PER_ROW) {
+        if (wave == 0 && lane < 16 * MT) {
+            row_scale_of[lane] = rstd_of_lane;
+            row_place_of[0][lane] = page_of_lane;
+            row_place_of[1][lane] = slot_of_lane;
+        }
+    }
     __syncthreads();
     if constexpr (ROPE) {
         static_assert(!ROPE || WAVES == 4, "a wave per accumulator row");
@@ -1651,6 +1689,11 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
         for (int mt = 0; mt < MT; ++mt) {
             const int ml = r0 + 16 * mt + (L & 15);
             if (ml >= r_end) continue;
+            if constexpr (LANE_PER_ROW) {
+                rope_rstd[mt] = row_scale_of[16 * mt + (L & 15)];
+                rope_page[mt] = row_place_of[0][16 * mt + (L & 15)];
+                rope_slot[mt] = row_place_of[1][16 * mt + (L & 15)];
+            }
             f32x4_t v0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, v1 = v0;
 #pragma unroll
             for (int w = 0; w < PARTS; ++w) {
@@ -2693,6 +2736,19 @@ static void launch_skinny(const GemmArgs& g, int epi, int mt, int nw, int waves,
 // 6.7; sums of two batches, 3,584 k, 2 rows 12.0 12.7, 17 rows 16.8 18.0; two row tiles of 2,048 k with sums 13.1 13.5).
 FX_API int fx_qkv_rope_weights_first(int M, int K, int sums) { return M <= 16 && sums >= 1 && sums <= 8 && (K > 1024 || (long)M * K >= 16384); }
 
+// Row tiles of 16 a block of the rotating product takes: the fewest with which its blocks are one round of the CUs, or else all rows' (a block fetches the operands of its row
+// tiles itself and finds weights that another block has fetched in the cache; what takes the time is the CU with the most blocks).  us with sums, 1 / 2 / 3 or 4 tiles a block:
+//   48 groups of columns (1,024 k)    32 rows 8.5 9.5, 48 rows 8.6 9.2 11.2, 64 rows 8.6 9.4 12.5
+//   144 (3,584 k)    24 rows 24.0 18.1, 48 rows 27.7 29.8 23.9, 64 rows 37.9 32.3 28.6
+//   192 (2,048 k)    24 rows 18.0 14.8, 33 rows 23.3 20.0 16.3, 48 rows 26.2 21.9 18.3, 64 rows 27.3 23.1 21.4     192 (4,096 k)    48 rows 42.6 35.4 26.3, 64 rows 44.6 37.5 31.2
+// (Two tiles a block from 17 rows on, as it was, with sums found by every lane: 64 rows of the four 10.5, 35.2, 25.8 and 39.5.)  The same bits whatever the tiles.
+FX_API int fx_qkv_rope_row_tiles(int M, int groups, int cus) {
+    const int tiles = ceil_div(M, 16);
+    for (int mt = 1; mt < tiles; ++mt)
+        if ((long)groups * ceil_div(tiles, mt) <= cus) return mt;
+    return tiles;
+}
+
 // The q/k/v product of up to 64 tokens with the rotation and the cache write in its epilogue (see GemmArgs):
 // bfloat16, C [M, (nh + 2 nkv) hd], bias [N] or null, row_ss as in fx_gemm.  head_dim and the rotary dimension
 // are multiples of 32.  k_pages [pages][nkv][bs][hd] and v_pages [pages][nkv][hd][bs], or both null.
@@ -2722,17 +2778,15 @@ FX_API int fx_qkv_rope(void* stream, const void* A, long lda, const void* W, lon
     g.rope_inv_freq = inv_freq ? inv_freq : (const float*)positions;      // (rot == 0: read, never used)
     g.rope_freq_factors = freq_factors;
     dim3 grid((nh + 2 * nkv) * (hd / 32), 1);
+    const int mt = fx_qkv_rope_row_tiles(M, (int)grid.x, fx_compute_units());
+    grid.y = ceil_div(M, 16 * mt);
+    hipStream_t s = (hipStream_t)stream;
     if (row_ss && fx_qkv_rope_weights_first(M, K, row_ss_n))
-        gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true, false, 2, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
-    else if (M <= 16) gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
-    else if (M <= 32) gemm_bf16_skinny_kernel<2, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
-    else {
-        // 33..64 rows: two blocks of 32 rows a column group rather than one of 64 (a wave fetches the operands of
-        // every row tile of its block itself: a decode step at 64 sequences 11.03 -> 10.94 ms; the second block
-        // finds the weights in the cache); the same bits
-        grid.y = 2;
-        gemm_bf16_skinny_kernel<2, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, (hipStream_t)stream>>>(g);
-    }
+        gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true, false, 2, true><<<grid, 256, 0, s>>>(g);
+    else if (mt == 1) gemm_bf16_skinny_kernel<1, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, s>>>(g);
+    else if (mt == 2) gemm_bf16_skinny_kernel<2, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, s>>>(g);
+    else if (mt == 3) gemm_bf16_skinny_kernel<3, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, s>>>(g);
+    else gemm_bf16_skinny_kernel<4, 4, 2, false, EPI_STORE, false, true><<<grid, 256, 0, s>>>(g);
     FX_CHECK_LAUNCH("qkv_rope");
     return 0;
 }

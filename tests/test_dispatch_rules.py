@@ -114,6 +114,16 @@ def test_weights_of_the_rotating_product_leave_first_with_sums_of_one_batch_and_
     assert not rule(16, 2048, 0) and not rule(16, 2056) and not rule(16, 3584) and rule(16, 3584, 8)
 
 
+def test_row_tiles_of_the_rotating_product():
+    """The fewest row tiles a block that keep its blocks within one round of the CUs, or else one block for all rows."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, groups, cus=256: load_library("gemm").fx_qkv_rope_row_tiles(m, groups, cus)
+    assert [rule(m, 192) for m in (1, 16, 17, 32, 33, 48, 49, 64)] == [1, 1, 2, 2, 3, 3, 4, 4]
+    assert [rule(m, 128) for m in (16, 17, 32, 33, 48, 49, 64)] == [1, 1, 1, 2, 2, 2, 2]
+    assert [rule(m, 64) for m in (17, 33, 49, 64)] == [1, 1, 1, 1] and [rule(m, 85) for m in (33, 48, 49, 64)] == [1, 1, 2, 2]
+    assert rule(64, 192, 1024) == 1 and rule(64, 300) == 4 and rule(16, 300) == 1
+
+
 def test_a_block_per_row_tile_while_such_blocks_are_one_a_cu():
     """The product of 33 to 128 plain rows: beyond 64 rows a second round of blocks is behind two row tiles a block."""
     from ferrox_amd.csrc.build import load_library

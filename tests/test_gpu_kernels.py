@@ -940,6 +940,19 @@ def test_qkv_product_that_rotates_and_writes_the_cache(later, T, H, nh, nkv, hd,
     assert not ops.can_qkv_rope(x, w, 65, hd, rot, False) and not ops.can_qkv_rope(x, w, T, hd, rot, True)
 
 
+@pytest.mark.parametrize("later", [False, True])
+@pytest.mark.parametrize("T", [33, 47, 48, 49, 63])
+@pytest.mark.parametrize("H,nh,tiles", [(264, 32, (3, 4)), (2312, 32, (3, 4)), (520, 4, (1, 1))])
+def test_rotating_product_of_several_row_tiles_a_block(later, T, H, nh, tiles):
+    """One, three and four row tiles a block, with rows of the last tile missing, K that ends in a piece, sums of up to eight and of ten numbers."""
+    from ferrox_amd import ops
+    from ferrox_amd.csrc.build import load_library
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    groups = (nh + 4) * 4
+    assert load_library("gemm").fx_qkv_rope_row_tiles(T, groups, cus) == tiles[T > 48] or cus != 256
+    test_qkv_product_that_rotates_and_writes_the_cache(later, T, H, nh, 2, 128, 16, 64, True)
+
+
 @pytest.mark.parametrize("T,H", [(16, 1032), (13, 1384), (9, 2000), (16, 2048), (1, 1032), (3, 2000), (16, 1024)])
 def test_rotating_product_whose_weights_leave_before_the_sums(T, H):
     """Sums of one batch and rows enough for it, K with and without a last part of a piece: the bits of the product and the rotation."""

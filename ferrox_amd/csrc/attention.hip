@@ -116,11 +116,12 @@ __device__ __forceinline__ BiasRow fetch_bias(const AttnArgs& a, int h, int dist
 // sequence (0: none).  Pages of other keys may have been given back.
 struct KeySpan {
     int begin, end, keep;
-    __device__ __forceinline__ bool has(int t) const { return t < end && (t >= begin || t < keep); }
+    // (`&` and `|`: with `&&` and `||` each comparison becomes a branch, 35 ns where it is taken)
+    __device__ __forceinline__ bool has(int t) const { return (t < end) & ((t >= begin) | (t < keep)); }
     // whether any of the n consecutive keys from t on is one of them
-    __device__ __forceinline__ bool touches(int t, int n) const { return t < end && (t + n > begin || t < keep); }
+    __device__ __forceinline__ bool touches(int t, int n) const { return (t < end) & ((t + n > begin) | (t < keep)); }
     // whether all of the 64 keys of the tile at t are
-    __device__ __forceinline__ bool holds_tile(int t) const { return t >= begin && t + 64 <= end; }
+    __device__ __forceinline__ bool holds_tile(int t) const { return (t >= begin) & (t + 64 <= end); }
 };
 // The tiles of 64 keys that a block walks over, in ascending order: those that hold kept first keys and lie
 // before the first tile of the span's stretch [begin, end), then that stretch's tiles.
@@ -213,6 +214,35 @@ struct PageLookup {
         return i < (unsigned)count ? copy[i] : table[blk];
     }
 };
+// Pages and slots of N keys: one branch for how a page's number is found and one for where its entry is (every lane takes part), not one a key (decode attention, a tile a wave,
+// us one a key / so: 16 heads of 128, one sequence of 2,060 keys 12.8 11.8, 8 30.6 29.4; 28 heads on 4, 8 sequences 17.0 15.9).
+template <int N>
+__device__ __forceinline__ void pages_of(const AttnArgs& a, const PageLookup& pl, const int (&key)[N], int (&page)[N], int (&slot)[N]) {
+    int blk[N];
+    if (a.bs_shift >= 0) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            blk[i] = key[i] >> a.bs_shift;
+            slot[i] = key[i] & (a.bs - 1);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            blk[i] = key[i] / a.bs;
+            slot[i] = key[i] - blk[i] * a.bs;
+        }
+    }
+    unsigned farthest = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) farthest = max(farthest, (unsigned)(blk[i] - pl.first));
+    if (pl.copy && __all(farthest < (unsigned)pl.count)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) page[i] = pl.copy[blk[i] - pl.first];
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) page[i] = pl.page(blk[i]);
+    }
+}
 // every thread of the block calls this; blocks [first_blk, last_blk] of the table are wanted
 __device__ __forceinline__ PageLookup stage_pages(const int* table, int* lds, int first_blk, int last_blk) {
     PageLookup pl;
@@ -609,7 +639,7 @@ __device__ __forceinline__ float softmax_step(f32x4_t (&sc)[4], int key0, int lo
         for (int r = 0; r < 4; ++r) {
             if (MASKED) {
                 const int key = key0 + 4 * kb + r;
-                sc[kb][r] = ((key >= lo || key < keep) && key <= hi) ? sc[kb][r] : NEG_INF;
+                sc[kb][r] = (((key >= lo) | (key < keep)) & (key <= hi)) ? sc[kb][r] : NEG_INF;
             }
             mt = fmaxf(mt, sc[kb][r]);
         }
@@ -711,32 +741,26 @@ struct WaveAttn {
         const bool edge = !span.holds_tile(kt0);      // some key of the tile is outside
         const bool vlive = span.touches(kg, 16);
         const int vkey = vlive ? kg : safe_group;
-        int vblk, vslot;
-        page_slot(a, vkey, vblk, vslot);
         // every page id of the tile is looked up before the first load leaves: a lookup that stands between two
         // groups of loads makes the second group wait for the first
-        const int vpage = pl.page(vblk);
-        int kpage[4], kslots[4];
-        bool klives[4];
         constexpr int KP = KS & ~1;      // k-steps that are loaded in pairs, whole lines of eight keys at a time
-        int kpage_a[4], kslots_a[4], kpage_b[4], kslots_b[4];
+        constexpr int NP = KP < KS ? 13 : 9;
+        int key_of[NP], page_of[NP], slot_of[NP];
+        bool klives[4];
+        key_of[0] = vkey;
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
             const int key0 = kt0 + 16 * (li >> 2) + 4 * kb + (li & 3);
             klives[kb] = span.has(key0);
-            int kblk;
-            if (KP < KS) {
-                page_slot(a, klives[kb] ? key0 : safe_group, kblk, kslots[kb]);
-                kpage[kb] = pl.page(kblk);
-            }
             // rows li % 8 and 8 + li % 8 of the block's 16 keys (row i is key 16 (i / 4) + 4 kb + i % 4 of the tile)
             const int key_a = kt0 + 16 * (l8 >> 2) + 4 * kb + (l8 & 3), key_b = key_a + 32;
-            page_slot(a, span.has(key_a) ? key_a : safe_group, kblk, kslots_a[kb]);
-            kpage_a[kb] = pl.page(kblk);
-            page_slot(a, span.has(key_b) ? key_b : safe_group, kblk, kslots_b[kb]);
-            kpage_b[kb] = pl.page(kblk);
+            key_of[1 + kb] = span.has(key_a) ? key_a : safe_group;
+            key_of[5 + kb] = span.has(key_b) ? key_b : safe_group;
+            if constexpr (KP < KS) key_of[9 + kb] = klives[kb] ? key0 : safe_group;
         }
-        const bf16* vbase = (const bf16*)a.v_pages + ((size_t)vpage * a.nkv + kvh) * vd * bs + vslot;
+        pages_of(a, pl, key_of, page_of, slot_of);
+        const int *kpage_a = page_of + 1, *kslots_a = slot_of + 1, *kpage_b = page_of + 5, *kslots_b = slot_of + 5;
+        const bf16* vbase = (const bf16*)a.v_pages + ((size_t)page_of[0] * a.nkv + kvh) * vd * bs + slot_of[0];
         uint4 vv[EARLY_V ? CB : 1][2];
         const uint32_t vmask = opaque_mask(vlive);
         if (EARLY_V) {
@@ -763,7 +787,7 @@ struct WaveAttn {
                 kf[kb][u + 1] = load_lines16(krb + (d < hd ? d : 0));
             }
             if (KP < KS) {
-                const bf16* kr = (const bf16*)a.k_pages + (((size_t)kpage[kb] * a.nkv + kvh) * bs + kslots[kb]) * hd;
+                const bf16* kr = (const bf16*)a.k_pages + (((size_t)page_of[NP - 4 + kb] * a.nkv + kvh) * bs + slot_of[NP - 4 + kb]) * hd;
                 const uint32_t kmask = opaque_mask(klives[kb]);
 #pragma unroll
                 for (int u = KP; u < KS; ++u) {
@@ -795,7 +819,7 @@ struct WaveAttn {
         // Heads too wide for their values to be fetched before the scores: the values arrive in groups of VG column
         // blocks, a group's loads issued together and a group ahead of the products that use them (the first one before
         // the softmax), so that a tile waits for memory CB / VG times and not once per column block.
-        constexpr int VG = CB < 4 ? CB : 4;
+        constexpr int VG = CB < 4 ? CB : (EARLY_V ? 4 : 8);      // (wide heads, groups of four / eight: 8 sequences of 2,060 latent keys 18.1 / 17.5 us, 64 41.1 / 38.7)
         uint4 ahead[EARLY_V ? 1 : VG][2];
         auto fetch_values = [&](int c0) {
 #pragma unroll
@@ -916,9 +940,9 @@ struct F32Attention {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const int k = kt0 + 16 * c + li, v = kt0 + 16 * c + 4 * g;
-                t[c] = (k < span.end) & ((k >= span.begin) | (k < span.keep)) ? k : safe;
+                t[c] = span.has(k) ? k : safe;
                 // (four keys of one page: the page is there if any of them is in the span)
-                t[4 + c] = (v < span.end) & ((v + 4 > span.begin) | (v < span.keep)) ? v : safe & ~3;
+                t[4 + c] = span.touches(v, 4) ? v : safe & ~3;
             }
             int (&slot)[8] = page_slots;
             if (a.bs_shift >= 0) {
@@ -1006,7 +1030,7 @@ struct F32Attention {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int t = kt0 + 16 * c + 4 * g + r;
-                        s[c][r] = (t <= to) & ((t >= from) | (t < a.keep_first)) ? s[c][r] : NEG_INF;
+                        s[c][r] = ((t <= to) & ((t >= from) | (t < a.keep_first))) ? s[c][r] : NEG_INF;
                     }
             }
             float top = NEG_INF;
@@ -1031,10 +1055,7 @@ struct F32Attention {
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int t = kt0 + 16 * c + 4 * g + r;
-                        inside |= ((t < span.end) & ((t >= span.begin) | (t < span.keep)) ? 1 : 0) << (4 * c + r);
-                    }
+                    for (int r = 0; r < 4; ++r) inside |= (span.has(kt0 + 16 * c + 4 * g + r) ? 1 : 0) << (4 * c + r);
             }
 #pragma unroll
             for (int pair = 0; pair < (NC + 1) / 2; ++pair) {
@@ -1246,32 +1267,63 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
     }
     if (n_waves == 1) {
         // one wave: nothing to merge, the rows go out from the registers that hold them (lane (li, g) has rows
-        // 4g .. 4g + 3 of columns 16 cb + li; a row's maximum and sum sit in the lanes whose li is the row)
+        // 4g .. 4g + 3 of columns 16 cb + li; a row's maximum and sum sit in the lanes whose li is the row).  Without gate and turns through a buffer whose end drops the
+        // columns past the value head and the rows past the group: a block's only tile is little longer than this end of it, and with a branch around each of the stores
+        // (and two more inside) 40 keys of 16 heads on one kv head of
+        // 256 took 14.3 us, so 11.0 (8 sequences of 2,060 keys 17.5 and 16.3; 28 heads of 128 on 4, 40 keys 8.7 and 6.9).
+        constexpr int CB = WaveAttn<HD, SHAPE>::CB, OUTSIDE = 1 << 30;
+        const int vd = a.vd;
+        const bool parts = a.splits > 1;
+        if (parts || !(a.gate || a.turns)) {
+            const size_t first = parts ? (((size_t)item * a.nh + h0) * a.splits + split) * vd : (size_t)tok * a.ldo + (size_t)h0 * vd;
+            const int row_len = parts ? a.splits * vd : vd, size = parts ? 4 : 2;
+            const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(parts ? (void*)(a.part_o + first) : (void*)((bf16*)a.out + first), 0, ((n - 1) * row_len + vd) * size, 0x00027000);
+            float m[4], l[4];
+            int at[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                m[r] = __shfl(w.m, 4 * g + r, 64);
+                l[r] = __shfl(w.l, 4 * g + r, 64);
+                at[r] = 4 * g + r < n ? (4 * g + r) * row_len * size : OUTSIDE;
+            }
+            if (parts) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    const int column = 16 * cb + li < vd ? 4 * (16 * cb + li) : OUTSIDE;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m[r] == NEG_INF ? 0.f : w.o[cb][r]), to, at[r] + column, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (li == 0 && 4 * g + r < n) {
+                        float* pml = a.part_ml + (((size_t)item * a.nh + h0 + 4 * g + r) * a.splits + split) * 2;
+                        pml[0] = m[r] == NEG_INF ? NEG_INF : m[r] * LN2;
+                        pml[1] = m[r] == NEG_INF ? 0.f : l[r];
+                    }
+                return;
+            }
+            float fin[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) fin[r] = finish_row<true>(a, h0 + min(4 * g + r, n - 1), m[r], l[r]);
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                const int column = 16 * cb + li < vd ? 2 * (16 * cb + li) : OUTSIDE;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, float_to_bf16(w.o[cb][r] * fin[r])), to, at[r] + column, 0, 0);
+            }
+            return;
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = 4 * g + r;
             const float m = __shfl(w.m, row, 64), l = __shfl(w.l, row, 64);
             if (row >= n) continue;
             const int h = h0 + row;
-            if (a.splits == 1) {
-                const float fin = finish_row<true>(a, h, m, l);
+            const float fin = finish_row<true>(a, h, m, l);
 #pragma unroll
-                for (int cb = 0; cb < WaveAttn<HD, SHAPE>::CB; ++cb) {
-                    const int d = 16 * cb + li;
-                    if (d < a.vd) store_lane<bf16>(a, tok, h, d, w.o[cb][r] * fin);
-                }
-            } else {
-                float* po = a.part_o + (((size_t)item * a.nh + h) * a.splits + split) * a.vd;
-#pragma unroll
-                for (int cb = 0; cb < WaveAttn<HD, SHAPE>::CB; ++cb) {
-                    const int d = 16 * cb + li;
-                    if (d < a.vd) po[d] = m == NEG_INF ? 0.f : w.o[cb][r];
-                }
-                if (li == 0) {
-                    float* pml = a.part_ml + (((size_t)item * a.nh + h) * a.splits + split) * 2;
-                    pml[0] = m == NEG_INF ? NEG_INF : m * LN2;
-                    pml[1] = m == NEG_INF ? 0.f : l;
-                }
+            for (int cb = 0; cb < CB; ++cb) {
+                const int d = 16 * cb + li;
+                if (d < vd) store_lane<bf16>(a, tok, h, d, w.o[cb][r] * fin);
             }
         }
         return;

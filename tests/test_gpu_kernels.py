@@ -1923,3 +1923,39 @@ def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2
     assert not ops.can_pair(first, ops.Product(y[:, 1:], w2[:, 1:], one, epi2)) and not ops.can_pair(first, ops.Product(y.float(), w2.float(), one, epi2))
     with pytest.raises(ops.KernelError):
         ops.gemm_pair(first, ops.Product(y, w2, h0, ops.EPI_RESID))
+
+
+@pytest.mark.parametrize("nh,nkv,hd,vd", [(5, 1, 64, 64), (16, 1, 256, 192), (34, 2, 64, 40), (7, 7, 128, 72), (28, 4, 128, 128), (16, 1, 256, 200)])
+@pytest.mark.parametrize("bs", [64, 16])
+def test_single_queries_of_one_wave_write_their_rows_and_columns_only(nh, nkv, hd, vd, bs):
+    """Blocks of one wave store through a buffer whose end drops what a block does not have: heads beyond the group, columns beyond the
+    value head, in outputs and in parts of several chunks.  Whatever stands around the outputs stays.  Probabilities and values are
+    rounded to bfloat16, and so is the output: 3 x 2^-9 of the largest value."""
+    from ferrox_amd import ops
+    lens = [1, 40, 64, 150]
+    blocks = [-(-n // bs) for n in lens]
+    g = torch.Generator().manual_seed(3)
+    ids = torch.randperm(sum(blocks) + 2, generator=g)
+    kp = rnd(len(ids), nkv, bs, hd, dtype=torch.bfloat16)
+    vp = rnd(len(ids), nkv, vd, bs, dtype=torch.bfloat16, seed=1)
+    table, used = torch.zeros(len(lens), max(blocks), dtype=torch.int32), 0
+    for s, n in enumerate(blocks):
+        table[s, :n] = ids[used:used + n].to(torch.int32)
+        used += n
+    q = rnd(len(lens), nh * hd, dtype=torch.bfloat16, seed=2)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    for most in (64, 150):      # keys: one chunk of 64, whose block writes the output, and three, whose blocks write parts
+        around = torch.full((len(lens) + 2, nh * vd + 16), 7.0, dtype=torch.bfloat16, device=DEV)
+        out = around[1:-1, 8:-8]
+        ops.attention_decode(q, out, kp, vp, table.to(DEV), i32([min(n, most) - 1 for n in lens]), i32([0, 1, 2, 3]), i32([0, 1, 2, 3]), nh, nkv, hd,
+                             bs, 0, hd ** -0.5, max_kv_len=most, chunk=64, v_dim=vd)
+        edge = around.clone()
+        edge[1:-1, 8:-8] = 7.0
+        assert bool((edge == 7.0).all())
+        for s, n in enumerate(lens):
+            n = min(n, most)
+            k = kp[table[s].long().to(DEV)].transpose(1, 2).reshape(-1, nkv, hd)[:n].double().repeat_interleave(nh // nkv, 1)
+            v = vp[table[s].long().to(DEV)].permute(0, 3, 1, 2).reshape(-1, nkv, vd)[:n].double().repeat_interleave(nh // nkv, 1)
+            p = torch.softmax((q[s].double().view(nh, 1, hd) * k.transpose(0, 1)).sum(-1) * hd ** -0.5, -1)
+            want = (p[..., None] * v.transpose(0, 1)).sum(1)
+            assert float((out[s].reshape(nh, vd).double() - want).abs().max()) <= 3 * 2 ** -9 * float(v.abs().max()), (s, most)

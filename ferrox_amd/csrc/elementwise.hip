@@ -325,6 +325,99 @@ FX_API int fx_rmsnorm(void* stream, int out_dtype, const float* h, const int* ro
 // [page][kv_head][value head size][slot], which is what the attention kernels read (a value head's size vd
 // may differ from head_dim, the size of a query and key head).
 // ---------------------------------------------------------------------------
+// Values of many tokens into their transposed pages: a block takes 64 tokens and 4 G pieces of G dimensions of the token's kv heads (G elements: 16 bytes), a thread G tokens of a
+// piece: one 16-byte load a token, G x G elements turned in registers, one 16-byte store a dimension, which with its neighbours' makes a whole line of a page.  The G tokens are those that
+// start at a multiple of G in a page, wherever that is in the step (behind decoded sequences a prompt starts at any token); tokens without G - 1 others go out element by element.
+// us, eight tokens of a head a block with a 2-byte load an element / so, rotation of q and k included: 16 heads of 128 in bfloat16, 1,024 tokens 8.5 / 7.0, 2,048 13.9 / 11.1, 2,048 behind
+// 15 decoded 27.1 / 13.8, 4,096 behind 7 50.6 / 20.9, in float32 700 13.9 / 9.3, 2,048 33.5 / 19.1.
+template <typename T>
+__device__ __forceinline__ void write_many_values(int b, const T* __restrict__ v, int ldv, const int* __restrict__ positions,
+                                                  const int* __restrict__ token_seq, const int* __restrict__ block_table,
+                                                  int max_blocks, T* __restrict__ v_pages, int n_tokens, int nkv, int bs, int vd) {
+    constexpr int G = 16 / sizeof(T), GROUPS = 64 / G, PIECES = 256 / GROUPS, NEAR = 8, N = 64 + 2 * NEAR;
+    __shared__ int pos_of[N], seq_of[N], leads[N];
+    const int tid = threadIdx.x, j = tid % GROUPS;
+    const int head_pieces = vd / G, window_blocks = (nkv * head_pieces + PIECES - 1) / PIECES;
+    const int t0 = b / window_blocks * 64, piece = b % window_blocks * PIECES + tid / GROUPS;
+    if (tid < N) {
+        const int t = t0 - NEAR + tid;
+        const bool there = (t >= 0) & (t < n_tokens);
+        const int at = min(max(t, 0), n_tokens - 1), pos = positions[at], seq = token_seq[at];
+        pos_of[tid] = there ? pos : -1;
+        seq_of[tid] = there ? seq : -1;
+    }
+    __syncthreads();
+    if (tid < N) {      // whether G tokens of one page start here
+        bool lead = (tid + G <= N) & (pos_of[tid] >= 0) & (pos_of[tid] % G == 0);
+#pragma unroll
+        for (int i = 1; i < G; ++i) {
+            const int k = min(tid + i, N - 1);
+            lead = lead & (pos_of[k] == pos_of[tid] + i) & (seq_of[k] == seq_of[tid]);
+        }
+        leads[tid] = lead;
+    }
+    __syncthreads();
+    if (piece >= nkv * head_pieces) return;
+    const int kh = piece / head_pieces, d0 = (piece - kh * head_pieces) * G;
+    const T* from = v + (size_t)kh * vd + d0;
+    int first = -1, alone = 0;      // the group that starts among the thread's G tokens; a bit for each of them that belongs to none
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+        const int at = NEAR + j * G + u, pos = pos_of[at];
+        if (leads[at]) first = at;
+        alone |= ((pos >= 0) & !leads[at - (pos & (G - 1))]) << u;
+    }
+    if (first >= 0) {
+        const int pos = pos_of[first], page = block_table[(size_t)seq_of[first] * max_blocks + pos / bs];
+        const T* src = from + (size_t)(t0 - NEAR + first) * ldv;
+        T* dst = v_pages + (((size_t)page * nkv + kh) * vd + d0) * bs + pos % bs;
+        uint4 row[G];
+#pragma unroll
+        for (int i = 0; i < G; ++i) row[i] = *(const uint4*)(src + (size_t)i * ldv);
+        auto word = [&](int i, int w) { return w == 0 ? row[i].x : w == 1 ? row[i].y : w == 2 ? row[i].z : row[i].w; };
+#pragma unroll
+        for (int d = 0; d < G; ++d) {
+            uint32_t o[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if constexpr (sizeof(T) == 4) {
+                    o[w] = word(w, d);
+                } else {
+                    const uint32_t lo = word(2 * w, d / 2), hi = word(2 * w + 1, d / 2);
+                    o[w] = d & 1 ? (lo >> 16) | (hi & 0xffff0000u) : (lo & 0xffffu) | (hi << 16);
+                }
+            }
+            *(uint4*)(dst + (size_t)d * bs) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+    }
+    while (alone) {      // four at a time (where fewer are left, the last of them again)
+        T* dst[4];
+        uint4 own[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int at = NEAR + j * G + __ffs(alone) - 1, pos = pos_of[at];
+            dst[i] = v_pages + (((size_t)block_table[(size_t)seq_of[at] * max_blocks + pos / bs] * nkv + kh) * vd + d0) * bs + pos % bs;
+            own[i] = *(const uint4*)(from + (size_t)(t0 - NEAR + at) * ldv);
+            const int rest = alone & (alone - 1);
+            alone = rest || i == 3 ? rest : alone;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            T e[G];
+            __builtin_memcpy(e, &own[i], 16);
+#pragma unroll
+            for (int d = 0; d < G; ++d) dst[i][(size_t)d * bs] = e[d];
+        }
+    }
+}
+// How many blocks that takes, or 0 where its 16-byte pieces do not fit or the step has fewer than two million bfloat16 or half a million float32 values: its two looks at the tokens around
+// come before its first load (us, eight tokens a block / 64: 512 tokens of 16 heads of 128 5.7 / 5.9, 700 7.2 / 7.8; float32, 128 decoded 7.6 / 8.7, 300 8.0 / 6.4).
+static long many_value_blocks(long T, int nkv, int vd, int bs, int dtype, const void* v, long ldv, const void* v_pages) {
+    const int G = dtype == FX_F32 ? 4 : 8;
+    if (T * nkv * vd < (dtype == FX_F32 ? 1L << 19 : 1L << 21) || bs % G || vd % G || ldv % G || (((uintptr_t)v | (uintptr_t)v_pages) % 16)) return 0;
+    return (T + 63) / 64 * (((long)nkv * (vd / G) + 4 * G - 1) / (4 * G));
+}
+
 // Values into their transposed pages: block b of ceil(T / 8) * nkv takes eight consecutive tokens of one kv head, so
 // that eight tokens that follow each other in one page go out as one 16-byte store per head dimension.
 template <typename T>
@@ -365,14 +458,15 @@ __device__ __forceinline__ void write_values(int b, const T* __restrict__ v, int
 // and cosines once and takes its part of the heads of q (in place) and of k (into its page); few
 // tokens get several blocks each, many tokens one.  The blocks after them write v: one block per (eight
 // consecutive tokens, kv head), so that eight tokens that follow each other in one page go out as
-// one 16-byte store per head dimension into the transposed page.
+// one 16-byte store per head dimension into the transposed page, or `write_many_values`.  (Eight blocks a CU: with the registers
+// of the values' part a rotating block of 2,048 tokens would have seven beside it.)
 template <typename T>
-__global__ __launch_bounds__(256) void rope_kv_write_kernel(
+__global__ __launch_bounds__(256, 8) void rope_kv_write_kernel(
     T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk, const T* __restrict__ v, int ldv,
     const int* __restrict__ positions, const int* __restrict__ token_seq,
     const int* __restrict__ block_table, int max_blocks, T* __restrict__ k_pages, T* __restrict__ v_pages,
     int n_tokens, int split, int nh, int nkv, int hd, int bs, int rot, int interleaved, const float* __restrict__ inv_freq, int vec8,
-    const float* __restrict__ freq_factors, int vd) {
+    const float* __restrict__ freq_factors, int vd, int many) {
     __shared__ float cs[128], sn[128];     // rot / 2 <= 128
     const int tid = threadIdx.x;
     const int half = rot >> 1;
@@ -441,7 +535,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
         return;
     }
     if (!v_pages) return;
-    write_values<T>(blockIdx.x - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
+    if (many) write_many_values<T>(blockIdx.x - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
+    else write_values<T>(blockIdx.x - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
 }
 
 FX_API int fx_rope_kv_write(void* stream, int dtype, void* q, int ldq, const void* k, int ldk,
@@ -458,7 +553,8 @@ FX_API int fx_rope_kv_write(void* stream, int dtype, void* q, int ldq, const voi
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const int split = T <= 32 ? 8 : (T <= 128 ? 2 : 1);
-    const long n_blocks = (long)T * split + (v_pages ? (long)((T + 7) / 8) * nkv : 0);
+    const long many = v_pages ? many_value_blocks(T, nkv, vd, bs, dtype, v, ldv, v_pages) : 0;
+    const long n_blocks = (long)T * split + (many ? many : v_pages ? (long)((T + 7) / 8) * nkv : 0);
     FX_REQUIRE(n_blocks < (1L << 31), "rope_kv_write: too many tokens and heads for one launch");
     const unsigned blocks = (unsigned)n_blocks;
     const int vec8 = dtype == FX_BF16 && !interleaved && rot % 16 == 0 && hd % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 &&
@@ -467,12 +563,12 @@ FX_API int fx_rope_kv_write(void* stream, int dtype, void* q, int ldq, const voi
         rope_kv_write_kernel<float><<<blocks, 256, 0, s>>>((float*)q, ldq, (const float*)k, ldk, (const float*)v, ldv,
                                                            positions, token_seq, block_table, max_blocks,
                                                            (float*)k_pages, (float*)v_pages, T, split, nh, nkv, hd, bs, rot,
-                                                           interleaved, inv_freq, 0, freq_factors, vd);
+                                                           interleaved, inv_freq, 0, freq_factors, vd, many > 0);
     else if (dtype == FX_BF16)
         rope_kv_write_kernel<bf16><<<blocks, 256, 0, s>>>((bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv,
                                                           positions, token_seq, block_table, max_blocks,
                                                           (bf16*)k_pages, (bf16*)v_pages, T, split, nh, nkv, hd, bs, rot,
-                                                          interleaved, inv_freq, vec8, freq_factors, vd);
+                                                          interleaved, inv_freq, vec8, freq_factors, vd, many > 0);
     else
         return fx_fail("rope_kv_write: unknown dtype %d", dtype);
     FX_CHECK_LAUNCH("rope_kv_write");

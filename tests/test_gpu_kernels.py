@@ -1959,3 +1959,30 @@ def test_single_queries_of_one_wave_write_their_rows_and_columns_only(nh, nkv, h
             p = torch.softmax((q[s].double().view(nh, 1, hd) * k.transpose(0, 1)).sum(-1) * hd ** -0.5, -1)
             want = (p[..., None] * v.transpose(0, 1)).sum(1)
             assert float((out[s].reshape(nh, vd).double() - want).abs().max()) <= 3 * 2 ** -9 * float(v.abs().max()), (s, most)
+
+
+@pytest.mark.parametrize("dtype,decoded,prompts", [(torch.bfloat16, 0, [1030]), (torch.bfloat16, 13, [700, 0, 345]), (torch.bfloat16, 1024, []),
+                                                   (torch.float32, 0, [260]), (torch.float32, 6, [131, 3, 140])])
+@pytest.mark.parametrize("nkv,vd,bs", [(16, 128, 64), (11, 192, 16), (16, 136, 20), (8, 264, 24)])
+def test_values_of_many_tokens_go_to_their_places(dtype, decoded, prompts, nkv, vd, bs):
+    """A step whose values go out in windows of 64 tokens: prompts that start at any token and any slot of a page, sequences of single
+    tokens, pages that hold a whole number of 16-byte pieces and (20) such that do not.  Every value is where its position says, and nothing else is written."""
+    from ferrox_amd import ops
+    starts = [5 * i % 61 for i in range(decoded)] + [37 * i for i in range(len(prompts))]
+    lens = [1] * decoded + prompts
+    seqs = [s for s, n in enumerate(lens) for _ in range(n)]
+    poss = [starts[s] + i for s, n in enumerate(lens) for i in range(n)]
+    T, per = len(seqs), max(poss) // bs + 1
+    assert T * nkv * vd >= (1 << 21 if dtype == torch.bfloat16 else 1 << 19)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table = torch.randperm(len(lens) * per, generator=torch.Generator().manual_seed(1)).to(torch.int32).view(len(lens), per).to(DEV)
+    hd = 32
+    buf = rnd(T, 2 * nkv * hd + nkv * vd, dtype=dtype)
+    q, k, v = buf[:, :nkv * hd], buf[:, nkv * hd:2 * nkv * hd], buf[:, 2 * nkv * hd:]
+    k_pages = torch.zeros(len(lens) * per, nkv, bs, hd, dtype=dtype, device=DEV)
+    v_pages = torch.full((len(lens) * per, nkv, vd, bs), 9.0, dtype=dtype, device=DEV)
+    want = v_pages.clone()
+    at, slot = table[seqs, [p // bs for p in poss]].long(), torch.tensor([p % bs for p in poss], device=DEV)
+    want[at, :, :, slot] = v.reshape(T, nkv, vd)
+    ops.rope_kv_write(q, k, v, i32(poss), i32(seqs), table, k_pages, v_pages, nkv, nkv, hd, bs, hd, 1e4, v_dim=vd)
+    assert torch.equal(v_pages, want)

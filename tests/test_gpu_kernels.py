@@ -1986,3 +1986,20 @@ def test_values_of_many_tokens_go_to_their_places(dtype, decoded, prompts, nkv, 
     want[at, :, :, slot] = v.reshape(T, nkv, vd)
     ops.rope_kv_write(q, k, v, i32(poss), i32(seqs), table, k_pages, v_pages, nkv, nkv, hd, bs, hd, 1e4, v_dim=vd)
     assert torch.equal(v_pages, want)
+
+
+@pytest.mark.parametrize("M", [33, 49, 64])
+@pytest.mark.parametrize("N,K,epi", [(6144, 2048, 0), (5184, 200, 0), (5200, 1192, 1), (5120, 640, 2), (12288, 128, 1), (2560, 1416, 3)])
+def test_products_of_four_row_tiles_have_the_bits_of_one(M, N, K, epi):
+    """33 to 64 rows in blocks of four row tiles and two sets of weight rows, with one piece of K a wave, several, a last part of one and waves
+    without any: the bits of the same rows sixteen at a time."""
+    from ferrox_amd import ops
+    a = rnd(M, K, dtype=torch.bfloat16)
+    w = rnd(N * (2 if epi == ops.EPI_GATED else 1), K, dtype=torch.bfloat16, seed=1, scale=0.05)
+    dtype = torch.bfloat16 if epi in (ops.EPI_STORE, ops.EPI_GATED) else torch.float32
+    whole = rnd(M, N, dtype=dtype, seed=2)
+    parts = whole.clone()
+    ops.gemm(a, w, epilogue=epi, out=whole)
+    for m in range(0, M, 16):
+        ops.gemm(a[m:m + 16], w, epilogue=epi, out=parts[m:m + 16])
+    assert torch.equal(whole, parts)

@@ -35,6 +35,8 @@ struct GemmArgs {
     void* C;
     long ldc;
     const float* row_scale;  // [M] or null, multiplies the product before it is added (EPI_RESID)
+    const float* then_add;   // EPI_RESID of up to 16 plain rows: [M, N] at a row distance of ld_then_add, added behind the product, or null
+    long ld_then_add;
     const int* a_rows;       // [M] or null: row of A to read for logical row m
     const int* c_rows;       // [M] or null: row of C to write for logical row m
     const int* expert_offsets;  // [E+1] or null
@@ -1452,7 +1454,8 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
     typedef __attribute__((ext_vector_type(V == 1 ? 2 : V))) float run_t;
     typedef run_t run_any_t __attribute__((aligned(4)));
     int m_of[IT];                                 // row of C, or -1
-    float old[IT][V], scale_of[IT], gate[IT][V];
+    constexpr bool THEN = EPI == EPI_RESID && MT == 1;
+    float old[IT][V], scale_of[IT], gate[IT][V], more[THEN ? IT : 1][V];
     RawElement bias_of[IT][V];
     auto tile_of = [&](int i) { return OUTS == 1 && V == 1 ? 0 : (tid + i * THREADS) / RUNS; };
     auto row_in_tile = [&](int i) { return V == 1 ? (tid + i * THREADS) / CW % 16 : (tid + i * THREADS) % RUNS / (4 / V) % 16; };
@@ -1478,6 +1481,13 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
                 } else {
 #pragma unroll
                     for (int r = 0; r < V; ++r) old[i][r] = from[min(first + r, g.N - 1)];
+                }
+            }
+            if constexpr (THEN) {
+                if (g.then_add) {
+                    const float* from = g.then_add + (size_t)m * g.ld_then_add;
+#pragma unroll
+                    for (int r = 0; r < V; ++r) more[i][r] = from[min(first + r, g.N - 1)];
                 }
             }
             if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_F32) {
@@ -1782,6 +1792,9 @@ __device__ __forceinline__ void skinny_block(const GemmArgs& g, const unsigned b
                             asm volatile("" : "+v"(o[r]));
                         }
                         o[r] = old[i][r] + o[r];
+                        if constexpr (THEN) {
+                            if (g.then_add) o[r] += more[i][r];
+                        }
                     } else {
                         o[r] = stored_c<decltype(kind)::value>(g, o[r], gate[i][r]);
                     }
@@ -1810,15 +1823,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(GemmArgs g
     skinny_block<MT, WAVES, NW, DUAL, EPI, NORM, ROPE, HALF, DEPTH, WEIGHTS_FIRST, false>(g, blockIdx.x, blockIdx.y);
 }
 
-// Two products of up to 16 plain rows that do not need each other, one launch: the first's blocks (gate/up, or a product that is added, in half sets of
+// Two products of up to 16 plain rows that do not need each other, one launch: the first's blocks (gate/up, or a product that is stored in float32, in half sets of
 // weight rows), then the second's (stored; in half or whole sets).  A step of few tokens is a chain of launches of 3 us and more that each wait for memory alone;
 // side by side they wait together, and the streams of the larger one go on meanwhile.  The same blocks, so the same bits.  us apart -> together: gate/up of 5,632 x 2,048 and
-// 1,024 x 2,048 1 row 14.6 -> 11.2, 8 rows 16.1 -> 13.2, 16 rows 18.6 -> 16.6; 2,048 x 5,632 added and 4,096 x 512 with its heads turned (a launch of its own before)
+// 1,024 x 2,048 1 row 14.6 -> 11.2, 8 rows 16.1 -> 13.2, 16 rows 18.6 -> 16.6; 2,048 x 5,632 and 4,096 x 512 with its heads turned (a launch of its own before)
 // 13.5 -> 8.0, 14.1 -> 8.9, 16.3 -> 10.9.
 template <bool GATED, int DEPTH, int NW2, int EPI2, bool HALF2>
 __global__ __launch_bounds__(256) void gemm_bf16_skinny_pair_kernel(GemmArgs a, GemmArgs b, int first) {
     if ((int)blockIdx.x < first)
-        skinny_block<1, 4, GATED ? 2 : 1, GATED, GATED ? EPI_GATED : EPI_RESID, false, false, true, DEPTH, false, false>(a, blockIdx.x, 0);
+        skinny_block<1, 4, GATED ? 2 : 1, GATED, GATED ? EPI_GATED : EPI_STORE_F32, false, false, true, DEPTH, false, false>(a, blockIdx.x, 0);
     else
         skinny_block<1, 4, NW2, false, EPI2, false, false, HALF2, HALF2 ? 4 : 2, false, EPI2 == EPI_STORE>(b, blockIdx.x - first, 0);
 }
@@ -2860,7 +2873,6 @@ static FewRows few_plain_rows(int M, int N, int K, bool dual, int cus) {
 struct FxProduct {
     const void *A, *W;
     void* C;
-    const float* row_scale;
     const int* turn_positions;
     const float* turn_inv_freq;
     long lda, ldc, up_offset;
@@ -2871,7 +2883,7 @@ struct FxProduct {
 FX_API int fx_gemm_pairs(int M, int epi, int N, int K, int epi2, int N2, int K2, int cus) {
     const FewRows f = few_plain_rows(M, N, K, epi == EPI_GATED, cus);
     return M >= 1 && M <= 16 && K % 8 == 0 && K2 % 8 == 0 && N2 < 65536 && N < 65536 && (epi2 == EPI_STORE || epi2 == EPI_STORE_F32) &&
-           f.half && (epi == EPI_RESID || (epi == EPI_GATED && f.deep));
+           f.half && (epi == EPI_STORE_F32 || (epi == EPI_GATED && f.deep));
 }
 FX_API int fx_gemm_pair(void* stream, const FxProduct* first, const FxProduct* second) {
     const int cus = fx_compute_units();
@@ -2887,7 +2899,7 @@ FX_API int fx_gemm_pair(void* stream, const FxProduct* first, const FxProduct* s
         FX_REQUIRE(p.turn_width == 0 || (i == 1 && p.epi == EPI_STORE && p.turn_positions && p.turn_inv_freq && p.turn_from >= 0 && p.turn_dims >= 0 && p.turn_from % 2 == 0 &&
                                          p.turn_dims % 2 == 0 && p.turn_width % 2 == 0 && p.turn_from + p.turn_dims <= p.turn_width && p.N % p.turn_width == 0),
                    "gemm_pair: %d turned dimensions from %d on of heads of %d", p.turn_dims, p.turn_from, p.turn_width);
-        g[i].A = p.A; g[i].lda = p.lda; g[i].W = p.W; g[i].C = p.C; g[i].ldc = p.ldc; g[i].up_offset = p.up_offset; g[i].row_scale = p.row_scale;
+        g[i].A = p.A; g[i].lda = p.lda; g[i].W = p.W; g[i].C = p.C; g[i].ldc = p.ldc; g[i].up_offset = p.up_offset;
         g[i].M = p.M; g[i].N = p.N; g[i].K = p.K; g[i].act = p.act; g[i].act_limit = p.act_limit; g[i].act_alpha = p.act_alpha; g[i].vec_ok = 1;
         if (p.turn_width) {
             g[i].rope_positions = p.turn_positions; g[i].rope_inv_freq = p.turn_inv_freq; g[i].act_alpha = p.turn_magnitude;
@@ -3008,7 +3020,8 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
                    int E, int M, int N, int K, const void* norm_w, int norm_dtype, float norm_eps,
                    const int* pair_ids, int pair_div, int n_always, int always_rows, int always_from_a, long kb_rows,
                    const float* row_ss, int row_ss_n, int act, int store_act, float act_limit, float act_alpha,
-                   const float* pre_scale, const int* pre_scale_rows, const float* out_gate, long ld_gate, int gate_div, int max_share) {
+                   const float* pre_scale, const int* pre_scale_rows, const float* out_gate, long ld_gate, int gate_div, int max_share,
+                   const float* then_add, long ld_then_add) {
     FX_REQUIRE((store_act == SACT_GATE) == (out_gate != nullptr) && (!out_gate || (gate_div >= 1 && ld_gate >= (long)gate_div * N)),
                "gemm: gated outputs need gate rows of %d x %d columns, got a row distance of %ld", gate_div, N, ld_gate);
     FX_REQUIRE(store_act >= 0 && store_act < SACT_COUNT && (store_act == 0 || ((epi == EPI_STORE || epi == EPI_STORE_F32) && !bias)),
@@ -3051,6 +3064,10 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
     FX_REQUIRE(kb_rows >= 0 && (kb_rows == 0 || (dtype == FX_BF16 && K % 64 == 0 && ((uintptr_t)W % 16) == 0 && lda % 8 == 0 &&
                                                  ((uintptr_t)A % 16) == 0 && (up_offset % K) == 0)),
                "gemm: weights in slabs of 64 k are bfloat16 with K a multiple of 64 and aligned operands");
+    FX_REQUIRE(!then_add || (dtype == FX_BF16 && epi == EPI_RESID && M <= 16 && !expert_offsets && !pair_ids && !c_rows && ld_then_add >= N && K % 8 == 0 && lda % 8 == 0 &&
+                             (((uintptr_t)A | (uintptr_t)W) % 16) == 0 && g_head_rows >= 16 && (g_plain_rows == 0 || g_plain_rows >= 16) && g_skinny_mt <= 1),
+               "gemm: rows to be added behind the product go with up to 16 aligned plain bfloat16 rows that are added");
+    g.then_add = then_add; g.ld_then_add = ld_then_add;
     g.n_always = n_always; g.always_rows = always_rows; g.always_from_a = always_from_a;
     FX_REQUIRE(n_always >= 0 && (n_always == 0 || (pair_ids && always_rows >= 1 && always_rows <= 16)),
                "gemm: experts that every row takes come with unsorted pairs and at most 16 rows");

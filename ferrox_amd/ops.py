@@ -130,7 +130,7 @@ _sigs = {
     ("gemm", "fx_gemm"): [c_void_p, c_int, c_int, c_void_p, c_long, c_void_p, c_long, c_long, c_void_p, c_int,
                           c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_int, c_long, c_void_p, c_int, c_int, c_int,
-                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int],
+                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_long],
     ("gemm", "fx_qkv_rope"): [c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_void_p, c_long, c_int, c_int,
                               c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
@@ -667,7 +667,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
          always: tuple | None = None, w_kblocked: bool = False, row_ss: tuple | None = None,
          activation: str = "silu", store_activation: str | None = None, activation_params: tuple = (0.0, 0.0),
          pre_scale: torch.Tensor | None = None, pre_scale_rows: torch.Tensor | None = None,
-         out_gate: tuple | None = None, max_share: int = 0) -> torch.Tensor:
+         out_gate: tuple | None = None, max_share: int = 0, then_add: torch.Tensor | None = None) -> torch.Tensor:
     """C[m, n] = sum_k a[m, k] * w[n, k] with an epilogue.
 
     `w` is [N, K], or [E, N, K] with `expert_offsets` [E+1] (rows sorted by expert).
@@ -699,6 +699,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
     is multiplied by sigmoid(logits[m // div, (m % div) * N + n]); div > 1 where the output's rows are parts of the gate's.
     `max_share` (with `expert_offsets`): a number of rows that no expert's share exceeds, if the caller knows one (a step's tokens, each
     of which takes an expert once): the order in which tiles are worked on depends on it, no result does.
+    `then_add` (float32 [M, N]; EPI_RESID of up to 16 plain bfloat16 rows): added to `out` behind the product, out = (out + product) + then_add.
     """
     gate_logits, gate_div = out_gate if out_gate is not None else (None, 0)
     if gate_logits is not None and (store_activation is not None or epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None
@@ -709,6 +710,9 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
         raise KernelError(f"gemm: stored activation '{store_activation}' is not one of {sorted(k for k in STORED_ACTIVATIONS if k)}")
     if store_activation is not None and (epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None):
         raise KernelError("gemm: a stored activation goes with the plain stored product without bias")
+    if then_add is not None and (then_add.dtype != torch.float32 or then_add.dim() != 2 or then_add.stride(1) != 1 or epilogue != EPI_RESID
+                                 or then_add.shape[0] < a.shape[0] or then_add.shape[1] < w.shape[0]):
+        raise KernelError("gemm: rows to be added behind the product are float32, as many as are added to")
     if row_ss is not None:
         ss = row_ss[0]
         if ss.dtype != torch.float32 or ss.dim() != 2 or not ss.is_contiguous() or ss.shape[0] != a.shape[0]:
@@ -785,7 +789,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
           _p(row_ss[0]) if row_ss is not None else None, row_ss[0].shape[1] if row_ss is not None else 0,
           ACTIVATIONS[activation], STORED_ACTIVATIONS[store_activation] if gate_logits is None else _SACT_GATE,
           float(activation_params[0]), float(activation_params[1]), _p(pre_scale), _p(_i32(pre_scale_rows, "pre_scale_rows")),
-          _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share))
+          _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share),
+          _p(then_add), then_add.stride(0) if then_add is not None else 0)
     return out
 
 
@@ -802,7 +807,6 @@ class Product:
     epilogue: int = EPI_STORE
     activation: str = "silu"
     activation_params: tuple = (0.0, 0.0)
-    row_scale: torch.Tensor | None = None
     turn: tuple | None = None
 
     def columns(self) -> int:
@@ -810,19 +814,18 @@ class Product:
 
     def launch(self) -> None:
         """By itself (without `turn`)."""
-        gemm(self.a, self.w, epilogue=self.epilogue, out=self.out, activation=self.activation, activation_params=self.activation_params,
-             row_scale=self.row_scale)
+        gemm(self.a, self.w, epilogue=self.epilogue, out=self.out, activation=self.activation, activation_params=self.activation_params)
 
 
 class _ProductArgs(Structure):
-    _fields_ = [(n, c_void_p) for n in ("A", "W", "C", "row_scale", "turn_positions", "turn_inv_freq")] + \
+    _fields_ = [(n, c_void_p) for n in ("A", "W", "C", "turn_positions", "turn_inv_freq")] + \
                [(n, c_long) for n in ("lda", "ldc", "up_offset")] + \
                [(n, c_int) for n in ("epi", "M", "N", "K", "act", "turn_width", "turn_from", "turn_dims")] + \
                [(n, c_float) for n in ("act_limit", "act_alpha", "turn_magnitude")]
 
 
 def can_pair(first: Product, second: Product) -> bool:
-    """Whether `gemm_pair` takes the two: up to 16 rows of bfloat16, the first gated or added in blocks of half sets of weight rows, the second stored."""
+    """Whether `gemm_pair` takes the two: up to 16 rows of bfloat16, the first gated or stored in float32 in blocks of half sets of weight rows, the second stored."""
     M = first.a.shape[0]
     if not 1 <= M <= PAIR_MAX_ROWS or second.a.shape[0] != M:
         return False
@@ -846,9 +849,7 @@ def gemm_pair(first: Product, second: Product) -> None:
             raise KernelError(f"gemm_pair: output {tuple(p.out.shape)} {p.out.dtype} does not fit [{M},{N}] {dtype}")
         if p.activation not in ACTIVATIONS:
             raise KernelError(f"gemm_pair: activation '{p.activation}' is not one of {sorted(ACTIVATIONS)}")
-        if p.row_scale is not None and (p.epilogue != EPI_RESID or p.row_scale.dtype != torch.float32 or p.row_scale.numel() < M):
-            raise KernelError("gemm_pair: a row scale is float32, a number per row of a product that is added")
-        g = _ProductArgs(A=_p(p.a), W=_p(p.w), C=_p(p.out), row_scale=_p(p.row_scale), lda=p.a.stride(0), ldc=p.out.stride(0),
+        g = _ProductArgs(A=_p(p.a), W=_p(p.w), C=_p(p.out), lda=p.a.stride(0), ldc=p.out.stride(0),
                          up_offset=N * K if p.epilogue == EPI_GATED else 0, epi=p.epilogue, M=M, N=N, K=K, act=ACTIVATIONS[p.activation],
                          act_limit=float(p.activation_params[0]), act_alpha=float(p.activation_params[1]))
         if p.turn is not None:

@@ -333,7 +333,7 @@ class PagedAttention(Mixer):
         w = self.qkv.weight
         cut = self.qw + self.kvw + self.vw
         qk, _ = matmul_with(ctx, x, w[:cut], epilogue=ops.EPI_STORE_F32)
-        rest = matmul_with(ctx, x, w[cut:])[0] if w.shape[0] > cut else None
+        rest = matmul(x, w[cut:]) if w.shape[0] > cut else None
         q = torch.empty((ctx.n_tokens, self.qw), dtype=ctx.act_dtype, device=qk.device)
         writes = self.own_kv and cache.writes
         debug.region("rope + cache write")

@@ -153,6 +153,7 @@ class StepContext:
     kv_bound: int = 0
     carry: object = None               # what a feed-forward hands on to the next block (its rows, normed), see PreNormBlock
     waiting: list = field(default_factory=list)      # products (ops.Product) that a block has left for its mixer's launches, see `linear.matmul_with`
+    owed: object = None                # float32 rows that one of them has stored, which the mixer's last product adds behind its own
     _memo: dict = field(default_factory=dict)
 
     def memo(self, key, make: Callable):
@@ -198,6 +199,11 @@ class Part:
     def children(self) -> list:
         """Sub-parts as [(prefix, part)]; a child's tensors are named prefix + its local names."""
         return []
+
+
+def keeps_methods(part: "Part", cls: type, *names: str) -> bool:
+    """Whether the part's methods are those of the class: neither a class derived from it nor the instance has put others in their place."""
+    return all(getattr(getattr(part, n), "__func__", None) is vars(cls)[n] for n in names)
 
 
 def walk_params(part: "Part", prefix: str = ""):

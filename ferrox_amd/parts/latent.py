@@ -27,7 +27,7 @@ import torch
 
 from .. import debug, limits, ops
 from .attention import attention_items
-from .base import MIXERS, NORMS, POSITION_ENCODINGS, Mixer, ParamSpec, PartSpec
+from .base import MIXERS, NORMS, POSITION_ENCODINGS, Mixer, ParamSpec, PartSpec, keeps_methods
 from .linear import Linear, matmul, matmul_with, same_dtype
 from .recurrent import longest_portion
 
@@ -170,6 +170,11 @@ class LatentAttention(Mixer):
         w = self.retain_window
         return (("window", w), w) if w else (("full",), None)
 
+    def adds_owed(self) -> bool:
+        """Whether `forward` adds ctx.owed behind its own output (its output product takes up to 16 bfloat16 rows with it)."""
+        w = self.o_proj.weight
+        return keeps_methods(self, LatentAttention, "forward") and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0
+
     def forward(self, x, ctx, cache, residual, out_scale: float | None = None, fresh: bool = False) -> None:
         """`out_scale`, `fresh` as `PagedAttention.forward` takes them."""
         T, H, D, P, R, V = ctx.n_tokens, self.n_heads, self.head_dim, self.rot_dim, self.kv_rank, self.v_dim
@@ -238,4 +243,5 @@ class LatentAttention(Mixer):
         if fresh:
             ops.fill_u32(residual, 0)
         scale = ops.constant_rows(heads.device, out_scale, T) if out_scale is not None and out_scale != 1.0 else None
-        self.o_proj(heads, epilogue=ops.EPI_RESID, out=residual, row_scale=scale)
+        self.o_proj(heads, epilogue=ops.EPI_RESID, out=residual, row_scale=scale, then_add=ctx.owed)
+        ctx.owed = None

@@ -26,12 +26,16 @@ def matmul(x: torch.Tensor, weight: torch.Tensor, *, epilogue: int = ops.EPI_STO
 
 def matmul_with(ctx, x: torch.Tensor, weight: torch.Tensor, *, epilogue: int = ops.EPI_STORE, turn=None):
     """(x @ weight^T stored, whether it has been turned as `turn` says): `matmul`, or, where a product that waits in ctx.waiting goes out with it, one
-    launch of both.  What waits reads nothing that this product writes, and this product nothing that what waits writes."""
+    launch of both.  What waits reads nothing that this product writes, and this product nothing that what waits writes.  What is stored for
+    the stream is owed to it then (ctx.owed)."""
     if ctx.waiting and x.dim() == 2 and x.shape[0] <= ops.PAIR_MAX_ROWS and epilogue in (ops.EPI_STORE, ops.EPI_STORE_F32):
         out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32 if epilogue == ops.EPI_STORE_F32 else weight.dtype, device=x.device)
         mine = ops.Product(x, weight, out, epilogue, turn=turn)
         if ops.can_pair(ctx.waiting[0], mine):
-            ops.gemm_pair(ctx.waiting.pop(0), mine)
+            first = ctx.waiting.pop(0)
+            ops.gemm_pair(first, mine)
+            if first.epilogue == ops.EPI_STORE_F32:
+                ctx.owed = first.out
             return out, turn is not None
     return matmul(x, weight, epilogue=epilogue), False
 

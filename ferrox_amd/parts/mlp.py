@@ -45,17 +45,24 @@ class GatedMLP(FeedForward):
 
     takes_fresh = True       # forward(..., fresh=True): `residual` holds nothing yet, the output is stored into it
 
-    def products(self, x, residual) -> list:
-        """What `forward` launches, in its order, for a caller that launches it beside other products (none where a weight is of another type than the rows)."""
+    def gate_up_product(self, x):
+        """The first product of `forward`, for a caller that launches it beside another (None where a weight is of another type than the rows)."""
         if not x.dtype == self.gate_up.weight.dtype == self.down.weight.dtype:
-            return []
-        act = torch.empty((x.shape[0], self.intermediate_size), dtype=self.gate_up.weight.dtype, device=x.device)
-        return [ops.Product(x, self.gate_up.weight, act, ops.EPI_GATED, self.activation, self.activation_params),
-                ops.Product(act, self.down.weight, residual, ops.EPI_RESID)]
+            return None
+        act = torch.empty((x.shape[0], self.intermediate_size), dtype=x.dtype, device=x.device)
+        return ops.Product(x, self.gate_up.weight, act, ops.EPI_GATED, self.activation, self.activation_params)
+
+    def down_product(self, act):
+        """The second one, stored in rows of its own, which the caller adds."""
+        out = torch.empty((act.shape[0], self.hidden_size), dtype=torch.float32, device=act.device)
+        return ops.Product(act, self.down.weight, out, ops.EPI_STORE_F32)
 
     def forward(self, x, ctx, residual, row_scale=None, fresh: bool = False) -> None:
         debug.region("mlp gate/up")
-        act = self._act(x)
+        self.add(self._act(x), residual, row_scale, fresh)
+
+    def add(self, act, residual, row_scale=None, fresh: bool = False) -> None:
+        """The rows of the gate/up product through the second one, into `residual`."""
         debug.region("mlp down")
         if fresh and row_scale is None:
             self.down(act, epilogue=ops.EPI_STORE_F32, out=residual)

@@ -574,3 +574,31 @@ def test_command_line_and_replay(tmp_path_factory):
     for step, want_rows in ((0, [la[0], la[16]]), (1, [lb[2]]), (2, [lb[3], la[29]])):
         got = torch.from_numpy(np.fromfile(os.path.join(out_dir, f"{step}.f32"), dtype="<f4").reshape(-1, V))
         assert float(u.row_errors(got, torch.stack(want_rows)).max()) <= u.LIMIT["float32"], step
+
+
+@pytest.mark.parametrize("rows", [1, 3, 16])
+def test_few_rows_add_the_mixer_and_then_the_feed_forward(monkeypatch, rows):
+    """The products of a layer's two sublayers share launches for up to 16 rows.  The stream has the bits that it has where each goes out by
+    itself: the mixer's output is added first, the feed-forward's to that."""
+    from ferrox_amd import ops
+    from ferrox_amd.config import presets
+    from ferrox_amd.engine.model import Model
+    from ferrox_amd.engine.runner import StepEntry
+    from ferrox_amd.models.registry import resolve
+    from ferrox_amd.weights.random_init import RandomSource
+    raw = presets.load("fokinex-2k")
+    raw = dict(raw, vocab=512, layers=raw["layers"][:4])           # (latent attention, one with the latents of another layer, attention beside a delta rule)
+    arch = resolve(raw)
+    model = Model(arch.build_spec(arch.config_class.from_dict(raw), None))
+    model.load(RandomSource(5, torch.bfloat16, "cuda:0"), torch.bfloat16, "cuda:0")
+    got = {}
+    for most in (ops.PAIR_MAX_ROWS, 0):
+        monkeypatch.setattr(ops, "PAIR_MAX_ROWS", most)
+        runner = runner_of(model, block_size=64, num_pages=rows, max_seqs=rows, use_graphs=False)
+        got[most] = []
+        for step in range(3):
+            for i in range(rows):
+                assert (step or runner.admit(i)) and runner.reserve(i, 1)
+            got[most].append(runner.step([StepEntry(i, [(37 * i + 11 * step) % 512], [0]) for i in range(rows)]).clone())
+    for a, b in zip(got[16], got[0]):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

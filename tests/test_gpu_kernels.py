@@ -1894,7 +1894,8 @@ def test_delta_rule_at_every_length_of_a_group(D, V, H, G):
 @pytest.mark.parametrize("M", [1, 4, 5, 16])
 @pytest.mark.parametrize("N2,K2,epi2", [(256, 128, 0), (1024, 2048, 1), (4096, 512, 0), (5120, 512, 1), (24, 64, 0)])
 def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2):
-    """Gate/up and an added product, each beside a stored one in half sets, whole sets and two of them, with the pairs of its heads turned and without."""
+    """Gate/up and a product stored in float32, each beside a stored one in half sets, whole sets and two of them, with the pairs of its heads turned and without; and
+    what adds the second one's rows behind its own: the bits of two additions."""
     from ferrox_amd import ops
     x, w_gu, w_down = rnd(M, 2048, dtype=torch.bfloat16), rnd(2 * 5632, 2048, dtype=torch.bfloat16, seed=1, scale=0.02), rnd(2048, 5632, dtype=torch.bfloat16, seed=2, scale=0.02)
     y, w2 = rnd(M, K2, dtype=torch.bfloat16, seed=3), rnd(N2, K2, dtype=torch.bfloat16, seed=4, scale=0.1)
@@ -1907,17 +1908,24 @@ def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2
     def stored():
         return torch.full((M, N2 + 8), 7.0, dtype=torch.bfloat16 if epi2 == 0 else torch.float32, device=DEV)
     act, h = ops.gemm(x, w_gu, epilogue=ops.EPI_GATED, activation="gelu_tanh"), h0.clone()
-    ops.gemm(act, w_down, epilogue=ops.EPI_RESID, out=h, row_scale=scale)
+    w_out = rnd(2048, 2048, dtype=torch.bfloat16, seed=7, scale=0.02)
+    for row_scale in (None, scale):
+        h, both = h0.clone(), h0.clone()
+        ops.gemm(x, w_out, epilogue=ops.EPI_RESID, out=h, row_scale=row_scale)
+        ops.gemm(act, w_down, epilogue=ops.EPI_RESID, out=h)
+        ops.gemm(x, w_out, epilogue=ops.EPI_RESID, out=both, row_scale=row_scale, then_add=ops.gemm(act, w_down, epilogue=ops.EPI_STORE_F32))
+        assert torch.equal(both, h)
+    down = ops.gemm(act, w_down, epilogue=ops.EPI_STORE_F32)
     plain2 = ops.gemm(y, w2, epilogue=epi2)
     for turn in (None, (positions, inv_freq, width, first_dim, n_dims, 1.25)) if epi2 == 0 else (None,):
         want = plain2.clone()
         if turn is not None:
             ops.latent_q_rot(want, want, positions, heads, first_dim, width - first_dim, n_dims, first_dim, inv_freq, 1.25)
-        got_act, got_h, one, two = torch.full((M, 5632), 7.0, dtype=torch.bfloat16, device=DEV), h0.clone(), stored(), stored()
+        got_act, got_down, one, two = torch.full((M, 5632), 7.0, dtype=torch.bfloat16, device=DEV), torch.empty_like(down), stored(), stored()
         first = ops.Product(x, w_gu, got_act, ops.EPI_GATED, "gelu_tanh")
         ops.gemm_pair(first, ops.Product(y, w2, one[:, :N2], epi2, turn=turn))
-        ops.gemm_pair(ops.Product(got_act, w_down, got_h, ops.EPI_RESID, row_scale=scale), ops.Product(y, w2, two[:, :N2], epi2, turn=turn))
-        assert torch.equal(got_act, act) and torch.equal(got_h, h)
+        ops.gemm_pair(ops.Product(got_act, w_down, got_down, ops.EPI_STORE_F32), ops.Product(y, w2, two[:, :N2], epi2, turn=turn))
+        assert torch.equal(got_act, act) and torch.equal(got_down, down)
         for out in (one, two):
             assert torch.equal(out[:, :N2], want) and bool((out[:, N2:] == 7).all()), turn is not None
     assert not ops.can_pair(first, ops.Product(y[:, 1:], w2[:, 1:], one, epi2)) and not ops.can_pair(first, ops.Product(y.float(), w2.float(), one, epi2))

@@ -1367,6 +1367,10 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
         f[u] = ((u < n_waves) & (ms[u] != NEG_INF)) ? e : 0.f;
         l += f[u] * (u < n_waves ? ls[u] : 0.f);
     }
+    auto value = [&](int u, int d) {      // (of a wave that is there: the last one's sum may be infinite, and an infinity with weight 0 is no 0)
+        const float v = from[u][d];
+        return u < n_waves ? v : 0.f;
+    };
     const int h = h0 + row;
     const bool last = a.splits == 1;
     const float fin = last ? finish_row<true>(a, h, m, l) : 1.f;
@@ -1376,8 +1380,8 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
             float o0 = 0.f, o1 = 0.f;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                o0 += f[u] * from[u][d];
-                o1 += f[u] * from[u][d + 1];
+                o0 += f[u] * value(u, d);
+                o1 += f[u] * value(u, d + 1);
             }
             o0 *= fin;
             o1 *= fin;
@@ -1389,7 +1393,7 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
     for (int d = sub; d < vd; d += per_row) {
         float o = 0.f;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) o += f[u] * from[u][d];
+        for (int u = 0; u < 8; ++u) o += f[u] * value(u, d);
         if (last) store_out<bf16>(a, tok, h, d, o * fin);
         else po[d] = o;
     }

@@ -1969,6 +1969,36 @@ def test_single_queries_of_one_wave_write_their_rows_and_columns_only(nh, nkv, h
             assert float((out[s].reshape(nh, vd).double() - want).abs().max()) <= 3 * 2 ** -9 * float(v.abs().max()), (s, most)
 
 
+@pytest.mark.parametrize("waves", [2, 3, 4])
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 16, 128), (28, 4, 128), (16, 4, 64), (8, 1, 256)])
+def test_an_infinite_value_stays_infinite_in_the_merge_of_a_blocks_waves(nh, nkv, hd, waves):
+    """A value of infinity in the keys of the first, a middle and the last of a block's waves, of which there are two and more: the outputs that take
+    it are infinite, and all others are as without it."""
+    from ferrox_amd import ops
+    bs, lens = 64, [129, 200, 300, 500]
+    per = 8
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table = torch.randperm(len(lens) * per, generator=torch.Generator().manual_seed(2)).to(torch.int32).view(len(lens), per).to(DEV)
+    kp = rnd(len(lens) * per, nkv, bs, hd, dtype=torch.bfloat16)
+    vp = rnd(len(lens) * per, nkv, hd, bs, dtype=torch.bfloat16, seed=1)
+    q = rnd(len(lens), nh * hd, dtype=torch.bfloat16, seed=2, scale=0.05)          # (no probability is near nothing)
+    def run(values):
+        out = torch.zeros(len(lens), nh * hd, dtype=torch.bfloat16, device=DEV)
+        ops.attention_decode(q, out, kp, values, table, i32([n - 1 for n in lens]), i32([0, 1, 2, 3]), i32([0, 1, 2, 3]), nh, nkv, hd, bs, 0,
+                             hd ** -0.5, max_kv_len=512, chunk=512, waves=waves)
+        return out.view(len(lens), nkv, nh // nkv, hd)
+    clean = run(vp)
+    assert torch.isfinite(clean).all()
+    for place in (lambda n: 0, lambda n: 70, lambda n: n // 2, lambda n: n - 1):
+        bad = vp.clone()
+        for s, n in enumerate(lens):
+            t = place(n)
+            bad[table[s, t // bs].long(), nkv - 1, 5, t % bs] = math.inf
+        got, want = run(bad), clean.clone()
+        want[:, nkv - 1, :, 5] = math.inf
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype,decoded,prompts", [(torch.bfloat16, 0, [1030]), (torch.bfloat16, 13, [700, 0, 345]), (torch.bfloat16, 1024, []),
                                                    (torch.float32, 0, [260]), (torch.float32, 6, [131, 3, 140])])
 @pytest.mark.parametrize("nkv,vd,bs", [(16, 128, 64), (11, 192, 16), (16, 136, 20), (8, 264, 24)])

@@ -123,7 +123,7 @@ class ParallelBlock(Block):
     def forward(self, h, ctx, cache):
         debug.region("norm")
         x = self.norm1.forward(h, ctx)
-        few = x.dtype == torch.bfloat16 and x.shape[0] <= ops.PAIR_MAX_ROWS and hasattr(self.ffn, "gate_up_product")
+        few = isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and x.shape[0] <= ops.PAIR_MAX_ROWS and hasattr(self.ffn, "gate_up_product")
         gate_up = self.ffn.gate_up_product(x) if few else None
         if gate_up is not None:
             ctx.waiting.append(gate_up)
@@ -141,6 +141,7 @@ class ParallelBlock(Block):
                 self.ffn.forward(x, ctx, h)
             return
         if launched == 0:
+            debug.region("mlp gate/up")          # (a launch that it shares is one of the mixer's stages)
             gate_up.launch()
         if launched < 2:
             self.ffn.add(gate_up.out, h)

@@ -6,7 +6,7 @@ from __future__ import annotations
 import torch
 
 from .. import debug, ops
-from .base import FEED_FORWARDS, FeedForward, ParamSpec
+from .base import FEED_FORWARDS, FeedForward, ParamSpec, keeps_methods
 from .linear import Linear, same_dtype
 
 
@@ -46,8 +46,10 @@ class GatedMLP(FeedForward):
     takes_fresh = True       # forward(..., fresh=True): `residual` holds nothing yet, the output is stored into it
 
     def gate_up_product(self, x):
-        """The first product of `forward`, for a caller that launches it beside another (None where a weight is of another type than the rows)."""
-        if not x.dtype == self.gate_up.weight.dtype == self.down.weight.dtype:
+        """The first product of `forward`, for a caller that launches it beside another and goes on with `down_product` or `add`.  None where a weight
+        is of another type than the rows, or where `forward` is not what is written here: the caller calls that."""
+        if not (keeps_methods(self, GatedMLP, "forward", "_act", "add") and type(self.gate_up) is type(self.down) is Linear
+                and x.dtype == self.gate_up.weight.dtype == self.down.weight.dtype):
             return None
         act = torch.empty((x.shape[0], self.intermediate_size), dtype=x.dtype, device=x.device)
         return ops.Product(x, self.gate_up.weight, act, ops.EPI_GATED, self.activation, self.activation_params)

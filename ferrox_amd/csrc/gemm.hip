@@ -3013,6 +3013,8 @@ FX_API int fx_gemm_grouped_tile(int per_group, int M, int N, int nonempty, int d
 }
 
 // dtype: type of A and W.  C is: T for EPI_STORE and EPI_GATED, float32 otherwise.
+// f32_instruction: a float32 product goes through the float32 matrix instruction whatever its sizes (a call that has its operands the other way round, rows of weights
+// against tokens as "weights": the rule by the weights' sizes would go by the tokens then).
 // max_share: rows sorted by expert, a number that no expert's rows exceed (0: none is known); the order of tiles depends on it, no result does.
 FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, const void* W, long w_stride,
                    long up_offset, const void* bias, int bias_dtype, void* C, long ldc,
@@ -3021,7 +3023,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
                    const int* pair_ids, int pair_div, int n_always, int always_rows, int always_from_a, long kb_rows,
                    const float* row_ss, int row_ss_n, int act, int store_act, float act_limit, float act_alpha,
                    const float* pre_scale, const int* pre_scale_rows, const float* out_gate, long ld_gate, int gate_div, int max_share,
-                   const float* then_add, long ld_then_add) {
+                   const float* then_add, long ld_then_add, int f32_instruction) {
     FX_REQUIRE((store_act == SACT_GATE) == (out_gate != nullptr) && (!out_gate || (gate_div >= 1 && ld_gate >= (long)gate_div * N)),
                "gemm: gated outputs need gate rows of %d x %d columns, got a row distance of %ld", gate_div, N, ld_gate);
     FX_REQUIRE(store_act >= 0 && store_act < SACT_COUNT && (store_act == 0 || ((epi == EPI_STORE || epi == EPI_STORE_F32) && !bias)),
@@ -3091,7 +3093,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         // x 5,632 18.5 -> 16.1, gate/up of 1,408 12.8 -> 9.1, a router of 61 8.2 -> 6.2; of 6,144 x 2,048, 768 of them, 15.9 -> 17.1).
         // Where it cannot take whole lines it stays behind tiles of 32 with sorted rows, and from three rows on with the head's.
         const bool lines = g.vec_ok && K % 32 == 0;
-        const bool split = g_f32_split >= 0 ? g_f32_split && K % 32 == 0 : fx_gemm_f32_split(N, K);
+        const bool split = !f32_instruction && (g_f32_split >= 0 ? g_f32_split && K % 32 == 0 : fx_gemm_f32_split(N, K));
         int tile = 0, mt = 1, nw = 2;
         if (g_f32_tile) tile = g_f32_tile == 1 ? 0 : g_f32_tile;
         else if (expert_offsets) tile = lines && group <= 2 ? 0 : (group <= 36 && !split ? 32 : 64);

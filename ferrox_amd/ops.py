@@ -130,7 +130,7 @@ _sigs = {
     ("gemm", "fx_gemm"): [c_void_p, c_int, c_int, c_void_p, c_long, c_void_p, c_long, c_long, c_void_p, c_int,
                           c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                           c_void_p, c_int, c_float, c_void_p, c_int, c_int, c_int, c_int, c_long, c_void_p, c_int, c_int, c_int,
-                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_long],
+                          c_float, c_float, c_void_p, c_void_p, c_void_p, c_long, c_int, c_int, c_void_p, c_long, c_int],
     ("gemm", "fx_qkv_rope"): [c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_void_p, c_long, c_int, c_int,
                               c_void_p, c_int, c_float, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p],
@@ -150,6 +150,7 @@ _sigs = {
                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     ("moe", "fx_moe_front"): [c_void_p, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_int,
                               c_int, c_int, c_int, c_int, c_float, c_float, c_int] + [c_void_p] * 9 + [c_int],
+    ("gemm", "fx_gemm_f32_split"): [c_int, c_int],
     ("gemm", "fx_gemm_pairs"): [c_int] * 8,
     ("gemm", "fx_gemm_pair"): [c_void_p, c_void_p, c_void_p],
     ("moe", "fx_moe_align"): [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int],
@@ -667,7 +668,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
          always: tuple | None = None, w_kblocked: bool = False, row_ss: tuple | None = None,
          activation: str = "silu", store_activation: str | None = None, activation_params: tuple = (0.0, 0.0),
          pre_scale: torch.Tensor | None = None, pre_scale_rows: torch.Tensor | None = None,
-         out_gate: tuple | None = None, max_share: int = 0, then_add: torch.Tensor | None = None) -> torch.Tensor:
+         out_gate: tuple | None = None, max_share: int = 0, then_add: torch.Tensor | None = None, f32_instruction: bool = False) -> torch.Tensor:
     """C[m, n] = sum_k a[m, k] * w[n, k] with an epilogue.
 
     `w` is [N, K], or [E, N, K] with `expert_offsets` [E+1] (rows sorted by expert).
@@ -700,6 +701,8 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
     `max_share` (with `expert_offsets`): a number of rows that no expert's share exceeds, if the caller knows one (a step's tokens, each
     of which takes an expert once): the order in which tiles are worked on depends on it, no result does.
     `then_add` (float32 [M, N]; EPI_RESID of up to 16 plain bfloat16 rows): added to `out` behind the product, out = (out + product) + then_add.
+    `f32_instruction`: float32 operands go through the float32 matrix instruction whatever their sizes (`f32_from_parts`): for a call whose `w` are not the
+    weights, so that the bits do not depend on how many rows stand side by side.
     """
     gate_logits, gate_div = out_gate if out_gate is not None else (None, 0)
     if gate_logits is not None and (store_activation is not None or epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None
@@ -790,8 +793,14 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
           ACTIVATIONS[activation], STORED_ACTIVATIONS[store_activation] if gate_logits is None else _SACT_GATE,
           float(activation_params[0]), float(activation_params[1]), _p(pre_scale), _p(_i32(pre_scale_rows, "pre_scale_rows")),
           _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share),
-          _p(then_add), then_add.stride(0) if then_add is not None else 0)
+          _p(then_add), then_add.stride(0) if then_add is not None else 0, int(f32_instruction))
     return out
+
+
+def f32_from_parts(n: int, k: int) -> bool:
+    """Whether a float32 product of [n, k] weights is worked out from bfloat16 parts of its operands (by the weights alone, whatever the rows)."""
+    fn, _ = _fn("gemm", "fx_gemm_f32_split")
+    return bool(fn(n, k))
 
 
 PAIR_MAX_ROWS = 16

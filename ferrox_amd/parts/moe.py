@@ -124,6 +124,15 @@ class SparseMoE(FeedForward):
             router = torch.cat(same_dtype([router, fetch(n["shared_gate"]).reshape(1, -1)]), dim=0)
         self.router = router.contiguous()
 
+    def _logits(self, x):
+        """The router's logits, float32 [T, outputs].  Few experts and many tokens: the router's rows are the short side of the product, so the kernel for
+        few rows streams the activations once, and the logits come out transposed.  A token's have the same bits either way: what would decide
+        by the weights' sizes how float32 numbers are multiplied is told not to, as it sees the tokens there."""
+        E, K = self.router.shape
+        if x.shape[0] > 64 and E <= 64 and self.router.dtype == x.dtype and not (x.dtype == torch.float32 and ops.f32_from_parts(E, K)):
+            return ops.gemm(self.router, x, epilogue=ops.EPI_STORE_F32, f32_instruction=True).t()
+        return matmul(x, self.router, epilogue=ops.EPI_STORE_F32)
+
     def _gated(self, weights, order=None) -> dict:
         """What the gate/up product is told beside its operands: the activation, and, where the weights act on the
         experts' input, the weights as a scale in front of it (`order`: the pair that each sorted row stands for)."""
@@ -223,10 +232,7 @@ class SparseMoE(FeedForward):
             # product's 2,048 weight rows give 16 tiles of 128 columns) beside launches that the host cannot
             # issue faster than the GPU runs them.
             debug.region("router")
-            if self.router.shape[0] <= 64 and self.router.dtype == x.dtype:      # (as below: the router's rows as the short side)
-                logits = ops.gemm(self.router, x, epilogue=ops.EPI_STORE_F32).t()
-            else:
-                logits = matmul(x, self.router, epilogue=ops.EPI_STORE_F32)
+            logits = self._logits(x)
             ids, weights, gate = ops.router_select(logits, self.n_experts, self.top_k, self.norm_topk_prob, self.gating,
                                                    self.has_shared_gate, weighting=self.weighting)
             S = self.shared_pieces
@@ -248,12 +254,7 @@ class SparseMoE(FeedForward):
                 join.record(side)
         if routed is None:
             debug.region("router")
-            if T > 64 and self.router.shape[0] <= 64 and self.router.dtype == x.dtype:
-                # few experts, many tokens: the router's rows are the short side of the product, so the
-                # kernel for few rows streams the activations once; the logits come out transposed
-                logits = ops.gemm(self.router, x, epilogue=ops.EPI_STORE_F32).t()
-            else:
-                logits = matmul(x, self.router, epilogue=ops.EPI_STORE_F32)
+            logits = self._logits(x)
             routed = ops.route(logits, self.n_experts, self.top_k, self.norm_topk_prob, self.gating,
                                self.has_shared_gate, weighting=self.weighting)
         ids, weights, gate, offsets, sorted_token, sorted_pair, _ = routed

@@ -234,3 +234,32 @@ def test_the_chunk_rule_leaves_the_callers_arguments_alone():
     body = src[src.index('"""', src.index('"""') + 3):]
     assert "waves =" not in body and "waves=" not in body.replace("int(waves)", "")
     assert "int(waves)" in body
+
+
+def test_float32_products_from_parts_by_the_weights_alone():
+    """Whole steps of 32 k, sums of 1,024 and more, weights of a million numbers; the router's product, whose rows stand where weights do, is left out of the
+    rule: no number of tokens changes how its float32 operands are multiplied."""
+    from types import SimpleNamespace
+    import torch
+    from ferrox_amd import ops
+    from ferrox_amd.csrc.build import load_library
+    from ferrox_amd.parts.moe import SparseMoE
+    rule = load_library("gemm").fx_gemm_f32_split
+    assert rule(2048, 2048) and rule(6144, 2048) and rule(1408, 2048) and rule(151936, 2048)
+    assert not rule(2048, 2056) and not rule(4096, 992) and not rule(60, 2048) and not rule(256, 2048)
+    asked = []
+
+    def gemm(a, w, *, f32_instruction=False, **kw):
+        asked.append((tuple(a.shape), tuple(w.shape), f32_instruction))
+        return torch.zeros(a.shape[0], w.shape[0])
+
+    moe, plain_gemm = SparseMoE(2048, 60, 4, 1408, True), ops.gemm
+    moe.router = torch.zeros(60, 2048)
+    try:
+        ops.gemm = gemm
+        for T in (1, 64, 65, 511, 512, 700, 4096):
+            assert moe._logits(torch.zeros(T, 2048)).shape == (T, 60)
+            rows, weights, instruction = asked.pop()
+            assert instruction or not rule(weights[0], weights[1]), T
+    finally:
+        ops.gemm = plain_gemm

@@ -601,3 +601,26 @@ def test_two_chaining_blocks_from_outside_equal_the_built_in_block(model_folders
         assert a.keys() == b.keys()
         for key in a:
             assert torch.equal(a[key], b[key]), f"{name} {dtype}: position {key} differs between the two ways of cutting a layer into blocks"
+
+
+@pytest.mark.parametrize("E", [8, 60])
+def test_a_float32_token_gets_the_same_bits_however_many_tokens_stand_beside_it(E):
+    """A step of many tokens has the router's rows as the short side of its product, of few tokens the tokens: the same sums in the same order, so the
+    same experts and the same weights."""
+    from types import SimpleNamespace
+    from ferrox_amd.parts.moe import SparseMoE
+    H, T = 2048, 700
+    moe = SparseMoE(H, E, 2, 32, True)
+    g = torch.Generator(device="cuda:0").manual_seed(E)
+    w = {n: torch.randn(s.shape, generator=g, device="cuda:0") * H ** -0.5 for n, s in moe.param_specs().items()}
+    moe.load(lambda n: w[n])
+    x = torch.randn(T, H, generator=g, device="cuda:0")
+
+    def run(a, b):
+        out = torch.zeros(b - a, H, device="cuda:0")
+        moe.forward(x[a:b], SimpleNamespace(act_dtype=torch.float32, carry=None), out)
+        return out
+
+    whole = run(0, T)
+    for cut in (1, 40, 65, 188, 350):
+        assert torch.equal(torch.cat([run(0, cut), run(cut, T)]), whole), cut

@@ -1887,7 +1887,9 @@ __device__ __forceinline__ f32x4_t f32_fetch_guarded(const float* row, int k, in
 // out the negative and subtracts it, so that what is cut off has either sign: else outputs are low by 5e-8 of their size, which the mean over a thousand keys brings out (decoded logits at 1,030 keys: 1.3e-6
 // off 64 bits instead of 0.8e-6).  Error against 64 bits, float32 instruction / taken apart: 2,048 k 2.9e-7 / 7.5e-8, 5,632 k 4.8e-7 / 7.3e-8, terms of one sign 8.9e-8 / 4.5e-8.
 // Parts of K (F32_PARTS, of whole pairs of steps) are added in their order, in the kernel for few rows and in tiles alike: a row's bits do not depend on which of them computes it.
-// Four columns of a row that hold an infinity, a NaN or a sum beyond float32 are worked out again on the float32 instruction: an infinity has no rest.
+// Four columns of a row that hold an infinity, a NaN or a sum beyond float32 are worked out again on the float32 instruction: an infinity has no rest.  And so are four of which one is below 2^-64
+// and not 0: bfloat16 ends where float32 does, so a number below 2^-110 loses the bits of its third part (at 2^-118 1.5e-5 of itself), at most 2^-126 of each.  Such losses come to less
+// than a rounding of a sum of 2^-64 and more while the rows' absolute sums are below 2^37; what is made of such numbers alone is smaller.
 __host__ __device__ __forceinline__ int f32_split_part_length(int K) { return ((K + F32_PARTS - 1) / F32_PARTS + 63) / 64 * 64; }
 typedef __attribute__((ext_vector_type(8))) __bf16 f32_part8_t;
 typedef __attribute__((ext_vector_type(2))) __bf16 f32_part2_t;
@@ -1959,8 +1961,18 @@ __device__ __forceinline__ f32x4_t f32_whole_sum(int K, const float* w_row, cons
     }
     return total + acc[0][0];
 }
-__device__ __forceinline__ bool f32_all_finite(f32x4_t v) {
-    return fabsf(v[0]) < INFINITY && fabsf(v[1]) < INFINITY && fabsf(v[2]) < INFINITY && fabsf(v[3]) < INFINITY;
+// Whether four sums of products taken apart stand (or eight, `other`): finite, and zero or not so small that numbers below 2^-110 may be what they are made of.  (In whole numbers, least and largest
+// of all: a comparison each, with what joins them, is a chain between the vector and the scalar unit at the end of a kernel of 5 us.)
+__device__ __forceinline__ bool f32_sums_stand(f32x4_t v, f32x4_t other) {
+    constexpr uint32_t LEAST = 2u * (127 - 64) << 23, INFINITE = 2u * 255 << 23;      // (without the sign, one place up)
+    uint32_t low = 0xffffffffu, high = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t a = __float_as_uint(v[i]) << 1, b = __float_as_uint(other[i]) << 1;
+        low = min(low, min(a - 1, b - 1));        // (0 becomes the largest)
+        high = max(high, max(a, b));
+    }
+    return (low >= LEAST - 1) & (high < INFINITE);
 }
 
 // What columns n .. n + 3 of logical row ml need on their way out besides the product: a kernel whose last wait is for its operands
@@ -2368,7 +2380,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(GemmArgs g) {
         for (int j = 0; j < NT; j += PER) {
             const int n = n0 + j / PER * 16 + 4 * gq;
             const f32x4_t v = total[i][j] + acc[i][j], v2 = ROLES ? other[wave * MB + i][lane] : DUAL ? total[i][j + PER - 1] + acc[i][j + PER - 1] : v;
-            if (!(f32_all_finite(v) && f32_all_finite(v2))) odd |= 1u << (i * (NT / PER) + j / PER);
+            if (!f32_sums_stand(v, DUAL ? v2 : v)) odd |= 1u << (i * (NT / PER) + j / PER);
             else f32_store4<DUAL, EPI>(g, f32_ask<DUAL, EPI>(g, ml, min(n, g.N - 1)), n, v, v2);
         }
     }
@@ -2523,7 +2535,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
         for (int p = 1; p < F32_PARTS; ++p) v2 += red[p][ti * NW + ta + PER - 1][lane];
     }
     if constexpr (SPLIT) {
-        const bool odd = finishes && !(f32_all_finite(v) && f32_all_finite(v2));
+        const bool odd = finishes && !f32_sums_stand(v, DUAL ? v2 : v);
         if (__ballot(odd)) {            // (the whole wave: the products take all its lanes)
             const int m = min(r0 + ti * 16 + li, r_end - 1), n = min(n0 + (DUAL ? ta >> 1 : ta) * CW + (HALF ? li & 7 : li), g.N - 1);
             const float *x_row = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda, *w_row = Wbase + (size_t)n * g.K;

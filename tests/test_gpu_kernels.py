@@ -218,6 +218,33 @@ def test_float32_parts_leave_what_is_not_finite_to_the_float32_instruction(tile)
         assert torch.equal(got[~odd], clean[~odd]) and bool(odd.any()) and not bool(odd.all())
 
 
+@pytest.mark.parametrize("tile", [1, 32, 64, 128])
+def test_float32_parts_leave_the_smallest_numbers_to_the_float32_instruction(tile):
+    """Rows of numbers whose parts are below what bfloat16 holds, weights and activations, and rows of nothing: the float32 instruction's bits, and those of the
+    rows beside them as without them."""
+    from ferrox_amd import debug, ops
+    M, N, K = 70, 72, 96
+    a, w = rnd(M, K), torch.cat([rnd(N, K, seed=1), rnd(N, K, seed=2)])
+    small_a, small_w = a.clone(), w.clone()
+    rows = {3: 2.0 ** -90, 4: 2.0 ** -108, 17: 2.0 ** -114, 20: 2.0 ** -119, 33: 2.0 ** -123, 66: 0.0}
+    for m, scale in rows.items():
+        small_a[m] *= scale
+    for n, scale in {8: 2.0 ** -90, 9: 2.0 ** -112, 10: 2.0 ** -118, 11: 2.0 ** -121}.items():         # (four columns of their own)
+        small_w[n] *= scale
+        small_w[N + n] *= scale
+    for kw, some in ((dict(epilogue=ops.EPI_STORE_F32), lambda x: x[:N].contiguous()), (dict(epilogue=ops.EPI_GATED, activation="relu"), lambda x: x)):
+        with debug.kernel_switch("gemm", "f32_tile", tile):
+            with debug.kernel_switch("gemm", "f32_split", 1):
+                clean, got = ops.gemm(a, some(w), **kw), ops.gemm(small_a, some(small_w), **kw)
+            with debug.kernel_switch("gemm", "f32_split", 0):
+                want = ops.gemm(small_a, some(small_w), **kw)
+        odd = torch.zeros(M, N, dtype=torch.bool, device=DEV)
+        odd[list(rows)] = True
+        odd[:, 8:12] = True
+        assert torch.equal(got[odd], want[odd]) and torch.equal(got[~odd], clean[~odd]), kw
+        assert bool((got[66] == 0).all())
+
+
 @pytest.mark.parametrize("T,E,k,I,H", [(1, 5, 2, 20, 36), (3, 60, 4, 96, 128), (90, 7, 3, 33, 50), (700, 4, 2, 64, 96)])
 def test_float32_grouped_products_have_the_same_bits_in_every_kernel(T, E, k, I, H):
     from ferrox_amd import debug, ops

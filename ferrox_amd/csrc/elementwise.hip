@@ -328,8 +328,8 @@ FX_API int fx_rmsnorm(void* stream, int out_dtype, const float* h, const int* ro
 // Values of many tokens into their transposed pages: a block takes 64 tokens and 4 G pieces of G dimensions of the token's kv heads (G elements: 16 bytes), a thread G tokens of a
 // piece: one 16-byte load a token, G x G elements turned in registers, one 16-byte store a dimension, which with its neighbours' makes a whole line of a page.  The G tokens are those that
 // start at a multiple of G in a page, wherever that is in the step (behind decoded sequences a prompt starts at any token); tokens without G - 1 others go out element by element.
-// us, eight tokens of a head a block with a 2-byte load an element / so, rotation of q and k included: 16 heads of 128 in bfloat16, 1,024 tokens 8.5 / 7.0, 2,048 13.9 / 11.1, 2,048 behind
-// 15 decoded 27.1 / 13.8, 4,096 behind 7 50.6 / 20.9, in float32 700 13.9 / 9.3, 2,048 33.5 / 19.1.
+// us with rows from memory, eight tokens of a head a block with a 2-byte load an element / so, rotation of q and k included: 16 heads of 128 in bfloat16, 1,024 tokens 10.0 / 8.3, 2,048 16.3 / 14.7,
+// 2,048 behind 15 decoded 35.4 / 18.6, 4,096 behind 7 66 / 26.4, in float32 700 20.5 / 13.6, 2,048 46.5 / 25.1.
 template <typename T>
 __device__ __forceinline__ void write_many_values(int b, const T* __restrict__ v, int ldv, const int* __restrict__ positions,
                                                   const int* __restrict__ token_seq, const int* __restrict__ block_table,
@@ -412,7 +412,7 @@ __device__ __forceinline__ void write_many_values(int b, const T* __restrict__ v
 }
 // How many blocks that takes, or 0 where its 16-byte pieces do not fit or the step has fewer than two million bfloat16 or half a million float32 values: its two looks at the tokens around
 // come before its first load (us, eight tokens a block / 64: 512 tokens of 16 heads of 128 5.7 / 5.9, 700 7.2 / 7.8; float32, 128 decoded 7.6 / 8.7, 300 8.0 / 6.4).
-static long many_value_blocks(long T, int nkv, int vd, int bs, int dtype, const void* v, long ldv, const void* v_pages) {
+FX_API long fx_many_value_blocks(long T, int nkv, int vd, int bs, int dtype, const void* v, long ldv, const void* v_pages) {
     const int G = dtype == FX_F32 ? 4 : 8;
     if (T * nkv * vd < (dtype == FX_F32 ? 1L << 19 : 1L << 21) || bs % G || vd % G || ldv % G || (((uintptr_t)v | (uintptr_t)v_pages) % 16)) return 0;
     return (T + 63) / 64 * (((long)nkv * (vd / G) + 4 * G - 1) / (4 * G));
@@ -454,24 +454,30 @@ __device__ __forceinline__ void write_values(int b, const T* __restrict__ v, int
     }
 }
 
-// The first T * split blocks rotate: `split` blocks share a token, each computes the angles' sines
+// T * split blocks rotate: `split` blocks share a token, each computes the angles' sines
 // and cosines once and takes its part of the heads of q (in place) and of k (into its page); few
-// tokens get several blocks each, many tokens one.  The blocks after them write v: one block per (eight
+// tokens get several blocks each, many tokens one.  Behind them stand blocks that write v: one block per (eight
 // consecutive tokens, kv head), so that eight tokens that follow each other in one page go out as
-// one 16-byte store per head dimension into the transposed page, or `write_many_values`.  (Eight blocks a CU: with the registers
-// of the values' part a rotating block of 2,048 tokens would have seven beside it.)
-template <typename T>
-__global__ __launch_bounds__(256, 8) void rope_kv_write_kernel(
+// one 16-byte store per head dimension into the transposed page.  Or, MANY, in front of them `value_blocks` blocks of `write_many_values`: fewer and longer ones, which
+// behind the others would be what the launch ends with (us with rows from memory, eight tokens a block / behind / in front: bfloat16, 16 heads of 128, 1,024 tokens 10.0 9.2 8.3, 2,048 16.3 18.0 14.7; 28
+// heads on 4, 4,096 tokens 20.7 23.6 19.2; float32, 4,096 tokens 84.7 46.5 44.6; 1,024 single tokens of 32 heads 192 201 201).
+template <typename T, bool MANY>
+__global__ __launch_bounds__(256) void rope_kv_write_kernel(
     T* __restrict__ q, int ldq, const T* __restrict__ k, int ldk, const T* __restrict__ v, int ldv,
     const int* __restrict__ positions, const int* __restrict__ token_seq,
     const int* __restrict__ block_table, int max_blocks, T* __restrict__ k_pages, T* __restrict__ v_pages,
     int n_tokens, int split, int nh, int nkv, int hd, int bs, int rot, int interleaved, const float* __restrict__ inv_freq, int vec8,
-    const float* __restrict__ freq_factors, int vd, int many) {
+    const float* __restrict__ freq_factors, int vd, int value_blocks) {
     __shared__ float cs[128], sn[128];     // rot / 2 <= 128
     const int tid = threadIdx.x;
     const int half = rot >> 1;
-    if ((int)blockIdx.x < n_tokens * split) {
-        const int t = blockIdx.x / split, part = blockIdx.x % split, step = 256 * split;
+    if (MANY && (int)blockIdx.x < value_blocks) {
+        write_many_values<T>(blockIdx.x, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
+        return;
+    }
+    const int block = blockIdx.x - (MANY ? value_blocks : 0);
+    if (MANY || block < n_tokens * split) {
+        const int t = block / split, part = block % split, step = 256 * split;
         const int pos = positions[t];
         for (int p = tid; p < half; p += 256) {
             float angle = (float)pos * inv_freq[p];
@@ -534,9 +540,7 @@ __global__ __launch_bounds__(256, 8) void rope_kv_write_kernel(
         }
         return;
     }
-    if (!v_pages) return;
-    if (many) write_many_values<T>(blockIdx.x - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
-    else write_values<T>(blockIdx.x - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
+    if (v_pages) write_values<T>(block - n_tokens * split, v, ldv, positions, token_seq, block_table, max_blocks, v_pages, n_tokens, nkv, bs, vd);
 }
 
 FX_API int fx_rope_kv_write(void* stream, int dtype, void* q, int ldq, const void* k, int ldk,
@@ -553,22 +557,22 @@ FX_API int fx_rope_kv_write(void* stream, int dtype, void* q, int ldq, const voi
     if (T == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     const int split = T <= 32 ? 8 : (T <= 128 ? 2 : 1);
-    const long many = v_pages ? many_value_blocks(T, nkv, vd, bs, dtype, v, ldv, v_pages) : 0;
+    const long many = v_pages ? fx_many_value_blocks(T, nkv, vd, bs, dtype, v, ldv, v_pages) : 0;
     const long n_blocks = (long)T * split + (many ? many : v_pages ? (long)((T + 7) / 8) * nkv : 0);
     FX_REQUIRE(n_blocks < (1L << 31), "rope_kv_write: too many tokens and heads for one launch");
     const unsigned blocks = (unsigned)n_blocks;
     const int vec8 = dtype == FX_BF16 && !interleaved && rot % 16 == 0 && hd % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 &&
                      ((uintptr_t)q % 16) == 0 && ((uintptr_t)k % 16) == 0 && (!k_pages || ((uintptr_t)k_pages % 16) == 0);
-    if (dtype == FX_F32)
-        rope_kv_write_kernel<float><<<blocks, 256, 0, s>>>((float*)q, ldq, (const float*)k, ldk, (const float*)v, ldv,
-                                                           positions, token_seq, block_table, max_blocks,
-                                                           (float*)k_pages, (float*)v_pages, T, split, nh, nkv, hd, bs, rot,
-                                                           interleaved, inv_freq, 0, freq_factors, vd, many > 0);
-    else if (dtype == FX_BF16)
-        rope_kv_write_kernel<bf16><<<blocks, 256, 0, s>>>((bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv,
-                                                          positions, token_seq, block_table, max_blocks,
-                                                          (bf16*)k_pages, (bf16*)v_pages, T, split, nh, nkv, hd, bs, rot,
-                                                          interleaved, inv_freq, vec8, freq_factors, vd, many > 0);
+    auto go = [&](auto* typed, auto with_many) {
+        typedef std::remove_pointer_t<decltype(typed)> T_;
+        rope_kv_write_kernel<T_, decltype(with_many)::value><<<blocks, 256, 0, s>>>((T_*)q, ldq, (const T_*)k, ldk, (const T_*)v, ldv, positions, token_seq, block_table, max_blocks,
+                                                                                   (T_*)k_pages, (T_*)v_pages, T, split, nh, nkv, hd, bs, rot, interleaved, inv_freq,
+                                                                                   dtype == FX_BF16 ? vec8 : 0, freq_factors, vd, (int)many);
+    };
+    if (dtype == FX_F32 && many) go((float*)nullptr, std::true_type{});
+    else if (dtype == FX_F32) go((float*)nullptr, std::false_type{});
+    else if (dtype == FX_BF16 && many) go((bf16*)nullptr, std::true_type{});
+    else if (dtype == FX_BF16) go((bf16*)nullptr, std::false_type{});
     else
         return fx_fail("rope_kv_write: unknown dtype %d", dtype);
     FX_CHECK_LAUNCH("rope_kv_write");

@@ -263,3 +263,19 @@ def test_float32_products_from_parts_by_the_weights_alone():
             assert instruction or not rule(weights[0], weights[1]), T
     finally:
         ops.gemm = plain_gemm
+
+
+def test_values_go_out_in_windows_of_64_tokens_from_a_number_of_them_on():
+    """Two million bfloat16 values or half a million float32 ones, where 16-byte pieces of rows and of pages fit; a block of 64 tokens takes 4 G pieces of G elements."""
+    import ctypes
+    from ferrox_amd.csrc.build import load_library
+    rule = load_library("elementwise").fx_many_value_blocks
+    rule.restype = ctypes.c_long
+    rule.argtypes = [ctypes.c_long] + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p]
+    f32, bf16 = 0, 1
+    assert rule(1024, 16, 128, 64, bf16, 4096, 6144, 4096) == 16 * 8 and rule(1023, 16, 128, 64, bf16, 4096, 6144, 4096) == 0
+    assert rule(256, 16, 128, 64, f32, 4096, 6144, 4096) == 4 * 32 and rule(255, 16, 128, 64, f32, 4096, 6144, 4096) == 0
+    assert rule(2048, 11, 136, 16, bf16, 4096, 6144, 4096) == 32 * 6                    # (187 pieces of 8, 32 a block)
+    for bs, vd, ldv, v, pages in ((20, 128, 6144, 4096, 4096), (64, 132, 6144, 4096, 4096), (64, 128, 6148, 4096, 4096), (64, 128, 6144, 4104, 4096), (64, 128, 6144, 4096, 4104)):
+        assert rule(4096, 16, vd, bs, bf16, v, ldv, pages) == 0
+    assert rule(4096, 16, 132, 20, f32, 4096, 6148, 4096) > 0

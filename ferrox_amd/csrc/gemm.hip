@@ -1925,6 +1925,21 @@ __device__ __forceinline__ F32Split f32_split8(f32x4_t lo, f32x4_t hi) {
     s.l = __builtin_bit_cast(f32_part8_t, make_uint4(l0.x, l0.y, l1.x, l1.y));
     return s;
 }
+// the operand of eight rows from a lane's four k: its own, then those of the lane that has the row's other 16 (taken apart once, then handed over)
+template <bool NEG>
+__device__ __forceinline__ F32Split f32_split_half(f32x4_t own) {
+    uint2 h, m, l;
+    f32_split4<NEG>(own, h, m, l);
+    auto both = [](uint2 v) {
+        const uint32_t x = __builtin_amdgcn_update_dpp(v.x, v.x, 0x128, 0xF, 0x3, false), y = __builtin_amdgcn_update_dpp(v.y, v.y, 0x128, 0xF, 0x3, false);      // (as `swap_halves<0x3>`)
+        return __builtin_bit_cast(f32_part8_t, make_uint4(v.x, v.y, x, y));
+    };
+    F32Split s;
+    s.h = both(h);
+    s.m = both(m);
+    s.l = both(l);
+    return s;
+}
 // 32 k of a tile: the small terms first
 #define FX_MFMA32(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 template <bool NEG, int MT, int NT>
@@ -2416,14 +2431,19 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     const int n0 = blockIdx.x * (DUAL ? CW / 2 : CW) * NW;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
     const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
-    const float* x_src[MT];
+    // SPLIT: the rows come in whole lines as well, the first load of 32 k with rows 0 .. 7 of a tile and the second with rows 8 .. 15, which a tile of up to eight rows does without
+    constexpr bool XLINES = LINES && SPLIT;
+    const float* x_src[MT][XLINES ? 2 : 1];
     constexpr int WR = LINES && !HALF ? 2 : 1;
     const float* w_src[NW][WR];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-        int m = r0 + i * 16 + li;
-        m = m < r_end ? m : r_end - 1;
-        x_src[i] = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda;
+#pragma unroll
+        for (int half = 0; half < (XLINES ? 2 : 1); ++half) {
+            int m = r0 + i * 16 + (XLINES ? (li & 7) + 8 * half : li);
+            m = m < r_end ? m : r_end - 1;
+            x_src[i][half] = (const float*)g.A + (size_t)(g.a_rows ? g.a_rows[m] : m) * g.lda + (XLINES ? (li >> 3) * 16 + gq * 4 : 0);
+        }
     }
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
@@ -2440,7 +2460,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     constexpr int STEP = 2;       // groups of 16 k that are on their way together
     f32x4_t w[2][STEP][NW], x[2][STEP][MT];
     const int k_full = k_first + (k_end - k_first) / 16 * 16;
-    auto fetch = [&](int b, int k0) {
+    auto fetch = [&](auto x_loads, int b, int k0) {
 #pragma unroll
         for (int c = 0; c < STEP; ++c) {
             const int kc = k0 + c * 16, k = (kc < k_full ? kc : k_full - 16) + gq * 4;
@@ -2455,7 +2475,10 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
                 }
             }
 #pragma unroll
-            for (int i = 0; i < MT; ++i) x[b][c][i] = f32_fetch<VEC>(x_src[i] + k);
+            for (int i = 0; i < MT; ++i) {
+                if constexpr (!XLINES) x[b][c][i] = f32_fetch<VEC>(x_src[i][0] + k);
+                else if (c < decltype(x_loads)::value) x[b][c][i] = f32_fetch<VEC>(x_src[i][c] + (k0 < k_full ? k0 : k_full - 32));
+            }
         }
     };
     // the tile that this wave finishes, and what that needs besides the product
@@ -2470,13 +2493,13 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int a = 0; a < NW; ++a) acc[i][a] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    if (k_first < k_full) {
-        fetch(0, k_first);
+    auto loop = [&](auto x_loads) {
+        fetch(x_loads, 0, k_first);
         for (int k0 = k_first; k0 < k_full; k0 += 2 * STEP * 16) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const int kb = k0 + b * STEP * 16;
-                fetch(b ^ 1, kb + STEP * 16);
+                fetch(x_loads, b ^ 1, kb + STEP * 16);
                 // what the lane multiplies of weight set a in group c of 16 k
                 auto own = [&](int c, int a) -> f32x4_t {
                     if constexpr (!LINES) return w[b][c][a];
@@ -2489,14 +2512,26 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
                     if (kb < k_full) {          // (whole steps of 32 k)
                         F32Split ws[NW], xs[MT];
 #pragma unroll
-                        for (int a = 0; a < NW; ++a) ws[a] = f32_split8<false>(own(0, a), own(1, a));
+                        for (int a = 0; a < NW; ++a) {
+                            if constexpr (HALF) ws[a] = f32_split_half<false>(w[b][0][a]);
+                            else ws[a] = f32_split8<false>(own(0, a), own(1, a));
+                        }
+                        auto rows_of = [&](auto neg, int i) {
+                            constexpr bool NEG = decltype(neg)::value;
+                            if constexpr (!XLINES) return f32_split8<NEG>(x[b][0][i], x[b][1][i]);
+                            else if constexpr (decltype(x_loads)::value == 1) return f32_split_half<NEG>(x[b][0][i]);
+                            else {
+                                const uint4 one = __builtin_bit_cast(uint4, x[b][0][i]), two = __builtin_bit_cast(uint4, x[b][1][i]);
+                                return f32_split8<NEG>(__builtin_bit_cast(f32x4_t, swap_halves<0xC>(one, two)), __builtin_bit_cast(f32x4_t, swap_halves<0x3>(two, one)));
+                            }
+                        };
                         if (b & 1) {
 #pragma unroll
-                            for (int i = 0; i < MT; ++i) xs[i] = f32_split8<true>(x[b][0][i], x[b][1][i]);
+                            for (int i = 0; i < MT; ++i) xs[i] = rows_of(std::true_type{}, i);
                             f32_split_multiply<true>(acc, ws, xs);
                         } else {
 #pragma unroll
-                            for (int i = 0; i < MT; ++i) xs[i] = f32_split8<false>(x[b][0][i], x[b][1][i]);
+                            for (int i = 0; i < MT; ++i) xs[i] = rows_of(std::false_type{}, i);
                             f32_split_multiply<false>(acc, ws, xs);
                         }
                     }
@@ -2512,12 +2547,16 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
                     }
             }
         }
+    };
+    if (k_first < k_full) {
+        if (XLINES && MT == 1 && r_end - r0 <= 8) loop(fx_int<1>{});
+        else loop(fx_int<2>{});
     }
     if (!LINES && !SPLIT && k_first < k_end && k_full < k_end) {       // the last, partial group of K
 #pragma unroll
         for (int a = 0; a < NW; ++a) w[0][0][a] = f32_fetch_guarded<VEC>(w_src[a][0], k_full + gq * 4, k_end);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) x[0][0][i] = f32_fetch_guarded<VEC>(x_src[i], k_full + gq * 4, k_end);
+        for (int i = 0; i < MT; ++i) x[0][0][i] = f32_fetch_guarded<VEC>(x_src[i][0], k_full + gq * 4, k_end);
         f32_multiply(acc, w[0][0], x[0][0]);
     }
 #pragma unroll

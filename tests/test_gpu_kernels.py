@@ -2068,3 +2068,25 @@ def test_products_of_four_row_tiles_have_the_bits_of_one(M, N, K, epi):
     for m in range(0, M, 16):
         ops.gemm(a[m:m + 16], w, epilogue=epi, out=parts[m:m + 16])
     assert torch.equal(whole, parts)
+
+
+@pytest.mark.parametrize("K", [96, 1056, 2112])
+@pytest.mark.parametrize("N", [8, 264, 2056])
+def test_few_float32_rows_from_parts_in_whole_lines_and_in_half(N, K):
+    """The product for few rows fetches up to eight rows of a tile with one load of whole lines and more with two: at 7, 8, 9, 15, 16, 17 and 25 rows, plain
+    and of experts with so many, the bits of tiles."""
+    from ferrox_amd import debug, ops
+    a, w = rnd(34, K), torch.stack([rnd(2 * N, K, seed=1), rnd(2 * N, K, seed=2)])
+    with debug.kernel_switch("gemm", "f32_split", 1):
+        for kw, some in ((dict(epilogue=ops.EPI_STORE_F32), lambda x: x[..., :N, :].contiguous()), (dict(epilogue=ops.EPI_GATED), lambda x: x)):
+            one, both = some(w[0]), some(w)
+            with debug.kernel_switch("gemm", "f32_tile", 32):
+                want, other = ops.gemm(a, one, **kw), ops.gemm(a, some(w[1]), **kw)
+            for rows in (1, 7, 8, 9, 15, 16, 17, 25, 32):
+                offsets = torch.tensor([0, rows, 34], dtype=torch.int32, device=DEV)
+                for half in (-1, 0, 1) if rows <= 16 else (-1,):
+                    with debug.kernel_switch("gemm", "f32_tile", 1), debug.kernel_switch("gemm", "skinny_half", half):
+                        assert torch.equal(ops.gemm(a[:rows], one, **kw), want[:rows]), (rows, half)
+                with debug.kernel_switch("gemm", "f32_tile", 1):
+                    got = ops.gemm(a, both, expert_offsets=offsets, n_rows=34, **kw)
+                assert torch.equal(got[:rows], want[:rows]) and torch.equal(got[rows:], other[rows:]), rows

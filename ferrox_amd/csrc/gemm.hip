@@ -2885,17 +2885,23 @@ FX_API int fx_gemm_half_sets(int M, int N, int dual, int sets, int cus) {
 }
 
 // Whether a float32 product is worked out from operands taken apart into bfloat16 ones (gemm_f32_split_kernel, and in the kernel for few rows): by the weights alone, so that the bits of a row
-// do not depend on the rows beside it.  Whole steps of 32 k; sums of 1,024 and more, where the error is a third of the float32 instruction's (it is level around 256); and weights of a million numbers, below which the
-// products are a few microseconds either way and some have their sums repeated elsewhere in the float32 order (`f32_ordered_dot`).
-FX_API int fx_gemm_f32_split(int N, int K) { return K % 32 == 0 && K >= 1024 && (long)N * K >= 1L << 20; }
+// do not depend on the rows beside it.  Whole steps of 32 k; sums of 1,024 and more, where the error is a third of the float32 instruction's (it is level around 256); and weights of more than a million numbers, up to which the
+// products are a few microseconds either way (us of 1,024 x 1,024, float32 instruction / taken apart: 1 row 4.5 4.6, 48 rows 13.4 14.4, 256 14.1 15.0, 512 18.6 16.2; of 512 x 2,048 1 row 6.1 6.2, 48 rows 23.6 23.5) and some have their sums repeated elsewhere in the float32 order (`f32_ordered_dot`).
+FX_API int fx_gemm_f32_split(int N, int K) { return K % 32 == 0 && K >= 1024 && (long)N * K > 1L << 20; }
 
 // The tile of such a product of plain rows, more than a few: its rows (32, 48 or 64) by 64 columns, or, as 128, 144 and 160, 64, 48 or 32 rows by 128
 // columns (dual: half as many of both matrices).  The time goes with how many blocks the busiest CU gets: us of a first block, of each further one and beside them, of 2,048 k
 // (1 to 6 blocks; up to 32 rows 32 x 64, one reading of the weights: 32 x 64 25 40 60 76 93 115; 48 x 64 34 50 70 88 104 131; 64 x 64 42 57 85 113 131 172; 32 x 128 49 70 107 137; 48 x 128 51 83 127 154 205 248; 64 x 128 59 92 141 184 229); other k in proportion.
+// (whether blocks of 64 columns, of dual 32 of both matrices, are at most one a CU)
+static bool fx_gemm_f32_one_round(int N, int dual, int cus) { return ceil_div(N, dual ? 32 : 64) <= cus; }
 FX_API int fx_gemm_f32_split_tile(int M, int N, int dual, int cus) {
     static const struct { int code, rows, columns; float first, each, beside; } kinds[] = {
         {32, 32, 64, 25, 18.5f, 4}, {48, 48, 64, 34, 20.5f, 8}, {64, 64, 64, 42, 28.3f, 0}, {160, 32, 128, 49, 33, 5}, {144, 48, 128, 51, 41, 3}, {128, 64, 128, 59, 46, 2}};
     if (M <= 32) return 32;
+    // Up to 64 rows while one row tile's blocks are one a CU: 32 x 64, two row tiles, where those are one block a CU too, else one row tile, so that the weights are read once, in whole lines and two stages ahead (us with weights from memory, float32
+    // instruction / 32 x 64 / so: 33 rows and gate/up of 5,632 42.6 43.3 37.7, of 8,192 50.2 53.3 38.6, 64 rows 44.2 45.8 43.1 and 51.4 55.4 45.9, 48 rows against 9,216 40.6 39.2 36.4; gate/up of 4,096, 256
+    // such blocks, 33 rows 31.0 26.9 37.4, 64 rows 31.9 27.8 43.0; with more blocks the table below is ahead of it: 64 rows against 40,960 weight rows 98 and 104).
+    if (M <= 64 && fx_gemm_f32_one_round(N, dual, cus)) return 2L * ceil_div(N, dual ? 32 : 64) <= cus ? 32 : 64;
     int best = 128;
     float least = INFINITY;
     for (const auto& k : kinds) {
@@ -3162,7 +3168,8 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
                 if (tile != 64) tile = 128;
                 else stream = group <= 12 ? 2 : (group <= 24 ? 1 : 0);
             } else if (!(tile == 32 || (split && (tile == 48 || tile == 128 || tile == 144 || tile == 160)))) tile = 64;
-            if (split && tile == 32 && M <= 32) stream = 1;
+            if (split && !expert_offsets && tile == 32 && M <= 32) stream = 1;
+            if (split && !expert_offsets && tile == 64 && M <= 64 && fx_gemm_f32_one_round(N, dual, (int)cus)) stream = 2;
         }
         if (!tile) {
             mt = group <= 16 ? 1 : 2;

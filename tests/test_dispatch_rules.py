@@ -237,7 +237,7 @@ def test_the_chunk_rule_leaves_the_callers_arguments_alone():
 
 
 def test_float32_products_from_parts_by_the_weights_alone():
-    """Whole steps of 32 k, sums of 1,024 and more, weights of a million numbers; the router's product, whose rows stand where weights do, is left out of the
+    """Whole steps of 32 k, sums of 1,024 and more, weights of more than a million numbers; the router's product, whose rows stand where weights do, is left out of the
     rule: no number of tokens changes how its float32 operands are multiplied."""
     from types import SimpleNamespace
     import torch
@@ -245,7 +245,7 @@ def test_float32_products_from_parts_by_the_weights_alone():
     from ferrox_amd.csrc.build import load_library
     from ferrox_amd.parts.moe import SparseMoE
     rule = load_library("gemm").fx_gemm_f32_split
-    assert rule(2048, 2048) and rule(6144, 2048) and rule(1408, 2048) and rule(151936, 2048)
+    assert rule(2048, 2048) and rule(6144, 2048) and rule(1408, 2048) and rule(151936, 2048) and rule(1025, 1024) and not rule(1024, 1024)
     assert not rule(2048, 2056) and not rule(4096, 992) and not rule(60, 2048) and not rule(256, 2048)
     asked = []
 
@@ -279,3 +279,15 @@ def test_values_go_out_in_windows_of_64_tokens_from_a_number_of_them_on():
     for bs, vd, ldv, v, pages in ((20, 128, 6144, 4096, 4096), (64, 132, 6144, 4096, 4096), (64, 128, 6148, 4096, 4096), (64, 128, 6144, 4104, 4096), (64, 128, 6144, 4096, 4104)):
         assert rule(4096, 16, vd, bs, bf16, v, ldv, pages) == 0
     assert rule(4096, 16, 132, 20, f32, 4096, 6148, 4096) > 0
+
+
+def test_tiles_of_float32_products_from_parts():
+    """Up to 32 rows tiles of 32; up to 64 rows one row tile, or two of 32 where those are one block a CU, while one row tile's blocks are; beyond that by what the CU with the most
+    blocks takes."""
+    from ferrox_amd.csrc.build import load_library
+    rule = lambda m, n, dual=0, cus=256: load_library("gemm").fx_gemm_f32_split_tile(m, n, dual, cus)
+    assert [rule(m, 6144) for m in (1, 32)] == [32, 32]
+    assert [rule(m, n) for m in (33, 64) for n in (2048, 8192, 8256, 16384)] == [32, 32, 64, 64] * 2
+    assert [rule(m, n, 1) for m in (33, 64) for n in (4096, 4128, 8192)] == [32, 64, 64] * 2
+    assert [rule(m, n) for m in (33, 64) for n in (16448, 40960)] == [48, 48, 64, 64]
+    assert rule(65, 2048) == 32 and rule(700, 6144) == 144 and rule(700, 2048) == 48 and rule(700, 1024) == 48

@@ -2090,3 +2090,30 @@ def test_few_float32_rows_from_parts_in_whole_lines_and_in_half(N, K):
                 with debug.kernel_switch("gemm", "f32_tile", 1):
                     got = ops.gemm(a, both, expert_offsets=offsets, n_rows=34, **kw)
                 assert torch.equal(got[:rows], want[:rows]) and torch.equal(got[rows:], other[rows:]), rows
+
+
+@pytest.mark.parametrize("K", [96, 128, 160, 192])
+@pytest.mark.parametrize("shares,stream", [((0, 1, 17, 8, 0, 12, 5, 3), 2), ((0, 1, 49, 0, 3, 17, 0, 26), 2), ((0, 1, 17, 49, 64, 3, 5, 30), 1), ((65, 0, 1, 17, 0, 49, 3, 50), 1),
+                                            ((130, 65, 64, 63, 0, 1, 17, 49), 0)])
+def test_float32_experts_from_parts_with_their_weights_in_whole_lines(K, shares, stream):
+    """Rows sorted by expert in tiles of 64: up to 12 rows an expert on average with whole lines two stages ahead, up to 24 one stage, beyond without; shares at the edges of row blocks
+    and tiles, none at all, every number of steps beside the stages.  The bits of the product for few rows, also beside operands that are not finite."""
+    from ferrox_amd import debug, ops
+    E, N, M = len(shares), 136, sum(shares)
+    average = -(-M // E)
+    assert (2 if average <= 12 else 1 if average <= 24 else 0) == stream
+    a, w = rnd(M, K), rnd(E, 2 * N, K, seed=1)
+    bad_a, bad_w = a.clone(), w.clone()
+    bad_a[M // 2, 5], bad_a[M - 1, K - 1], bad_w[2, 17, 3], bad_w[5, N + 30, 0] = math.inf, math.nan, -math.inf, math.nan
+    offsets = torch.tensor([sum(shares[:e]) for e in range(E + 1)], dtype=torch.int32, device=DEV)
+    for x, weights in ((a, w), (bad_a, bad_w)):
+        for kw, some in ((dict(epilogue=ops.EPI_STORE_F32), lambda t: t[:, :N].contiguous()), (dict(epilogue=ops.EPI_GATED), lambda t: t)):
+            got = {}
+            for split, tile in ((1, 1), (1, 0), (1, 64), (1, 128), (0, 0)):
+                with debug.kernel_switch("gemm", "f32_split", split), debug.kernel_switch("gemm", "f32_tile", tile):
+                    got[split, tile] = torch.nan_to_num(ops.gemm(x, some(weights), expert_offsets=offsets, n_rows=M, **kw), nan=7e30, posinf=8e30, neginf=-8e30)
+            for tile in (0, 64, 128):
+                assert torch.equal(got[1, tile], got[1, 1]), (tile, kw)
+            odd = got[0, 0].abs() > 1e30
+            assert torch.equal(got[1, 1][odd], got[0, 0][odd])
+            close(got[1, 1][~odd], got[0, 0][~odd], torch.float32, "float32 instruction")

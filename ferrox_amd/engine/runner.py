@@ -126,11 +126,12 @@ class DecodeGraph:
             # GB in the cache costs a recording several hundred milliseconds)
             main, side = torch.cuda.current_stream(), runner.capture_stream
             side.wait_stream(main)
+            ctx = self._context(runner)         # (its events go when the recording that they are part of has ended)
             try:
                 with torch.cuda.stream(side):
                     graph.capture_begin()
                     try:
-                        self.logits = model.forward(self._context(runner), caches)
+                        self.logits = model.forward(ctx, caches)
                     finally:
                         graph.capture_end()
             finally:

@@ -154,6 +154,7 @@ class StepContext:
     carry: object = None               # what a feed-forward hands on to the next block (its rows, normed), see PreNormBlock
     waiting: list = field(default_factory=list)      # products (ops.Product) that a block has left for its mixer's launches, see `linear.matmul_with`
     owed: object = None                # float32 rows that one of them has stored, which the mixer's last product adds behind its own
+    events: list = field(default_factory=list)       # what the step's launches on other streams wait for: kept until the step has been launched, or its recording has ended
     _memo: dict = field(default_factory=dict)
 
     def memo(self, key, make: Callable):

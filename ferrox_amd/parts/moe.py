@@ -246,6 +246,7 @@ class SparseMoE(FeedForward):
             # blocks of one fill the CUs that the last round of the other's tiles leaves idle
             main, side = torch.cuda.current_stream(), side_stream(x.device)
             fork, join = torch.cuda.Event(), torch.cuda.Event()
+            ctx.events += (fork, join)      # (a recording goes on behind this call, and these two are part of it)
             fork.record(main)
             side.wait_event(fork)
             with torch.cuda.stream(side):

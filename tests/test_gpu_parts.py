@@ -618,7 +618,7 @@ def test_a_float32_token_gets_the_same_bits_however_many_tokens_stand_beside_it(
 
     def run(a, b):
         out = torch.zeros(b - a, H, device="cuda:0")
-        moe.forward(x[a:b], SimpleNamespace(act_dtype=torch.float32, carry=None), out)
+        moe.forward(x[a:b], SimpleNamespace(act_dtype=torch.float32, carry=None, events=[]), out)
         return out
 
     whole = run(0, T)

@@ -63,3 +63,46 @@ def test_a_step_that_was_never_recorded_waits_for_nothing(made):
     runner = make(0)
     DecodeGraph(runner, 1, 64)
     assert log == []
+
+
+def test_events_of_a_step_live_until_its_recording_has_ended(made, monkeypatch):
+    """What a part leaves in the context's events, the events of launches on another stream, is there when the recording ends, and gone once the step is recorded."""
+    import contextlib
+    import weakref
+    make, log = made
+
+    class Event:
+        pass
+
+    class Graph:
+        def capture_begin(self):
+            log.append("begin")
+
+        def capture_end(self):
+            log.append(("end", seen[-1]() is not None))
+
+        def reset(self):
+            pass
+
+    seen = []
+
+    def forward(ctx, caches):
+        event = Event()
+        ctx.events.append(event)
+        seen.append(weakref.ref(event))
+        return torch.zeros(1, 4)
+
+    stream = NS(wait_stream=lambda s: None)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", Graph)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: stream)
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "Event", lambda: NS(record=lambda: None, synchronize=lambda: None))
+    runner = make(0)
+    runner.manager.pack_decode = lambda *a, **kw: None
+    runner.storage = NS(pad_pages=[], pad_slot=0, caches=None)
+    runner.model, runner.vocab_size, runner.before_launch, runner.capture_stream = NS(forward=forward), 4, None, stream
+    runner.act_dtype, runner.block_size = torch.float32, 64
+    step = DecodeGraph(runner, 1, 64)
+    step.run(runner, [NS(want=[0], tokens=[1], req="a")])
+    assert log == ["wait", "begin", ("end", True)] and step.graph is not None
+    assert seen[-1]() is None and seen[0]() is None

@@ -2363,18 +2363,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(GemmArgs g) {
         }
     };
     const int n_blocks = (min(TM, r_end - r0) + 15) >> 4;
-    if constexpr (MB == 8) {
-        if (n_blocks <= 2) loop(fx_int<2>{});
-        else if (n_blocks <= 4) loop(fx_int<4>{});
-        else if (n_blocks <= 6) loop(fx_int<6>{});
-        else loop(fx_int<8>{});
-    } else {
-        if (n_blocks == 1) loop(fx_int<1>{});
-        else if (MB == 2 || n_blocks == 2) loop(fx_int<2>{});
-        else if constexpr (MB > 2) {
-            if (n_blocks == 3) loop(fx_int<3>{});
-            else loop(fx_int<4>{});
-        }
+    if (n_blocks == 1) loop(fx_int<1>{});
+    else if (MB == 2 || n_blocks == 2) loop(fx_int<2>{});
+    else if constexpr (MB > 2) {
+        if (n_blocks == 3) loop(fx_int<3>{});
+        else loop(fx_int<4>{});
     }
     f32x4_t(*other)[64] = (f32x4_t(*)[64]) & Xs[0][0][0][0][0];       // ROLES: up's sums, MB blocks of each of two waves
     if constexpr (ROLES) {
@@ -2714,9 +2707,13 @@ static void launch_f32(const GemmArgs& g, bool split, int tile, int stream, int 
         else if (tile == 32) {
             if (VEC && stream) gemm_f32_split_kernel<32, 1, 2, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
             else gemm_f32_split_kernel<32, 1, 2, DUAL, EPI, VEC, false><<<grid, 256, 0, s>>>(g);
-        } else if (VEC && stream == 2) gemm_f32_split_kernel<64, 1, 2, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
-        else if (VEC && stream) gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, VEC, VEC><<<grid, 256, 0, s>>>(g);
-        else gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, VEC, false><<<grid, 256, 0, s>>>(g);
+        } else if constexpr (VEC) {
+            if (stream == 2) gemm_f32_split_kernel<64, 1, 2, DUAL, EPI, true, true><<<grid, 256, 0, s>>>(g);
+            else if (stream) gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, true, true><<<grid, 256, 0, s>>>(g);
+            else gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, true, false><<<grid, 256, 0, s>>>(g);
+        } else {
+            gemm_f32_split_kernel<64, 1, 1, DUAL, EPI, false, false><<<grid, 256, 0, s>>>(g);
+        }
     } else if (tile == 64) gemm_f32_tiled_kernel<64, 64, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
     else if (tile == 32) gemm_f32_tiled_kernel<32, DUAL ? 64 : 32, DUAL, EPI, VEC><<<grid, 256, 0, s>>>(g);
     else if (VEC && g.K % 32 == 0) {
@@ -2749,9 +2746,11 @@ static void launch_skinny_cfg(const GemmArgs& g, int epi, int m_tiles, hipStream
 }
 
 // mt: row tiles per block (1, 2, 4); nw: 16-row weight sets per wave; waves: 4 or 8 split K (1 or 2 with one row tile).
+// half sets: four pieces on their way where that is a wave's whole part of K, or where rows are so few that their operands do not fill the way
+static bool four_pieces(int M, int K) { return K <= 2048 || M <= 4; }
 static void launch_skinny(const GemmArgs& g, int epi, int mt, int nw, int waves, bool half, int m_tiles, hipStream_t s) {
-    if (half) {      // (four pieces on their way where that is a wave's whole part of K, or where rows are so few that their operands do not fill the way)
-        const bool deep = g.K <= 2048 || g.M <= 4;
+    if (half) {
+        const bool deep = four_pieces(g.M, g.K);
         if (epi == EPI_GATED) {
             if (deep) launch_skinny_cfg<1, 4, 2, true, 4>(g, epi, m_tiles, s);
             else launch_skinny_cfg<1, 4, 2, true>(g, epi, m_tiles, s);
@@ -2912,17 +2911,21 @@ FX_API int fx_gemm_f32_split_tile(int M, int N, int dual, int cus) {
     return best;
 }
 
-// How the product for few rows takes up to 16 plain rows: sets of weight rows a wave has, half sets or whole ones, pieces of K on their way.
+// How the product for few rows takes up to 16 plain rows: sets of weight rows a wave has, waves a block, half sets or whole ones, pieces of K on their way (half sets only).  Two
+// sets share the activations that they multiply and halve the blocks' fixed work; one where two would leave too few blocks to keep the memory busy, or where a row or two
+// meet so many weight rows that the blocks are plenty either way.
 struct FewRows {
-    int sets;
+    int sets, waves;
     bool half, deep;
 };
 static FewRows few_plain_rows(int M, int N, int K, bool dual, int cus) {
     FewRows f;
     f.sets = dual || ceil_div(N, 32) >= 160 ? 2 : 1;
     if (!dual && M <= 2 && ceil_div(N, 16) >= 4096) f.sets = 1;
-    f.half = (K >= 2048 || ceil_div(N, 8) <= cus) && fx_gemm_half_sets(M, N, dual, f.sets, cus);
-    f.deep = K <= 2048 || M <= 4;
+    if ((g_skinny_nw == 1 && !dual) || g_skinny_nw == 2) f.sets = g_skinny_nw;
+    f.waves = g_skinny_waves == 8 || g_skinny_waves == 2 || g_skinny_waves == 1 ? g_skinny_waves : 4;
+    f.half = f.waves == 4 && (g_skinny_half >= 0 ? g_skinny_half != 0 : (K >= 2048 || ceil_div(N, 8) <= cus) && fx_gemm_half_sets(M, N, dual, f.sets, cus));
+    f.deep = four_pieces(M, K);
     return f;
 }
 
@@ -2940,7 +2943,7 @@ struct FxProduct {
 FX_API int fx_gemm_pairs(int M, int epi, int N, int K, int epi2, int N2, int K2, int cus) {
     const FewRows f = few_plain_rows(M, N, K, epi == EPI_GATED, cus);
     return M >= 1 && M <= 16 && K % 8 == 0 && K2 % 8 == 0 && N2 < 65536 && N < 65536 && (epi2 == EPI_STORE || epi2 == EPI_STORE_F32) &&
-           f.half && (epi == EPI_STORE_F32 || (epi == EPI_GATED && f.deep));
+           f.waves == 4 && f.half && (epi == EPI_STORE_F32 || (epi == EPI_GATED && f.deep));
 }
 FX_API int fx_gemm_pair(void* stream, const FxProduct* first, const FxProduct* second) {
     const int cus = fx_compute_units();
@@ -3252,6 +3255,12 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
                                      fx_gemm_row_tile_blocks(M, N, fx_compute_units());
         if (row_tile_blocks) mt = 1;
         if (g_skinny_mt && !pair_ids) mt = g_skinny_mt;
+        if (!expert_offsets && !pair_ids && !norm_w && M <= 16 && mt == 1) {
+            const FewRows f = few_plain_rows(M, N, K, dual, fx_compute_units());
+            launch_skinny(g, epi, 1, f.sets, f.waves, f.half, 1, s);
+            FX_CHECK_LAUNCH("gemm_bf16_skinny");
+            return 0;
+        }
         const int m_tiles = pair_ids ? (M < E ? M : E) + M / 16 + n_always
                                      : M / (16 * mt) + (expert_offsets ? nonempty : (M % (16 * mt) != 0));
         // two sets of weight rows per wave share the activations they multiply and halve the blocks' fixed
@@ -3270,10 +3279,7 @@ FX_API int fx_gemm(void* stream, int dtype, int epi, const void* A, long lda, co
         int waves = 4;
         if (expert_offsets && mt == 1) waves = 2;      // sorted, up to 16 rows per expert: 152 against 159 us at 64 tokens
         if (g_skinny_waves == 8 || g_skinny_waves == 4 || g_skinny_waves == 2 || g_skinny_waves == 1) waves = g_skinny_waves;
-        const bool half = g_skinny_half >= 0 ? g_skinny_half && M <= 16 && !expert_offsets && !pair_ids && !norm_w && waves == 4 && mt == 1
-                                             : !expert_offsets && !pair_ids && !norm_w && waves == 4 && mt == 1 && (K >= 2048 || ceil_div(N, 8) <= fx_compute_units()) &&
-                                                   fx_gemm_half_sets(M, N, dual, nw, fx_compute_units());
-        launch_skinny(g, epi, mt, nw, waves, half, m_tiles, s);
+        launch_skinny(g, epi, mt, nw, waves, false, m_tiles, s);
         FX_CHECK_LAUNCH("gemm_bf16_skinny");
         return 0;
     }

@@ -291,3 +291,23 @@ def test_tiles_of_float32_products_from_parts():
     assert [rule(m, n, 1) for m in (33, 64) for n in (4096, 4128, 8192)] == [32, 64, 64] * 2
     assert [rule(m, n) for m in (33, 64) for n in (16448, 40960)] == [48, 48, 64, 64]
     assert rule(65, 2048) == 32 and rule(700, 6144) == 144 and rule(700, 2048) == 48 and rule(700, 1024) == 48
+
+
+def test_which_products_of_few_rows_share_a_launch():
+    """A gate/up product or one that is stored in float32, in half sets of weight rows by four waves, beside one that is stored; a switch that gives the first another kernel
+    leaves both to launches of their own."""
+    from ferrox_amd import debug
+    from ferrox_amd.csrc.build import load_library
+    lib = load_library("gemm")
+    stored, stored_f32, added, gated = 0, 1, 2, 3
+    pairs = lambda m, epi, n, k, epi2=stored_f32, n2=1024, k2=2048: bool(lib.fx_gemm_pairs(m, epi, n, k, epi2, n2, k2, 256))
+    assert all(pairs(m, gated, 5632, 2048) and pairs(m, stored_f32, 2048, 5632, stored, 4096, 768) for m in (1, 5, 16))
+    assert not any(pairs(m, gated, 5632, 2048) for m in (0, 17, 64))
+    assert not pairs(8, added, 2048, 5632) and not pairs(8, stored, 2048, 5632) and not pairs(8, gated, 5632, 2048, added) and not pairs(8, gated, 5632, 2048, gated)
+    assert not pairs(8, gated, 5632, 2052) and not pairs(8, gated, 5632, 2048, stored, 1024, 2044) and not pairs(8, gated, 5632, 2048, stored, 65536)
+    assert pairs(4, gated, 5632, 4096) and not pairs(5, gated, 5632, 4096)                # (four pieces on their way)
+    for m, n, dual, sets in ((8, 5632, 1, 2), (8, 2048, 0, 1), (8, 24576, 0, 2), (16, 40960, 1, 2)):       # as the rule for half sets has it
+        assert pairs(m, gated if dual else stored_f32, n, 2048) == bool(lib.fx_gemm_half_sets(m, n, dual, sets, 256))
+    for key, value in (("skinny_half", 0), ("skinny_waves", 8)):
+        with debug.kernel_switch("gemm", key, value):
+            assert not pairs(8, gated, 5632, 2048) and not pairs(8, stored_f32, 2048, 5632, stored, 4096, 768)

@@ -1271,17 +1271,21 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
         // columns past the value head and the rows past the group: a block's only tile is little longer than this end of it, and with a branch around each of the stores
         // (and two more inside) 40 keys of 16 heads on one kv head of
         // 256 took 14.3 us, so 11.0 (8 sequences of 2,060 keys 17.5 and 16.3; 28 heads of 128 on 4, 40 keys 8.7 and 6.9).
-        constexpr int CB = WaveAttn<HD, SHAPE>::CB, OUTSIDE = 1 << 30;
+        // A block of one row leaves out the three that lanes hold beside it (16 heads of 128, one sequence of 300 keys, scores capped, 10.6 -> 10.1 us; 16 of 64, 64 sequences of 300 keys
+        // 22.2 -> 21.9, and 21.1 with branches here and in front of the loads: a wave of narrow heads walks five tiles there, and asks for its keys' pages together in each).
+        constexpr int CB = WaveAttn<HD, SHAPE>::CB;
+        constexpr uint32_t OUTSIDE = 1u << 30;       // (a row and a column that do not exist: 2^31, past any end)
         const int vd = a.vd;
         const bool parts = a.splits > 1;
-        if (parts || !(a.gate || a.turns)) {
+        auto store_rows = [&](auto rows) {
+            constexpr int R = decltype(rows)::value;
             const size_t first = parts ? (((size_t)item * a.nh + h0) * a.splits + split) * vd : (size_t)tok * a.ldo + (size_t)h0 * vd;
             const int row_len = parts ? a.splits * vd : vd, size = parts ? 4 : 2;
             const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(parts ? (void*)(a.part_o + first) : (void*)((bf16*)a.out + first), 0, ((n - 1) * row_len + vd) * size, 0x00027000);
-            float m[4], l[4];
-            int at[4];
+            float m[R], l[R];
+            uint32_t at[R];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
+            for (int r = 0; r < R; ++r) {
                 m[r] = __shfl(w.m, 4 * g + r, 64);
                 l[r] = __shfl(w.l, 4 * g + r, 64);
                 at[r] = 4 * g + r < n ? (4 * g + r) * row_len * size : OUTSIDE;
@@ -1289,12 +1293,12 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
             if (parts) {
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb) {
-                    const int column = 16 * cb + li < vd ? 4 * (16 * cb + li) : OUTSIDE;
+                    const uint32_t column = 16 * cb + li < vd ? 4 * (16 * cb + li) : OUTSIDE;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m[r] == NEG_INF ? 0.f : w.o[cb][r]), to, at[r] + column, 0, 0);
+                    for (int r = 0; r < R; ++r) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(m[r] == NEG_INF ? 0.f : w.o[cb][r]), to, at[r] + column, 0, 0);
                 }
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+                for (int r = 0; r < R; ++r)
                     if (li == 0 && 4 * g + r < n) {
                         float* pml = a.part_ml + (((size_t)item * a.nh + h0 + 4 * g + r) * a.splits + split) * 2;
                         pml[0] = m[r] == NEG_INF ? NEG_INF : m[r] * LN2;
@@ -1302,15 +1306,19 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
                     }
                 return;
             }
-            float fin[4];
+            float fin[R];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) fin[r] = finish_row<true>(a, h0 + min(4 * g + r, n - 1), m[r], l[r]);
+            for (int r = 0; r < R; ++r) fin[r] = finish_row<true>(a, h0 + min(4 * g + r, n - 1), m[r], l[r]);
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) {
-                const int column = 16 * cb + li < vd ? 2 * (16 * cb + li) : OUTSIDE;
+                const uint32_t column = 16 * cb + li < vd ? 2 * (16 * cb + li) : OUTSIDE;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, float_to_bf16(w.o[cb][r] * fin[r])), to, at[r] + column, 0, 0);
+                for (int r = 0; r < R; ++r) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, float_to_bf16(w.o[cb][r] * fin[r])), to, at[r] + column, 0, 0);
             }
+        };
+        if (parts || !(a.gate || a.turns)) {
+            if (n == 1) store_rows(std::integral_constant<int, 1>{});
+            else store_rows(std::integral_constant<int, 4>{});
             return;
         }
 #pragma unroll
@@ -1349,59 +1357,64 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
     const int per_row = blockDim.x / n;
     const int row = threadIdx.x / per_row, sub = threadIdx.x - row * per_row;
     if (row >= n) return;
-    // (waves past the last stand for it with weight 0: all reads of a step of this on their way together.  In loops over the waves that there are each
+    // (up to four waves or up to eight; waves past the last stand for it with weight 0: all reads of a step of this on their way together.  In loops over the waves that there are each
     // read was waited for, us: 16 heads of 128, one sequence of 2,060 keys 11.9, so 11.3, 8 29.8 and 29.0; 28 heads on 4, 8 sequences 16.0 and 15.3.)
-    const float* from[8];
-    float ms[8], ls[8], f[8], m = NEG_INF, l = 0.f;
+    auto merge = [&](auto most) {
+        constexpr int W = decltype(most)::value;
+        const float* from[W];
+        float ms[W], ls[W], f[W], m = NEG_INF, l = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        from[u] = wave_out + ((size_t)min(u, n_waves - 1) * n + row) * stride;
-        ms[u] = from[u][HD];
-        ls[u] = from[u][HD + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) m = fmaxf(m, ms[u]);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const float e = __builtin_amdgcn_exp2f(ms[u] - m);
-        f[u] = ((u < n_waves) & (ms[u] != NEG_INF)) ? e : 0.f;
-        l += f[u] * (u < n_waves ? ls[u] : 0.f);
-    }
-    auto value = [&](int u, int d) {      // (of a wave that is there: the last one's sum may be infinite, and an infinity with weight 0 is no 0)
-        const float v = from[u][d];
-        return u < n_waves ? v : 0.f;
-    };
-    const int h = h0 + row;
-    const bool last = a.splits == 1;
-    const float fin = last ? finish_row<true>(a, h, m, l) : 1.f;
-    float* po = a.part_o + (((size_t)item * a.nh + h) * a.splits + split) * vd;
-    if (last && a.turns) {      // pairs of columns, which are turned back together
-        for (int d = 2 * sub; d < vd; d += 2 * per_row) {
-            float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                o0 += f[u] * value(u, d);
-                o1 += f[u] * value(u, d + 1);
-            }
-            o0 *= fin;
-            o1 *= fin;
-            store_out<bf16>(a, tok, h, d, turned_back(a, tok, d, o0, o1));
-            store_out<bf16>(a, tok, h, d + 1, turned_back(a, tok, d + 1, o1, o0));
+        for (int u = 0; u < W; ++u) {
+            from[u] = wave_out + ((size_t)min(u, n_waves - 1) * n + row) * stride;
+            ms[u] = from[u][HD];
+            ls[u] = from[u][HD + 1];
         }
-        return;
-    }
-    for (int d = sub; d < vd; d += per_row) {
-        float o = 0.f;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) o += f[u] * value(u, d);
-        if (last) store_out<bf16>(a, tok, h, d, o * fin);
-        else po[d] = o;
-    }
-    if (!last && sub == 0) {
-        float* pml = a.part_ml + (((size_t)item * a.nh + h) * a.splits + split) * 2;
-        pml[0] = m == NEG_INF ? NEG_INF : m * LN2;
-        pml[1] = l;
-    }
+        for (int u = 0; u < W; ++u) m = fmaxf(m, ms[u]);
+#pragma unroll
+        for (int u = 0; u < W; ++u) {
+            const float e = __builtin_amdgcn_exp2f(ms[u] - m);
+            f[u] = ((u < n_waves) & (ms[u] != NEG_INF)) ? e : 0.f;
+            l += f[u] * (u < n_waves ? ls[u] : 0.f);
+        }
+        auto value = [&](int u, int d) {      // (of a wave that is there: the last one's sum may be infinite, and an infinity with weight 0 is no 0)
+            const float v = from[u][d];
+            return u < n_waves ? v : 0.f;
+        };
+        const int h = h0 + row;
+        const bool last = a.splits == 1;
+        const float fin = last ? finish_row<true>(a, h, m, l) : 1.f;
+        float* po = a.part_o + (((size_t)item * a.nh + h) * a.splits + split) * vd;
+        if (last && a.turns) {      // pairs of columns, which are turned back together
+            for (int d = 2 * sub; d < vd; d += 2 * per_row) {
+                float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+                for (int u = 0; u < W; ++u) {
+                    o0 += f[u] * value(u, d);
+                    o1 += f[u] * value(u, d + 1);
+                }
+                o0 *= fin;
+                o1 *= fin;
+                store_out<bf16>(a, tok, h, d, turned_back(a, tok, d, o0, o1));
+                store_out<bf16>(a, tok, h, d + 1, turned_back(a, tok, d + 1, o1, o0));
+            }
+            return;
+        }
+        for (int d = sub; d < vd; d += per_row) {
+            float o = 0.f;
+#pragma unroll
+            for (int u = 0; u < W; ++u) o += f[u] * value(u, d);
+            if (last) store_out<bf16>(a, tok, h, d, o * fin);
+            else po[d] = o;
+        }
+        if (!last && sub == 0) {
+            float* pml = a.part_ml + (((size_t)item * a.nh + h) * a.splits + split) * 2;
+            pml[0] = m == NEG_INF ? NEG_INF : m * LN2;
+            pml[1] = l;
+        }
+    };
+    if (n_waves <= 4) merge(std::integral_constant<int, 4>{});
+    else merge(std::integral_constant<int, 8>{});
 }
 
 // A head's row of biases for a block that walks over many tiles is copied to LDS (dynamic, sized by the launch): a load from

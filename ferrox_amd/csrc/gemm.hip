@@ -4,7 +4,7 @@
 //
 //  * bfloat16: MFMA 16x16x32 tiles, float32 accumulators.
 //  * float32 : MFMA 16x16x4 in float32, or every operand as the sum of three bfloat16
-//    numbers on the bfloat16 instruction, with no larger error (see `f32_split8`).
+//    numbers on the bfloat16 instruction, with a smaller error in sums of a thousand terms (see `f32_split8`).
 //
 // In both, one output element's products are added in an order that the sizes of the
 // weights fix, whatever the tile shape and whatever else is in the batch, so a float32
@@ -1880,8 +1880,10 @@ __device__ __forceinline__ f32x4_t f32_fetch_guarded(const float* row, int k, in
 // float32 products as bfloat16 ones
 // ---------------------------------------------------------------------------
 // A float32 is the sum of three bfloat16 numbers h + m + l, each the rest of the ones before it rounded to nearest (8 + 8 + 8 bits and two signs hold
-// its 24 bits), and a product of two such sums has six terms down to 2^-18 of it: hh, hm, mh, mm, hl, lh; what is left out, ml, lm and ll, is
-// 2^-26 of the product or less and of either sign (6e-9 of a sum's norm, where rounding a float32 product takes 3e-8).  The matrix instruction adds 32 bfloat16 products in 16 cycles where the float32 one adds
+// its 24 bits; Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations", 2019), and a product of two such sums has six terms
+// down to 2^-18 of it: hh, hm, mh, mm, hl, lh.  What is left out, ml, lm and ll, can be 2^-24 of a product (just above a power of two in both) and is of either sign: 6e-9 of a sum's norm, where
+// rounding a float32 product takes 3e-8.  Of few terms the cut-off weighs more than the roundings that it saves: rows with one number that is not 0 are off by 5.0e-8 of themselves instead of 2.5e-8, with eight
+// 7.2e-8 instead of 5.5e-8, from some 64 on it is level, then less.  The matrix instruction adds 32 bfloat16 products in 16 cycles where the float32 one adds
 // four in 32, so six terms take 96 cycles instead of 256.
 // The instruction cuts a sum off below instead of rounding it, so a step's 32 k start from zero, small terms first, and are added to the sums so far with an add that rounds; and every second step works
 // out the negative and subtracts it, so that what is cut off has either sign: else outputs are low by 5e-8 of their size, which the mean over a thousand keys brings out (decoded logits at 1,030 keys: 1.3e-6
@@ -2411,7 +2413,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(GemmArgs g) {
 // with the non-temporal hint, the halves changing places before the products (`load_lines16`).  Bound by the stream of the weights: 4 rows
 // against 6,144 x 2,048 15.5 us, gate/up of 5,632 24.3, 15 experts' gate/up 63 (5.5 TB/s), the head of 151,936 235 (5.3 TB/s).  With half
 // lines and steps of 64 k these took 17.6, 30.0, 75 and 275: twice the registers a step leave half the waves, and it
-// is waves, not deeper loads, that keep memory busy (steps of 128 k: 19.9, 33.3, 95 and 329).
+// is waves, not deeper loads, that keep memory busy (steps of 128 k: 19.9, 33.3, 95 and 329).  SPLIT, us for 4 rows: 6,144 x 2,048 13.2, gate/up of 5,632 23.0, the head 204; with three steps on their way
+// 2,048 x 2,048 8.0 instead of 7.1 and the head 277, with the next step taken apart beside this one's products 7.7 and 218.
 template <int MT, int NW, bool DUAL, int EPI, bool VEC, bool LINES, bool HALF = false, bool SPLIT = false>
 __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     static_assert(!DUAL || NW % 2 == 0, "dual mode multiplies two matrices");
@@ -2425,6 +2428,7 @@ __global__ __launch_bounds__(512) void gemm_f32_skinny_kernel(GemmArgs g) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 15, gq = lane >> 4;
     const float* Wbase = (const float*)g.W + (size_t)expert * g.w_stride;
     // SPLIT: the rows come in whole lines as well, the first load of 32 k with rows 0 .. 7 of a tile and the second with rows 8 .. 15, which a tile of up to eight rows does without
+    // (2,048 x 5,632, 1 row 14.3 -> 13.2 us, 8 rows 15.4 -> 14.1, 32 rows 48.2 -> 44.1; 16 rows of half sets, where nothing hides that the halves change places, 18.8 and 18.9)
     constexpr bool XLINES = LINES && SPLIT;
     const float* x_src[MT][XLINES ? 2 : 1];
     constexpr int WR = LINES && !HALF ? 2 : 1;
@@ -2884,7 +2888,7 @@ FX_API int fx_gemm_half_sets(int M, int N, int dual, int sets, int cus) {
 }
 
 // Whether a float32 product is worked out from operands taken apart into bfloat16 ones (gemm_f32_split_kernel, and in the kernel for few rows): by the weights alone, so that the bits of a row
-// do not depend on the rows beside it.  Whole steps of 32 k; sums of 1,024 and more, where the error is a third of the float32 instruction's (it is level around 256); and weights of more than a million numbers, up to which the
+// do not depend on the rows beside it.  Whole steps of 32 k; sums of 1,024 and more, where the error is a half to a sixth of the float32 instruction's (it is level around 64); and weights of more than a million numbers, up to which the
 // products are a few microseconds either way (us of 1,024 x 1,024, float32 instruction / taken apart: 1 row 4.5 4.6, 48 rows 13.4 14.4, 256 14.1 15.0, 512 18.6 16.2; of 512 x 2,048 1 row 6.1 6.2, 48 rows 23.6 23.5) and some have their sums repeated elsewhere in the float32 order (`f32_ordered_dot`).
 FX_API int fx_gemm_f32_split(int N, int K) { return K % 32 == 0 && K >= 1024 && (long)N * K > 1L << 20; }
 

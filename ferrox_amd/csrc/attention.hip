@@ -747,18 +747,34 @@ struct WaveAttn {
         constexpr int NP = KP < KS ? 13 : 9;
         int key_of[NP], page_of[NP], slot_of[NP];
         bool klives[4];
-        key_of[0] = vkey;
+        // rows li % 8 and 8 + li % 8 of the block's 16 keys (row i is key 16 (i / 4) + 4 kb + i % 4 of the tile)
+        const int row0 = 16 * (li >> 2) + (li & 3), row_a = 16 * (l8 >> 2) + (l8 & 3), row_b = row_a + 32;
+        if (SHAPE == 0 && !edge && a.bs_shift >= 6) {
+            // every key is there and on one page: a wave that walks many tiles has no time for more (16 heads of 128, 72 sequences of 2,054 keys 227 us without this, so 210, one sequence of 2,060 the
+            // same; heads of 64, 64 sequences of 300 keys 22.0 and 19.7).  Scores that go through a cap or slopes leave no registers for a second way (28 heads on 4, 24 sequences 26.6 and 28.6).
+            const int page = pl.page(kt0 >> a.bs_shift), slot = kt0 & (a.bs - 1);
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            const int key0 = kt0 + 16 * (li >> 2) + 4 * kb + (li & 3);
-            klives[kb] = span.has(key0);
-            // rows li % 8 and 8 + li % 8 of the block's 16 keys (row i is key 16 (i / 4) + 4 kb + i % 4 of the tile)
-            const int key_a = kt0 + 16 * (l8 >> 2) + 4 * kb + (l8 & 3), key_b = key_a + 32;
-            key_of[1 + kb] = span.has(key_a) ? key_a : safe_group;
-            key_of[5 + kb] = span.has(key_b) ? key_b : safe_group;
-            if constexpr (KP < KS) key_of[9 + kb] = klives[kb] ? key0 : safe_group;
+            for (int i = 0; i < NP; ++i) page_of[i] = page;
+            slot_of[0] = slot + 16 * g;
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) {
+                klives[kb] = true;
+                slot_of[1 + kb] = slot + row_a + 4 * kb;
+                slot_of[5 + kb] = slot + row_b + 4 * kb;
+                if constexpr (KP < KS) slot_of[9 + kb] = slot + row0 + 4 * kb;
+            }
+        } else {
+            key_of[0] = vkey;
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) {
+                const int key0 = kt0 + row0 + 4 * kb, key_a = kt0 + row_a + 4 * kb, key_b = kt0 + row_b + 4 * kb;
+                klives[kb] = span.has(key0);
+                key_of[1 + kb] = span.has(key_a) ? key_a : safe_group;
+                key_of[5 + kb] = span.has(key_b) ? key_b : safe_group;
+                if constexpr (KP < KS) key_of[9 + kb] = klives[kb] ? key0 : safe_group;
+            }
+            pages_of(a, pl, key_of, page_of, slot_of);
         }
-        pages_of(a, pl, key_of, page_of, slot_of);
         const int *kpage_a = page_of + 1, *kslots_a = slot_of + 1, *kpage_b = page_of + 5, *kslots_b = slot_of + 5;
         const bf16* vbase = (const bf16*)a.v_pages + ((size_t)page_of[0] * a.nkv + kvh) * vd * bs + slot_of[0];
         uint4 vv[EARLY_V ? CB : 1][2];

@@ -1961,7 +1961,7 @@ def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2
 
 
 @pytest.mark.parametrize("nh,nkv,hd,vd", [(5, 1, 64, 64), (16, 1, 256, 192), (34, 2, 64, 40), (7, 7, 128, 72), (28, 4, 128, 128), (16, 1, 256, 200)])
-@pytest.mark.parametrize("bs", [64, 16])
+@pytest.mark.parametrize("bs", [64, 16, 128, 96])
 def test_single_queries_of_one_wave_write_their_rows_and_columns_only(nh, nkv, hd, vd, bs):
     """Blocks of one wave store through a buffer whose end drops what a block does not have: heads beyond the group, columns beyond the
     value head, in outputs and in parts of several chunks.  Whatever stands around the outputs stays.  Probabilities and values are

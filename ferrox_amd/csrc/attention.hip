@@ -724,8 +724,10 @@ struct WaveAttn {
         }
     }
 
+    // WALKS: for waves that walk many tiles (see `fx_attn_wave_walks`)
     // keys [kt0, kt0 + 64); this lane's row sees key t iff t <= hi and (lo <= t or t < span.keep) (hi < lo: row unused)
     // `slope`, `qpos`, `head`: the row's distance penalty, its query's position and its head, where the scores are shaped
+    template <bool WALKS>
     __device__ __forceinline__ void tile(const AttnArgs& a, const PageLookup& pl, int kvh, int kt0, const KeySpan& span,
                                          int lo, int hi, float slope, int qpos, int head) {
         const int kv_end = span.end;
@@ -749,16 +751,18 @@ struct WaveAttn {
         bool klives[4];
         // rows li % 8 and 8 + li % 8 of the block's 16 keys (row i is key 16 (i / 4) + 4 kb + i % 4 of the tile)
         const int row0 = 16 * (li >> 2) + (li & 3), row_a = 16 * (l8 >> 2) + (l8 & 3), row_b = row_a + 32;
-        if (SHAPE == 0 && !edge && a.bs_shift >= 6) {
-            // every key is there and on one page: a wave that walks many tiles has no time for more (16 heads of 128, 72 sequences of 2,054 keys 227 us without this, so 210, one sequence of 2,060 the
-            // same; heads of 64, 64 sequences of 300 keys 22.0 and 19.7).  Scores that go through a cap or slopes leave no registers for a second way (28 heads on 4, 24 sequences 26.6 and 28.6).
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) klives[kb] = (WALKS && !edge) || span.has(kt0 + row0 + 4 * kb);
+        if ((!WALKS || !edge) && a.bs_shift >= 6) {
+            // the tile is on one page, which is there, as some key of it is: one lookup, and slots that follow each other (what stands in those of other keys is masked below).
+            // Nine lookups a tile took 16 heads of 128 and one sequence of 2,060 keys in a trace of the step 10.1 us a launch, this 9.7; four waves of heads of 128 with values of 64, 8 sequences, 26.3 and 25.5.
+            // In waves that walk many tiles it is for tiles whose keys are all there.
             const int page = pl.page(kt0 >> a.bs_shift), slot = kt0 & (a.bs - 1);
 #pragma unroll
             for (int i = 0; i < NP; ++i) page_of[i] = page;
             slot_of[0] = slot + 16 * g;
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
-                klives[kb] = true;
                 slot_of[1 + kb] = slot + row_a + 4 * kb;
                 slot_of[5 + kb] = slot + row_b + 4 * kb;
                 if constexpr (KP < KS) slot_of[9 + kb] = slot + row0 + 4 * kb;
@@ -768,7 +772,6 @@ struct WaveAttn {
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
                 const int key0 = kt0 + row0 + 4 * kb, key_a = kt0 + row_a + 4 * kb, key_b = kt0 + row_b + 4 * kb;
-                klives[kb] = span.has(key0);
                 key_of[1 + kb] = span.has(key_a) ? key_a : safe_group;
                 key_of[5 + kb] = span.has(key_b) ? key_b : safe_group;
                 if constexpr (KP < KS) key_of[9 + kb] = klives[kb] ? key0 : safe_group;
@@ -1206,7 +1209,7 @@ __global__ __launch_bounds__(64) void attn_mfma_tile_kernel(AttnArgs a) {
     const KeySpan span = {kv_begin, kv_end, a.keep_first};
     const TileWalk walk = tile_walk(span);
     const float slope = a.slopes ? a.slopes[h] : 0.f;
-    for (int ti = 0; ti < walk.n; ++ti) w.tile(a, pl, kvh, walk.start(ti), span, lo, hi, slope, max(hi, 0), h);
+    for (int ti = 0; ti < walk.n; ++ti) w.template tile<false>(a, pl, kvh, walk.start(ti), span, lo, hi, slope, max(hi, 0), h);
     const float fin = li < n ? finish_row<true>(a, h, w.m, w.l) : 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1225,7 +1228,7 @@ __global__ __launch_bounds__(64) void attn_mfma_tile_kernel(AttnArgs a) {
 // decode, several waves per block: block = (item, kv head x group block of 16 query heads, split);
 // its waves take the split's tiles of 64 keys in turn and their results are merged through LDS in
 // wave order.  With one split the block writes the output itself, no second launch.
-template <int HD, int MAX_THREADS, int SHAPE>
+template <int HD, int MAX_THREADS, int SHAPE, bool WALKS = false>
 __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(AttnArgs a) {
     extern __shared__ float wave_out[];      // [waves][rows][HD + 2]: o, then m and l
     // The grid is (heads, items, splits): blocks go to the eight XCDs in turn, so with the heads fastest every
@@ -1279,7 +1282,7 @@ __global__ __launch_bounds__(MAX_THREADS) void attn_mfma_decode_block_kernel(Att
         const TileWalk walk = tile_walk(span);
         const int lo = row_ok ? kv_begin : 1, hi = row_ok ? kv_end - 1 : 0;
         const float slope = (a.slopes && row_ok) ? a.slopes[h0 + li] : 0.f;      // (a row is a query head here)
-        for (int ti = wave; ti < walk.n; ti += n_waves) w.tile(a, pl, kvh, walk.start(ti), span, lo, hi, slope, p, h0 + min(li, n - 1));
+        for (int ti = wave; ti < walk.n; ti += n_waves) w.template tile<WALKS>(a, pl, kvh, walk.start(ti), span, lo, hi, slope, p, h0 + min(li, n - 1));
     }
     if (n_waves == 1) {
         // one wave: nothing to merge, the rows go out from the registers that hold them (lane (li, g) has rows
@@ -2468,6 +2471,12 @@ static void launch_merge(const AttnArgs& a, dim3 grid, hipStream_t s) {
     else attn_decode_merge_kernel<T, false><<<grid, threads, 2 * ((a.splits + 15) & ~15) * sizeof(float), s>>>(a);
 }
 
+// Whether a decode block's waves walk many tiles of plain scores: 16 and more each of the longest sequence that the launch can have, of heads of up to 64 five.  They look a page up apart from the tiles at the span's ends,
+// which costs a wave of few tiles the time to fetch that code (8 sequences of 2,050 keys in a trace of the step 31.1 us a launch, 34.6) and is ahead where a launch is at the
+// rate of memory (us without / with: 16 heads of 128 64 sequences in a trace 192 and 168, 72 sequences of 2,054 keys 223 and 207; heads of 64 64 sequences 90.8 and 86.6, 128 of 200 keys 26.1 and 24.6; the other way 96 sequences of 2,060 keys
+// 223 and 228; from nine tiles on 12 sequences of 8,000 keys 123.2 and 125.7).
+FX_API int fx_attn_wave_walks(long keys, int waves, int hd) { return (keys + 63) / 64 >= (hd <= 64 ? 5L : 16L) * waves; }
+
 static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, void* out, long ldo,
                               const void* k_pages, const void* v_pages, const int* block_table, int max_blocks,
                               const int* positions, const int* item_seq, const int* item_tok, int n_items,
@@ -2535,6 +2544,13 @@ static int attn_decode_launch(void* stream, int dtype, const void* q, long ldq, 
         const size_t shm = (size_t)nw * rows * (hdc + 2) * 4;
         by_shape(a, [&](auto shape) {
             constexpr int SH = decltype(shape)::value;
+            if constexpr (SH == 0) {
+                if (hd > 32 && hd <= 128 && fx_attn_wave_walks(own, nw, hd)) {
+                    if (hd <= 64) attn_mfma_decode_block_kernel<64, 512, SH, true><<<gridm, nw * 64, shm, s>>>(a);
+                    else attn_mfma_decode_block_kernel<128, 512, SH, true><<<gridm, nw * 64, shm, s>>>(a);
+                    return;
+                }
+            }
             if (hd <= 32) attn_mfma_decode_block_kernel<32, 512, SH><<<gridm, nw * 64, shm, s>>>(a);
             else if (hd <= 64) attn_mfma_decode_block_kernel<64, 512, SH><<<gridm, nw * 64, shm, s>>>(a);
             else if (hd <= 128) attn_mfma_decode_block_kernel<128, 512, SH><<<gridm, nw * 64, shm, s>>>(a);

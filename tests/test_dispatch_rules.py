@@ -311,3 +311,13 @@ def test_which_products_of_few_rows_share_a_launch():
     for key, value in (("skinny_half", 0), ("skinny_waves", 8)):
         with debug.kernel_switch("gemm", key, value):
             assert not pairs(8, gated, 5632, 2048) and not pairs(8, stored_f32, 2048, 5632, stored, 4096, 768)
+
+
+def test_waves_that_walk_many_tiles_of_keys():
+    """16 tiles of 64 keys and more a wave, by the longest sequence that a launch can have; of heads of up to 64 five."""
+    import ctypes
+    from ferrox_amd.csrc.build import load_library
+    rule = load_library("attention").fx_attn_wave_walks
+    rule.argtypes = [ctypes.c_long, ctypes.c_int, ctypes.c_int]
+    assert [rule(keys, waves, 128) for keys, waves in ((960, 1), (961, 1), (2560, 1), (2560, 2), (2560, 4), (4032, 4), (4033, 4))] == [0, 1, 1, 1, 0, 0, 1]
+    assert [rule(keys, waves, 64) for keys, waves in ((256, 1), (257, 1), (512, 2), (577, 2), (2560, 8), (2561, 8))] == [0, 1, 0, 1, 1, 1]

@@ -2117,3 +2117,35 @@ def test_float32_experts_from_parts_with_their_weights_in_whole_lines(K, shares,
             odd = got[0, 0].abs() > 1e30
             assert torch.equal(got[1, 1][odd], got[0, 0][odd])
             close(got[1, 1][~odd], got[0, 0][~odd], torch.float32, "float32 instruction")
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(16, 16, 64), (16, 16, 128), (28, 4, 128), (12, 12, 48), (8, 1, 256)])
+@pytest.mark.parametrize("S,longest", [(3, 1300), (72, 1300), (70, 150)])
+@pytest.mark.parametrize("window,keep,softcap", [(0, 0, 0.0), (300, 0, 0.0), (200, 70, 0.0), (0, 0, 20.0)])
+def test_single_queries_on_pages_that_hold_whole_tiles(nh, nkv, hd, S, longest, window, keep, softcap):
+    """Pages of 64 and 128 positions, where a tile of keys has one page, against pages of 16, where every key has its own: the same bits, in waves that walk
+    one tile and many.  What no query may see, the other positions of a sequence's pages, is not a number."""
+    from ferrox_amd import ops
+    lens = [max(1, longest - (53 * i) % longest) for i in range(S)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    width = -(-longest // 128) * 128
+    t = torch.arange(width, device=DEV)[None]
+    n = torch.tensor(lens, device=DEV)[:, None]
+    sees = (t < n) & ((t >= n - window) | (t < keep) if window else t >= 0)
+    k, v = rnd(S, width, nkv, hd, dtype=torch.bfloat16), rnd(S, width, nkv, hd, dtype=torch.bfloat16, seed=1)
+    k[~sees], v[~sees] = math.nan, math.nan
+    q = rnd(S, nh * hd, dtype=torch.bfloat16, seed=2)
+    got = []
+    for bs in (16, 64, 128):
+        per = width // bs
+        table = torch.randperm(S * per, generator=torch.Generator().manual_seed(bs)).to(DEV)
+        kp = torch.empty(S * per, nkv, bs, hd, dtype=torch.bfloat16, device=DEV)
+        vp = torch.empty(S * per, nkv, hd, bs, dtype=torch.bfloat16, device=DEV)
+        kp[table] = k.view(S * per, bs, nkv, hd).transpose(1, 2)
+        vp[table] = v.view(S * per, bs, nkv, hd).permute(0, 2, 3, 1)
+        out = torch.zeros(S, nh * hd, dtype=torch.bfloat16, device=DEV)
+        seqs = i32(list(range(S)))
+        ops.attention_decode(q, out, kp, vp, table.to(torch.int32).view(S, per), i32([m - 1 for m in lens]), seqs, seqs, nh, nkv, hd, bs, window, hd ** -0.5,
+                             max_kv_len=longest, keep_first=keep, softcap=softcap)
+        got.append(out)
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

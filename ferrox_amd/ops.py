@@ -714,7 +714,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
     if store_activation is not None and (epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None):
         raise KernelError("gemm: a stored activation goes with the plain stored product without bias")
     if then_add is not None and (then_add.dtype != torch.float32 or then_add.dim() != 2 or then_add.stride(1) != 1 or epilogue != EPI_RESID
-                                 or then_add.shape[0] < a.shape[0] or then_add.shape[1] < w.shape[0]):
+                                 or then_add.shape[0] < a.shape[0] or then_add.shape[1] < w.shape[0] or not then_add.is_cuda):
         raise KernelError("gemm: rows to be added behind the product are float32, as many as are added to")
     if row_ss is not None:
         ss = row_ss[0]
@@ -793,7 +793,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
           ACTIVATIONS[activation], STORED_ACTIVATIONS[store_activation] if gate_logits is None else _SACT_GATE,
           float(activation_params[0]), float(activation_params[1]), _p(pre_scale), _p(_i32(pre_scale_rows, "pre_scale_rows")),
           _p(gate_logits), gate_logits.stride(0) if gate_logits is not None else 0, int(gate_div), int(max_share),
-          _p(then_add), then_add.stride(0) if then_add is not None else 0, int(f32_instruction))
+          None if then_add is None else then_add.data_ptr(), 0 if then_add is None else then_add.stride(0), f32_instruction)
     return out
 
 

@@ -713,7 +713,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, *, epilogue: int = EPI_STORE, out: to
         raise KernelError(f"gemm: stored activation '{store_activation}' is not one of {sorted(k for k in STORED_ACTIVATIONS if k)}")
     if store_activation is not None and (epilogue not in (EPI_STORE, EPI_STORE_F32) or bias is not None):
         raise KernelError("gemm: a stored activation goes with the plain stored product without bias")
-    if then_add is not None and (then_add.dtype != torch.float32 or then_add.dim() != 2 or then_add.stride(1) != 1 or epilogue != EPI_RESID
+    if then_add is not None and (then_add.dtype != torch.float32 or then_add.dim() != 2 or w.dim() != 2 or then_add.stride(1) != 1 or epilogue != EPI_RESID
                                  or then_add.shape[0] < a.shape[0] or then_add.shape[1] < w.shape[0] or not then_add.is_cuda):
         raise KernelError("gemm: rows to be added behind the product are float32, as many as are added to")
     if row_ss is not None:

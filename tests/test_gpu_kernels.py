@@ -1943,6 +1943,12 @@ def test_pairs_of_few_row_products_have_the_bits_of_two_launches(M, N2, K2, epi2
         ops.gemm(x, w_out, epilogue=ops.EPI_RESID, out=both, row_scale=row_scale, then_add=ops.gemm(act, w_down, epilogue=ops.EPI_STORE_F32))
         assert torch.equal(both, h)
     down = ops.gemm(act, w_down, epilogue=ops.EPI_STORE_F32)
+    for bad in (dict(epilogue=ops.EPI_STORE_F32, then_add=down), dict(epilogue=ops.EPI_RESID, out=h, then_add=down[:, :2047]), dict(epilogue=ops.EPI_RESID, out=h, then_add=down.bfloat16()),
+                dict(epilogue=ops.EPI_RESID, out=h, then_add=down.cpu()), dict(epilogue=ops.EPI_RESID, out=h, then_add=down[:M - 1])):
+        with pytest.raises(ops.KernelError):
+            ops.gemm(x, w_out, **bad)
+    with pytest.raises(ops.KernelError):
+        ops.gemm(rnd(17, 2048, dtype=torch.bfloat16), w_out, epilogue=ops.EPI_RESID, out=rnd(17, 2048), then_add=rnd(17, 2048))
     plain2 = ops.gemm(y, w2, epilogue=epi2)
     for turn in (None, (positions, inv_freq, width, first_dim, n_dims, 1.25)) if epi2 == 0 else (None,):
         want = plain2.clone()
